@@ -158,8 +158,7 @@ struct vecsz_ctx {
     HostBuf vpin;
     // decompress scratch
     // dec_small: decoder summary, symbol and zero totals, list counts (kDecSmall*)
-    DevBuf tabs, sub_b, sub_e, sub_cnt, sub_zeros, sub_lj, sub_ls, sub_ln, sym_off, zero_off, scan_tmp, scan_tot,
-        dec_small, flagged, nflagged;
+    DevBuf tabs, sub_b, sub_e, sub_cz, sub_list, sub_ln, unit_off, scan_tmp, scan_tot, dec_small, flagged, nflagged;
     // host staging
     DevBuf stage_in, stage_out;
     HostBuf pin, pin2, pin_tab;
@@ -405,13 +404,19 @@ CScratch small_scratch(CScratch s, uint8_t* block, int dict) {
     return s;
 }
 
-// The small state of a single-field decompress in one block, so that each
-// host check is one copy: [decoder summary | symbol and zero totals | the
-// three re-decode list counts].
-constexpr size_t kDecSmallTotals = 64;
-constexpr size_t kDecSmallLists = 96;
-constexpr size_t kDecSmallBytes = 112;
-static_assert(sizeof(DecSummary) <= kDecSmallTotals, "decoder summary fits its slot");
+// The small state of a single-field decompress in one block: [decoder
+// summary | the re-decode list counters].
+constexpr size_t kDecSmallLists = 128;
+constexpr size_t kDecSmallBytes = kDecSmallLists + kListCountBytes;
+static_assert(sizeof(DecSummary) <= kDecSmallLists, "decoder summary fits its slot");
+
+// Whether the list pass `pass` reads holds entries (counters: the host's copy).
+bool any_listed(const uint8_t* counters, uint32_t pass) {
+    const uint32_t* n = reinterpret_cast<const uint32_t*>(counters) + list_slot(pass);
+    for (uint32_t i = 0; i < kMaxStripes; i++)
+        if (n[i * kCounterWords]) return true;
+    return false;
+}
 
 // ---- allocation-free compress (vecsz_compress_noalloc)
 //
@@ -1054,10 +1059,13 @@ int decompress_device(vecsz_ctx* c, const vecsz_params* p, const uint8_t* d_in, 
     } else {
         const uint64_t T = stream_bytes * 8;
         const uint64_t nsub = std::max<uint64_t>(1, (T + kSubBits - 1) / kSubBits);
-        if (!c->sub_b.ensure(nsub * 8) || !c->sub_e.ensure(nsub * 8) || !c->sub_cnt.ensure(nsub * 4) ||
-            !c->sub_zeros.ensure(nsub * 4) || !c->sub_lj.ensure(nsub * 8) || !c->sub_ls.ensure(nsub * 16) ||
-            !c->sym_off.ensure(nsub * 8) || !c->zero_off.ensure(nsub * 8) ||
-            !c->scan_tmp.ensure(((nsub + 4095) / 4096 + 1) * 16) || !c->dec_small.ensure(kDecSmallBytes))
+        const uint64_t nunits = decode_write_units(nsub);
+        SubState ss{};  // jbase 0: list entries are this field's subsequence numbers
+        list_stripes(decode_sync_units(nsub), &ss.nstripe, &ss.stripe_cap);
+        const uint64_t list_cap = ss.nstripe * ss.stripe_cap;
+        if (!c->sub_b.ensure(nsub) || !c->sub_e.ensure(nsub) || !c->sub_cz.ensure(nsub * 4) ||
+            !c->sub_list.ensure(list_cap * 16) || !c->unit_off.ensure((nunits + 1) * 16) ||
+            !c->dec_small.ensure(kDecSmallBytes))
             return fail(c, VECSZ_ENOMEM, "device scratch allocation failed");
         // Decode tables in one pinned staging copy: the compact form when the
         // symbols fit 12 bits (the kernels keep its deeper tables in LDS when
@@ -1087,22 +1095,18 @@ int decompress_device(vecsz_ctx* c, const vecsz_params* p, const uint8_t* d_in, 
         da.sub = t16 ? nullptr : c->tabs.as<uint32_t>() + dt.lut.size();
         da.lut16 = t16 ? c->tabs.as<uint16_t>() : nullptr;
         da.sub16 = t16 ? c->tabs.as<uint16_t>() + dt.lut16.size() : nullptr;
-        da.n_sub16 = t16 && dt.sub16.size() <= kMaxSub16 ? (uint32_t)dt.sub16.size() : 0;
+        da.n_sub16 = t16 ? (uint32_t)std::min<size_t>(dt.sub16.size(), kMaxSub16) : 0;
         da.nsub = nsub;
         da.outliers = d_outl;
         da.n_outlier = nout;
-        SubState ss{};  // jbase 0: list entries are this field's subsequence numbers
-        ss.b = c->sub_b.as<uint64_t>();
-        ss.e = c->sub_e.as<uint64_t>();
-        ss.cnt = c->sub_cnt.as<uint32_t>();
-        ss.zer = c->sub_zeros.as<uint32_t>();
-        ss.list_j[0] = c->sub_lj.as<uint32_t>();
-        ss.list_j[1] = c->sub_lj.as<uint32_t>() + nsub;
-        ss.list_start[0] = c->sub_ls.as<uint64_t>();
-        ss.list_start[1] = c->sub_ls.as<uint64_t>() + nsub;
+        ss.b = c->sub_b.as<uint8_t>();
+        ss.e = c->sub_e.as<uint8_t>();
+        ss.cz = c->sub_cz.as<uint32_t>();
+        ss.list[0] = c->sub_list.as<uint64_t>();
+        ss.list[1] = c->sub_list.as<uint64_t>() + list_cap;
         ss.list_n = reinterpret_cast<uint32_t*>(c->dec_small.as<uint8_t>() + kDecSmallLists);
         DecSummary* dsum = c->dec_small.as<DecSummary>();
-        uint64_t* stot = reinterpret_cast<uint64_t*>(c->dec_small.as<uint8_t>() + kDecSmallTotals);
+        uint64_t* off = c->unit_off.as<uint64_t>();
         if (d_index) {
             StageScope s(c, "decode_indexed");
             Recon1D r1{d_out, B, R, eb.twoeb, ra.halo, ra.halo_stride};
@@ -1114,44 +1118,46 @@ int decompress_device(vecsz_ctx* c, const vecsz_params* p, const uint8_t* d_in, 
             StageScope s(c, "decode_sync");
             launch_decode_sync(da, ss, dsum, c->stream);
         }
-        // Re-decode passes, two without a host check (most streams need one or
-        // none), then the scan and the write pass, which do nothing unless the
-        // list the third pass would read is empty: in the common case the
-        // decode needs one host check, after the write.  Otherwise passes run
+        // Re-decode passes, a few without a host check, then the scan and the
+        // write pass, which do nothing unless the list the next pass would
+        // read is empty: in the common case the decode needs one host check,
+        // after the write.  (The longest chain of wrong starts grows with
+        // their number: the 1 GiB field needs three or four passes, a 26 MB
+        // one two; a pass over empty lists takes about 4 us, a host check
+        // with its repeated launches about 35.)  Otherwise passes run
         // in growing batches between host checks while the lists ask for more
         // (each pass resolves at least the first subsequence of every chain,
         // so nsub passes suffice), and then the scan and the write again.
-        constexpr uint32_t kPassesAhead = 2;
+        const uint32_t ahead = nsub < (1u << 17) ? 2 : nsub < (1u << 21) ? 3 : 4;
         uint32_t pass = 0;
         {
             StageScope s(c, "decode_redo");
-            for (; pass < kPassesAhead; pass++) launch_decode_pass(da, ss, pass, dsum, c->stream);
+            for (; pass < ahead; pass++) launch_decode_pass(da, ss, pass, dsum, c->stream);
         }
         auto scan_write = [&](const uint32_t* guard) {
             {
                 StageScope s(c, "decode_scan");
-                launch_scan_u32x2(ss.cnt, ss.zer, nsub, c->sym_off.as<uint64_t>(), c->zero_off.as<uint64_t>(),
-                                  c->scan_tmp.as<uint64_t>(), stot, c->stream, guard);
+                launch_decode_offsets(ss, nsub, off, c->stream, guard);
             }
             StageScope s(c, "decode_write");
-            launch_decode_write(da, ss, c->sym_off.as<uint64_t>(), c->zero_off.as<uint64_t>(), codes, sparse, dsum,
-                                c->stream, guard);
+            launch_decode_write(da, ss, off, codes, sparse, dsum, c->stream, guard);
         };
-        scan_write(ss.list_n + pass % 3);
+        scan_write(ss.list_n + list_slot(pass));
         // the reconstruction goes in behind the write pass, under the same
         // guard, before the host check: in the common case the check then
         // waits on the whole decompress
-        if (!fused_1d) reconstruct(ss.list_n + pass % 3);
+        if (!fused_1d) reconstruct(ss.list_n + list_slot(pass));
         HIPCHK(c, hipGetLastError());
         DecSummary ds;
-        uint64_t tot[2];
-        uint32_t left = 0;
-        auto check = [&]() -> int {  // summary, symbol totals and the pending list count
+        uint64_t tot;
+        bool left = false;
+        auto check = [&]() -> int {  // summary, the pending list count and the symbol total
             HIPCHK(c, hipMemcpyAsync(h, c->dec_small.p, kDecSmallBytes, hipMemcpyDeviceToHost, c->stream));
+            HIPCHK(c, hipMemcpyAsync(h + kDecSmallBytes, off + 2 * nunits, 8, hipMemcpyDeviceToHost, c->stream));
             HIPCHK(c, hipStreamSynchronize(c->stream));
             memcpy(&ds, h, sizeof(ds));
-            memcpy(tot, h + kDecSmallTotals, 16);
-            memcpy(&left, h + kDecSmallLists + 4 * (pass % 3), 4);
+            memcpy(&tot, h + kDecSmallBytes, 8);
+            left = any_listed(h + kDecSmallLists, pass);
             return ds.error ? fail(c, VECSZ_ECORRUPT, "bitstream does not decode") : VECSZ_OK;
         };
         if (int rc2 = check()) return rc2;
@@ -1170,7 +1176,7 @@ int decompress_device(vecsz_ctx* c, const vecsz_params* p, const uint8_t* d_in, 
             HIPCHK(c, hipGetLastError());
             if (int rc2 = check()) return rc2;
         }
-        if (tot[0] < n) return fail(c, VECSZ_ECORRUPT, "bitstream holds fewer symbols than the field");
+        if (tot < n) return fail(c, VECSZ_ECORRUPT, "bitstream holds fewer symbols than the field");
         }
     }
 
@@ -2007,7 +2013,7 @@ static int decompress_batch_fused_run(vecsz_ctx* c, int nf, const vecsz_params* 
         if (status[k] || c->db_dt[k].root_leaf) continue;
         const DecodeTables& dt = c->db_dt[k];
         if (dt.lut16.empty()) t16 = false;
-        if (dt.sub16.size() <= kMaxSub16) max_sub16 = std::max<uint32_t>(max_sub16, (uint32_t)dt.sub16.size());
+        max_sub16 = std::max<uint32_t>(max_sub16, (uint32_t)std::min<size_t>(dt.sub16.size(), kMaxSub16));
     }
     max_sub16 = batch_sub16_in_lds(max_sub16);
     std::vector<uint64_t> off(nf, 0), toff(nf, 0), fl_off(nf, 0);
@@ -2046,7 +2052,7 @@ static int decompress_batch_fused_run(vecsz_ctx* c, int nf, const vecsz_params* 
             toff[k] = tab_tot;
             tab_tot += t16 ? ((dt.lut16.size() + dt.sub16.size()) * 2 + 15) / 16 * 16
                            : ((dt.lut.size() + dt.sub.size()) * 4 + 15) / 16 * 16;
-            F.s.jbase = (uint32_t)sb[k];
+            F.s.jbase = sb[k];
             su[k + 1] = su[k] + decode_sync_units(F.a.nsub);
             wu[k + 1] = wu[k] + decode_write_units(F.a.nsub);
             sb[k + 1] = sb[k] + F.a.nsub;
@@ -2076,32 +2082,30 @@ static int decompress_batch_fused_run(vecsz_ctx* c, int nf, const vecsz_params* 
         F.out = d_out[k];
     }
     nsub_tot = sb[nf];
-    if (nsub_tot > 0xFFFFFFF0ull) return fail(c, VECSZ_EINVAL, "batch too large");  // u32 list entries
+    if (nsub_tot > 0xFFFFFFF0ull) return fail(c, VECSZ_EINVAL, "batch too large");  // u32 list counts
     const size_t st_bytes = st.size() * 8, fd_bytes = (size_t)nf * sizeof(DecField);
     const uint64_t nsub_alloc = std::max<uint64_t>(nsub_tot, 1);
+    SubState S{};
+    list_stripes(std::max<uint64_t>(su[nf], 1), &S.nstripe, &S.stripe_cap);
+    const uint64_t list_cap = S.nstripe * S.stripe_cap;
     if (!c->codes.ensure(ntot * 2 + 64) || !c->sparse.ensure(ntot * 4 + 64) || !c->tabs.ensure(tab_tot + 64) ||
-        !c->sub_b.ensure(nsub_alloc * 8) || !c->sub_e.ensure(nsub_alloc * 8) || !c->sub_cnt.ensure(nsub_alloc * 4) ||
-        !c->sub_zeros.ensure(nsub_alloc * 4) || !c->sub_lj.ensure(nsub_alloc * 8) ||
-        !c->sub_ls.ensure(nsub_alloc * 16) || !c->sub_ln.ensure(16) || !c->sym_off.ensure(nsub_alloc * 8) ||
-        !c->zero_off.ensure(nsub_alloc * 8) || !c->scan_tmp.ensure(((nsub_alloc + 4095) / 4096 + 1) * 16) ||
-        !c->scan_tot.ensure(16) || !c->flagged.ensure(fl_tot * 4 + 64) || !c->db_nfl.ensure((size_t)nf * 4) ||
+        !c->sub_b.ensure(nsub_alloc) || !c->sub_e.ensure(nsub_alloc) || !c->sub_cz.ensure(nsub_alloc * 4) ||
+        !c->sub_list.ensure(list_cap * 16) || !c->sub_ln.ensure(kListCountBytes) || !c->unit_off.ensure((wu[nf] + 1) * 16) ||
+        !c->flagged.ensure(fl_tot * 4 + 64) || !c->db_nfl.ensure((size_t)nf * 4) ||
         !c->db_sums.ensure((size_t)nf * sizeof(DecSummary)) || !c->db_tot.ensure((size_t)nf * 8) ||
         !c->db_desc.ensure(fd_bytes) || !c->db_start.ensure(st_bytes))
         return fail(c, VECSZ_ENOMEM, "device scratch allocation failed");
     if (!c->db_pin.ensure(fd_bytes + st_bytes + tab_tot + 64) ||
-        !c->db_back.ensure((size_t)nf * (sizeof(DecSummary) + 8) + 64))
+        !c->db_back.ensure((size_t)nf * (sizeof(DecSummary) + 8) + kListCountBytes))
         return fail(c, VECSZ_ENOMEM, "pinned buffer");
-    SubState S{};
-    S.b = c->sub_b.as<uint64_t>();
-    S.e = c->sub_e.as<uint64_t>();
-    S.cnt = c->sub_cnt.as<uint32_t>();
-    S.zer = c->sub_zeros.as<uint32_t>();
-    S.list_j[0] = c->sub_lj.as<uint32_t>();
-    S.list_j[1] = c->sub_lj.as<uint32_t>() + nsub_alloc;
-    S.list_start[0] = c->sub_ls.as<uint64_t>();
-    S.list_start[1] = c->sub_ls.as<uint64_t>() + nsub_alloc;
+    S.b = c->sub_b.as<uint8_t>();
+    S.e = c->sub_e.as<uint8_t>();
+    S.cz = c->sub_cz.as<uint32_t>();
+    S.list[0] = c->sub_list.as<uint64_t>();
+    S.list[1] = c->sub_list.as<uint64_t>() + list_cap;
     S.list_n = c->sub_ln.as<uint32_t>();
     S.jbase = 0;
+    uint64_t* uoff = c->unit_off.as<uint64_t>();
     uint8_t* tab_h = c->db_pin.as<uint8_t>() + fd_bytes + st_bytes;
     for (int k = 0; k < nf; k++) {
         DecField& F = fd[k];
@@ -2115,15 +2119,11 @@ static int decompress_batch_fused_run(vecsz_ctx* c, int nf, const vecsz_params* 
         const uint64_t s0 = sb[k];
         F.s.b = S.b + s0;
         F.s.e = S.e + s0;
-        F.s.cnt = S.cnt + s0;
-        F.s.zer = S.zer + s0;
-        for (int q = 0; q < 2; q++) {
-            F.s.list_j[q] = S.list_j[q];
-            F.s.list_start[q] = S.list_start[q];
-        }
+        F.s.cz = S.cz + s0;
+        for (int q = 0; q < 2; q++) F.s.list[q] = S.list[q];
         F.s.list_n = S.list_n;
-        F.sym_off = c->sym_off.as<uint64_t>() + s0;
-        F.zero_off = c->zero_off.as<uint64_t>() + s0;
+        F.s.nstripe = S.nstripe;
+        F.s.stripe_cap = S.stripe_cap;
         if (dt.root_leaf) continue;
         uint8_t* tp = tab_h + toff[k];
         uint8_t* tdev = c->tabs.as<uint8_t>() + toff[k];
@@ -2132,7 +2132,7 @@ static int decompress_batch_fused_run(vecsz_ctx* c, int nf, const vecsz_params* 
             memcpy(tp + dt.lut16.size() * 2, dt.sub16.data(), dt.sub16.size() * 2);
             F.a.lut16 = reinterpret_cast<const uint16_t*>(tdev);
             F.a.sub16 = reinterpret_cast<const uint16_t*>(tdev) + dt.lut16.size();
-            F.a.n_sub16 = max_sub16 && dt.sub16.size() <= max_sub16 ? (uint32_t)dt.sub16.size() : 0;
+            F.a.n_sub16 = (uint32_t)std::min<size_t>(dt.sub16.size(), max_sub16);
         } else {
             memcpy(tp, dt.lut.data(), dt.lut.size() * 4);
             memcpy(tp + dt.lut.size() * 4, dt.sub.data(), dt.sub.size() * 4);
@@ -2154,7 +2154,7 @@ static int decompress_batch_fused_run(vecsz_ctx* c, int nf, const vecsz_params* 
     if (tab_tot) HIPCHK(c, hipMemcpyAsync(c->tabs.p, tab_h, tab_tot, hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipMemsetAsync(c->db_sums.p, 0, (size_t)nf * sizeof(DecSummary), c->stream));
     HIPCHK(c, hipMemsetAsync(c->db_nfl.p, 0, (size_t)nf * 4, c->stream));
-    HIPCHK(c, hipMemsetAsync(c->sub_ln.p, 0, 16, c->stream));
+    HIPCHK(c, hipMemsetAsync(c->sub_ln.p, 0, kListCountBytes, c->stream));
 
     // 4. decode: one-symbol trees by a fill; the others by the batch passes
     {
@@ -2168,7 +2168,7 @@ static int decompress_batch_fused_run(vecsz_ctx* c, int nf, const vecsz_params* 
     }
     DecSummary* sums_h = c->db_back.as<DecSummary>();
     uint64_t* tot_h = reinterpret_cast<uint64_t*>(c->db_back.as<uint8_t>() + (size_t)nf * sizeof(DecSummary));
-    uint32_t* left_h = reinterpret_cast<uint32_t*>(tot_h + nf);
+    uint8_t* left_h = reinterpret_cast<uint8_t*>(tot_h + nf);
     uint64_t max_nsub = 0;
     for (int k = 0; k < nf; k++) max_nsub = std::max<uint64_t>(max_nsub, fd[k].a.nsub);
     if (nsub_tot) {
@@ -2176,17 +2176,17 @@ static int decompress_batch_fused_run(vecsz_ctx* c, int nf, const vecsz_params* 
         uint32_t pass = 0;
         {
             StageScope s(c, "decode_redo");
-            for (; pass < kPassesAhead; pass++) launch_decode_pass_multi(t16, fdd, sb_d, nf, S, pass, nsub_tot, c->stream);
+            for (; pass < kPassesAhead; pass++) launch_decode_pass_multi(t16, fdd, sb_d, nf, S, pass, c->stream);
         }
         HIPCHK(c, hipGetLastError());
         uint32_t batch = 2;
         for (;;) {
-            HIPCHK(c, hipMemcpyAsync(left_h, S.list_n + pass % 3, 4, hipMemcpyDeviceToHost, c->stream));
+            HIPCHK(c, hipMemcpyAsync(left_h, S.list_n, kListCountBytes, hipMemcpyDeviceToHost, c->stream));
             HIPCHK(c, hipStreamSynchronize(c->stream));
-            if (*left_h == 0) break;
+            if (!any_listed(left_h, pass)) break;
             if (pass > max_nsub + 2) return fail(c, VECSZ_ECORRUPT, "subsequence boundaries do not converge");
             StageScope s(c, "decode_redo");
-            for (uint32_t b = 0; b < batch; b++) launch_decode_pass_multi(t16, fdd, sb_d, nf, S, pass++, nsub_tot, c->stream);
+            for (uint32_t b = 0; b < batch; b++) launch_decode_pass_multi(t16, fdd, sb_d, nf, S, pass++, c->stream);
             batch = std::min<uint32_t>(2 * batch, 16);
         }
         // fields whose stream does not decode are left out of the write pass
@@ -2215,14 +2215,13 @@ static int decompress_batch_fused_run(vecsz_ctx* c, int nf, const vecsz_params* 
         }
         {
             StageScope s(c, "decode_scan");
-            launch_scan_u32x2(S.cnt, S.zer, nsub_tot, c->sym_off.as<uint64_t>(), c->zero_off.as<uint64_t>(),
-                              c->scan_tmp.as<uint64_t>(), c->scan_tot.as<uint64_t>(), c->stream);
+            launch_decode_offsets_multi(fdd, wu_d, nf, wu[nf], uoff, c->stream);
         }
         {
             StageScope s(c, "decode_write");
-            launch_decode_write_multi(t16, max_sub16, fdd, wu_d, nf, wu[nf], c->stream);
+            launch_decode_write_multi(t16, max_sub16, fdd, wu_d, nf, wu[nf], uoff, c->stream);
         }
-        launch_dec_field_totals(fdd, nf, c->db_tot.as<uint64_t>(), c->stream);
+        launch_dec_field_totals(wu_d, nf, uoff, c->db_tot.as<uint64_t>(), c->stream);
         HIPCHK(c, hipGetLastError());
     }
     {
@@ -2433,10 +2432,12 @@ int vecsz_decompress_batch(vecsz_ctx* c, int nfields, const vecsz_params* p, con
     auto prep = [&](vecsz_ctx* w) {
         (void)hipSetDevice(w->device);
         const uint64_t nsub = bmax * 8 / kSubBits + 2;
-        return w->codes.ensure(nmax * 2 + 64) && w->sparse.ensure(nmax * 4 + 64) && w->sub_b.ensure(nsub * 8) &&
-               w->sub_e.ensure(nsub * 8) && w->sub_cnt.ensure(nsub * 4) && w->sub_zeros.ensure(nsub * 4) &&
-               w->sub_lj.ensure(nsub * 8) && w->sub_ls.ensure(nsub * 16) && w->sub_ln.ensure(16) &&
-               w->sym_off.ensure(nsub * 8) && w->zero_off.ensure(nsub * 8);
+        uint32_t nstripe;
+        uint64_t cap;
+        list_stripes(decode_sync_units(nsub), &nstripe, &cap);
+        return w->codes.ensure(nmax * 2 + 64) && w->sparse.ensure(nmax * 4 + 64) && w->sub_b.ensure(nsub) &&
+               w->sub_e.ensure(nsub) && w->sub_cz.ensure(nsub * 4) && w->sub_list.ensure(nstripe * cap * 16) &&
+               w->unit_off.ensure((decode_write_units(nsub) + 1) * 16);
     };
     return run_batch(c, nfields, weight.data(), status, prep, [&](vecsz_ctx* w, int k) {
         if (!d_in[k] || !d_out[k]) return fail(w, VECSZ_EINVAL, "NULL field");
@@ -2463,7 +2464,7 @@ uint64_t request_bytes(int kind, const vecsz_params* p, uint64_t in_bytes, uint6
         return 4 * n + out_cap + 6 * n + 24 * nch + (uint64_t)768 * p->dict_size * 4 + (1 << 20);
     }
     const uint64_t nsub = in_bytes * 8 / kSubBits + 2;
-    return in_bytes + 4 * out_cap + 6 * out_cap + 50 * nsub + (1 << 20);
+    return in_bytes + 4 * out_cap + 6 * out_cap + 24 * nsub + (1 << 20);
 }
 
 struct Request {

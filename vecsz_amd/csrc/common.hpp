@@ -12,9 +12,7 @@ constexpr int kChunk = 1024;       // symbols per encode chunk (one wavefront)
 constexpr int kSymPerThread = kChunk / kWave;  // 16 consecutive symbols per lane
 constexpr int kLutBits = 12;       // first-level decode table width
 constexpr int kSubTabBits = 4;     // width of each deeper decode table
-constexpr int kSubBits = 1024;     // bits per decode subsequence
-constexpr int kCkptBits = 128;     // decoder checkpoint window
-constexpr int kCkpts = kSubBits / kCkptBits;
+constexpr int kSubBits = 512;      // bits per decode subsequence
 
 // Error-bound family computed on the device from the value range
 // (ChangeToRelativeMode + InitializeErrorBoundFamily, src/types.cc:49-60,
@@ -138,6 +136,31 @@ __device__ __forceinline__ void mem_sync() {
     __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
     __syncthreads();
 }
+
+// DPP move (GFX9 encodings): lanes without a source, or in rows outside
+// ROWS, read 0.  Every lane of the wavefront must be active.
+template <int CTRL, int ROWS = 0xF>
+__device__ __forceinline__ uint32_t dpp_move(uint32_t v) {
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xF, false);
+}
+
+// Inclusive scan of 32-bit values over the wavefront in six DPP steps and no
+// LDS traffic: row_shr 1, 2, 4, 8 scan each row of 16 lanes, row_bcast:15
+// adds row 0's total to row 1 and row 2's to row 3, row_bcast:31 adds the
+// total of rows 0-1 to rows 2-3.  OR = true gives the OR-scan.
+template <bool OR = false>
+__device__ __forceinline__ uint32_t wave_scan_dpp(uint32_t v) {
+    auto op = [](uint32_t a, uint32_t b) { return OR ? (a | b) : (a + b); };
+    v = op(v, dpp_move<0x111>(v));
+    v = op(v, dpp_move<0x112>(v));
+    v = op(v, dpp_move<0x114>(v));
+    v = op(v, dpp_move<0x118>(v));
+    v = op(v, dpp_move<0x142, 0xA>(v));
+    v = op(v, dpp_move<0x143, 0xC>(v));
+    return v;
+}
+
+__device__ __forceinline__ uint32_t lane63(uint32_t v) { return (uint32_t)__builtin_amdgcn_readlane((int)v, 63); }
 
 // Field of work unit u in a batch: the f with start[f] <= u < start[f + 1]
 // (start is nondecreasing, start[0] = 0, start[nf] = total units > u).

@@ -113,31 +113,49 @@ struct DecodeArgs {
 };
 
 struct SubState {
-    uint64_t* b;      // true start bit of each subsequence (first codeword start >= j * kSubBits)
-    uint64_t* e;      // its end: first codeword start >= (j + 1) * kSubBits
-    uint32_t* cnt;    // codewords starting in [b, e)
-    uint32_t* zer;    // of which decode to symbol 0
+    // Of subsequence j (its target: bit (j + 1) * kSubBits, or the stream's
+    // end): how far past bit j * kSubBits its first codeword starts, and how
+    // far past its target the one after its last (both below 64, a codeword's
+    // length); codewords starting in between | those of them that decode to
+    // symbol 0 << 16 (at most kSubBits each).
+    uint8_t* b;
+    uint8_t* e;
+    uint32_t* cz;
     // Re-decode lists, used in alternation by successive passes: subsequence
-    // list_j[.][k] to re-decode from bit list_start[.][k] (nsub entries each),
-    // and entry counts in a ring of three (pass p reads list_n[p % 3]).
-    uint32_t* list_j[2];
-    uint64_t* list_start[2];
+    // jbase + j | its start (as b) << 48.  A list is nstripe stripes of
+    // stripe_cap entries, each with a counter of its own (list_count): a
+    // counter that every wavefront adds to is a queue at one cache line, at
+    // about 10 ns an addition.
+    uint64_t* list[2];
     uint32_t* list_n;
-    // List entries hold jbase + j: 0 for one field; in a batch the arrays
-    // above are views of one field's part of batch-wide arrays, and jbase is
-    // the batch-wide number of its subsequence 0 (the lists are batch-wide).
-    uint32_t jbase = 0;
+    uint32_t nstripe;
+    uint64_t stripe_cap;
+    // 0 for one field; in a batch b, e and cz are views of one field's part
+    // of batch-wide arrays, and jbase is the batch-wide number of its
+    // subsequence 0 (the lists are batch-wide).
+    uint64_t jbase = 0;
 };
 
+// Counters of a ring of three lists (pass p reads slot p % 3), each on a
+// cache line of its own.
+constexpr uint32_t kMaxStripes = 32;
+constexpr uint32_t kCounterWords = 32;
+constexpr size_t kListCountBytes = (size_t)3 * kMaxStripes * kCounterWords * 4;
+__host__ __device__ inline uint32_t list_slot(uint32_t pass) { return pass % 3 * kMaxStripes * kCounterWords; }
+// Stripes of the lists for `units` sync workgroups, and their entries.
+void list_stripes(uint64_t units, uint32_t* nstripe, uint64_t* cap);
 void launch_decode_sync(const DecodeArgs& a, SubState s, DecSummary* sum, hipStream_t st);
 // Re-decode pass `pass` over the list the previous pass (or the sync pass) built.
 void launch_decode_pass(const DecodeArgs& a, SubState s, uint32_t pass, DecSummary* sum, hipStream_t st);
-// guard (nullable): every kernel of the scan does nothing while *guard is nonzero.
 void launch_scan_u32x2(const uint32_t* a, const uint32_t* b, uint64_t n, uint64_t* oa, uint64_t* ob, uint64_t* block_tmp,
-                       uint64_t* totals, hipStream_t st, const uint32_t* guard = nullptr);
-void launch_decode_write(const DecodeArgs& a, SubState s, const uint64_t* sym_off, const uint64_t* zero_off,
-                         uint16_t* codes, float* sparse, DecSummary* sum, hipStream_t st,
-                         const uint32_t* guard = nullptr);
+                       uint64_t* totals, hipStream_t st);
+// Codewords and zeros before each write unit (decode_write_units(nsub) units
+// of consecutive subsequences): off[2 u], off[2 u + 1], the totals behind the
+// last.  guard (nullable): nothing runs while any of the kMaxStripes counters
+// from there on (a list_slot) is nonzero.
+void launch_decode_offsets(const SubState& s, uint64_t nsub, uint64_t* off, hipStream_t st, const uint32_t* guard = nullptr);
+void launch_decode_write(const DecodeArgs& a, SubState s, const uint64_t* off, uint16_t* codes, float* sparse,
+                         DecSummary* sum, hipStream_t st, const uint32_t* guard = nullptr);
 void launch_fill_u16(uint16_t* p, uint64_t n, uint16_t v, hipStream_t st);
 // Decode with a decode index (index = its kIdxHead header words first): codes
 // and outliers as k_decode_write leaves them.
@@ -164,7 +182,7 @@ struct ReconArgs {
     uint64_t ntiles_x, ntiles_y, ntiles_z;
     const float* halo;  // as DQArgs::halo; nullptr = the +0.0 halo
     uint64_t halo_stride, hb0, hb1;
-    const uint32_t* guard = nullptr;  // nonzero *guard: the launch does nothing
+    const uint32_t* guard = nullptr;  // as launch_decode_offsets
 };
 void launch_reconstruct(int ndim, int B, const uint16_t* codes, const float* sparse, float* out, const ReconArgs& a,
                         uint32_t* flagged, uint32_t* nflagged, int grid, hipStream_t st);
@@ -172,9 +190,8 @@ void launch_reconstruct_fallback(int ndim, int B, const uint16_t* codes, const f
                                  const ReconArgs& a, const uint32_t* flagged, const uint32_t* nflagged, hipStream_t st);
 
 // Batched decompress: one field as the batch kernels see it.  The
-// subsequence state, the code-count prefixes and the re-decode lists are
-// batch-wide arrays (a field's subsequences are numbered from sub0); s,
-// sym_off and zero_off are views of its part.
+// subsequence state and the re-decode lists are batch-wide arrays; s holds
+// views of the field's part.
 // 64 x per wavefront (kRcN), four x per lane with vector (kRcNx4) or element
 // (kRcNx4u) loads and stores.
 enum ReconKind { kRc1 = 0, kRc1x4, kRc2, kRc2x4, kRc3, kRc3x4, kRc1x4u, kRc2x4u, kRc3x4u, kRcKinds };
@@ -183,8 +200,6 @@ int recon_kind_ndim(int kind);
 struct DecField {
     DecodeArgs a;              // nsub = 0: nothing to decode on the device
     SubState s;
-    const uint64_t* sym_off;
-    const uint64_t* zero_off;
     uint16_t* codes;
     float* sparse;
     float* out;
@@ -204,13 +219,17 @@ uint32_t batch_sub16_in_lds(uint32_t max_sub16);
 void launch_decode_sync_multi(bool t16, uint32_t max_sub16, const DecField* fd, const uint64_t* start, int nf,
                               uint64_t nunits, hipStream_t st);
 // sub_start: batch-wide number of each field's subsequence 0 (nf + 1 entries);
-// S: the batch-wide lists (list_j, list_start, list_n).
+// S: the batch-wide lists (list, list_n).
 void launch_decode_pass_multi(bool t16, const DecField* fd, const uint64_t* sub_start, int nf, SubState S,
-                              uint32_t pass, uint64_t nsub_tot, hipStream_t st);
+                              uint32_t pass, hipStream_t st);
+// start: per-field write unit starts (nf + 1), nunits = start[nf]; off as
+// launch_decode_offsets, over the units of every field.
+void launch_decode_offsets_multi(const DecField* fd, const uint64_t* start, int nf, uint64_t nunits, uint64_t* off,
+                                 hipStream_t st);
 void launch_decode_write_multi(bool t16, uint32_t max_sub16, const DecField* fd, const uint64_t* start, int nf,
-                               uint64_t nunits, hipStream_t st);
+                               uint64_t nunits, const uint64_t* off, hipStream_t st);
 // Symbols each field's subsequences hold (tot[f]).
-void launch_dec_field_totals(const DecField* fd, int nf, uint64_t* tot, hipStream_t st);
+void launch_dec_field_totals(const uint64_t* start, int nf, const uint64_t* off, uint64_t* tot, hipStream_t st);
 // One reconstruction form over its fields' tiles (start: per-field tile starts).
 void launch_reconstruct_multi(int kind, int B, const DecField* fd, const uint64_t* start, int nf, uint64_t ntiles,
                               hipStream_t st);

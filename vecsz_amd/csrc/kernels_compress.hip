@@ -854,31 +854,6 @@ __device__ __forceinline__ T wave_incl_scan(T v) {
     return v;
 }
 
-// DPP move (GFX9 encodings): lanes without a source, or in rows outside
-// ROWS, read 0.  Every lane of the wavefront must be active.
-template <int CTRL, int ROWS = 0xF>
-__device__ __forceinline__ uint32_t dpp_move(uint32_t v) {
-    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROWS, 0xF, false);
-}
-
-// Inclusive scan of 32-bit values over the wavefront in six DPP steps and no
-// LDS traffic: row_shr 1, 2, 4, 8 scan each row of 16 lanes, row_bcast:15
-// adds row 0's total to row 1 and row 2's to row 3, row_bcast:31 adds the
-// total of rows 0-1 to rows 2-3.  OR = true gives the OR-scan.
-template <bool OR = false>
-__device__ __forceinline__ uint32_t wave_scan_dpp(uint32_t v) {
-    auto op = [](uint32_t a, uint32_t b) { return OR ? (a | b) : (a + b); };
-    v = op(v, dpp_move<0x111>(v));
-    v = op(v, dpp_move<0x112>(v));
-    v = op(v, dpp_move<0x114>(v));
-    v = op(v, dpp_move<0x118>(v));
-    v = op(v, dpp_move<0x142, 0xA>(v));
-    v = op(v, dpp_move<0x143, 0xC>(v));
-    return v;
-}
-
-__device__ __forceinline__ uint32_t lane63(uint32_t v) { return (uint32_t)__builtin_amdgcn_readlane((int)v, 63); }
-
 // Exclusive scan across a 256-thread workgroup; returns the thread's prefix and
 // the workgroup total through *total.
 template <typename T>

@@ -3,19 +3,17 @@
 //   Huffman decode (decode_withTree/decode, src/huffman.hh:343-372, :679-691)
 //   as a chunk-parallel, self-synchronising decode of the archive's single
 //   MSB-first bitstream, cut into subsequences of kSubBits bits:
-//     k_decode_sync   a workgroup stages 256 subsequences in LDS; each thread
-//                     decodes its own from the assumed start j*kSubBits and
-//                     records checkpoints (first codeword start in every
-//                     kCkptBits window, with the symbol and zero counts before
-//                     it); then it continues from its own end into the next
-//                     subsequence until a codeword start meets a checkpoint,
-//                     after which both decodes agree, and writes the next
-//                     subsequence's true start, end and counts
-//                     (after kContBits bits without a meeting point it
-//                     gives up and lists the subsequence)
-//     k_decode_pass   listed subsequences re-decode in full from their true
-//                     starts, from LDS-staged rows; a moved end lists the
-//                     successor for the next pass, until no list is left
+//     k_decode_sync   each thread finds a subsequence's first codeword by
+//                     decoding from kLeadBits before it (two decodes of one
+//                     stream soon agree, wherever they started), then
+//                     decodes the subsequence: start, end and counts.  A
+//                     start other than the end its predecessor found lists
+//                     the subsequence
+//     k_decode_pass   listed subsequences re-decode from their predecessor's
+//                     end; a moved end lists the successor for the next
+//                     pass, until no list is left
+//     k_decode_sums,  codeword and zero counts per write unit, and their
+//     k_decode_scan   prefixes
 //     k_decode_write  final decode from the true starts: quant codes in
 //                     16-byte stores + outlier scatter
 //                     (src/vecsz_interface.hh:313-317)
@@ -34,13 +32,27 @@ namespace vsz {
 
 __device__ __forceinline__ uint32_t lane_id2() { return __lane_id(); }
 
+// Pointers with their address space in the type: a pointer that may be either
+// LDS or global (or that was loaded from memory) is read by FLAT loads, which
+// wait for every global access the wavefront has in flight, its own stores
+// among them.
+#define VSZ_LDS __attribute__((address_space(3)))
+#define VSZ_GLOBAL __attribute__((address_space(1)))
+typedef uint32_t U32x4 __attribute__((ext_vector_type(4)));
+typedef uint16_t U16x2 __attribute__((ext_vector_type(2)));
+using LdsU16 = const VSZ_LDS uint16_t*;
+using GlobalU8 = const VSZ_GLOBAL uint8_t*;
+using GlobalU16 = const VSZ_GLOBAL uint16_t*;
+using GlobalU32 = const VSZ_GLOBAL uint32_t*;
+using GlobalU32x4 = const VSZ_GLOBAL U32x4*;
+
 // The bitstream in "aligned space": word w is the big-endian u32 at byte 4w
 // of the 16-byte aligned address at or before the stream start; stream bit p
 // is aligned-space bit p + shift0.  Bytes before the stream belong to the
 // archive header; bytes at or past the stream end are never read and count
 // as zero.
 struct StreamView {
-    const uint8_t* base;
+    GlobalU8 base;
     uint32_t shift0;
     uint64_t nbytes;  // readable bytes from base (through the stream end)
 
@@ -48,36 +60,39 @@ struct StreamView {
         // pointer arithmetic (not an integer round trip) keeps the global
         // address space visible to the compiler: global_load, not flat_load
         const uint32_t mis = (uint32_t)(reinterpret_cast<uintptr_t>(stream) & 15);
-        base = stream - mis;
+        base = (GlobalU8)(stream - mis);
         shift0 = 8 * mis;
         nbytes = mis + stream_bits / 8;
     }
     __device__ __forceinline__ uint32_t word(uint64_t w) const {
         const uint64_t b = 4 * w;
-        if (b + 4 <= nbytes) return __builtin_bswap32(reinterpret_cast<const uint32_t*>(base)[w]);
+        if (b + 4 <= nbytes) return __builtin_bswap32(((GlobalU32)base)[w]);
         uint32_t v = 0;
         for (int i = 0; i < 4; i++) v = (v << 8) | (b + i < nbytes ? base[b + i] : 0u);
         return v;
     }
 };
 
-// Staged words are stored in rows of 33: the 32 words of one 1024-bit
-// subsequence followed by a copy of the next row's first word.  Threads of a
-// wavefront, each at its own subsequence, then read different LDS banks, and
-// any two consecutive words sit side by side (one ds_read2).
-__device__ __forceinline__ uint32_t pad_idx(uint32_t w) { return w + (w >> 5); }
+// Staged words are stored in rows of 17: the 16 words of one subsequence
+// followed by a copy of the next row's first word.  Threads of a wavefront,
+// each at its own subsequence, then read different LDS banks, and any two
+// consecutive words sit side by side (one ds_read2).
+constexpr uint32_t kSubWords = kSubBits / 32;
+__device__ __forceinline__ uint32_t pad_idx(uint32_t w) { return w + w / kSubWords; }
 
 // 32-bit window whose MSB is bit `lp` of the staged words.
 __device__ __forceinline__ uint32_t win32(const uint32_t* st, uint32_t lp) {
     const uint32_t i0 = pad_idx(lp >> 5);
     return __builtin_elementwise_fshl(st[i0], st[i0 + 1], lp & 31);
 }
-struct PadWin {  // the rows-of-33 staging above
+struct PadWin {  // the rows staging above
     const uint32_t* st;
+    __device__ __forceinline__ uint32_t word(uint32_t w) const { return st[pad_idx(w)]; }
     __device__ __forceinline__ uint32_t operator()(uint32_t lp) const { return win32(st, lp); }
 };
 struct RowWin {  // plain consecutive words
     const uint32_t* row;
+    __device__ __forceinline__ uint32_t word(uint32_t w) const { return row[w]; }
     __device__ __forceinline__ uint32_t operator()(uint32_t lp) const {
         const uint32_t i0 = lp >> 5;
         return __builtin_elementwise_fshl(row[i0], row[i0 + 1], lp & 31);
@@ -94,355 +109,396 @@ struct GlobalWin {
     }
 };
 
-// One codeword at position p, 32-bit tables: first level in LDS, deeper
-// levels (codes longer than kLutBits) from the global sub-tables.  len = 0
-// marks an invalid path.
-template <typename Win, typename P>
-__device__ __forceinline__ uint32_t decode_sym(const Win& win, P p, const uint32_t* lut,
-                                               const uint32_t* __restrict__ sub, uint32_t& len) {
-    uint32_t e = lut[(uint32_t)(win(p) >> (64 - kLutBits))];
-    if (e & kLutSlow) {
-        P q = p + kLutBits;
-        for (int lv = 0; lv < 16 && (e & kLutSlow); lv++) {
-            e = sub[(e & 0x7FFFFFFFu) + (uint32_t)(win(q) >> (64 - kSubTabBits))];
-            q += kSubTabBits;
-        }
-    }
-    len = (e & kLutSlow) ? 0u : (e >> 16) & 0x7F;
-    return e & 0xFFFF;
+// Whether a list is not empty (every lane of the wavefront calls it).
+__device__ __forceinline__ bool listed(const uint32_t* guard) {
+    if (!guard) return false;
+    const uint32_t lane = lane_id2();
+    return __any(lane < kMaxStripes && ((GlobalU32)guard)[(lane % kMaxStripes) * kCounterWords] != 0);
 }
 
-// The same with the compact 16-bit tables, every level in LDS.
-template <typename Win, typename P>
-__device__ __forceinline__ uint32_t decode_sym16(const Win& win, P p, const uint16_t* lut, const uint16_t* sub,
-                                                 uint32_t& len) {
-    uint32_t e = lut[(uint32_t)(win(p) >> (64 - kLutBits))];
-    len = e >> 12;
-    if (len == 0) {
-        P q = p + kLutBits;
-        for (int lv = 0; lv < 16; lv++) {
-            e = sub[((e & 0xFFF) << kSubTabBits) + (uint32_t)(win(q) >> (64 - kSubTabBits))];
-            if (e >> 12) {
-                len = (uint32_t)(q - p) + (e >> 12);
-                break;
-            }
-            q += kSubTabBits;
-        }
-    }
-    return e & 0xFFF;
+// Appends to the list of slot `slot` the lanes with `on` (a subsequence and
+// its start), in stripe `stripe`: one counter addition per wavefront.
+__device__ __forceinline__ void list_append(const SubState& s, uint32_t pass, uint32_t stripe, bool on, uint64_t j,
+                                            uint32_t first) {
+    const uint64_t m = __ballot(on);
+    if (!m) return;
+    const uint32_t lane = lane_id2();
+    const int lead = __builtin_ctzll(m);
+    uint32_t k = 0;
+    if ((int)lane == lead) k = atomicAdd(&s.list_n[list_slot(pass) + stripe * kCounterWords], (uint32_t)__popcll(m));
+    k = (uint32_t)__builtin_amdgcn_readlane((int)k, lead);
+    if (on)
+        s.list[pass & 1][stripe * s.stripe_cap + k + __popcll(m & ((1ull << lane) - 1))] = (s.jbase + j) | ((uint64_t)first << 48);
 }
 
-// Decode tables as a kernel sees them; load() copies what lives in LDS to
-// the front of the dynamic LDS area and returns the words it used.
+// Decode tables as a kernel sees them.
+//   look(w)     first-level entry of the codeword at the top of w
+//   escape(e)   the codeword is longer than the first level (32-bit tables:
+//               or invalid): resolve() walks the deeper tables
+//   len, sym    of an entry (sym: bits above the symbol may be set for the
+//               packing helpers below)
+//   resolve     e, l <- entry and length of the codeword at lp whose first
+//               32 bits (at least 16 of them valid) are w; l = 0: invalid.
+//               win is read for the bits past those
 template <bool T16>
 struct Decoder;
 
 template <>
 struct Decoder<true> {
     const uint16_t* lut;
-    const uint16_t* sub;
-    __device__ __forceinline__ uint32_t load(uint32_t* lds, const DecodeArgs& a) {
-        uint16_t* l = reinterpret_cast<uint16_t*>(lds);
-        const uint32_t nl = 1u << kLutBits, ns = a.n_sub16;
-        for (uint32_t i = threadIdx.x; i < nl; i += blockDim.x) l[i] = a.lut16[i];
-        for (uint32_t i = threadIdx.x; i < ns; i += blockDim.x) l[nl + i] = a.sub16[i];
-        lut = l;
-        sub = ns ? l + nl : a.sub16;  // n_sub16 0: the deeper tables stay in global memory
-        return (nl + ns + 1) / 2;
+    LdsU16 sub_lds;  // the first n_lds entries of the deeper tables
+    GlobalU16 sub;   // all of them
+    uint32_t n_lds;
+    // The tables are in LDS at lds (TableCopy); returns the words they take.
+    __device__ __forceinline__ uint32_t attach(const uint32_t* lds, const DecodeArgs& a) {
+        lut = reinterpret_cast<const uint16_t*>(lds);
+        sub_lds = (LdsU16)(lut + (1u << kLutBits));
+        sub = (GlobalU16)a.sub16;
+        n_lds = a.n_sub16;
+        return ((1u << kLutBits) + n_lds) / 2;
     }
-    template <typename Win, typename P>
-    __device__ __forceinline__ uint32_t operator()(const Win& w, P p, uint32_t& len) const {
-        return decode_sym16(w, p, lut, sub, len);
-    }
-    // Decodes the codeword at staged bit lp; len = 0: invalid path.  The
-    // window covers codewords of up to 32 bits; longer ones re-read.
-    __device__ __forceinline__ uint32_t take_at(const uint32_t* st, uint32_t lp, uint32_t& len) const {
-        return take_w(PadWin{st}, lp, len);
+    __device__ __forceinline__ uint32_t look(uint32_t w) const { return lut[w >> (32 - kLutBits)]; }
+    static __device__ __forceinline__ bool escape(uint32_t e) { return e < 4096; }
+    static __device__ __forceinline__ uint32_t len(uint32_t e) { return e >> 12; }
+    static __device__ __forceinline__ uint32_t sym(uint32_t e) { return e & 0xFFF; }
+    // Two symbols as the halves of a word.
+    static __device__ __forceinline__ uint32_t pack(uint32_t a, uint32_t b) { return (a | (b << 16)) & 0x0FFF0FFFu; }
+    // Entry i of the deeper tables.  The empty asm makes a global read's wait
+    // part of its own branch: behind the join the wavefronts that read LDS
+    // alone would wait too, for all of their stores in flight.
+    __device__ __forceinline__ uint32_t deeper(uint32_t i) const {
+        uint32_t e;
+        if (i < n_lds) {
+            e = sub_lds[i];
+        } else {
+            e = sub[i];
+            asm volatile("" : "+v"(e));
+        }
+        return e;
     }
     template <typename W>
-    __device__ __forceinline__ uint32_t take_w(const W& win, uint32_t lp, uint32_t& len) const {
-        return take_v(win, win(lp), lp, len);
-    }
-    // w: the 32 bits from lp (the window is read again only past them)
-    template <typename W>
-    __device__ __forceinline__ uint32_t take_v(const W& win, uint32_t w, uint32_t lp, uint32_t& len) const {
-        uint32_t e = lut[w >> (32 - kLutBits)];
-        uint32_t l = e >> 12;
-        if (l == 0) {
-            uint32_t used = kLutBits;
-            for (int lv = 0; lv < 16; lv++) {
-                const uint32_t idx = used + kSubTabBits <= 32 ? (w << used) >> (32 - kSubTabBits)
-                                                              : win(lp + used) >> (32 - kSubTabBits);
-                e = sub[((e & 0xFFF) << kSubTabBits) + idx];
-                if (e >> 12) {
-                    l = used + (e >> 12);
-                    break;
-                }
-                used += kSubTabBits;
+    __device__ __forceinline__ void resolve(const W& win, uint32_t w, uint32_t lp, uint32_t& e, uint32_t& l) const {
+        e = deeper((e << kSubTabBits) | ((w << kLutBits) >> (32 - kSubTabBits)));
+        l = e >> 12;
+        if (l != 0) {
+            l += kLutBits;
+            return;
+        }
+        l = 1;  // (every walk of a full tree ends at a leaf)
+        uint32_t used = kLutBits + kSubTabBits;
+#pragma unroll 1
+        for (int lv = 1; lv < 16; lv++, used += kSubTabBits) {
+            e = deeper((e << kSubTabBits) | (win(lp + used) >> (32 - kSubTabBits)));
+            if (e >> 12) {
+                l = used + (e >> 12);
+                break;
             }
         }
-        len = l;
-        return e & 0xFFF;
     }
 };
 
 template <>
 struct Decoder<false> {
     const uint32_t* lut;
-    const uint32_t* sub;
-    __device__ __forceinline__ uint32_t load(uint32_t* lds, const DecodeArgs& a) {
-        const uint32_t nl = 1u << kLutBits;
-        for (uint32_t i = threadIdx.x; i < nl; i += blockDim.x) lds[i] = a.lut[i];
+    GlobalU32 sub;
+    __device__ __forceinline__ uint32_t attach(const uint32_t* lds, const DecodeArgs& a) {
         lut = lds;
-        sub = a.sub;
-        return nl;
+        sub = (GlobalU32)a.sub;
+        return 1u << kLutBits;
     }
-    template <typename Win, typename P>
-    __device__ __forceinline__ uint32_t operator()(const Win& w, P p, uint32_t& len) const {
-        return decode_sym(w, p, lut, sub, len);
-    }
-    __device__ __forceinline__ uint32_t take_at(const uint32_t* st, uint32_t lp, uint32_t& len) const {
-        return take_w(PadWin{st}, lp, len);
-    }
+    __device__ __forceinline__ uint32_t look(uint32_t w) const { return lut[w >> (32 - kLutBits)]; }
+    static __device__ __forceinline__ bool escape(uint32_t e) { return (int32_t)e <= 0; }
+    static __device__ __forceinline__ uint32_t len(uint32_t e) { return e >> 16; }
+    static __device__ __forceinline__ uint32_t sym(uint32_t e) { return e & 0xFFFF; }
+    static __device__ __forceinline__ uint32_t pack(uint32_t a, uint32_t b) { return (a & 0xFFFF) | (b << 16); }
     template <typename W>
-    __device__ __forceinline__ uint32_t take_w(const W& win, uint32_t lp, uint32_t& len) const {
-        return take_v(win, win(lp), lp, len);
-    }
-    template <typename W>
-    __device__ __forceinline__ uint32_t take_v(const W& win, uint32_t w, uint32_t lp, uint32_t& len) const {
-        uint32_t e = lut[w >> (32 - kLutBits)];
-        if (e & kLutSlow) {
-            uint32_t used = kLutBits;
-            for (int lv = 0; lv < 16 && (e & kLutSlow); lv++) {
-                const uint32_t idx = used + kSubTabBits <= 32 ? (w << used) >> (32 - kSubTabBits)
-                                                              : win(lp + used) >> (32 - kSubTabBits);
-                e = sub[(e & 0x7FFFFFFFu) + idx];
-                used += kSubTabBits;
-            }
+    __device__ __forceinline__ void resolve(const W& win, uint32_t, uint32_t lp, uint32_t& e, uint32_t& l) const {
+        uint32_t used = kLutBits;
+#pragma unroll 1
+        for (int lv = 0; lv < 16 && (e & kLutSlow); lv++, used += kSubTabBits) {
+            e = sub[(e & ~kLutSlow) + (win(lp + used) >> (32 - kSubTabBits))];
+            asm volatile("" : "+v"(e));  // (its wait, as in Decoder<true>::deeper)
         }
-        len = (e & kLutSlow) ? 0u : (e >> 16) & 0x7F;
-        return e & 0xFFFF;
+        l = (e & kLutSlow) ? 0u : (e >> 16) & 0x7F;
     }
 };
 
-constexpr int kSyncWg = 256;                                     // subsequences decoded per workgroup
-constexpr int kSyncStride = kSyncWg - 1;                         // ... whose results it writes
-constexpr uint32_t kStageWords = kSyncWg * (kSubBits / 32) + 12;  // + shift0 and the tail read by the last codewords
-constexpr uint32_t kStageLds = kStageWords + kStageWords / 32 + 1;
-constexpr int kCkStride = kCkpts + 1;                            // odd row stride: one bank per thread
-constexpr uint32_t kNoCkpt = 0xFF;                               // window without a codeword start
-// Bits a continuation decodes before it gives up and lists the subsequence
-// for a full re-decode: most continuations meet a checkpoint within a few
-// windows (a meeting shows at the first codeword start of the window after
-// the two decodes agree, so the budget must span more than one window
-// whatever the code lengths), and a wavefront otherwise waits for its
-// slowest lane.
-constexpr uint32_t kContBits = 288;
+// Copies the tables a kernel keeps in LDS (compact: the first level and the
+// n_sub16 entries behind it, a multiple of 16) with NT threads.  fetch()
+// issues every load of a thread and put() stores them, so a workgroup can
+// have its tables and its bits in flight together and waits for one memory
+// latency; a copy loop of one load per round waited for one latency per
+// round, which was most of a workgroup's time (the indexed decode of the
+// 512^3 field at 1e-3: 0.28 -> 0.16 ms).
+template <bool T16, uint32_t NT>
+struct TableCopy {
+    static constexpr uint32_t kVecs = (((1u << kLutBits) + (T16 ? kMaxSub16 : 0)) * (T16 ? 2 : 4) / 16 + NT - 1) / NT;
+    U32x4 v[kVecs];
+    uint32_t n;
+    __device__ __forceinline__ void fetch(const DecodeArgs& a) {
+        n = T16 ? ((1u << kLutBits) + a.n_sub16) / 8 : (1u << kLutBits) / 4;
+        const GlobalU32x4 src = T16 ? (GlobalU32x4)a.lut16 : (GlobalU32x4)a.lut;
+#pragma unroll
+        for (uint32_t m = 0; m < kVecs; m++)
+            if (threadIdx.x + m * NT < n) v[m] = src[threadIdx.x + m * NT];
+    }
+    __device__ __forceinline__ void put(uint32_t* lds) const {
+#pragma unroll
+        for (uint32_t m = 0; m < kVecs; m++)
+            if (threadIdx.x + m * NT < n) reinterpret_cast<U32x4*>(lds)[threadIdx.x + m * NT] = v[m];
+    }
+};
 
-// Stages NW aligned-space words starting at w0 (a multiple of 4) into the
-// padded layout.  Every thread issues all of its 16-byte loads before the
-// first LDS write, so the workgroup waits for one memory latency, not one per
-// word.
-template <uint32_t NW>
-__device__ __forceinline__ void stage_words(uint32_t* st, const StreamView& sv, uint64_t w0) {
-    constexpr uint32_t kVec = (NW + 4 * kSyncWg - 1) / (4 * kSyncWg);  // uint4 per thread
-    uint4 v[kVec];
-    const uint4* src = reinterpret_cast<const uint4*>(sv.base) + w0 / 4;
-    if (4 * (w0 + kVec * 4 * kSyncWg) <= sv.nbytes) {
-        // whole range inside the stream: unconditional loads, all in flight together
-#pragma unroll
-        for (uint32_t m = 0; m < kVec; m++) v[m] = src[threadIdx.x + m * kSyncWg];
-#pragma unroll
-        for (uint32_t m = 0; m < kVec; m++)
-            v[m] = make_uint4(__builtin_bswap32(v[m].x), __builtin_bswap32(v[m].y), __builtin_bswap32(v[m].z),
-                              __builtin_bswap32(v[m].w));
-    } else {
-#pragma unroll
-        for (uint32_t m = 0; m < kVec; m++) {
-            const uint64_t w = w0 + 4 * (threadIdx.x + m * kSyncWg);
-            v[m] = make_uint4(sv.word(w), sv.word(w + 1), sv.word(w + 2), sv.word(w + 3));
+// A lane's place in its staged bits: words iw, iw + 1 and iw + 2 are held in
+// registers, iw the word before bit lp - 1 ends ((lp - 1) >> 5, so that the
+// window at lp is one alignbit: 1 to 32 bits into a).  The word that a step
+// will need is read one step ahead, so a codeword waits for its table
+// lookup only, not for the window before it.
+struct BitCursor {
+    uint32_t a, b, c;
+    int32_t iw;
+    template <typename W>
+    __device__ __forceinline__ void seek(const W& win, uint32_t lp) {
+        iw = (int32_t)(lp - 1) >> 5;
+        a = iw >= 0 ? win.word((uint32_t)iw) : 0u;
+        b = win.word((uint32_t)(iw + 1));
+        c = win.word((uint32_t)(iw + 2));
+    }
+    __device__ __forceinline__ uint32_t window(uint32_t lp) const { return __builtin_amdgcn_alignbit(a, b, 0u - lp); }
+    // To the new position lp (forward).
+    template <typename W>
+    __device__ __forceinline__ void advance(const W& win, uint32_t lp) {
+        const int32_t w = (int32_t)(lp - 1) >> 5;
+        if (w > iw + 1) {  // more than 32 bits: a long codeword
+            seek(win, lp);
+        } else {
+            const bool over = w != iw;
+            a = over ? b : a;
+            b = over ? c : b;
+            c = win.word((uint32_t)(w + 2));
+            iw = w;
         }
     }
+};
+
+// The two codewords from lp on: entries e[], lengths l[] (0: invalid path).
+// One window serves both: its 32 bits hold a codeword of at most 16 bits and
+// the first 16 of the next, which is as far as the first two table levels
+// look.
+template <bool T16, typename W>
+__device__ __forceinline__ void decode_pair(const Decoder<T16>& dec, const W& win, const BitCursor& cur, uint32_t lp,
+                                            uint32_t* e, uint32_t* l) {
+    using D = Decoder<T16>;
+    const uint32_t w = cur.window(lp);
+    e[0] = dec.look(w);
+    l[0] = D::len(e[0]);
+    uint32_t w2 = w << (l[0] & 31);
+    if (D::escape(e[0])) {
+        dec.resolve(win, w, lp, e[0], l[0]);
+        w2 = l[0] <= 16 ? w << l[0] : win(lp + l[0]);
+    }
+    e[1] = dec.look(w2);
+    l[1] = D::len(e[1]);
+    if (D::escape(e[1])) dec.resolve(win, w2, lp + l[0], e[1], l[1]);
+}
+template <bool T16, typename W>
+__device__ __forceinline__ uint32_t decode_one(const Decoder<T16>& dec, const W& win, uint32_t w, uint32_t lp,
+                                               uint32_t& l) {
+    uint32_t e = dec.look(w);
+    l = Decoder<T16>::len(e);
+    if (Decoder<T16>::escape(e)) dec.resolve(win, w, lp, e, l);
+    return Decoder<T16>::sym(e);
+}
+
+// Codewords and zeros (outliers) of the codewords that start in [lp, end),
+// added to cnt and z; lp ends at the first start at or past end, cur with it.
+// Returns whether an invalid codeword was met (it counts as one of one bit).
+template <bool T16, typename W>
+__device__ __forceinline__ bool decode_count(const Decoder<T16>& dec, const W& win, BitCursor& cur, uint32_t& lp,
+                                             uint32_t end, uint32_t& cnt, uint32_t& z) {
+    using D = Decoder<T16>;
+    bool bad = false;
+    while (lp < end) {
+        uint32_t e[2], l[2];
+        decode_pair<T16>(dec, win, cur, lp, e, l);
+        if constexpr (!T16) {  // (the compact tables hold no invalid path)
+            bad |= l[0] == 0;
+            l[0] = max(l[0], 1u);
+        }
+        const bool two = lp + l[0] < end;
+        if constexpr (!T16) {
+            bad |= two & (l[1] == 0);
+            l[1] = max(l[1], 1u);
+        }
+        cnt += two ? 2u : 1u;
+        lp += l[0] + (two ? l[1] : 0u);
+        const uint32_t s0 = D::sym(e[0]), s1 = D::sym(e[1]);
+        if (min(s0, s1) == 0) z += (uint32_t)(s0 == 0) + (uint32_t)(two & (s1 == 0));
+        cur.advance(win, lp);
+    }
+    return bad;
+}
+
+// Whether either half of w is 0 after taking the halves' minima with those of
+// more words (pk_min).
+__device__ __forceinline__ uint32_t pk_min(uint32_t a, uint32_t b) {
+    return __builtin_bit_cast(uint32_t, __builtin_elementwise_min(__builtin_bit_cast(U16x2, a), __builtin_bit_cast(U16x2, b)));
+}
+__device__ __forceinline__ bool pk_has_zero(uint32_t w) { return ((w & 0xFFFFu) == 0) | ((w >> 16) == 0); }
+
+// Stages aligned-space words from w0 (a multiple of 4) with NT threads, at
+// most VECS 16-byte vectors each: fetch() issues every load, the put()s store
+// (see TableCopy).  Vectors past the stream's readable bytes are zero, the
+// one that holds its end is read word by word.
+template <uint32_t VECS, uint32_t NT>
+struct StageCopy {
+    U32x4 v[VECS];
+    __device__ __forceinline__ void fetch(const StreamView& sv, uint64_t w0, uint32_t nvec) {
+        const GlobalU32x4 src = (GlobalU32x4)sv.base + w0 / 4;
+        // whole vectors from w0 on, of those wanted
+        const uint64_t whole = sv.nbytes / 16 > w0 / 4 ? sv.nbytes / 16 - w0 / 4 : 0;
+        const uint32_t lim = (uint32_t)min<uint64_t>(whole, nvec);
 #pragma unroll
-    for (uint32_t m = 0; m < kVec; m++) {
-        const uint32_t k = 4 * (threadIdx.x + m * kSyncWg);
-        if (k < NW) {
-            // four consecutive words never straddle a 32-word row
-            uint32_t* d = st + pad_idx(k);
-            d[0] = v[m].x;
-            d[1] = v[m].y;
-            d[2] = v[m].z;
-            d[3] = v[m].w;
-            if ((k & 31) == 0 && k > 0) d[-1] = v[m].x;  // the previous row's copy of its successor
+        for (uint32_t m = 0; m < VECS; m++) {
+            v[m] = U32x4{0, 0, 0, 0};
+            if (threadIdx.x + m * NT < lim) v[m] = src[threadIdx.x + m * NT];
+        }
+#pragma unroll
+        for (uint32_t m = 0; m < VECS; m++)
+            v[m] = U32x4{__builtin_bswap32(v[m].x), __builtin_bswap32(v[m].y), __builtin_bswap32(v[m].z),
+                         __builtin_bswap32(v[m].w)};
+        if (lim < nvec && (sv.nbytes & 15)) {
+#pragma unroll
+            for (uint32_t m = 0; m < VECS; m++) {
+                if (threadIdx.x + m * NT == lim) {
+                    const uint64_t w = w0 + 4 * lim;
+                    v[m] = U32x4{sv.word(w), sv.word(w + 1), sv.word(w + 2), sv.word(w + 3)};
+                }
+            }
         }
     }
-}
+    // Into rows (pad_idx), the first nw words.
+    __device__ __forceinline__ void put_rows(uint32_t* st, uint32_t nw) const {
+#pragma unroll
+        for (uint32_t m = 0; m < VECS; m++) {
+            const uint32_t k = 4 * (threadIdx.x + m * NT);
+            if (k < nw) {
+                // four consecutive words never straddle a row
+                uint32_t* d = st + pad_idx(k);
+                d[0] = v[m].x;
+                d[1] = v[m].y;
+                d[2] = v[m].z;
+                d[3] = v[m].w;
+                if (k % kSubWords == 0 && k > 0) d[-1] = v[m].x;  // the previous row's copy of its successor
+            }
+        }
+    }
+    // Into consecutive words (16-byte aligned).
+    __device__ __forceinline__ void put(uint32_t* st, uint32_t nvec) const {
+#pragma unroll
+        for (uint32_t m = 0; m < VECS; m++)
+            if (threadIdx.x + m * NT < nvec) reinterpret_cast<U32x4*>(st)[threadIdx.x + m * NT] = v[m];
+    }
+};
 
-// Checkpoint word: bits 0..7 offset of the first codeword start in the
-// window (kNoCkpt: none), 8..18 codewords before it, 19..29 zeros before it.
-__device__ __forceinline__ uint32_t ckpt(uint32_t off, uint32_t cnt, uint32_t z) {
-    return off | (cnt << 8) | (z << 19);
-}
-
-// Dynamic LDS words of the sync kernel after the tables.
-constexpr uint32_t kSyncLdsWords = kStageLds + kSyncWg * kCkStride + 2 * kSyncWg;
+constexpr uint32_t kSyncWg = 512;             // subsequences decoded per workgroup
+constexpr uint32_t kSyncStride = kSyncWg - 1;  // ... whose results it writes (the first one's belong to the workgroup before)
+// Bits decoded before a subsequence to find its first codeword.
+constexpr uint32_t kLeadBits = 288;
+static_assert(kLeadBits <= kSubBits, "the lead lies in one row");
+// A row for the first subsequence's lead, and the tail its last codewords'
+// windows read: the last starts before bit kSubBits + shift0 (<= 120) of its
+// row, the second of its pair up to 64 bits later, and a decode reads at most
+// 72 + 64 bits on (the deepest table walk of an invalid path, words read ahead).
+constexpr uint32_t kSyncStageWords = (kSyncWg + 1) * kSubWords + 12;
+constexpr uint32_t kSyncStageLds = kSyncStageWords + kSyncStageWords / kSubWords + 1;
+constexpr uint32_t kSyncLdsWords = kSyncStageLds + kSyncWg;  // dynamic LDS after the tables
 
 // Workgroup `unit` of the sync pass: subsequences unit * kSyncStride on.
 template <bool T16>
 __device__ __forceinline__ void decode_sync_unit(const DecodeArgs& a, const SubState& s, DecSummary* sum,
-                                                 uint64_t unit) {
-    extern __shared__ uint32_t lds[];
+                                                 uint64_t unit, uint32_t stripe) {
+    extern __shared__ __align__(16) uint32_t lds[];
     Decoder<T16> dec;
-    uint32_t* st = lds + dec.load(lds, a);
-    uint32_t* ck = st + kStageLds;
-    uint32_t* own_cz = ck + kSyncWg * kCkStride;  // own codeword count | zero count << 16 (both <= kSubBits)
-    uint32_t* own_e = own_cz + kSyncWg;
+    uint32_t* st = lds + dec.attach(lds, a);
+    uint32_t* own_e = st + kSyncStageLds;
     StreamView sv;
     sv.setup(a.stream, a.stream_bits);
     const uint64_t J0 = unit * kSyncStride;
-    stage_words<kStageWords>(st, sv, J0 * (kSubBits / 32));
+    // the stage starts one row before subsequence J0 (but not before the stream)
+    const uint64_t Jst = J0 ? J0 - 1 : 0;
+    {
+        TableCopy<T16, kSyncWg> tc;
+        StageCopy<(kSyncStageWords + 4 * kSyncWg - 1) / (4 * kSyncWg), kSyncWg> sc;
+        tc.fetch(a);
+        sc.fetch(sv, Jst * kSubWords, (kSyncStageWords + 3) / 4);
+        tc.put(lds);
+        sc.put_rows(st, kSyncStageWords);
+    }
     lds_sync();
     const uint32_t t = threadIdx.x;
     const uint64_t j = J0 + t;
-    // local position of stream bit p: p - J0*kSubBits + shift0
-    auto local = [&](uint64_t p) -> uint32_t { return (uint32_t)(p - J0 * kSubBits) + sv.shift0; };
+    const bool live = j < a.nsub;
     bool bad = false;
-
-    // 1. own decode from the assumed start, with checkpoints
-    if (j < a.nsub) {
-        const uint32_t s0 = t * kSubBits + sv.shift0;
-        const uint32_t e0 = local(min((j + 1) * (uint64_t)kSubBits, a.stream_bits));
-#pragma unroll
-        for (int k = 0; k < kCkpts; k++) ck[t * kCkStride + k] = kNoCkpt;
-        // minl: the shortest codeword length seen (0: an invalid path), a
-        // per-lane minimum rather than a flag the loop merges across lanes
-        uint32_t lp = s0, cnt = 0, z = 0, last_k = 0xFFFFFFFFu, minl = ~0u;
-        while (lp < e0) {
-            // the first codeword start in a window is its checkpoint; the
-            // other codewords write the row's pad slot (never read), so the
-            // record needs no branch
-            const uint32_t rel = lp - s0;
-            const uint32_t kk = rel / kCkptBits;
-            ck[t * kCkStride + (kk != last_k ? kk : (uint32_t)kCkpts)] = ckpt(rel % kCkptBits, cnt, z);
-            last_k = kk;
-            uint32_t len;
-            const uint32_t sym = dec.take_at(st, lp, len);
-            minl = min(minl, len);
-            lp += max(len, 1u);
-            cnt++;
-            z += sym == 0;
+    // stage bits: the subsequence's first bit, its first codeword, its target
+    const uint32_t s0 = (uint32_t)(j - Jst) * kSubBits + sv.shift0;
+    uint32_t first = s0, e0 = s0, cnt = 0, z = 0, lp = s0;
+    if (live) {
+        const PadWin win{st};
+        e0 += (uint32_t)min<uint64_t>(kSubBits, a.stream_bits - j * kSubBits);
+        BitCursor cur;
+        if (j) {
+            lp = s0 - kLeadBits;
+            cur.seek(win, lp);
+            uint32_t lc = 0, lz = 0;
+            (void)decode_count<T16>(dec, win, cur, lp, s0, lc, lz);  // (an invalid path here is a wrong start's)
+            first = lp;
+        } else {  // the stream starts with a codeword
+            cur.seek(win, lp);
         }
-        bad |= minl == 0;
-        own_cz[t] = cnt | (z << 16);
+        bad = decode_count<T16>(dec, win, cur, lp, e0, cnt, z);
         own_e[t] = lp;
-        if (j == 0) {  // the stream's first subsequence starts at a true boundary
-            s.b[0] = 0;
-            s.e[0] = (uint64_t)lp - sv.shift0;
-            s.cnt[0] = cnt;
-            s.zer[0] = z;
-        }
     }
     lds_sync();
-
-    // 2. continuation into subsequence j + 1 from this thread's own end
-    if (t < kSyncStride && j + 1 < a.nsub) {
-        const uint32_t u = t + 1;
-        const uint32_t su = u * kSubBits + sv.shift0;
-        const uint32_t eu = local(min((j + 2) * (uint64_t)kSubBits, a.stream_bits));
-        const uint32_t q0 = own_e[t];
-        uint32_t cc = 0, cz = 0, minl = ~0u, e = 0;
-        uint32_t q = q0;
-        bool hit = false;
-        // One exit, taken when the budget is spent, past u's end, or at a
-        // codeword start that meets u's checkpoint; which one is worked out
-        // after the loop (exits that each set their own results cost the
-        // divergent loop a set of lane masks per exit and iteration).  Past
-        // the budget or u's end the read goes to the row's pad slot and is
-        // not used.
-        for (;;) {
-            const uint32_t rel = q - su;
-            e = ck[u * kCkStride + min(rel / kCkptBits, (uint32_t)kCkpts)];
-            const bool stop = (q - q0 >= kContBits) | (q >= eu);
-            hit = !stop && (e & 0xFF) == rel % kCkptBits;
-            if (stop | hit) break;
-            uint32_t len;
-            const uint32_t sym = dec.take_at(st, q, len);
-            minl = min(minl, len);
-            q += max(len, 1u);
-            cc++;
-            cz += sym == 0;
-        }
-        bad |= minl == 0;
-        const bool capped = !hit && q - q0 >= kContBits;
-        bool met = hit;
-        uint32_t before_c = 0, before_z = 0;
-        if (hit) {
-            before_c = (e >> 8) & 0x7FF;
-            before_z = e >> 19;
-        } else if (!capped && q == own_e[u]) {  // past u's end, at u's own end
-            met = true;
-            before_c = own_cz[u] & 0xFFFF;
-            before_z = own_cz[u] >> 16;
-        }
-        const uint64_t base = J0 * kSubBits - sv.shift0;
-        s.b[j + 1] = base + q0;
-        if (capped) {
-            // re-decoded in full from q0 by the first pass, which then compares
-            // its end with the own end that j + 2's continuation started from
-            s.e[j + 1] = base + own_e[u];
-            const uint32_t k = atomicAdd(&s.list_n[0], 1u);
-            s.list_j[0][k] = s.jbase + (uint32_t)(j + 1);
-            s.list_start[0][k] = base + q0;
-        } else if (met) {
-            s.cnt[j + 1] = cc + (own_cz[u] & 0xFFFF) - before_c;
-            s.zer[j + 1] = cz + (own_cz[u] >> 16) - before_z;
-            s.e[j + 1] = base + own_e[u];
-        } else {
-            // the continuation decoded all of j + 1 from its true start; the
-            // check of j + 2 started from j + 1's own (different) end
-            s.cnt[j + 1] = cc;
-            s.zer[j + 1] = cz;
-            s.e[j + 1] = base + q;
-            if (j + 2 < a.nsub) {
-                const uint32_t k = atomicAdd(&s.list_n[0], 1u);
-                s.list_j[0][k] = s.jbase + (uint32_t)(j + 2);
-                s.list_start[0][k] = base + q;
-            }
-        }
+    bool wrong = false;
+    uint32_t pred = s0;
+    if (live && (t > 0 || j == 0)) {
+        s.b[j] = (uint8_t)(first - s0);
+        s.e[j] = (uint8_t)(lp - e0);
+        s.cz[j] = cnt | (z << 16);
+        if (t > 0) pred = own_e[t - 1];
+        wrong = t > 0 && pred != first;
+        if (bad && !wrong) atomicOr(&sum->error, 1u);
     }
-    if (bad) atomicOr(&sum->error, 1u);
+    list_append(s, 0, stripe, wrong, j, pred - s0);
 }
 
 template <bool T16>
-__global__ void __launch_bounds__(256) k_decode_sync(DecodeArgs a, SubState s, DecSummary* sum) {
-    decode_sync_unit<T16>(a, s, sum, blockIdx.x);
+__global__ void __launch_bounds__(kSyncWg) k_decode_sync(DecodeArgs a, SubState s, DecSummary* sum) {
+    decode_sync_unit<T16>(a, s, sum, blockIdx.x, blockIdx.x % s.nstripe);
 }
 
-// Re-decode pass: each listed subsequence j is decoded in full from its
-// listed start (the true end of j - 1); this gives its start, counts and
-// end.  An end other than the one j + 1's data was computed from lists j + 1,
-// from that end, for the next pass.  Chains shorten by at least one per
-// pass.  Workgroups take 256 entries at a time, one per thread; a thread
-// stages its entry's row (the subsequence plus the tail its last codeword
-// may read) in LDS with independent 16-byte loads, all in flight together,
-// then decodes it.  (Staging rows with coalesced word loads, one dependent
-// load of the entry number per word, put a memory latency per word on the
-// round.)
+// Re-decode pass: each listed subsequence j is decoded from its listed start
+// (the true end of j - 1); this gives its start, counts and end.  An end other
+// than the one j + 1's data was computed from lists j + 1, from that end, for
+// the next pass.  Chains shorten by at least one per pass.  Workgroups take
+// 256 entries at a time, one per thread; a thread stages its entry's row (the
+// subsequence plus the tail its last codeword may read) in LDS with
+// independent 16-byte loads, all in flight together, then decodes it.
 //
-// A row is aligned-space words 32 j .. 32 j + kRowWords - 1, 16-byte aligned
-// like the stream base: the decode starts at local bit start + shift0 - 1024 j
-// (>= 0, since a subsequence's true start is at or past its first bit), the
-// last codeword starts before local bit 1024 + shift0 (<= 1144), and a
-// decode reads at most 72 + 32 bits past a codeword start (the deepest
-// table walk of an invalid path), so the last word read is word 38.
-constexpr uint32_t kRowWords = 40;   // ten 16-byte loads
-constexpr uint32_t kRowStride = 41;  // odd: the lanes' reads of one word index fall in different banks
-constexpr uint32_t kPassGrid = 1024;  // persistent workgroups of a pass (at most ~3 resident per CU)
+// A row is aligned-space words 16 j .. 16 j + kRowWords - 1, 16-byte aligned
+// like the stream base: the last codeword starts before local bit 512 +
+// shift0 (<= 632), the second of its pair up to 64 bits later, and a decode
+// reads at most 72 + 64 bits on (see kSyncStageWords), so the last word read
+// is word 25.
+constexpr uint32_t kRowWords = 28;    // seven 16-byte loads
+constexpr uint32_t kRowStride = 29;   // odd: the lanes' reads of one word index fall in different banks
+constexpr uint32_t kPassGrid = 1024;  // persistent workgroups of a pass (at most ~4 resident per CU)
 __device__ __forceinline__ void stage_row(uint32_t* __restrict__ row, const StreamView& sv, uint64_t j) {
-    const uint64_t w0 = j * (kSubBits / 32);
+    const uint64_t w0 = j * kSubWords;
     if (4 * (w0 + kRowWords) <= sv.nbytes) {
-        const uint4* src = reinterpret_cast<const uint4*>(sv.base) + w0 / 4;
-        uint4 v[kRowWords / 4];
+        const GlobalU32x4 src = (GlobalU32x4)sv.base + w0 / 4;
+        U32x4 v[kRowWords / 4];
 #pragma unroll
         for (uint32_t m = 0; m < kRowWords / 4; m++) v[m] = src[m];
 #pragma unroll
@@ -456,78 +512,69 @@ __device__ __forceinline__ void stage_row(uint32_t* __restrict__ row, const Stre
         for (uint32_t w = 0; w < kRowWords; w++) row[w] = sv.word(w0 + w);
     }
 }
-// Entries e0 .. e0 + 255 (those below m) of pass `pass`'s list: one entry
-// per thread, staged in the thread's own LDS row.
+// Entry `ent` (jbase taken off its number) of pass `pass`'s list, in the
+// thread's own LDS row.  Returns whether j + 1 (set) is to be listed, from
+// over bits past its first.
 template <bool T16>
-__device__ __forceinline__ void redecode_entries(const DecodeArgs& a, const SubState& s, uint32_t pass,
-                                                 const Decoder<T16>& dec, uint32_t* rows, const StreamView& sv,
-                                                 uint64_t e0, uint32_t m, bool& bad) {
-    const uint32_t* lj = s.list_j[pass & 1];
-    const uint64_t* ls = s.list_start[pass & 1];
-    uint32_t* oj = s.list_j[(pass + 1) & 1];
-    uint64_t* os = s.list_start[(pass + 1) & 1];
-    uint32_t* on = &s.list_n[(pass + 1) % 3];
-    const uint32_t ne = (uint32_t)min<uint64_t>(256, m - e0);
-    if (threadIdx.x < ne) {
-        const uint64_t j = lj[e0 + threadIdx.x];
-        const uint64_t start = ls[e0 + threadIdx.x];
-        stage_row(rows + threadIdx.x * kRowStride, sv, j);  // the thread's own row: no barrier
-        const uint64_t rowbit = j * kSubBits;  // aligned-space bit of word 0
-        const RowWin win{rows + threadIdx.x * kRowStride};
-        const uint64_t target = min((j + 1) * (uint64_t)kSubBits, a.stream_bits);
-        const uint32_t tl = (uint32_t)(target + sv.shift0 - rowbit);
-        uint32_t lp = (uint32_t)(start + sv.shift0 - rowbit);
-        uint32_t cnt = 0, z = 0, minl = ~0u;
-        while (lp < tl) {
-            uint32_t len;
-            const uint32_t sym = dec.take_w(win, lp, len);
-            minl = min(minl, len);
-            lp += max(len, 1u);
-            cnt++;
-            z += sym == 0;
-        }
-        bad |= minl == 0;
-        const uint64_t pos = rowbit + lp - sv.shift0;
-        s.b[j] = start;
-        s.cnt[j] = cnt;
-        s.zer[j] = z;
-        if (pos != s.e[j]) {
-            s.e[j] = pos;
-            if (j + 1 < a.nsub) {
-                const uint32_t k = atomicAdd(on, 1u);
-                oj[k] = (uint32_t)(j + 1);
-                os[k] = pos;
-            }
-        }
-    }
-}
-
-template <bool T16>
-__global__ void __launch_bounds__(256) k_decode_pass(DecodeArgs a, SubState s, uint32_t pass, DecSummary* sum) {
-    const uint32_t m = s.list_n[pass % 3];
-    if (blockIdx.x == 0 && threadIdx.x == 0) s.list_n[(pass + 2) % 3] = 0;  // the list after next
-    if ((uint64_t)blockIdx.x * 256 >= m) return;  // whole workgroup
-    extern __shared__ uint32_t lds[];
-    Decoder<T16> dec;
-    uint32_t* rows = lds + dec.load(lds, a);
+__device__ __forceinline__ bool redecode_entry(const DecodeArgs& a, const SubState& s, const Decoder<T16>& dec,
+                                               uint32_t* row, uint64_t ent, DecSummary* sum, uint64_t& next,
+                                               uint32_t& over) {
+    const uint64_t j = (ent & ((1ull << 48) - 1)) - s.jbase;
+    const uint32_t first = (uint32_t)(ent >> 48);
     StreamView sv;
     sv.setup(a.stream, a.stream_bits);
-    bool bad = false;
+    stage_row(row, sv, j);  // the thread's own row: no barrier
+    const RowWin win{row};
+    const uint32_t tl = (uint32_t)min<uint64_t>(kSubBits, a.stream_bits - j * kSubBits) + sv.shift0;
+    uint32_t lp = first + sv.shift0, cnt = 0, z = 0;
+    BitCursor cur;
+    cur.seek(win, lp);
+    if (decode_count<T16>(dec, win, cur, lp, tl, cnt, z)) atomicOr(&sum->error, 1u);
+    over = lp - tl;
+    next = j + 1;
+    s.b[j] = (uint8_t)first;
+    s.cz[j] = cnt | (z << 16);
+    if (over == s.e[j]) return false;
+    s.e[j] = (uint8_t)over;
+    return next < a.nsub;
+}
+
+// Workgroup b takes entries of stripe b % nstripe.  (Whole wavefronts go
+// round together: list_append.)
+template <bool T16>
+__global__ void __launch_bounds__(256) k_decode_pass(DecodeArgs a, SubState s, uint32_t pass, DecSummary* sum) {
+    const uint32_t stripe = blockIdx.x % s.nstripe, nb = gridDim.x / s.nstripe, b = blockIdx.x / s.nstripe;
+    const uint32_t m = s.list_n[list_slot(pass) + stripe * kCounterWords];
+    if (b == 0 && threadIdx.x == 0) s.list_n[list_slot(pass + 2) + stripe * kCounterWords] = 0;  // the list after next
+    if ((uint64_t)b * 256 >= m) return;  // whole workgroup
+    extern __shared__ __align__(16) uint32_t lds[];
+    Decoder<T16> dec;
+    uint32_t* rows = lds + dec.attach(lds, a);
+    {
+        TableCopy<T16, 256> tc;
+        tc.fetch(a);
+        tc.put(lds);
+    }
     lds_sync();  // the tables
-    for (uint64_t e0 = blockIdx.x * 256ull; e0 < m; e0 += (uint64_t)gridDim.x * 256)
-        redecode_entries<T16>(a, s, pass, dec, rows, sv, e0, m, bad);
-    if (bad) atomicOr(&sum->error, 1u);
+    for (uint64_t e0 = b * 256ull + (threadIdx.x & ~63u); e0 < m; e0 += nb * 256ull) {
+        const uint64_t e = e0 + lane_id2();
+        bool on = false;
+        uint64_t next = 0;
+        uint32_t over = 0;
+        if (e < m)
+            on = redecode_entry<T16>(a, s, dec, rows + threadIdx.x * kRowStride,
+                                     s.list[pass & 1][stripe * s.stripe_cap + e], sum, next, over);
+        list_append(s, pass + 1, stripe, on, next, over);
+    }
 }
 
 // Device-wide exclusive scan of two u32 arrays into u64 offsets.
 constexpr int kScanPer = 4;
 constexpr int kScanBlock = 1024 * kScanPer;
 
-// guard (nullable): the scan does nothing while *guard is nonzero.
 __global__ void __launch_bounds__(1024) k_scan_local(const uint32_t* __restrict__ a, const uint32_t* __restrict__ b,
                                                      uint64_t n, uint64_t* __restrict__ oa, uint64_t* __restrict__ ob,
-                                                     uint64_t* __restrict__ bsum, const uint32_t* guard) {
-    if (guard && *guard) return;
+                                                     uint64_t* __restrict__ bsum) {
     __shared__ uint64_t sa[16], sbb[16];
     const uint64_t base = blockIdx.x * (uint64_t)kScanBlock + threadIdx.x * kScanPer;
     uint64_t va[kScanPer], vb[kScanPer], ta = 0, tb = 0;
@@ -582,9 +629,7 @@ __global__ void __launch_bounds__(1024) k_scan_local(const uint32_t* __restrict_
 
 // Exclusive scan of the per-block sums, 1024 at a time on one workgroup
 // (an LDS Hillis-Steele scan per pass, carried across passes).
-__global__ void __launch_bounds__(1024) k_scan_blocks(uint64_t* __restrict__ bsum, uint64_t nb, uint64_t* __restrict__ totals,
-                                                      const uint32_t* guard) {
-    if (guard && *guard) return;
+__global__ void __launch_bounds__(1024) k_scan_blocks(uint64_t* __restrict__ bsum, uint64_t nb, uint64_t* __restrict__ totals) {
     __shared__ uint64_t sa[1024], sb[1024];
     const uint32_t t = threadIdx.x;
     uint64_t ca = 0, cb = 0;
@@ -616,8 +661,7 @@ __global__ void __launch_bounds__(1024) k_scan_blocks(uint64_t* __restrict__ bsu
 }
 
 __global__ void __launch_bounds__(1024) k_scan_add(uint64_t* __restrict__ oa, uint64_t* __restrict__ ob, uint64_t n,
-                                                   const uint64_t* __restrict__ bsum, const uint32_t* guard) {
-    if (guard && *guard) return;
+                                                   const uint64_t* __restrict__ bsum) {
     const uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
     if (i < n) {
         const uint64_t blk = i / kScanBlock;
@@ -655,7 +699,7 @@ __device__ __forceinline__ IdxSpan idx_span(const uint64_t* __restrict__ index, 
     IdxSpan sp;
     sp.bs = bs;
     sp.be = be;
-    sp.w_lo = (bs + sv.shift0) >> 5;
+    sp.w_lo = (bs + sv.shift0) >> 7 << 2;  // (16-byte aligned)
     sp.nwords = be >= bs ? ((be + sv.shift0) >> 5) - sp.w_lo + kIdxSpanPad : 0;
     sp.fits = be >= bs && sp.nwords <= kIdxSpanWords;
     return sp;
@@ -709,9 +753,12 @@ __global__ void __launch_bounds__(256) k_decode_indexed(DecodeArgs a, const uint
     // per 16-byte piece of output
     constexpr uint32_t kFlush = R1D ? 16 : kIdxFlush;
     constexpr uint32_t kPer16 = R1D ? 4 : 8;
-    extern __shared__ uint32_t lds[];
+    extern __shared__ __align__(16) uint32_t lds[];
     Decoder<T16> dec;
-    const uint32_t tw = dec.load(lds, a);
+    const uint32_t tw = dec.attach(lds, a);
+    TableCopy<T16, 256> tc;
+    tc.fetch(a);
+    tc.put(lds);
     const uint32_t lane = threadIdx.x & 63;
     uint32_t* stage = lds + tw + (threadIdx.x >> 6) * kIdxStageWords;
     lds_sync();
@@ -741,7 +788,7 @@ __global__ void __launch_bounds__(256) k_decode_indexed(DecodeArgs a, const uint
     // already loaded (about 14 codewords of decode ahead of their use)
     auto load4 = [&](uint64_t q) -> uint4 {
         if (16 * (q + 1) <= sv.nbytes) {
-            const uint4 v = reinterpret_cast<const uint4*>(sv.base)[q];
+            const U32x4 v = ((GlobalU32x4)sv.base)[q];
             return make_uint4(__builtin_bswap32(v.x), __builtin_bswap32(v.y), __builtin_bswap32(v.z),
                               __builtin_bswap32(v.w));
         }
@@ -799,7 +846,7 @@ __global__ void __launch_bounds__(256) k_decode_indexed(DecodeArgs a, const uint
                 // lp - cw.b0 < 32 here: the codeword's first 32 bits are in buf
                 const uint32_t w = (uint32_t)((cw.buf << (lp - cw.b0)) >> 32);
                 uint32_t len;
-                const uint32_t sym = dec.take_v(cw, w, lp, len);
+                const uint32_t sym = decode_one<T16>(dec, cw, w, lp, len);
                 // past ns (or at an invalid codeword, an error) the lane
                 // stays where it is: lp ends at the segment's end
                 const bool in = u + k < ns;
@@ -915,10 +962,18 @@ __global__ void __launch_bounds__(256) k_decode_indexed_staged(DecodeArgs a, con
     sv.setup(a.stream, a.stream_bits);
     const IdxSpan sp = idx_span(index, L, total_bits, sv, blockIdx.x);
     if (!sp.fits) return;  // (the whole workgroup)
-    extern __shared__ uint32_t lds[];
+    extern __shared__ __align__(16) uint32_t lds[];
     Decoder<T16> dec;
-    uint32_t* stage = lds + dec.load(lds, a);
-    for (uint32_t i = threadIdx.x; i < (uint32_t)sp.nwords; i += 256) stage[i] = sv.word(sp.w_lo + i);
+    uint32_t* stage = lds + dec.attach(lds, a);
+    {
+        TableCopy<T16, 256> tc;
+        StageCopy<(kIdxSpanWords + 4 * 256 - 1) / (4 * 256), 256> sc;
+        const uint32_t nvec = ((uint32_t)sp.nwords + 3) / 4;
+        tc.fetch(a);
+        sc.fetch(sv, sp.w_lo, nvec);
+        tc.put(lds);
+        sc.put(stage, nvec);
+    }
     lds_sync();
     const uint64_t g = blockIdx.x * 256ull + threadIdx.x;
     if (g >= L.nseg) return;  // no barrier follows
@@ -938,13 +993,24 @@ __global__ void __launch_bounds__(256) k_decode_indexed_staged(DecodeArgs a, con
     // the loops count symbols, so an invalid codeword (len 0, an error)
     // needs no forced progress; a damaged stream stays within kIdxSpanOver
     // words past the span
-    uint32_t minl = ~0u;  // shortest codeword length seen (0: an invalid path)
+    BitCursor cur;
+    cur.seek(win, lp);
+    // one codeword, or two as the halves of a word
     auto next = [&]() -> uint32_t {
         uint32_t len;
-        const uint32_t sym = dec.take_w(win, lp, len);
-        minl = min(minl, len);
+        const uint32_t sym = decode_one<T16>(dec, win, cur.window(lp), lp, len);
+        if constexpr (!T16) bad |= len == 0;
         lp += len;
+        cur.advance(win, lp);
         return sym;
+    };
+    auto next2 = [&]() -> uint32_t {
+        uint32_t e[2], l[2];
+        decode_pair<T16>(dec, win, cur, lp, e, l);
+        if constexpr (!T16) bad |= (l[0] == 0) | (l[1] == 0);
+        lp += l[0] + l[1];
+        cur.advance(win, lp);
+        return Decoder<T16>::pack(e[0], e[1]);
     };
     auto outlier = [&](uint64_t i) {
         if (rank < a.n_outlier)
@@ -964,19 +1030,21 @@ __global__ void __launch_bounds__(256) k_decode_indexed_staged(DecodeArgs a, con
         };
         const uint32_t nfull16 = ns & ~15u;
         for (uint32_t G = 0; G < nfull16; G += 16) {
-            uint32_t c[16], omask = 0;
+            uint32_t c[16], least = ~0u;
 #pragma unroll
-            for (int k = 0; k < 16; k++) {
-                c[k] = next();
-                omask |= (uint32_t)(c[k] == 0) << k;
+            for (int k = 0; k < 16; k += 2) {
+                const uint32_t w = next2();
+                least = pk_min(least, w);
+                c[k] = w & 0xFFFF;
+                c[k + 1] = w >> 16;
             }
             float ov[16];
 #pragma unroll
             for (int k = 0; k < 16; k++) ov[k] = 0.f;
-            if (omask) {
+            if (pk_has_zero(least)) {
 #pragma unroll
                 for (int k = 0; k < 16; k++) {
-                    if ((omask >> k) & 1) {
+                    if (c[k] == 0) {
                         if (rank < a.n_outlier)
                             ov[k] = read_f32_bytes(a.outliers + 4 * rank);
                         else
@@ -1009,19 +1077,17 @@ __global__ void __launch_bounds__(256) k_decode_indexed_staged(DecodeArgs a, con
         const uint32_t nfull = ns & ~7u;  // whole units
         for (uint32_t G = 0; G < nfull; G += 32) {
             // outliers are rare: one test per group, then in symbol order
-            uint32_t w[16], omask = 0;
+            uint32_t w[16], least = ~0u;
 #pragma unroll
             for (int u = 0; u < 4; u++) {
                 const bool mine = G + 8 * u < nfull;  // differs across lanes only for the field's last segment
 #pragma unroll
-                for (int m = 0; m < 4; m++) w[4 * u + m] = 0;
+                for (int m = 0; m < 4; m++) w[4 * u + m] = ~0u;
                 if (mine) {
 #pragma unroll
                     for (int m = 0; m < 4; m++) {
-                        const uint32_t lo = next();
-                        const uint32_t hi = next();
-                        omask |= ((uint32_t)(lo == 0) | ((uint32_t)(hi == 0) << 1)) << (8 * u + 2 * m);
-                        w[4 * u + m] = lo | (hi << 16);
+                        w[4 * u + m] = next2();
+                        least = pk_min(least, w[4 * u + m]);
                     }
                 }
             }
@@ -1030,9 +1096,10 @@ __global__ void __launch_bounds__(256) k_decode_indexed_staged(DecodeArgs a, con
                 if (G + 8 * u < nfull)
                     *reinterpret_cast<uint4*>(codes + s0 + G + 8 * u) =
                         make_uint4(w[4 * u], w[4 * u + 1], w[4 * u + 2], w[4 * u + 3]);
-            if (omask) {
+            if (pk_has_zero(least)) {
+#pragma unroll
                 for (int k = 0; k < 32; k++)
-                    if ((omask >> k) & 1) outlier(s0 + G + k);
+                    if (((w[k / 2] >> (16 * (k & 1))) & 0xFFFF) == 0) outlier(s0 + G + k);
             }
         }
         for (uint32_t i = nfull; i < ns; i++) {  // the field's last, partial unit
@@ -1041,62 +1108,168 @@ __global__ void __launch_bounds__(256) k_decode_indexed_staged(DecodeArgs a, con
             if (sym == 0) outlier(s0 + i);
         }
     }
-    bad |= minl == 0;
     // the segment ends where the next one starts
     if (!bad) bad = span_lo + lp - sv.shift0 != end;
     if (bad) atomicOr(&sum->error, 1u);
 }
 
-// Final decode.  Thread j decodes cnt[j] codewords from its true start b[j]
-// out of the workgroup's staged bits: its symbols are [O, E), O = sym_off[j].
+// Codewords and zeros of each write unit (kWriteWg consecutive subsequences),
+// a wavefront per unit: sums[2 u], sums[2 u + 1].  A batch's units are
+// numbered across its fields.
+constexpr uint32_t kWriteWg = 512;
+static_assert(kWriteWg % 64 == 0, "a unit is whole wavefronts");
+__device__ __forceinline__ void decode_sums_unit(const uint32_t* __restrict__ cz, uint64_t nsub, uint64_t unit,
+                                                 uint64_t* __restrict__ sums) {
+    const uint32_t lane = lane_id2();
+    uint32_t c = 0, z = 0;
+#pragma unroll
+    for (uint32_t i = 0; i < kWriteWg / 64; i++) {
+        const uint64_t j = unit * kWriteWg + i * 64 + lane;
+        const uint32_t v = j < nsub ? cz[j] : 0u;
+        c += v & 0xFFFF;
+        z += v >> 16;
+    }
+    c = wave_scan_dpp(c);
+    z = wave_scan_dpp(z);
+    if (lane == 63) {
+        sums[0] = c;
+        sums[1] = z;
+    }
+}
+__global__ void __launch_bounds__(256) k_decode_sums(SubState s, uint64_t nsub, uint64_t nunits,
+                                                     uint64_t* __restrict__ sums, const uint32_t* guard) {
+    if (listed(guard)) return;
+    const uint64_t u = blockIdx.x * 4ull + (threadIdx.x >> 6);
+    if (u < nunits) decode_sums_unit(s.cz, nsub, u, sums + 2 * u);
+}
+
+// Exclusive prefixes of nunits pairs in place, the totals behind the last
+// (one workgroup, kScanUnits pairs per thread and round).
+constexpr uint32_t kScanUnits = 8;
+__global__ void __launch_bounds__(1024) k_decode_scan(uint64_t* __restrict__ off, uint64_t nunits, const uint32_t* guard) {
+    if (listed(guard)) return;
+    __shared__ uint64_t sh[2][16];
+    const uint32_t t = threadIdx.x, lane = t & 63, w = t >> 6;
+    uint64_t carry[2] = {0, 0};
+    for (uint64_t base = 0; base < nunits; base += 1024 * kScanUnits) {
+        const uint64_t u0 = base + t * kScanUnits;
+        uint64_t v[kScanUnits][2], run[2] = {0, 0};
+#pragma unroll
+        for (uint32_t i = 0; i < kScanUnits; i++)
+            for (int q = 0; q < 2; q++) v[i][q] = u0 + i < nunits ? off[2 * (u0 + i) + q] : 0;
+#pragma unroll
+        for (uint32_t i = 0; i < kScanUnits; i++)
+            for (int q = 0; q < 2; q++) {
+                const uint64_t x = v[i][q];
+                v[i][q] = run[q];  // before unit u0 + i, from u0
+                run[q] += x;
+            }
+        uint64_t pre[2] = {run[0], run[1]};
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1)
+            for (int q = 0; q < 2; q++) {
+                const uint64_t x = __shfl_up(pre[q], d);
+                if (lane >= (uint32_t)d) pre[q] += x;
+            }
+        if (lane == 63) {
+            sh[0][w] = pre[0];
+            sh[1][w] = pre[1];
+        }
+        lds_sync();
+        uint64_t tot[2] = {0, 0};
+        for (int q = 0; q < 2; q++) {
+            pre[q] += carry[q] - run[q];
+            for (uint32_t i = 0; i < 16; i++) {
+                if (i < w) pre[q] += sh[q][i];
+                tot[q] += sh[q][i];
+            }
+        }
+        lds_sync();
+#pragma unroll
+        for (uint32_t i = 0; i < kScanUnits; i++)
+            if (u0 + i < nunits)
+                for (int q = 0; q < 2; q++) off[2 * (u0 + i) + q] = pre[q] + v[i][q];
+        for (int q = 0; q < 2; q++) carry[q] += tot[q];
+    }
+    if (t < 2) off[2 * nunits + t] = carry[t];
+}
+
+// Final decode.  Thread j decodes the codewords of subsequence j from its
+// true start out of the workgroup's staged bits: its symbols are [O, E), O
+// the unit's offset plus a scan of the unit's counts.
 // Output goes out in whole 16-byte units of 8 symbols: the thread whose range
 // holds a unit's first symbol writes the unit, decoding on past E into the
 // following subsequences where the unit ends beyond it (the decode is on the
 // true path there), and skips the symbols before its first unit (written by
 // a predecessor).  Only the field's last unit may be partial.
-//
-// A workgroup (256 threads) takes kWriteWg = 240 subsequences, so its LDS
-// (the 8 KiB first-level table and ~31 KiB of staged bits) stays under
-// 40 KiB and four workgroups fit a CU instead of three: the decode is
-// latency-bound, and the resident lanes count for more than the 16 that
-// only help stage.
-constexpr uint32_t kWriteWg = 240;
-constexpr uint32_t kWriteStageWords = kWriteWg * (kSubBits / 32) + 32;  // + up to 7 codewords past the last range
-constexpr uint32_t kWriteStageLds = kWriteStageWords + kWriteStageWords / 32 + 3;
-// sym_off / zero_off: exclusive prefixes of the subsequences' codeword and
-// zero counts, counted from the field's subsequence 0 (entry 0 is the base
-// subtracted: 0 for one field, the earlier fields' totals in a batch).
+constexpr uint32_t kWriteStageWords = kWriteWg * kSubWords + 32;  // + up to 7 codewords past the last range
+constexpr uint32_t kWriteStageLds = kWriteStageWords + kWriteStageWords / kSubWords + 1;
+constexpr uint32_t kWriteLdsWords = kWriteStageLds + 2 * (kWriteWg / 64);  // dynamic LDS after the tables
+// base, off: the field's first unit's offsets and this unit's (field_base of
+// a batch's earlier fields is subtracted).
 template <bool T16>
 __device__ __forceinline__ void decode_write_unit(const DecodeArgs& a, const SubState& s,
-                                                  const uint64_t* __restrict__ sym_off,
-                                                  const uint64_t* __restrict__ zero_off, uint16_t* __restrict__ codes,
-                                                  float* __restrict__ sparse, DecSummary* sum, uint64_t unit,
-                                                  const uint32_t* guard = nullptr) {
-    if (guard && *guard) return;  // (the whole workgroup)
-    extern __shared__ uint32_t lds[];
+                                                  const uint64_t* __restrict__ base, const uint64_t* __restrict__ off,
+                                                  uint16_t* __restrict__ codes, float* __restrict__ sparse,
+                                                  DecSummary* sum, uint64_t unit) {
+    extern __shared__ __align__(16) uint32_t lds[];
     Decoder<T16> dec;
-    uint32_t* st = lds + dec.load(lds, a);
+    uint32_t* st = lds + dec.attach(lds, a);
+    uint32_t* wsum = st + kWriteStageLds;  // counts and zeros of each wavefront
     StreamView sv;
     sv.setup(a.stream, a.stream_bits);
     const uint64_t J0 = unit * kWriteWg;
-    stage_words<kWriteStageWords>(st, sv, J0 * (kSubBits / 32));
-    lds_sync();
     const uint64_t j = J0 + threadIdx.x;
-    if (threadIdx.x >= kWriteWg || j >= a.nsub) return;
-    uint32_t lp = (uint32_t)(s.b[j] - J0 * kSubBits) + sv.shift0;
-    const uint64_t O = sym_off[j] - sym_off[0];
-    const uint64_t E = min(O + s.cnt[j], a.n);
-    uint64_t rank = zero_off[j] - zero_off[0];
+    const bool live = j < a.nsub;
+    uint32_t cz, first;
+    {
+        TableCopy<T16, kWriteWg> tc;
+        StageCopy<(kWriteStageWords + 4 * kWriteWg - 1) / (4 * kWriteWg), kWriteWg> sc;
+        tc.fetch(a);
+        sc.fetch(sv, J0 * kSubWords, (kWriteStageWords + 3) / 4);
+        cz = live ? s.cz[j] : 0u;
+        first = live ? s.b[j] : 0u;
+        tc.put(lds);
+        sc.put_rows(st, kWriteStageWords);
+    }
+    const uint32_t ic = wave_scan_dpp(cz & 0xFFFF), iz = wave_scan_dpp(cz >> 16);
+    const uint32_t w = threadIdx.x >> 6;
+    if (lane_id2() == 63) {
+        wsum[2 * w] = ic;
+        wsum[2 * w + 1] = iz;
+    }
+    lds_sync();
+    if (!live) return;
+    uint64_t O = off[0] - base[0] + ic - (cz & 0xFFFF);
+    uint64_t rank = off[1] - base[1] + iz - (cz >> 16);
+    for (uint32_t i = 0; i < w; i++) {
+        O += wsum[2 * i];
+        rank += wsum[2 * i + 1];
+    }
+    const uint64_t E = min<uint64_t>(O + (cz & 0xFFFF), a.n);
+    uint32_t lp = threadIdx.x * kSubBits + first + sv.shift0;
     bool bad = false;
     // the loops below count symbols, so an invalid codeword (len 0, an
     // error) needs no forced progress
-    uint32_t minl = ~0u;  // shortest codeword length seen (0: an invalid path)
+    const PadWin win{st};
+    BitCursor cur;
+    cur.seek(win, lp);
+    // one codeword, or two as the halves of a word
     auto next = [&]() -> uint32_t {
         uint32_t len;
-        const uint32_t sym = dec.take_at(st, lp, len);
-        minl = min(minl, len);
+        const uint32_t sym = decode_one<T16>(dec, win, cur.window(lp), lp, len);
+        if constexpr (!T16) bad |= len == 0;
         lp += len;
+        cur.advance(win, lp);
         return sym;
+    };
+    auto next2 = [&]() -> uint32_t {
+        uint32_t e[2], l[2];
+        decode_pair<T16>(dec, win, cur, lp, e, l);
+        if constexpr (!T16) bad |= (l[0] == 0) | (l[1] == 0);
+        lp += l[0] + l[1];
+        cur.advance(win, lp);
+        return Decoder<T16>::pack(e[0], e[1]);
     };
     auto outlier = [&](uint64_t i) {
         if (rank < a.n_outlier)
@@ -1110,7 +1283,7 @@ __device__ __forceinline__ void decode_write_unit(const DecodeArgs& a, const Sub
     for (; i < E && i < W0; i++)          // a predecessor's unit: decode, count zeros, skip
         rank += next() == 0;
     if (W0 < E) {
-        const uint64_t W1 = min((E + 7) & ~7ull, a.n);
+        const uint64_t W1 = min<uint64_t>((E + 7) & ~7ull, a.n);
         const uint64_t Wf = W0 + ((W1 - W0) & ~7ull);  // end of the whole units
         // Whole units go out in groups of four (64 bytes) held in registers
         // and stored back to back: the L2 then sees long runs of each lane's
@@ -1119,20 +1292,18 @@ __device__ __forceinline__ void decode_write_unit(const DecodeArgs& a, const Sub
         // at the lane's first unit, so only its last group is partial.
         for (uint64_t G = W0; G < Wf; G += 32) {
             // outliers are rare: one test per group, then in symbol order
-            uint32_t w[16], omask = 0;
+            uint32_t w[16], least = ~0u;
 #pragma unroll
             for (int u = 0; u < 4; u++) {
                 const uint64_t iu = G + 8 * u;
                 const bool mine = iu < Wf;  // differs across lanes only in a last group
 #pragma unroll
-                for (int m = 0; m < 4; m++) w[4 * u + m] = 0;
+                for (int m = 0; m < 4; m++) w[4 * u + m] = ~0u;
                 if (mine) {
 #pragma unroll
                     for (int m = 0; m < 4; m++) {
-                        const uint32_t lo = next();
-                        const uint32_t hi = next();
-                        omask |= ((uint32_t)(lo == 0) | ((uint32_t)(hi == 0) << 1)) << (8 * u + 2 * m);
-                        w[4 * u + m] = lo | (hi << 16);
+                        w[4 * u + m] = next2();
+                        least = pk_min(least, w[4 * u + m]);
                     }
                 }
             }
@@ -1143,9 +1314,10 @@ __device__ __forceinline__ void decode_write_unit(const DecodeArgs& a, const Sub
                     *reinterpret_cast<uint4*>(codes + iu) =
                         make_uint4(w[4 * u], w[4 * u + 1], w[4 * u + 2], w[4 * u + 3]);
             }
-            if (omask) {
+            if (pk_has_zero(least)) {
+#pragma unroll
                 for (int k = 0; k < 32; k++)
-                    if ((omask >> k) & 1) outlier(G + k);
+                    if (((w[k / 2] >> (16 * (k & 1))) & 0xFFFF) == 0) outlier(G + k);
             }
         }
         i = Wf;
@@ -1155,15 +1327,15 @@ __device__ __forceinline__ void decode_write_unit(const DecodeArgs& a, const Sub
             if (sym == 0) outlier(i);
         }
     }
-    bad |= minl == 0;
     if (bad) atomicOr(&sum->error, 1u);
 }
 
 template <bool T16>
-__global__ void __launch_bounds__(256) k_decode_write(DecodeArgs a, SubState s, const uint64_t* __restrict__ sym_off,
-                                                      const uint64_t* __restrict__ zero_off, uint16_t* __restrict__ codes,
-                                                      float* __restrict__ sparse, DecSummary* sum, const uint32_t* guard) {
-    decode_write_unit<T16>(a, s, sym_off, zero_off, codes, sparse, sum, blockIdx.x, guard);
+__global__ void __launch_bounds__(kWriteWg) k_decode_write(DecodeArgs a, SubState s, const uint64_t* __restrict__ off,
+                                                           uint16_t* __restrict__ codes, float* __restrict__ sparse,
+                                                           DecSummary* sum, const uint32_t* guard) {
+    if (listed(guard)) return;
+    decode_write_unit<T16>(a, s, off, off + 2 * (uint64_t)blockIdx.x, codes, sparse, sum, blockIdx.x);
 }
 
 __global__ void k_fill_u16(uint16_t* p, uint64_t n, uint16_t v) {
@@ -1311,7 +1483,7 @@ template <int B, bool PAD = false>
 __global__ void __launch_bounds__(256) k_recon_3d(const uint16_t* __restrict__ codes, const float* __restrict__ sparse,
                                                   float* __restrict__ out, ReconArgs a, uint32_t* flagged,
                                                   uint32_t* nflagged) {
-    if (a.guard && *a.guard) return;  // decode output not final: a later launch redoes this
+    if (listed(a.guard)) return;  // decode output not final: a later launch redoes this
     const uint64_t ntiles = a.ntiles_x * a.ntiles_y * a.ntiles_z;
     const uint64_t wave = blockIdx.x * 4ull + (threadIdx.x >> 6);
     const uint64_t nwaves = gridDim.x * 4ull;
@@ -1372,7 +1544,7 @@ template <int B, bool PAD = false>
 __global__ void __launch_bounds__(256) k_recon_2d(const uint16_t* __restrict__ codes, const float* __restrict__ sparse,
                                                   float* __restrict__ out, ReconArgs a, uint32_t* flagged,
                                                   uint32_t* nflagged) {
-    if (a.guard && *a.guard) return;  // decode output not final: a later launch redoes this
+    if (listed(a.guard)) return;  // decode output not final: a later launch redoes this
     const uint64_t ntiles = a.ntiles_x * a.ntiles_y;
     const uint64_t wave = blockIdx.x * 4ull + (threadIdx.x >> 6);
     const uint64_t nwaves = gridDim.x * 4ull;
@@ -1420,7 +1592,7 @@ template <int B, bool PAD = false>
 __global__ void __launch_bounds__(256) k_recon_1d(const uint16_t* __restrict__ codes, const float* __restrict__ sparse,
                                                   float* __restrict__ out, ReconArgs a, uint32_t* flagged,
                                                   uint32_t* nflagged) {
-    if (a.guard && *a.guard) return;  // decode output not final: a later launch redoes this
+    if (listed(a.guard)) return;  // decode output not final: a later launch redoes this
     const uint64_t ntiles = a.ntiles_x;
     const uint64_t wave = blockIdx.x * 4ull + (threadIdx.x >> 6);
     const uint64_t nwaves = gridDim.x * 4ull;
@@ -1496,7 +1668,7 @@ __global__ void __launch_bounds__(64) k_recon_fallback(int ndim, int B, const ui
                                                        const float* __restrict__ sparse, float* __restrict__ out,
                                                        ReconArgs a, const uint32_t* __restrict__ flagged,
                                                        const uint32_t* __restrict__ nflagged) {
-    if (a.guard && *a.guard) return;  // decode output not final: a later launch redoes this
+    if (listed(a.guard)) return;  // decode output not final: a later launch redoes this
     recon_fallback_blocks(ndim, B, codes, sparse, out, a, flagged, nflagged,
                           blockIdx.x * (uint64_t)blockDim.x + threadIdx.x, (uint64_t)gridDim.x * blockDim.x);
 }
@@ -1653,7 +1825,7 @@ template <int ND, int B, bool ALN>
 __global__ void __launch_bounds__(256) k_recon_x4(const uint16_t* __restrict__ codes, const float* __restrict__ sparse,
                                                   float* __restrict__ out, ReconArgs a, uint32_t* flagged,
                                                   uint32_t* nflagged) {
-    if (a.guard && *a.guard) return;  // decode output not final: a later launch redoes this
+    if (listed(a.guard)) return;  // decode output not final: a later launch redoes this
     const uint64_t ntx = (a.d0 + 255) / 256;
     const uint64_t nty = ND >= 2 ? a.ntiles_y : 1, ntz = ND >= 3 ? a.ntiles_z : 1;
     const uint64_t ntiles = ntx * nty * ntz;
@@ -1673,23 +1845,33 @@ __global__ void __launch_bounds__(256) k_recon_x4(const uint16_t* __restrict__ c
 // descriptor reads are scalar.
 
 template <bool T16>
-__global__ void __launch_bounds__(256) k_decode_sync_multi(const DecField* __restrict__ fd,
+__global__ void __launch_bounds__(kSyncWg) k_decode_sync_multi(const DecField* __restrict__ fd,
                                                            const uint64_t* __restrict__ start, int nf) {
     const uint64_t u = blockIdx.x;
     const int f = field_of(start, nf, u);
     const DecodeArgs a = fd[f].a;
     const SubState s = fd[f].s;
-    decode_sync_unit<T16>(a, s, fd[f].sum, u - start[f]);
+    decode_sync_unit<T16>(a, s, fd[f].sum, u - start[f], (uint32_t)(u % s.nstripe));
+}
+
+__global__ void __launch_bounds__(256) k_decode_sums_multi(const DecField* __restrict__ fd,
+                                                           const uint64_t* __restrict__ start, int nf,
+                                                           uint64_t* __restrict__ sums) {
+    const uint64_t u = blockIdx.x * 4ull + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    if (u >= start[nf]) return;
+    const int f = field_of(start, nf, u);
+    decode_sums_unit(fd[f].s.cz, fd[f].a.nsub, u - start[f], sums + 2 * u);
 }
 
 template <bool T16>
-__global__ void __launch_bounds__(256) k_decode_write_multi(const DecField* __restrict__ fd,
-                                                            const uint64_t* __restrict__ start, int nf) {
+__global__ void __launch_bounds__(kWriteWg) k_decode_write_multi(const DecField* __restrict__ fd,
+                                                                 const uint64_t* __restrict__ start, int nf,
+                                                                 const uint64_t* __restrict__ off) {
     const uint64_t u = blockIdx.x;
     const int f = field_of(start, nf, u);
     const DecodeArgs a = fd[f].a;
     const SubState s = fd[f].s;
-    decode_write_unit<T16>(a, s, fd[f].sym_off, fd[f].zero_off, fd[f].codes, fd[f].sparse, fd[f].sum, u - start[f]);
+    decode_write_unit<T16>(a, s, off + 2 * start[f], off + 2 * u, fd[f].codes, fd[f].sparse, fd[f].sum, u - start[f]);
 }
 
 // The decode tables of a field read from global memory (entries of one
@@ -1700,14 +1882,16 @@ template <>
 __device__ __forceinline__ Decoder<true> global_decoder<true>(const DecodeArgs& a) {
     Decoder<true> d;
     d.lut = a.lut16;
-    d.sub = a.sub16;
+    d.sub_lds = nullptr;
+    d.sub = (GlobalU16)a.sub16;
+    d.n_lds = 0;
     return d;
 }
 template <>
 __device__ __forceinline__ Decoder<false> global_decoder<false>(const DecodeArgs& a) {
     Decoder<false> d;
     d.lut = a.lut;
-    d.sub = a.sub;
+    d.sub = (GlobalU32)a.sub;
     return d;
 }
 
@@ -1718,65 +1902,32 @@ template <bool T16>
 __global__ void __launch_bounds__(256) k_decode_pass_multi(const DecField* __restrict__ fd,
                                                            const uint64_t* __restrict__ sub_start, int nf, SubState S,
                                                            uint32_t pass) {
-    const uint32_t m = S.list_n[pass % 3];
-    if (blockIdx.x == 0 && threadIdx.x == 0) S.list_n[(pass + 2) % 3] = 0;  // the list after next
-    if ((uint64_t)blockIdx.x * 256 >= m) return;                            // whole workgroup
+    const uint32_t stripe = blockIdx.x % S.nstripe, nb = gridDim.x / S.nstripe, b = blockIdx.x / S.nstripe;
+    const uint32_t m = S.list_n[list_slot(pass) + stripe * kCounterWords];
+    if (b == 0 && threadIdx.x == 0) S.list_n[list_slot(pass + 2) + stripe * kCounterWords] = 0;  // the list after next
+    if ((uint64_t)b * 256 >= m) return;  // whole workgroup
     __shared__ uint32_t rows[256 * kRowStride];
-    const uint32_t* lj = S.list_j[pass & 1];
-    const uint64_t* ls = S.list_start[pass & 1];
-    uint32_t* oj = S.list_j[(pass + 1) & 1];
-    uint64_t* os = S.list_start[(pass + 1) & 1];
-    uint32_t* on = &S.list_n[(pass + 1) % 3];
-    for (uint64_t e0 = blockIdx.x * 256ull; e0 < m; e0 += (uint64_t)gridDim.x * 256) {
-        const uint32_t ne = (uint32_t)min<uint64_t>(256, m - e0);
-        if (threadIdx.x < ne) {
-            const uint32_t J = lj[e0 + threadIdx.x];
-            const int f = field_of(sub_start, nf, J);
+    for (uint64_t e0 = b * 256ull + (threadIdx.x & ~63u); e0 < m; e0 += nb * 256ull) {
+        const uint64_t e = e0 + lane_id2();
+        bool on = false;
+        uint64_t next = 0;
+        uint32_t over = 0;
+        if (e < m) {
+            const uint64_t ent = S.list[pass & 1][stripe * S.stripe_cap + e];
+            const int f = field_of(sub_start, nf, ent & ((1ull << 48) - 1));
             const DecodeArgs& a = fd[f].a;
-            const SubState& s = fd[f].s;
-            const Decoder<T16> dec = global_decoder<T16>(a);
-            StreamView sv;
-            sv.setup(a.stream, a.stream_bits);
-            const uint64_t j = J - sub_start[f];
-            const uint64_t start = ls[e0 + threadIdx.x];
-            stage_row(rows + threadIdx.x * kRowStride, sv, j);  // the thread's own row: no barrier
-            const uint64_t rowbit = j * kSubBits;  // aligned-space bit of word 0
-            const RowWin win{rows + threadIdx.x * kRowStride};
-            const uint64_t target = min((j + 1) * (uint64_t)kSubBits, a.stream_bits);
-            const uint32_t tl = (uint32_t)(target + sv.shift0 - rowbit);
-            uint32_t lp = (uint32_t)(start + sv.shift0 - rowbit);
-            uint32_t cnt = 0, z = 0, minl = ~0u;
-            while (lp < tl) {
-                uint32_t len;
-                const uint32_t sym = dec.take_w(win, lp, len);
-                minl = min(minl, len);
-                lp += max(len, 1u);
-                cnt++;
-                z += sym == 0;
-            }
-            const bool bad = minl == 0;
-            const uint64_t pos = rowbit + lp - sv.shift0;
-            s.b[j] = start;
-            s.cnt[j] = cnt;
-            s.zer[j] = z;
-            if (pos != s.e[j]) {
-                s.e[j] = pos;
-                if (j + 1 < a.nsub) {
-                    const uint32_t k = atomicAdd(on, 1u);
-                    oj[k] = J + 1;
-                    os[k] = pos;
-                }
-            }
-            if (bad) atomicOr(&fd[f].sum->error, 1u);
+            on = redecode_entry<T16>(a, fd[f].s, global_decoder<T16>(a), rows + threadIdx.x * kRowStride, ent,
+                                     fd[f].sum, next, over);
+            next += fd[f].s.jbase;
         }
+        list_append(S, pass + 1, stripe, on, next, over);  // (S.jbase 0)
     }
 }
 
-__global__ void k_dec_field_totals(const DecField* __restrict__ fd, int nf, uint64_t* __restrict__ tot) {
+__global__ void k_dec_field_totals(const uint64_t* __restrict__ start, int nf, const uint64_t* __restrict__ off,
+                                   uint64_t* __restrict__ tot) {
     const int f = blockIdx.x * blockDim.x + threadIdx.x;
-    if (f >= nf) return;
-    const uint64_t ns = fd[f].a.nsub;
-    tot[f] = ns ? fd[f].sym_off[ns - 1] + fd[f].s.cnt[ns - 1] - fd[f].sym_off[0] : 0;
+    if (f < nf) tot[f] = off[2 * start[f + 1]] - off[2 * start[f]];
 }
 
 template <int KIND, int B>
@@ -1845,13 +1996,13 @@ static size_t table_lds_bytes(const DecodeArgs& a, bool t16) {
 // memory.
 static DecodeArgs with_lds_sub16(DecodeArgs a, size_t own_bytes) {
     if (!a.lut16 || !a.n_sub16) return a;
-    constexpr size_t kCuLds = 160 * 1024, kGranule = 1024;  // (workgroup LDS counted in whole KiB, conservatively)
+    constexpr size_t kCuLds = 160 * 1024, kGranule = 1280;  // LDS is allocated in units of 1280 bytes
     DecodeArgs b = a;
     b.n_sub16 = 0;
-    auto granules = [](size_t bytes) { return (bytes + kGranule - 1) / kGranule * kGranule; };
-    const size_t without = granules(table_lds_bytes(b, true) + own_bytes);
-    const size_t with = granules(table_lds_bytes(a, true) + own_bytes);
-    if (kCuLds / with < kCuLds / without) a.n_sub16 = 0;
+    const size_t bare = table_lds_bytes(b, true) + own_bytes;
+    const size_t share = kCuLds / ((bare + kGranule - 1) / kGranule * kGranule);  // workgroups per CU
+    const size_t room = kCuLds / share / kGranule * kGranule - bare;
+    a.n_sub16 = (uint32_t)std::min<size_t>(a.n_sub16, room / 2 & ~(size_t)((1u << kSubTabBits) - 1));
     return a;
 }
 
@@ -1883,6 +2034,13 @@ void launch_decode_sync(const DecodeArgs& a0, SubState s, DecSummary* sum, hipSt
     else
         hipLaunchKernelGGL(k_decode_sync<false>, grid, dim3(kSyncWg), lds, st, a, s, sum);
 }
+void list_stripes(uint64_t units, uint32_t* nstripe, uint64_t* cap) {
+    *nstripe = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(kMaxStripes, units));
+    *cap = (units + *nstripe - 1) / *nstripe * kSyncWg;
+}
+static unsigned pass_grid(const SubState& s) {
+    return s.nstripe * (unsigned)std::max<uint64_t>(1, std::min<uint64_t>(kPassGrid / s.nstripe, (s.stripe_cap + 255) / 256));
+}
 void launch_decode_pass(const DecodeArgs& a0, SubState s, uint32_t pass, DecSummary* sum, hipStream_t st) {
     allow_big_lds(k_decode_pass<true>);
     allow_big_lds(k_decode_pass<false>);
@@ -1890,7 +2048,7 @@ void launch_decode_pass(const DecodeArgs& a0, SubState s, uint32_t pass, DecSumm
     const DecodeArgs a = with_lds_sub16(a0, (size_t)256 * kRowStride * 4);
     const size_t lds = table_lds_bytes(a, t16) + (size_t)256 * kRowStride * 4;
     // persistent workgroups; those past the listed count return at once
-    const dim3 grid((unsigned)std::min<uint64_t>(kPassGrid, std::max<uint64_t>(1, grid_for(a.nsub, 256))));
+    const dim3 grid(pass_grid(s));
     if (t16)
         hipLaunchKernelGGL(k_decode_pass<true>, grid, dim3(256), lds, st, a, s, pass, sum);
     else
@@ -1949,27 +2107,29 @@ void launch_decode_indexed(const DecodeArgs& a0, const uint64_t* index, uint64_t
 #undef DI
 }
 void launch_scan_u32x2(const uint32_t* a, const uint32_t* b, uint64_t n, uint64_t* oa, uint64_t* ob, uint64_t* block_tmp,
-                       uint64_t* totals, hipStream_t st, const uint32_t* guard) {
+                       uint64_t* totals, hipStream_t st) {
     const uint64_t nb = (n + kScanBlock - 1) / kScanBlock;
-    hipLaunchKernelGGL(k_scan_local, dim3((unsigned)nb), dim3(1024), 0, st, a, b, n, oa, ob, block_tmp, guard);
-    hipLaunchKernelGGL(k_scan_blocks, dim3(1), dim3(1024), 0, st, block_tmp, nb, totals, guard);
-    hipLaunchKernelGGL(k_scan_add, dim3(grid_for(n, 1024)), dim3(1024), 0, st, oa, ob, n, block_tmp, guard);
+    hipLaunchKernelGGL(k_scan_local, dim3((unsigned)nb), dim3(1024), 0, st, a, b, n, oa, ob, block_tmp);
+    hipLaunchKernelGGL(k_scan_blocks, dim3(1), dim3(1024), 0, st, block_tmp, nb, totals);
+    hipLaunchKernelGGL(k_scan_add, dim3(grid_for(n, 1024)), dim3(1024), 0, st, oa, ob, n, block_tmp);
 }
-void launch_decode_write(const DecodeArgs& a0, SubState s, const uint64_t* sym_off, const uint64_t* zero_off,
-                         uint16_t* codes, float* sparse, DecSummary* sum, hipStream_t st,
-                         const uint32_t* guard) {
+void launch_decode_offsets(const SubState& s, uint64_t nsub, uint64_t* off, hipStream_t st, const uint32_t* guard) {
+    const uint64_t nu = decode_write_units(nsub);
+    hipLaunchKernelGGL(k_decode_sums, dim3(grid_for(nu, 4)), dim3(256), 0, st, s, nsub, nu, off, guard);
+    hipLaunchKernelGGL(k_decode_scan, dim3(1), dim3(1024), 0, st, off, nu, guard);
+}
+void launch_decode_write(const DecodeArgs& a0, SubState s, const uint64_t* off, uint16_t* codes, float* sparse,
+                         DecSummary* sum, hipStream_t st, const uint32_t* guard) {
     allow_big_lds(k_decode_write<true>);
     allow_big_lds(k_decode_write<false>);
     const bool t16 = a0.lut16 != nullptr;
-    const DecodeArgs a = with_lds_sub16(a0, (size_t)kWriteStageLds * 4);
-    const size_t lds = table_lds_bytes(a, t16) + (size_t)kWriteStageLds * 4;
+    const DecodeArgs a = with_lds_sub16(a0, (size_t)kWriteLdsWords * 4);
+    const size_t lds = table_lds_bytes(a, t16) + (size_t)kWriteLdsWords * 4;
     const dim3 grid((unsigned)decode_write_units(a.nsub));
     if (t16)
-        hipLaunchKernelGGL(k_decode_write<true>, grid, dim3(kSyncWg), lds, st, a, s, sym_off, zero_off, codes, sparse,
-                           sum, guard);
+        hipLaunchKernelGGL(k_decode_write<true>, grid, dim3(kWriteWg), lds, st, a, s, off, codes, sparse, sum, guard);
     else
-        hipLaunchKernelGGL(k_decode_write<false>, grid, dim3(kSyncWg), lds, st, a, s, sym_off, zero_off, codes, sparse,
-                           sum, guard);
+        hipLaunchKernelGGL(k_decode_write<false>, grid, dim3(kWriteWg), lds, st, a, s, off, codes, sparse, sum, guard);
 }
 void launch_fill_u16(uint16_t* p, uint64_t n, uint16_t v, hipStream_t st) {
     unsigned g = (unsigned)std::min<uint64_t>(grid_for(n, 256), 8192);
@@ -2061,7 +2221,8 @@ uint32_t batch_sub16_in_lds(uint32_t max_sub16) {
     DecodeArgs probe{};
     probe.lut16 = reinterpret_cast<const uint16_t*>(&probe);  // (only tested for null)
     probe.n_sub16 = max_sub16;
-    return with_lds_sub16(probe, (size_t)kSyncLdsWords * 4).n_sub16;
+    return std::min(with_lds_sub16(probe, (size_t)kSyncLdsWords * 4).n_sub16,
+                    with_lds_sub16(probe, (size_t)kWriteLdsWords * 4).n_sub16);
 }
 
 void launch_decode_sync_multi(bool t16, uint32_t max_sub16, const DecField* fd, const uint64_t* start, int nf,
@@ -2078,29 +2239,36 @@ void launch_decode_sync_multi(bool t16, uint32_t max_sub16, const DecField* fd, 
         hipLaunchKernelGGL(k_decode_sync_multi<false>, dim3((unsigned)nunits), dim3(kSyncWg), lds, st, fd, start, nf);
 }
 void launch_decode_pass_multi(bool t16, const DecField* fd, const uint64_t* sub_start, int nf, SubState S,
-                              uint32_t pass, uint64_t nsub_tot, hipStream_t st) {
+                              uint32_t pass, hipStream_t st) {
     // persistent workgroups; those past the listed count return at once
-    const dim3 grid((unsigned)std::min<uint64_t>(kPassGrid, std::max<uint64_t>(1, grid_for(nsub_tot, 256))));
+    const dim3 grid(pass_grid(S));
     if (t16)
         hipLaunchKernelGGL(k_decode_pass_multi<true>, grid, dim3(256), 0, st, fd, sub_start, nf, S, pass);
     else
         hipLaunchKernelGGL(k_decode_pass_multi<false>, grid, dim3(256), 0, st, fd, sub_start, nf, S, pass);
 }
+void launch_decode_offsets_multi(const DecField* fd, const uint64_t* start, int nf, uint64_t nunits, uint64_t* off,
+                                 hipStream_t st) {
+    if (nunits)
+        hipLaunchKernelGGL(k_decode_sums_multi, dim3(grid_for(nunits, 4)), dim3(256), 0, st, fd, start, nf, off);
+    hipLaunchKernelGGL(k_decode_scan, dim3(1), dim3(1024), 0, st, off, nunits, (const uint32_t*)nullptr);
+}
 void launch_decode_write_multi(bool t16, uint32_t max_sub16, const DecField* fd, const uint64_t* start, int nf,
-                               uint64_t nunits, hipStream_t st) {
+                               uint64_t nunits, const uint64_t* off, hipStream_t st) {
     allow_big_lds(k_decode_write_multi<true>);
     allow_big_lds(k_decode_write_multi<false>);
     if (!nunits) return;
     DecodeArgs probe{};
     probe.n_sub16 = max_sub16;
-    const size_t lds = table_lds_bytes(probe, t16) + (size_t)kWriteStageLds * 4;
+    const size_t lds = table_lds_bytes(probe, t16) + (size_t)kWriteLdsWords * 4;
     if (t16)
-        hipLaunchKernelGGL(k_decode_write_multi<true>, dim3((unsigned)nunits), dim3(kSyncWg), lds, st, fd, start, nf);
+        hipLaunchKernelGGL(k_decode_write_multi<true>, dim3((unsigned)nunits), dim3(kWriteWg), lds, st, fd, start, nf, off);
     else
-        hipLaunchKernelGGL(k_decode_write_multi<false>, dim3((unsigned)nunits), dim3(kSyncWg), lds, st, fd, start, nf);
+        hipLaunchKernelGGL(k_decode_write_multi<false>, dim3((unsigned)nunits), dim3(kWriteWg), lds, st, fd, start, nf, off);
 }
-void launch_dec_field_totals(const DecField* fd, int nf, uint64_t* tot, hipStream_t st) {
-    if (nf > 0) hipLaunchKernelGGL(k_dec_field_totals, dim3(grid_for((uint64_t)nf, 256)), dim3(256), 0, st, fd, nf, tot);
+void launch_dec_field_totals(const uint64_t* start, int nf, const uint64_t* off, uint64_t* tot, hipStream_t st) {
+    if (nf > 0)
+        hipLaunchKernelGGL(k_dec_field_totals, dim3(grid_for((uint64_t)nf, 256)), dim3(256), 0, st, start, nf, off, tot);
 }
 int recon_kind_ndim(int kind) {
     switch (kind) {
