@@ -1,8 +1,8 @@
 // Pad values of the padding modes (src/utils/padding.hh; src/dualquant.hh:36-46,
 // :226-246, :553-573; src/vecsz_interface.hh:70-90, :287-298).
 //
-//   k_pad_blocks     one thread per block of the reference's block grid
-//                    ((d + B + 1) / B blocks per dimension, src/dimensions.hh:31):
+//   k_pad_blocks     the blocks of the reference's block grid ((d + B + 1) / B
+//                    blocks per dimension, src/dimensions.hh:31):
 //                    find_pad_value over the block (block mode) or over its
 //                    first row / column / planes (edge mode), in the
 //                    reference's loop order, then the block_pad / edge_pad
@@ -26,25 +26,29 @@ namespace {
 
 // find_max / find_min / find_avg (src/utils/padding.hh:65-119) as a running
 // fold in the reference's order: max / min keep the first value and replace
-// it by a strictly larger / smaller one; avg sums in float.
+// it by a strictly larger / smaller one; avg sums in float.  add(): the next
+// n values, `stride` apart.
 struct Find {
     int type;
-    float m, sum;
+    float m;
     bool first;
-    __device__ explicit Find(int t) : type(t), m(0.f), sum(0.f), first(true) {}
-    __device__ __forceinline__ void add(float v) {
-        if (first) {
-            m = v;
-            first = false;
+    __device__ explicit Find(int t) : type(t), m(0.f), first(true) {}
+    __device__ __forceinline__ void add(const float* v, uint32_t n, uint32_t stride) {
+        if (first && type != kPadAvg) m = v[0];
+        first = false;
+        if (type == kPadMax) {
+#pragma unroll 8
+            for (uint32_t s = 0; s < n; s++) m = (v[s * stride] > m) ? v[s * stride] : m;
+        } else if (type == kPadMin) {
+#pragma unroll 8
+            for (uint32_t s = 0; s < n; s++) m = (v[s * stride] < m) ? v[s * stride] : m;
+        } else {
+#pragma unroll 32
+            for (uint32_t s = 0; s < n; s++) m = m + v[s * stride];
         }
-        if (type == kPadMax) m = (v > m) ? v : m;
-        else if (type == kPadMin) m = (v < m) ? v : m;
-        else sum = sum + v;
     }
     __device__ __forceinline__ float result(uint64_t count, float constant) const {
-        if (type == kPadConst) return constant;
-        if (type == kPadAvg) return sum / (float)count;
-        return m;
+        return type == kPadConst ? constant : type == kPadAvg ? m / (float)count : m;
     }
 };
 
@@ -59,79 +63,94 @@ __device__ __forceinline__ double pad_rd(const PadArgs& a) { return a.ebd ? a.eb
 
 }  // namespace
 
-__global__ void __launch_bounds__(256) k_pad_blocks(PadArgs a, float* __restrict__ pad_out, float* __restrict__ halo) {
-    const uint64_t nb = a.hb0 * a.hb1 * a.hb2;
-    const uint64_t id = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
-    if (id >= nb) return;
-    const uint64_t b0 = id % a.hb0, b1 = (id / a.hb0) % a.hb1, b2 = id / (a.hb0 * a.hb1);
-    const uint64_t B = (uint64_t)a.B;
-    const uint64_t x0 = b0 * B, y0 = b1 * B, z0 = b2 * B;
+// One pad value is a fold over a sequence of L = B, B^2 or B^3 elements (a
+// power of two): the block's elements in block mode, and in edge mode
+// blockIdx.y picks one of
+//   2D (find_edge_pad_value, src/utils/padding.hh:145-206): the first row, the
+//      first column; halo (i == 0) ? row value : column value
+//   3D: the z = 0 plane (x fastest), the x = 0 plane (y fastest), the y = 0
+//      plane (x fastest); halo (k == 0) ? p0 : (j == 0) ? p1 : p2
+// avg adds in float, so a sequence's order is fixed and its fold is one
+// lane's chain.  What can be spread is the reading: a workgroup takes
+// kPadTile / S blocks and stages S = min(L, 256) elements of each per round
+// (x fastest: whole row pieces of B floats per load), the next round's loads
+// in flight while one lane per block folds this round's out of LDS.  A thread
+// that read its own block's elements waited for memory on each
+// (201 x 333 x 413, B 16, block avg: 1033 -> 74 us).
+constexpr uint32_t kPadTile = 4096;
+constexpr uint32_t kPadPer = kPadTile / 256;  // loads per thread and round
+constexpr uint32_t kPadLgMaxS = 8, kPadMaxS = 1u << kPadLgMaxS;
+
+__global__ void __launch_bounds__(256) k_pad_blocks(PadArgs a, uint32_t lb, uint32_t lS, uint64_t L, uint32_t nseq,
+                                                    float* __restrict__ pad_out, float* __restrict__ halo) {
+    __shared__ float tile[kPadTile + kPadMaxS];  // element s of block g at s * (G + 1) + g
+    const uint32_t B = 1u << lb, S = 1u << lS, G = kPadTile >> lS, t = threadIdx.x, face = blockIdx.y;
+    const uint64_t nb = a.hb0 * a.hb1 * a.hb2, id0 = (uint64_t)blockIdx.x * G;
     const uint64_t sy = a.d0, sz = a.d0 * a.d1;
-    auto val = [&](uint64_t i, uint64_t j, uint64_t k) -> float {
-        const uint64_t x = x0 + i, y = y0 + j, z = z0 + k;
-        return (x < a.d0 && y < a.d1 && z < a.d2) ? a.x[x + y * sy + z * sz] : 0.f;
-    };
-    const double rd = pad_rd(a);
-    const bool cst = a.type == kPadConst;
-    float hz, hy, hx;
-    if (a.ndim == 1) {
-        // 1D block and edge padding keep the raw value (src/dualquant.hh:37-42)
-        Find f(a.type);
-        if (!cst)
-            for (uint64_t i = 0; i < B; i++) f.add(val(i, 0, 0));
-        const float p = f.result(B, a.constant);
-        pad_out[id] = p;
-        hz = hy = hx = p;
-    } else if (a.mode == kPadBlock) {
-        Find f(a.type);
-        const uint64_t nz = a.ndim >= 3 ? B : 1;
-        if (!cst)
-            for (uint64_t k = 0; k < nz; k++)
-                for (uint64_t j = 0; j < B; j++)
-                    for (uint64_t i = 0; i < B; i++) f.add(val(i, j, k));
-        const float p = pad_q_block(f.result(B * B * nz, a.constant), rd);
-        pad_out[id] = p;
-        hz = hy = hx = p;
-    } else if (a.ndim == 2) {
-        // find_edge_pad_value (src/utils/padding.hh:145-206): the first row,
-        // then the first column; halo (i == 0) ? row value : column value
-        Find fr(a.type), fc(a.type);
-        if (!cst) {
-            for (uint64_t i = 0; i < B; i++) fr.add(val(i, 0, 0));
-            for (uint64_t j = 0; j < B; j++) fc.add(val(0, j, 0));
-        }
-        const float p0 = pad_q_block(fr.result(B, a.constant), rd);
-        const float p1 = pad_q_block(fc.result(B, a.constant), rd);
-        pad_out[2 * id] = p0;
-        pad_out[2 * id + 1] = p1;
-        hz = 0.f;
-        hx = p0;
-        hy = p1;
-    } else {
-        // 3D: the z = 0 plane (x fastest), the x = 0 plane (y fastest) and
-        // the y = 0 plane (x fastest); halo (k == 0) ? p0 : (j == 0) ? p1 : p2
-        Find f0(a.type), f1(a.type), f2(a.type);
-        if (!cst) {
-            for (uint64_t j = 0; j < B; j++)
-                for (uint64_t i = 0; i < B; i++) f0.add(val(i, j, 0));
-            for (uint64_t j = 0; j < B; j++)
-                for (uint64_t i = 0; i < B; i++) f1.add(val(0, i, j));
-            for (uint64_t j = 0; j < B; j++)
-                for (uint64_t i = 0; i < B; i++) f2.add(val(i, 0, j));
-        }
-        const float p0 = pad_q_block(f0.result(B * B, a.constant), rd);
-        const float p1 = pad_q_block(f1.result(B * B, a.constant), rd);
-        const float p2 = pad_q_block(f2.result(B * B, a.constant), rd);
-        pad_out[3 * id] = p0;
-        pad_out[3 * id + 1] = p1;
-        pad_out[3 * id + 2] = p2;
-        hz = p0;
-        hy = p1;
-        hx = p2;
+    // Element s of a sequence is (p0, p1, p2) in base B; a round's first s is a
+    // multiple of S, so its part of p1 and p2 is one for the workgroup and a
+    // thread's loads keep their own: an offset, and how many rows and planes
+    // from there the field has (0: a block that starts past the field).
+    // (A thread's loads are 256 apart and S divides 256, so they share s.)
+    const uint32_t s = t & (S - 1), p0 = s & (B - 1), p1 = s >> lb & (B - 1), p2 = s >> (2 * lb);
+    const bool edge = nseq > 1, yz = edge && face > 0;  // yz: p1 counts planes
+    uint64_t off[kPadPer];
+    uint32_t ny[kPadPer], nz[kPadPer];
+#pragma unroll
+    for (uint32_t m = 0; m < kPadPer; m++) {
+        uint32_t i = p0, j = p1, k = p2;
+        if (edge && face == 1) i = 0, j = p0, k = p1;
+        if (edge && face == 2) j = 0, k = p1;
+        const uint64_t id = id0 + ((t + 256 * m) >> lS);
+        const uint64_t x = id % a.hb0 * B + i, y = id / a.hb0 % a.hb1 * B + j, z = id / (a.hb0 * a.hb1) * B + k;
+        off[m] = x + y * sy + z * sz;
+        const bool in = id < nb && x < a.d0 && y < a.d1 && z < a.d2;
+        ny[m] = in ? (uint32_t)min<uint64_t>(a.d1 - y, B) : 0u;
+        nz[m] = in ? (uint32_t)min<uint64_t>(a.d2 - z, B) : 0u;
     }
-    halo[3 * id] = hz;
-    halo[3 * id + 1] = hy;
-    halo[3 * id + 2] = hx;
+    float v[kPadPer];
+    auto fetch = [&](uint64_t s0) {
+        const uint32_t r1 = (uint32_t)(s0 >> lb) & (B - 1), r2 = (uint32_t)(s0 >> (2 * lb));
+        const uint32_t yr = yz ? 0 : r1, zr = yz ? r1 : r2;
+        const float* src = a.x + yr * sy + zr * sz;
+#pragma unroll
+        for (uint32_t m = 0; m < kPadPer; m++) {
+            v[m] = 0.f;
+            if (yr < ny[m] && zr < nz[m]) v[m] = src[off[m]];
+        }
+    };
+    // a thread folds block t, and block t + 256 where there are as many
+    Find f0(a.type), f1(a.type);
+    if (a.type != kPadConst) {
+        fetch(0);
+        for (uint64_t s0 = 0; s0 < L; s0 += S) {
+            lds_sync();
+#pragma unroll
+            for (uint32_t m = 0; m < kPadPer; m++) {
+                tile[s * (G + 1) + ((t + 256 * m) >> lS)] = v[m];
+            }
+            lds_sync();
+            if (s0 + S < L) fetch(s0 + S);
+            if (t < G) f0.add(tile + t, S, G + 1);
+            if (t + 256 < G) f1.add(tile + t + 256, S, G + 1);
+        }
+    }
+    const double rd = pad_rd(a);
+    for (uint32_t g = t; g < G; g += 256) {
+        const uint64_t id = id0 + g;
+        if (id >= nb) break;
+        float p = (g == t ? f0 : f1).result(L, a.constant);
+        if (a.ndim > 1) p = pad_q_block(p, rd);  // (1D keeps the raw value, src/dualquant.hh:37-42)
+        pad_out[nseq * id + face] = p;
+        if (nseq == 1) {
+            halo[3 * id] = halo[3 * id + 1] = halo[3 * id + 2] = p;
+        } else if (nseq == 2) {
+            halo[3 * id + (face == 0 ? 2 : 1)] = p;
+            if (face == 0) halo[3 * id] = 0.f;
+        } else {
+            halo[3 * id + face] = p;
+        }
+    }
 }
 
 // scratch: [0] ordered max, [1] ordered min (u32), [2..3] first zero index (u64)
@@ -281,7 +300,14 @@ __global__ void __launch_bounds__(256) k_pad_halo(int ndim, int mode, const floa
 
 void launch_pad_blocks(const PadArgs& a, float* pad_out, float* halo, hipStream_t st) {
     const uint64_t nb = a.hb0 * a.hb1 * a.hb2;
-    hipLaunchKernelGGL(k_pad_blocks, dim3((unsigned)((nb + 255) / 256)), dim3(256), 0, st, a, pad_out, halo);
+    const uint32_t nseq = a.mode == kPadEdge && a.ndim > 1 ? (uint32_t)a.ndim : 1u;
+    const uint32_t lb = (uint32_t)__builtin_ctz((unsigned)a.B);
+    // block mode: B^ndim elements; edge mode: B^(ndim - 1) (1D: as block mode)
+    const uint32_t lL = lb * (uint32_t)(nseq == 1 ? a.ndim : a.ndim - 1);
+    const uint32_t lS = std::min(lL, kPadLgMaxS);
+    const uint64_t G = kPadTile >> lS;
+    hipLaunchKernelGGL(k_pad_blocks, dim3((unsigned)((nb + G - 1) / G), nseq), dim3(256), 0, st, a, lb, lS, 1ull << lL,
+                       nseq, pad_out, halo);
 }
 
 void launch_pad_global(const PadArgs& a, void* scratch, float* pad_out, float* halo, hipStream_t st) {
