@@ -629,6 +629,8 @@ int compress_run(vecsz_ctx* c, const vecsz_params* p, const float* d_in, uint8_t
     }
     const bool x4 = pmode == VECSZ_PAD_NONE && dualquant_use_x4(ndim, B, d_in, d0, d1, d2, false);
     const uint64_t tiles_x = x4 ? (d0 + 255) / 256 : a.ntiles_x;
+    a.zs = dualquant_planes(ndim, B, tiles_x * a.ntiles_y * a.ntiles_z);
+    if (ndim >= 3) a.ntiles_z = (d2 + a.zs - 1) / a.zs;
     const uint64_t work = ndim == 1 ? ((n + 7) / 8 + 63) / 64 : tiles_x * a.ntiles_y * a.ntiles_z;
     const int grid_cap = NA ? std::min(c->dq_grid, kNaDqGrid) : c->dq_grid;
     const int grid = (int)std::max<uint64_t>(1, std::min<uint64_t>((work + 3) / 4, (uint64_t)grid_cap));
@@ -1567,6 +1569,12 @@ static int compress_batch_fused_run(vecsz_ctx* c, int nf, const vecsz_params* p,
     uint64_t* dqk = rg0 + 2 * (nf + 1);  // dqk + kind * (nf + 1) for each DqKind
     std::vector<char> dev_range(nf, 0);
     BatchField* fdd = c->b_desc.as<BatchField>();
+    uint64_t tiles3 = 0;  // 3D tiles of whole blocks
+    for (int k = 0; k < nf; k++) {
+        const uint64_t *d = p[k].dims, w = dualquant_use_x4(3, B, d_in[k], d[0], d[1], d[2], true) ? 256 : 64;
+        if (p[k].ndim == 3) tiles3 += (d[0] + w - 1) / w * ((d[1] + B - 1) / B) * ((d[2] + B - 1) / B);
+    }
+    const int zs = dualquant_planes(3, B, tiles3);
     for (int k = 0; k < nf; k++) {
         const vecsz_params& q = p[k];
         const int ndim = q.ndim;
@@ -1593,7 +1601,8 @@ static int compress_batch_fused_run(vecsz_ctx* c, int nf, const vecsz_params* p,
         const bool x4 = dualquant_use_x4(ndim, B, d_in[k], d0, d1, d2, true);
         a.ntiles_x = x4 ? (d0 + 255) / 256 : (d0 + 63) / 64;
         a.ntiles_y = ndim >= 2 ? (d1 + B - 1) / B : 1;
-        a.ntiles_z = ndim >= 3 ? (d2 + B - 1) / B : 1;
+        a.zs = zs;
+        a.ntiles_z = ndim >= 3 ? (d2 + zs - 1) / zs : 1;
         if (dev_range[k]) {
             f.range = c->b_range.as<uint32_t>() + 2 * k;
             f.ebd = c->b_ebd.as<EbDev>() + k;

@@ -42,6 +42,7 @@ struct DQArgs {
     int reverse;           // visit tiles last-to-first (reuses what a preceding pass left in cache)
     const EbDev* ebd;      // when set, r_f / r_d come from here (r2r range computed on the device)
     uint64_t ntiles_x, ntiles_y, ntiles_z;
+    int zs;                // 3D: planes of a tile (divides the block size; dq_planes)
     // Padding: halo values {z face, y face, x face} of block (bx, by, bz) at
     // halo + halo_stride * (bx + hb0 * (by + hb1 * bz)), blocks counted on the
     // reference's grid ((d + B + 1) / B per dimension); halo_stride 0 = one

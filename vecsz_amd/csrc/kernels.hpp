@@ -24,6 +24,8 @@ void launch_dualquant(int ndim, int B, const float* in, uint16_t* codes, float* 
 // A single field takes the element-load form only when it has enough
 // 4-wide tiles to fill the chip; a batch (tiles of many fields) always does.
 bool dualquant_use_x4(int ndim, int B, const float* in, uint64_t d0, uint64_t d1, uint64_t d2, bool batched);
+// Planes of a 3D tile (DQArgs::zs) where whole blocks would make `tiles` tiles.
+int dualquant_planes(int ndim, int B, uint64_t tiles);
 bool dualquant_x4_aligned(const float* in, uint64_t d0);
 // grid_cap: most workgroups of a launch (a tuned launch shape; the output
 // does not depend on it).

@@ -300,6 +300,26 @@ __device__ __forceinline__ Halo load_halo(const DQArgs& a, bool xin, uint64_t x,
     return h;
 }
 
+// Rows of a tile, kRowsAhead at a time, the next ones' loads in flight while
+// these are processed: a wavefront that loaded each row as it came to it
+// waited for memory on every row, and a small or mid-sized field has too few
+// wavefronts to hide that (201 x 333 x 413, B 16, padded: 182 -> 84 us;
+// 25 x 25 x 26: 32 -> 27 us).
+constexpr int kRowsAhead = 8;
+template <class T>
+struct RowsAhead {
+    T cur[kRowsAhead], next[kRowsAhead];
+    __device__ __forceinline__ void take() {
+#pragma unroll
+        for (int r = 0; r < kRowsAhead; r++) cur[r] = next[r];
+    }
+    template <class F>
+    __device__ __forceinline__ void ahead(const F& load) {
+#pragma unroll
+        for (int r = 0; r < kRowsAhead; r++) next[r] = load(r);
+    }
+};
+
 // PAD: the halo cells hold pad values instead of +0.0 (src/dualquant.hh:
 // 226-246, :553-573): a neighbour across the block's z face reads h.z, else
 // across its y face h.y, else h.x (src/utils/padding.hh:245, :290).
@@ -313,29 +333,50 @@ __device__ __forceinline__ void dq3_tile(const float* __restrict__ in, uint16_t*
         const uint64_t ty = (t / a.ntiles_x) % a.ntiles_y;
         const uint64_t tz = t / (a.ntiles_x * a.ntiles_y);
         const uint64_t x = tx * 64 + lane;
-        const uint64_t y0 = ty * B, z0 = tz * B;
+        const uint64_t y0 = ty * B, z0 = tz * a.zs;
+        const int zb = (int)(z0 % B);  // the tile's first plane in its block
         const bool xin = x < a.d0;
         const bool scal = x >= a.x8;  // partial x-group: scalar path
         const bool xstart = (x % B) == 0;
         const float thr = scal ? a.thr_scalar : a.thr_vec;
         Halo h{0.f, 0.f, 0.f};
-        if constexpr (PAD) h = load_halo(a, xin, x, B, ty, tz);
+        if constexpr (PAD) h = load_halo(a, xin, x, B, ty, z0 / B);
+        const int nz = (int)min<uint64_t>(a.zs, a.d2 - z0);
+        RowsAhead<float> rows;
+        auto load = [&](int zz, int yy) -> float {
+            return xin && zz < nz && y0 + yy < a.d1 ? __builtin_nontemporal_load(&in[x + (y0 + yy) * sy + (z0 + zz) * sz]) : 0.f;
+        };
         float prevplane[B];
 #pragma unroll
         for (int j = 0; j < B; j++) prevplane[j] = 0.f;
-        for (int zz = 0; zz < B; zz++) {
-            const uint64_t z = z0 + zz;
-            if (z >= a.d2) break;
+        if (zb > 0) {  // the plane before the tile is the block's too
+#pragma unroll
+            for (int j = 0; j < B; j++) prevplane[j] = load(-1, j);
+        }
+        rows.ahead([&](int r) { return load(0, r); });
+        if (zb > 0) {
+#pragma unroll
+            for (int j = 0; j < B; j++)
+                prevplane[j] = scal ? prequant_scalar(prevplane[j], a.r_d) : prequant_vec(prevplane[j], a.r_f);
+        }
+        for (int zi = 0; zi < nz; zi++) {
+            const uint64_t z = z0 + zi;
+            const int zz = zb + zi;            // the plane in its block
             float qrow = 0.f, xrow = 0.f;      // q and X of row y-1 (this plane)
             float zrow = 0.f, xzrow = 0.f;     // Z and XZ of row y-1
             const float hyz = zz > 0 ? h.y : h.z;  // the y-face halo of this plane's first row
 #pragma unroll
             for (int yy = 0; yy < B; yy++) {
                 const uint64_t y = y0 + yy;
+                if (yy % kRowsAhead == 0) {
+                    rows.take();
+                    const int ny = yy + kRowsAhead < B ? yy + kRowsAhead : 0;
+                    rows.ahead([&](int r) { return load(ny ? zi : zi + 1, ny + r); });
+                }
                 if (y < a.d1) {
                     const uint64_t idx = x + y * sy + z * sz;
                     const bool ok = xin;
-                    float v = ok ? __builtin_nontemporal_load(&in[idx]) : 0.f;
+                    const float v = rows.cur[yy % kRowsAhead];
                     float q = scal ? prequant_scalar(v, a.r_d) : prequant_vec(v, a.r_f);
                     float X = wave_shr1(q);
                     float Z = zz > 0 ? prevplane[yy] : h.z;
@@ -418,12 +459,21 @@ __device__ __forceinline__ void dq2_tile(const float* __restrict__ in, uint16_t*
         Halo h{0.f, 0.f, 0.f};
         if constexpr (PAD) h = load_halo(a, xin, x, B, ty, 0);
         float qrow = 0.f, xrow = 0.f;
+        RowsAhead<float> rows;
+        auto load = [&](int yy) -> float {
+            return xin && yy < B && y0 + yy < a.d1 ? __builtin_nontemporal_load(&in[x + (y0 + yy) * a.d0]) : 0.f;
+        };
+        rows.ahead([&](int r) { return load(r); });
 #pragma unroll
         for (int yy = 0; yy < B; yy++) {
             const uint64_t y = y0 + yy;
+            if (yy % kRowsAhead == 0) {
+                rows.take();
+                rows.ahead([&](int r) { return load(yy + kRowsAhead + r); });
+            }
             if (y < a.d1) {
                 const uint64_t idx = x + y * a.d0;
-                float v = xin ? __builtin_nontemporal_load(&in[idx]) : 0.f;
+                const float v = rows.cur[yy % kRowsAhead];
                 float q = prequant_vec(v, a.r_f);
                 float W = wave_shr1(q);
                 if (xstart) W = h.x;
@@ -534,24 +584,36 @@ __device__ __forceinline__ void dq3_x4_tile(const float* __restrict__ in, uint16
     const bool xstart = (x % B) == 0;
     const float thr = scal ? a.thr_scalar : a.thr_vec;
     const int ny = (int)min((uint64_t)B, a.d1 - y0);
-    const int nz = (int)min((uint64_t)B, a.d2 - z0);
+    const int nz = (int)min((uint64_t)a.zs, a.d2 - z0);
+    const int zb = (int)(z0 % B);  // the tile's first plane in its block
     float pp[B][4];
 #pragma unroll
-    for (int j = 0; j < B; j++)
-#pragma unroll
-        for (int k = 0; k < 4; k++) pp[j][k] = 0.f;
+    for (int j = 0; j < B; j++) {
+        // the plane before the tile where it is the block's too
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (zb > 0 && xin && j < ny) v = load_x4<ALN>(in + x + (y0 + j) * sy + (z0 - 1) * sz, nv);
+        pp[j][0] = v.x, pp[j][1] = v.y, pp[j][2] = v.z, pp[j][3] = v.w;
+    }
     // rows of the next plane are loaded while the current one is processed
     float4 vnext[B];
 #pragma unroll
     for (int yy = 0; yy < B; yy++)
         vnext[yy] = (xin && yy < ny) ? load_x4<ALN>(in + x + (y0 + yy) * sy + z0 * sz, nv)
                                      : make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int zz = 0; zz < nz; zz++) {
-        const uint64_t z = z0 + zz;
+    if (zb > 0) {
+#pragma unroll
+        for (int j = 0; j < B; j++)
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+                pp[j][k] = (SCAL && scal) ? prequant_scalar(pp[j][k], a.r_d) : prequant_vec(pp[j][k], a.r_f);
+    }
+    for (int zi = 0; zi < nz; zi++) {
+        const uint64_t z = z0 + zi;
+        const int zz = zb + zi;  // the plane in its block
         float4 vrow[B];
 #pragma unroll
         for (int yy = 0; yy < B; yy++) vrow[yy] = vnext[yy];
-        if (zz + 1 < nz) {
+        if (zi + 1 < nz) {
 #pragma unroll
             for (int yy = 0; yy < B; yy++)
                 vnext[yy] = (xin && yy < ny) ? load_x4<ALN>(in + x + (y0 + yy) * sy + (z + 1) * sz, nv)
@@ -635,9 +697,9 @@ __device__ __forceinline__ void dq3_x4_at(const float* __restrict__ in, uint16_t
     const uint64_t x = tx * 256 + 4 * lane;
     // the partial x-group only exists in the last tile column
     if (tx * 256 + 256 > a.x8 && a.x8 < a.d0)
-        dq3_x4_tile<B, true, ALN>(in, codes, sparse, H, a, x, ty * B, tz * B);
+        dq3_x4_tile<B, true, ALN>(in, codes, sparse, H, a, x, ty * B, tz * a.zs);
     else
-        dq3_x4_tile<B, false, ALN>(in, codes, sparse, H, a, x, ty * B, tz * B);
+        dq3_x4_tile<B, false, ALN>(in, codes, sparse, H, a, x, ty * B, tz * a.zs);
 }
 
 template <int B, bool ALN, bool COLD>
@@ -678,11 +740,22 @@ __device__ __forceinline__ void dq2_x4_tile(const float* __restrict__ in, uint16
         const bool lost = x >= a.x8;
         const bool xstart = (x % B) == 0;
         float qr[4] = {0.f, 0.f, 0.f, 0.f}, xr[4] = {0.f, 0.f, 0.f, 0.f};
-        for (int yy = 0; yy < B; yy++) {
+        RowsAhead<float4> rows;
+        auto load = [&](int yy) -> float4 {
+            return xin && yy < B && y0 + yy < a.d1 ? load_x4<ALN, true>(in + x + (y0 + yy) * a.d0, nv)
+                                                   : make_float4(0.f, 0.f, 0.f, 0.f);
+        };
+        rows.ahead([&](int r) { return load(r); });
+        for (int y8 = 0; y8 < B && y0 + y8 < a.d1; y8 += kRowsAhead) {
+            rows.take();
+            rows.ahead([&](int r) { return load(y8 + kRowsAhead + r); });
+#pragma unroll
+            for (int r = 0; r < kRowsAhead; r++) {
+            const int yy = y8 + r;
             const uint64_t y = y0 + yy;
             if (y >= a.d1) break;
             const uint64_t idx = x + y * a.d0;
-            float4 v = xin ? load_x4<ALN, true>(in + idx, nv) : make_float4(0.f, 0.f, 0.f, 0.f);
+            const float4 v = rows.cur[r];
             float q[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
             for (int k = 0; k < 4; k++) q[k] = prequant_vec(q[k], a.r_f);
@@ -715,6 +788,7 @@ __device__ __forceinline__ void dq2_x4_tile(const float* __restrict__ in, uint16
             for (int k = 0; k < 4; k++) {
                 qr[k] = q[k];
                 xr[k] = W[k];
+            }
             }
         }
     }
@@ -2011,6 +2085,19 @@ bool dualquant_use_x4(int ndim, int B, const float* in, uint64_t d0, uint64_t d1
     return tiles >= 2048;
 }
 
+// A wavefront walks its tile plane by plane, so a field of few tiles leaves
+// most of the chip idle for B planes' worth of latency.  A tile may stop
+// inside its blocks: the next one then reads the plane before it again (the
+// prediction needs prequantized input only, nothing the other tile computed).
+// Tiles are halved while there are fewer than 16 per CU, down to two planes
+// (three read): 25 x 25 x 26 ran 27 us on 16 tiles of 8 planes, 18 us on 64
+// of 2; 201 x 333 x 413 with B 16 84 us on 1,911 of 16, 73 us on 3,675 of 8.
+int dualquant_planes(int ndim, int B, uint64_t tiles) {
+    int zs = B;
+    if (ndim == 3)
+        for (; zs > 2 && tiles < 4096; tiles *= 2) zs /= 2;
+    return zs;
+}
 
 void launch_dualquant(int ndim, int B, const float* in, uint16_t* codes, float* sparse, unsigned long long* hist,
                       uint32_t* partials, const DQArgs& a0, int grid, hipStream_t st) {
