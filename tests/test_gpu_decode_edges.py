@@ -78,3 +78,63 @@ def test_many_long_codewords(gpu_ctx, common):
     counts = [1 + i % 3 for i in range(3900)]
     counts[1950 - common // 2: 1950 + common // 2] = [4000] * common
     _check(gpu_ctx, _field(counts, seed=common))
+
+
+def _sections(a):
+    """(archive bytes, offset of the Huffman section, its size, outlier count)."""
+    nd = int(np.frombuffer(a[:4], np.int32)[0])
+    pad, huff, nout = (int(v) for v in np.frombuffer(a[4 * nd + 12: 4 * nd + 36], np.uint64))
+    return 4 * nd + 36 + 4 * pad, huff, nout
+
+
+def _renumbered(a, seed):
+    """The archive with its tree's nodes (but the root) in another order."""
+    h, huff, _ = _sections(a)
+    nc = int.from_bytes(a[h: h + 4], "big")
+    w = 1 if nc <= 256 else 2
+    ty = np.uint8 if w == 1 else np.uint16
+    t = h + 9
+    left, right = (np.frombuffer(a[t + i * nc * w: t + (i + 1) * nc * w], ty).astype(np.int64) for i in (0, 1))
+    sym = np.frombuffer(a[t + 2 * nc * w: t + 2 * nc * w + 4 * nc], np.uint32)
+    leaf = np.frombuffer(a[t + 2 * nc * w + 4 * nc: t + 2 * nc * w + 5 * nc], np.uint8)
+    to = np.concatenate([[0], 1 + np.random.default_rng(seed).permutation(nc - 1)])
+    out = [np.empty(nc, ty), np.empty(nc, ty), np.empty(nc, np.uint32), np.empty(nc, np.uint8)]
+    out[0][to] = np.where(left > 0, to[left], 0)
+    out[1][to] = np.where(right > 0, to[right], 0)
+    out[2][to], out[3][to] = sym, leaf
+    return a[:t] + b"".join(o.tobytes() for o in out) + a[t + nc * (2 * w + 5):]
+
+
+# trees whose nodes are not numbered parents first: the host builds their
+# tables (the device leaves them), alone, with an index and in a batch
+@pytest.mark.parametrize("nsym", [40, 900])
+def test_other_node_orders(gpu_ctx, nsym):
+    counts = [1 + (i * i) % 37 for i in range(nsym)]
+    x = _field(counts, seed=nsym)
+    xt = torch.from_numpy(x).cuda()
+    a, _, idx = gpu_ctx.compress_indexed(xt, 0.5, "abs")
+    ref = gpu_ctx.decompress(a, "abs")
+    b = torch.from_numpy(np.frombuffer(_renumbered(a.cpu().numpy().tobytes(), nsym), np.uint8).copy()).cuda()
+    assert not torch.equal(a, b)
+    for y in [gpu_ctx.decompress(b, "abs"), gpu_ctx.decompress(b, "abs", index=idx),
+              *gpu_ctx.decompress_batch([a, b, a], "abs")]:
+        assert torch.equal(y.view(torch.int32), ref.view(torch.int32))
+
+
+# a stream that is a byte short is refused, also where the codewords that a
+# table entry holds at once would reach past its end
+@pytest.mark.parametrize("tail", [0, 5, 64, 600])
+def test_short_stream(gpu_ctx, tail):
+    from vecsz_amd import VecszError
+
+    x = np.concatenate([_field([3] * 64 + [2000], seed=tail), np.zeros(tail, np.float32)])
+    a, _ = gpu_ctx.compress(torch.from_numpy(x).cuda(), 0.5, "abs")
+    raw = a.cpu().numpy().tobytes()
+    h, huff, nout = _sections(raw)
+    nd = int(np.frombuffer(raw[:4], np.int32)[0])
+    cut = raw[: 4 * nd + 20] + np.uint64(huff - 1).tobytes() + raw[4 * nd + 28: h + huff - 1] + raw[h + huff:]
+    c = torch.from_numpy(np.frombuffer(cut, np.uint8).copy()).cuda()
+    with pytest.raises(VecszError):
+        gpu_ctx.decompress(c, "abs")
+    with pytest.raises(VecszError):
+        gpu_ctx.decompress_batch([a, c], "abs")

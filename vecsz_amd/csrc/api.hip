@@ -7,8 +7,8 @@
 //   header + tree H2D -> k_chunk_bits -> chunk scan -> k_enc_summary -> k_pack
 //   Batches: the same stages once for all fields (k_*_multi launches).
 // Decompress (vecsz::interface::Decompress, src/vecsz_interface.hh:232-375):
-//   header + tree D2H -> decode tables -> k_decode_sync -> k_decode_pass
-//   (re-decode of listed subsequences, until no list remains) -> scan
+//   header D2H -> k_decode_tables -> k_decode_sync -> k_decode_pass
+//   (re-decode of listed subsequences, until no list remains) -> offsets
 //   -> k_decode_write -> k_recon_* [-> fallback]
 #include <hip/hip_runtime.h>
 
@@ -143,10 +143,9 @@ struct vecsz_ctx {
     GraphSlot b_graph[2];
     // fused batch decompress: field descriptors, unit starts, head copies,
     // gathered heads, summaries, symbol totals, fallback counts; pinned
-    // staging of the same; decode tables per field
-    DevBuf db_desc, db_start, db_hc, db_heads, db_sums, db_tot, db_nfl;
+    // staging of the same
+    DevBuf db_desc, db_start, db_hc, db_heads, db_sums, db_tot, db_nfl, db_meta, db_jobs;
     HostBuf db_pin, db_hpin, db_back;
-    std::vector<DecodeTables> db_dt;
     Codebook cb;
     DecodeTables dt;  // kept between calls: its vectors keep their capacity
     // metadata of the last successful compress
@@ -405,10 +404,12 @@ CScratch small_scratch(CScratch s, uint8_t* block, int dict) {
 }
 
 // The small state of a single-field decompress in one block: [decoder
-// summary | the re-decode list counters].
+// summary | state of the device-built tables | the re-decode list counters].
+constexpr size_t kDecSmallTables = 64;
 constexpr size_t kDecSmallLists = 128;
 constexpr size_t kDecSmallBytes = kDecSmallLists + kListCountBytes;
-static_assert(sizeof(DecSummary) <= kDecSmallLists, "decoder summary fits its slot");
+static_assert(sizeof(DecSummary) <= kDecSmallTables && kDecSmallTables + sizeof(TableMeta) <= kDecSmallLists,
+              "the slots hold their structs");
 
 // Whether the list pass `pass` reads holds entries (counters: the host's copy).
 bool any_listed(const uint8_t* counters, uint32_t pass) {
@@ -899,6 +900,12 @@ int parse_meta(const uint8_t* h, uint64_t avail, uint64_t total, int* ndim, uint
     return VECSZ_OK;
 }
 
+// Trees whose decode tables the device builds (k_decode_tables): more than
+// one symbol, and the compact tables' limits.
+bool device_tables_ok(uint32_t nodes, int dict_size) {
+    return nodes > 1 && nodes <= kMaxTreeNodes && dict_size <= kMaxLdsBook;
+}
+
 bool tree_is_full(const DecodeTables& dt) {
     // every internal node reachable from the root has both children
     std::vector<uint32_t> stk{0};
@@ -920,16 +927,19 @@ bool tree_is_full(const DecodeTables& dt) {
 // d_index (nullable): a decode index written by compress_device for this
 // archive (index_words words); the decode then starts every segment at its
 // first codeword instead of synchronising.
+// host_tables: the device could not build this archive's tables.
 int decompress_device(vecsz_ctx* c, const vecsz_params* p, const uint8_t* d_in, uint64_t in_bytes, float* d_out,
-                      uint64_t out_cap, const uint64_t* d_index = nullptr, uint64_t index_words = 0) {
+                      uint64_t out_cap, const uint64_t* d_index = nullptr, uint64_t index_words = 0,
+                      bool host_tables = false) {
     int rc = check_params(c, p, false);
     if (rc) return rc;
     HIPCHK(c, hipSetDevice(c->device));
     timing_begin(c);
-    // One round trip for the metadata, the Huffman header and (for trees of
-    // up to ~14,000 nodes) the tree itself; a larger tree takes a second copy.
-    constexpr uint64_t kHeadRead = 1 << 17;
-    if (!c->pin.ensure(kHeadRead + 64)) return fail(c, VECSZ_ENOMEM, "pinned buffer");
+    // One round trip for the metadata and the Huffman header; where the host
+    // builds the tables, a second copy brings the tree.
+    constexpr uint64_t kHeadRead = 256;
+    if (!c->pin.ensure(std::max<uint64_t>(kHeadRead + 64, kDecSmallBytes + 64)))
+        return fail(c, VECSZ_ENOMEM, "pinned buffer");
     uint8_t* h = c->pin.as<uint8_t>();
     const uint64_t head_avail = std::min<uint64_t>(in_bytes, kHeadRead);
     HIPCHK(c, hipMemcpyAsync(h, d_in, head_avail, hipMemcpyDeviceToHost, c->stream));
@@ -956,9 +966,11 @@ int decompress_device(vecsz_ctx* c, const vecsz_params* p, const uint8_t* d_in, 
     const uint8_t* d_huff = d_in + mb + 4 * pad_len;
     if (huff_size < 8) return fail(c, VECSZ_ECORRUPT, "Huffman section too short");
     DecodeTables& dt = c->dt;
+    dt.root_leaf = false;
     uint64_t tb = 0;
+    uint32_t nodes = 0;
+    bool t16 = false;  // compact tables, built on the device
     {
-        HostTimer ht(c, "host_tables");
         const uint64_t hoff = mb + 4 * pad_len;
         const uint8_t* hp = h + hoff;
         if (hoff + 8 > head_avail) {
@@ -970,17 +982,19 @@ int decompress_device(vecsz_ctx* c, const vecsz_params* p, const uint8_t* d_in, 
         }
         int32_t ncs = (int32_t)(((uint32_t)hp[0] << 24) | ((uint32_t)hp[1] << 16) | ((uint32_t)hp[2] << 8) | hp[3]);
         if (ncs <= 0) return fail(c, VECSZ_ECORRUPT, "Huffman node count");
-        tb = tree_byte_size((uint64_t)ncs);
+        nodes = (uint32_t)ncs;
+        tb = tree_byte_size(nodes);
         if (8 + tb > huff_size) return fail(c, VECSZ_ECORRUPT, "Huffman tree truncated");
-        if (hoff + 8 + tb > head_avail) {
+        t16 = !host_tables && device_tables_ok(nodes, p->dict_size);
+        if (!t16) {
+            HostTimer ht(c, "host_tables");
             if (!c->pin2.ensure(8 + tb)) return fail(c, VECSZ_ENOMEM, "pinned buffer");
-            hp = c->pin2.as<uint8_t>();
             HIPCHK(c, hipMemcpyAsync(c->pin2.p, d_huff, 8 + tb, hipMemcpyDeviceToHost, c->stream));
             HIPCHK(c, hipStreamSynchronize(c->stream));
+            rc = build_decode_tables(c->pin2.as<uint8_t>(), huff_size, dt);
+            if (rc) return fail(c, rc, "Huffman tree is corrupt");
+            if (!dt.root_leaf && !tree_is_full(dt)) return fail(c, VECSZ_ECORRUPT, "Huffman tree is not full");
         }
-        rc = build_decode_tables(hp, huff_size, dt);
-        if (rc) return fail(c, rc, "Huffman tree is corrupt");
-        if (!dt.root_leaf && !tree_is_full(dt)) return fail(c, VECSZ_ECORRUPT, "Huffman tree is not full");
     }
 
     if (!c->codes.ensure(n * 2 + 64) || !c->sparse.ensure(n * 4 + 64))
@@ -1063,41 +1077,44 @@ int decompress_device(vecsz_ctx* c, const vecsz_params* p, const uint8_t* d_in, 
         const uint64_t nsub = std::max<uint64_t>(1, (T + kSubBits - 1) / kSubBits);
         const uint64_t nunits = decode_write_units(nsub);
         SubState ss{};  // jbase 0: list entries are this field's subsequence numbers
-        list_stripes(decode_sync_units(nsub), &ss.nstripe, &ss.stripe_cap);
+        list_stripes(decode_sync_units(nsub), &ss);
         const uint64_t list_cap = ss.nstripe * ss.stripe_cap;
         if (!c->sub_b.ensure(nsub) || !c->sub_e.ensure(nsub) || !c->sub_cz.ensure(nsub * 4) ||
             !c->sub_list.ensure(list_cap * 16) || !c->unit_off.ensure((nunits + 1) * 16) ||
             !c->dec_small.ensure(kDecSmallBytes))
             return fail(c, VECSZ_ENOMEM, "device scratch allocation failed");
-        // Decode tables in one pinned staging copy: the compact form when the
-        // symbols fit 12 bits (the kernels keep its deeper tables in LDS when
-        // they fit beside the first-level table, else read them in global
-        // memory), else 32-bit.
-        const bool t16 = !dt.lut16.empty();
-        const size_t tab_bytes = t16 ? (dt.lut16.size() + dt.sub16.size()) * 2 : (dt.lut.size() + dt.sub.size()) * 4;
-        if (!c->tabs.ensure(tab_bytes + 16) || !c->pin_tab.ensure(tab_bytes + 16))
-            return fail(c, VECSZ_ENOMEM, "decode table allocation failed");
-        // (the previous call's copy out of pin_tab finished before that call's
-        // mid-call synchronisation)
-        uint8_t* tp = c->pin_tab.as<uint8_t>();
-        if (t16) {
-            memcpy(tp, dt.lut16.data(), dt.lut16.size() * 2);
-            memcpy(tp + dt.lut16.size() * 2, dt.sub16.data(), dt.sub16.size() * 2);
-        } else {
-            memcpy(tp, dt.lut.data(), dt.lut.size() * 4);
-            memcpy(tp + dt.lut.size() * 4, dt.sub.data(), dt.sub.size() * 4);
-        }
-        HIPCHK(c, hipMemcpyAsync(c->tabs.p, tp, tab_bytes, hipMemcpyHostToDevice, c->stream));
-        HIPCHK(c, hipMemsetAsync(c->dec_small.p, 0, kDecSmallBytes, c->stream));
         DecodeArgs da;
         da.stream = d_stream;
         da.stream_bits = T;
         da.n = n;
-        da.lut = t16 ? nullptr : c->tabs.as<uint32_t>();
-        da.sub = t16 ? nullptr : c->tabs.as<uint32_t>() + dt.lut.size();
-        da.lut16 = t16 ? c->tabs.as<uint16_t>() : nullptr;
-        da.sub16 = t16 ? c->tabs.as<uint16_t>() + dt.lut16.size() : nullptr;
-        da.n_sub16 = t16 ? (uint32_t)std::min<size_t>(dt.sub16.size(), kMaxSub16) : 0;
+        da.lut = da.sub = nullptr;
+        da.tabs = nullptr;
+        da.meta = nullptr;
+        da.n_sub16 = 0;
+        HIPCHK(c, hipMemsetAsync(c->dec_small.p, 0, kDecSmallBytes, c->stream));
+        if (t16) {
+            const uint32_t cap = std::min<uint32_t>(kMaxSubTabs, nodes / 2);
+            if (!c->tabs.ensure(table_words(cap) * 2)) return fail(c, VECSZ_ENOMEM, "decode table allocation failed");
+            da.tabs = c->tabs.as<uint16_t>();
+            da.meta = reinterpret_cast<const TableMeta*>(c->dec_small.as<uint8_t>() + kDecSmallTables);
+            StageScope s(c, "decode_tables");
+            launch_decode_tables({d_huff, nodes, cap, c->tabs.as<uint16_t>(), const_cast<TableMeta*>(da.meta),
+                                  reinterpret_cast<uint32_t*>(c->dec_small.as<uint8_t>() + kDecSmallLists)},
+                                 c->stream);
+        } else {
+            // host-built tables, through one pinned staging copy (the previous
+            // call's copy out of pin_tab finished before that call's mid-call
+            // synchronisation)
+            const size_t tab_bytes = (dt.lut.size() + dt.sub.size()) * 4;
+            if (!c->tabs.ensure(tab_bytes + 16) || !c->pin_tab.ensure(tab_bytes + 16))
+                return fail(c, VECSZ_ENOMEM, "decode table allocation failed");
+            uint8_t* tp = c->pin_tab.as<uint8_t>();
+            memcpy(tp, dt.lut.data(), dt.lut.size() * 4);
+            memcpy(tp + dt.lut.size() * 4, dt.sub.data(), dt.sub.size() * 4);
+            HIPCHK(c, hipMemcpyAsync(c->tabs.p, tp, tab_bytes, hipMemcpyHostToDevice, c->stream));
+            da.lut = c->tabs.as<uint32_t>();
+            da.sub = da.lut + dt.lut.size();
+        }
         da.nsub = nsub;
         da.outliers = d_outl;
         da.n_outlier = nout;
@@ -1152,6 +1169,7 @@ int decompress_device(vecsz_ctx* c, const vecsz_params* p, const uint8_t* d_in, 
         HIPCHK(c, hipGetLastError());
         DecSummary ds;
         uint64_t tot;
+        TableMeta tm;
         bool left = false;
         auto check = [&]() -> int {  // summary, the pending list count and the symbol total
             HIPCHK(c, hipMemcpyAsync(h, c->dec_small.p, kDecSmallBytes, hipMemcpyDeviceToHost, c->stream));
@@ -1159,10 +1177,13 @@ int decompress_device(vecsz_ctx* c, const vecsz_params* p, const uint8_t* d_in, 
             HIPCHK(c, hipStreamSynchronize(c->stream));
             memcpy(&ds, h, sizeof(ds));
             memcpy(&tot, h + kDecSmallBytes, 8);
+            memcpy(&tm, h + kDecSmallTables, sizeof(tm));
             left = any_listed(h + kDecSmallLists, pass);
             return ds.error ? fail(c, VECSZ_ECORRUPT, "bitstream does not decode") : VECSZ_OK;
         };
         if (int rc2 = check()) return rc2;
+        if (tm.status)  // (nothing has run behind the tables)
+            return decompress_device(c, p, d_in, in_bytes, d_out, out_cap, nullptr, 0, true);
         if (left) {
             for (uint32_t batch = 2; left; batch = std::min<uint32_t>(2 * batch, 16)) {
                 if (pass > nsub + 2) return fail(c, VECSZ_ECORRUPT, "subsequence boundaries do not converge");
@@ -1184,10 +1205,13 @@ int decompress_device(vecsz_ctx* c, const vecsz_params* p, const uint8_t* d_in, 
 
     if (!fused_1d && !recon_issued) reconstruct(nullptr);
     HIPCHK(c, hipGetLastError());
-    if (indexed) HIPCHK(c, hipMemcpyAsync(h, c->dec_small.p, sizeof(DecSummary), hipMemcpyDeviceToHost, c->stream));
+    if (indexed) HIPCHK(c, hipMemcpyAsync(h, c->dec_small.p, kDecSmallLists, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     timing_end(c);
     if (indexed) {
+        TableMeta tm;
+        memcpy(&tm, h + kDecSmallTables, sizeof(tm));
+        if (tm.status) return decompress_device(c, p, d_in, in_bytes, d_out, out_cap, d_index, index_words, true);
         DecSummary ds;
         memcpy(&ds, h, sizeof(ds));
         if (ds.error) return fail(c, VECSZ_ECORRUPT, "bitstream does not decode with its decode index");
@@ -1910,13 +1934,12 @@ static int compress_batch_fused(vecsz_ctx* c, int nf, const vecsz_params* p, con
 
 // Fused batch decompress: every field shares the block size and a dictionary
 // of at most kMaxLdsBook, and has no pad section.  One copy brings every
-// archive's metadata, Huffman header and tree to the host (the tree of such
-// a dictionary is at most tree_byte_size(2 dict - 1) bytes), the decode
-// tables are built on host threads and go back in one copy, and then each
-// stage is one launch over all fields: the sync pass, the re-decode passes
-// over one batch-wide list, one scan over every subsequence of the batch,
-// the write pass, and the reconstruction (one launch per tile form) with its
-// fp32 fallback.  Outputs are the single-field path's.
+// archive's metadata and Huffman header to the host, and then each stage is
+// one launch over all fields: the decode tables (a workgroup per tree), the
+// sync pass, the re-decode passes, the offsets, the write pass, and the
+// reconstruction (one launch per tile form) with its fp32 fallback.  A field
+// whose tables the device could not build takes the per-field path behind
+// the batch.  Outputs are the single-field path's.
 static bool dbatch_fusable(const vecsz_ctx* c, int nf, const vecsz_params* p, const uint8_t* const* d_in,
                            float* const* d_out) {
     if (nf < 2 || nf > 4096) return false;
@@ -1937,8 +1960,11 @@ static int decompress_batch_fused_run(vecsz_ctx* c, int nf, const vecsz_params* 
     timing_begin(c);
     const int B = p[0].block, dict = p[0].dict_size, R = dict / 2;
 
-    // 1. the head of every archive (metadata, Huffman header, tree) in one copy
-    const uint64_t head_max = meta_bytes(3) + 8 + tree_byte_size(2 * (uint64_t)dict - 1);
+    // 1. the head of every archive (metadata, Huffman header, a tree of one
+    // node) in one copy
+    const uint64_t tree_max = meta_bytes(3) + 8 + tree_byte_size(2 * (uint64_t)dict - 1);
+    const uint64_t head_max = 128;
+    static_assert(4 * (3 + 1) + 8 + 24 + 8 + 14 <= 128, "a 3D header and a one-node tree fit");
     std::vector<HeadCopy> hc(nf);
     uint64_t htot = 0;
     for (int k = 0; k < nf; k++) {
@@ -1958,13 +1984,17 @@ static int decompress_batch_fused_run(vecsz_ctx* c, int nf, const vecsz_params* 
     HIPCHK(c, hipMemcpyAsync(c->db_hpin.p, c->db_heads.p, htot, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
 
-    // 2. headers, then the decode tables on host threads
+    // 2. headers; one-symbol trees
     struct Hdr {
         int ndim;
         uint64_t dims[3], n, pad_len, huff_size, nout, tb;
         double ebu;
+        uint32_t nodes;
+        bool root_leaf;
+        uint32_t root_sym;
     };
     std::vector<Hdr> hd(nf);
+    std::vector<char> redo(nf, 0);  // fields for the per-field path
     const uint8_t* heads = c->db_hpin.as<uint8_t>();
     for (int k = 0; k < nf; k++) {
         Hdr& h = hd[k];
@@ -1989,42 +2019,22 @@ static int decompress_batch_fused_run(vecsz_ctx* c, int nf, const vecsz_params* 
             const uint8_t* q = hp + mb;
             const int32_t ncs = (int32_t)(((uint32_t)q[0] << 24) | ((uint32_t)q[1] << 16) | ((uint32_t)q[2] << 8) | q[3]);
             h.tb = ncs > 0 ? tree_byte_size((uint64_t)ncs) : 0;
-            // a tree beyond what the dictionary allows cannot be in the head read
-            if (ncs <= 0 || 8 + h.tb > h.huff_size || mb + 8 + h.tb > hc[k].len) status[k] = VECSZ_ECORRUPT;
-        }
-    }
-    if ((int)c->db_dt.size() < nf) c->db_dt.resize(nf);
-    {
-        HostTimer ht(c, "host_tables");
-        std::atomic<int> next{0};
-        auto body = [&]() {
-            for (int k; (k = next.fetch_add(1)) < nf;) {
-                if (status[k]) continue;
-                DecodeTables& dt = c->db_dt[k];
-                if (build_decode_tables(heads + hc[k].off + meta_bytes(hd[k].ndim), hd[k].huff_size, dt) ||
-                    (!dt.root_leaf && !tree_is_full(dt)))
+            h.nodes = ncs > 0 ? (uint32_t)ncs : 0;
+            // (a tree beyond what the dictionary allows is not looked at)
+            if (ncs <= 0 || 8 + h.tb > h.huff_size || mb + 8 + h.tb > std::min<uint64_t>(in_bytes[k], tree_max)) {
+                status[k] = VECSZ_ECORRUPT;
+            } else if (h.nodes == 1) {
+                if (build_decode_tables(q, h.huff_size, c->dt) || (!c->dt.root_leaf && !tree_is_full(c->dt)))
                     status[k] = VECSZ_ECORRUPT;
+                h.root_leaf = c->dt.root_leaf;
+                h.root_sym = c->dt.root_sym;
             }
-        };
-        const int hw = (int)std::max(1u, std::thread::hardware_concurrency());
-        const int nt = std::max(1, std::min(nf, std::max(c->nworkers, std::min(16, hw))));
-        std::vector<std::thread> th;
-        for (int t = 1; t < nt; t++) th.emplace_back(body);
-        body();
-        for (auto& t : th) t.join();
+        }
     }
 
     // 3. layout: code / outlier regions (64-element aligned), tables,
     // subsequences, fallback block lists, unit and tile starts
-    bool t16 = true;
-    uint32_t max_sub16 = 0;
-    for (int k = 0; k < nf; k++) {
-        if (status[k] || c->db_dt[k].root_leaf) continue;
-        const DecodeTables& dt = c->db_dt[k];
-        if (dt.lut16.empty()) t16 = false;
-        max_sub16 = std::max<uint32_t>(max_sub16, (uint32_t)std::min<size_t>(dt.sub16.size(), kMaxSub16));
-    }
-    max_sub16 = batch_sub16_in_lds(max_sub16);
+    const uint32_t n_sub16 = batch_sub16_in_lds();
     std::vector<uint64_t> off(nf, 0), toff(nf, 0), fl_off(nf, 0);
     uint64_t ntot = 0, tab_tot = 0, nsub_tot = 0, fl_tot = 0;
     const size_t ns = (size_t)nf + 1;
@@ -2045,7 +2055,6 @@ static int decompress_batch_fused_run(vecsz_ctx* c, int nf, const vecsz_params* 
         for (int kind = 0; kind < kRcKinds; kind++) rk[kind * ns + k + 1] = rk[kind * ns + k];
         if (status[k]) continue;
         const Hdr& h = hd[k];
-        const DecodeTables& dt = c->db_dt[k];
         off[k] = ntot;
         ntot += (h.n + 63) / 64 * 64;
         F.ndim = h.ndim;
@@ -2053,19 +2062,18 @@ static int decompress_batch_fused_run(vecsz_ctx* c, int nf, const vecsz_params* 
         F.a.n_outlier = h.nout;
         const uint8_t* d_huff = d_in[k] + meta_bytes(h.ndim);
         F.a.outliers = d_huff + h.huff_size;
-        if (!dt.root_leaf) {
+        if (!h.root_leaf) {
             const uint64_t stream_bytes = h.huff_size - 8 - h.tb;
             F.a.stream = d_huff + 8 + h.tb;
             F.a.stream_bits = stream_bytes * 8;
             F.a.nsub = std::max<uint64_t>(1, (F.a.stream_bits + kSubBits - 1) / kSubBits);
             toff[k] = tab_tot;
-            tab_tot += t16 ? ((dt.lut16.size() + dt.sub16.size()) * 2 + 15) / 16 * 16
-                           : ((dt.lut.size() + dt.sub.size()) * 4 + 15) / 16 * 16;
+            tab_tot += table_words(std::min<uint32_t>(kMaxSubTabs, h.nodes / 2));
             F.s.jbase = sb[k];
             su[k + 1] = su[k] + decode_sync_units(F.a.nsub);
             wu[k + 1] = wu[k] + decode_write_units(F.a.nsub);
             sb[k + 1] = sb[k] + F.a.nsub;
-        } else if (dt.root_sym == 0 && h.nout < h.n) {
+        } else if (h.root_sym == 0 && h.nout < h.n) {
             status[k] = VECSZ_ECORRUPT;  // every element an outlier, but fewer outliers than elements
             continue;
         }
@@ -2094,18 +2102,25 @@ static int decompress_batch_fused_run(vecsz_ctx* c, int nf, const vecsz_params* 
     if (nsub_tot > 0xFFFFFFF0ull) return fail(c, VECSZ_EINVAL, "batch too large");  // u32 list counts
     const size_t st_bytes = st.size() * 8, fd_bytes = (size_t)nf * sizeof(DecField);
     const uint64_t nsub_alloc = std::max<uint64_t>(nsub_tot, 1);
+    // a re-decode list stripe per sync unit
     SubState S{};
-    list_stripes(std::max<uint64_t>(su[nf], 1), &S.nstripe, &S.stripe_cap);
+    S.nstripe = (uint32_t)std::max<uint64_t>(su[nf], 1);
+    S.stripe_cap = sync_unit_subs();
+    S.counter_words = 1;
+    S.slot_words = S.nstripe;
     const uint64_t list_cap = S.nstripe * S.stripe_cap;
-    if (!c->codes.ensure(ntot * 2 + 64) || !c->sparse.ensure(ntot * 4 + 64) || !c->tabs.ensure(tab_tot + 64) ||
+    const size_t count_bytes = (size_t)3 * S.slot_words * 4;
+    const size_t job_bytes = (size_t)nf * sizeof(TableJob), meta_all = (size_t)nf * sizeof(TableMeta);
+    if (!c->codes.ensure(ntot * 2 + 64) || !c->sparse.ensure(ntot * 4 + 64) || !c->tabs.ensure(tab_tot * 2 + 64) ||
         !c->sub_b.ensure(nsub_alloc) || !c->sub_e.ensure(nsub_alloc) || !c->sub_cz.ensure(nsub_alloc * 4) ||
-        !c->sub_list.ensure(list_cap * 16) || !c->sub_ln.ensure(kListCountBytes) || !c->unit_off.ensure((wu[nf] + 1) * 16) ||
+        !c->sub_list.ensure(list_cap * 16) || !c->sub_ln.ensure(count_bytes) || !c->unit_off.ensure((wu[nf] + 1) * 16) ||
+        !c->db_meta.ensure(meta_all + 64) || !c->db_jobs.ensure(job_bytes) ||
         !c->flagged.ensure(fl_tot * 4 + 64) || !c->db_nfl.ensure((size_t)nf * 4) ||
         !c->db_sums.ensure((size_t)nf * sizeof(DecSummary)) || !c->db_tot.ensure((size_t)nf * 8) ||
         !c->db_desc.ensure(fd_bytes) || !c->db_start.ensure(st_bytes))
         return fail(c, VECSZ_ENOMEM, "device scratch allocation failed");
-    if (!c->db_pin.ensure(fd_bytes + st_bytes + tab_tot + 64) ||
-        !c->db_back.ensure((size_t)nf * (sizeof(DecSummary) + 8) + kListCountBytes))
+    if (!c->db_pin.ensure(fd_bytes + st_bytes + job_bytes + 64) ||
+        !c->db_back.ensure((size_t)nf * (sizeof(DecSummary) + 8) + meta_all + count_bytes / 3 + 64))
         return fail(c, VECSZ_ENOMEM, "pinned buffer");
     S.b = c->sub_b.as<uint8_t>();
     S.e = c->sub_e.as<uint8_t>();
@@ -2115,11 +2130,10 @@ static int decompress_batch_fused_run(vecsz_ctx* c, int nf, const vecsz_params* 
     S.list_n = c->sub_ln.as<uint32_t>();
     S.jbase = 0;
     uint64_t* uoff = c->unit_off.as<uint64_t>();
-    uint8_t* tab_h = c->db_pin.as<uint8_t>() + fd_bytes + st_bytes;
+    std::vector<TableJob> jobs(nf, TableJob{});
     for (int k = 0; k < nf; k++) {
         DecField& F = fd[k];
         if (status[k]) continue;
-        const DecodeTables& dt = c->db_dt[k];
         F.codes = c->codes.as<uint16_t>() + off[k];
         F.sparse = c->sparse.as<float>() + off[k];
         F.flagged = c->flagged.as<uint32_t>() + fl_off[k];
@@ -2133,51 +2147,52 @@ static int decompress_batch_fused_run(vecsz_ctx* c, int nf, const vecsz_params* 
         F.s.list_n = S.list_n;
         F.s.nstripe = S.nstripe;
         F.s.stripe_cap = S.stripe_cap;
-        if (dt.root_leaf) continue;
-        uint8_t* tp = tab_h + toff[k];
-        uint8_t* tdev = c->tabs.as<uint8_t>() + toff[k];
-        if (t16) {
-            memcpy(tp, dt.lut16.data(), dt.lut16.size() * 2);
-            memcpy(tp + dt.lut16.size() * 2, dt.sub16.data(), dt.sub16.size() * 2);
-            F.a.lut16 = reinterpret_cast<const uint16_t*>(tdev);
-            F.a.sub16 = reinterpret_cast<const uint16_t*>(tdev) + dt.lut16.size();
-            F.a.n_sub16 = (uint32_t)std::min<size_t>(dt.sub16.size(), max_sub16);
-        } else {
-            memcpy(tp, dt.lut.data(), dt.lut.size() * 4);
-            memcpy(tp + dt.lut.size() * 4, dt.sub.data(), dt.sub.size() * 4);
-            F.a.lut = reinterpret_cast<const uint32_t*>(tdev);
-            F.a.sub = reinterpret_cast<const uint32_t*>(tdev) + dt.lut.size();
-        }
+        F.s.counter_words = S.counter_words;
+        F.s.slot_words = S.slot_words;
+        if (hd[k].root_leaf) continue;
+        uint16_t* tabs = c->tabs.as<uint16_t>() + toff[k];
+        F.a.tabs = tabs;
+        F.a.meta = c->db_meta.as<TableMeta>() + k;
+        F.a.n_sub16 = n_sub16;
+        const uint32_t cap = std::min<uint32_t>(kMaxSubTabs, hd[k].nodes / 2);
+        jobs[k] = {d_in[k] + meta_bytes(hd[k].ndim), hd[k].nodes, cap, tabs, c->db_meta.as<TableMeta>() + k, nullptr};
     }
     DecField* fdd = c->db_desc.as<DecField>();
     uint64_t* std_ = c->db_start.as<uint64_t>();
     const uint64_t* su_d = std_;
     const uint64_t* wu_d = std_ + ns;
-    const uint64_t* sb_d = std_ + 2 * ns;
     const uint64_t* rk_d = std_ + 3 * ns;
     memcpy(c->db_pin.p, fd.data(), fd_bytes);
     memcpy(c->db_pin.as<uint8_t>() + fd_bytes, st.data(), st_bytes);
     HIPCHK(c, hipMemcpyAsync(c->db_desc.p, c->db_pin.p, fd_bytes, hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipMemcpyAsync(c->db_start.p, c->db_pin.as<uint8_t>() + fd_bytes, st_bytes, hipMemcpyHostToDevice,
                              c->stream));
-    if (tab_tot) HIPCHK(c, hipMemcpyAsync(c->tabs.p, tab_h, tab_tot, hipMemcpyHostToDevice, c->stream));
+    uint8_t* jobs_h = c->db_pin.as<uint8_t>() + fd_bytes + st_bytes;
+    memcpy(jobs_h, jobs.data(), job_bytes);
+    HIPCHK(c, hipMemcpyAsync(c->db_jobs.p, jobs_h, job_bytes, hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipMemsetAsync(c->db_sums.p, 0, (size_t)nf * sizeof(DecSummary), c->stream));
     HIPCHK(c, hipMemsetAsync(c->db_nfl.p, 0, (size_t)nf * 4, c->stream));
-    HIPCHK(c, hipMemsetAsync(c->sub_ln.p, 0, kListCountBytes, c->stream));
+    HIPCHK(c, hipMemsetAsync(c->db_meta.p, 0, meta_all, c->stream));
+    HIPCHK(c, hipMemsetAsync(c->sub_ln.p, 0, count_bytes, c->stream));
 
     // 4. decode: one-symbol trees by a fill; the others by the batch passes
     {
+        StageScope s(c, "decode_tables");
+        launch_decode_tables_multi(c->db_jobs.as<TableJob>(), nf, c->stream);
+    }
+    {
         StageScope s(c, "decode_sync");
         for (int k = 0; k < nf; k++) {
-            if (status[k] || !c->db_dt[k].root_leaf) continue;
-            launch_fill_u16(fd[k].codes, hd[k].n, (uint16_t)c->db_dt[k].root_sym, c->stream);
-            if (c->db_dt[k].root_sym == 0) launch_scatter_all_outliers(fd[k].a.outliers, hd[k].n, fd[k].sparse, c->stream);
+            if (status[k] || !hd[k].root_leaf) continue;
+            launch_fill_u16(fd[k].codes, hd[k].n, (uint16_t)hd[k].root_sym, c->stream);
+            if (hd[k].root_sym == 0) launch_scatter_all_outliers(fd[k].a.outliers, hd[k].n, fd[k].sparse, c->stream);
         }
-        launch_decode_sync_multi(t16, max_sub16, fdd, su_d, nf, su[nf], c->stream);
+        launch_decode_sync_multi(n_sub16, fdd, su_d, nf, su[nf], c->stream);
     }
     DecSummary* sums_h = c->db_back.as<DecSummary>();
     uint64_t* tot_h = reinterpret_cast<uint64_t*>(c->db_back.as<uint8_t>() + (size_t)nf * sizeof(DecSummary));
-    uint8_t* left_h = reinterpret_cast<uint8_t*>(tot_h + nf);
+    TableMeta* meta_h = reinterpret_cast<TableMeta*>(tot_h + nf);
+    uint32_t* left_h = reinterpret_cast<uint32_t*>(meta_h + nf);
     uint64_t max_nsub = 0;
     for (int k = 0; k < nf; k++) max_nsub = std::max<uint64_t>(max_nsub, fd[k].a.nsub);
     if (nsub_tot) {
@@ -2185,36 +2200,40 @@ static int decompress_batch_fused_run(vecsz_ctx* c, int nf, const vecsz_params* 
         uint32_t pass = 0;
         {
             StageScope s(c, "decode_redo");
-            for (; pass < kPassesAhead; pass++) launch_decode_pass_multi(t16, fdd, sb_d, nf, S, pass, c->stream);
+            for (; pass < kPassesAhead; pass++)
+                launch_decode_pass_multi(n_sub16, fdd, su_d, nf, su[nf], pass, c->stream);
         }
         HIPCHK(c, hipGetLastError());
         uint32_t batch = 2;
         for (;;) {
-            HIPCHK(c, hipMemcpyAsync(left_h, S.list_n, kListCountBytes, hipMemcpyDeviceToHost, c->stream));
+            HIPCHK(c, hipMemcpyAsync(left_h, list_counter(S, pass, 0), (size_t)S.nstripe * 4, hipMemcpyDeviceToHost, c->stream));
+            HIPCHK(c, hipMemcpyAsync(sums_h, c->db_sums.p, (size_t)nf * sizeof(DecSummary), hipMemcpyDeviceToHost, c->stream));
+            HIPCHK(c, hipMemcpyAsync(meta_h, c->db_meta.p, meta_all, hipMemcpyDeviceToHost, c->stream));
             HIPCHK(c, hipStreamSynchronize(c->stream));
-            if (!any_listed(left_h, pass)) break;
+            if (std::all_of(left_h, left_h + S.nstripe, [](uint32_t n) { return n == 0; })) break;
             if (pass > max_nsub + 2) return fail(c, VECSZ_ECORRUPT, "subsequence boundaries do not converge");
             StageScope s(c, "decode_redo");
-            for (uint32_t b = 0; b < batch; b++) launch_decode_pass_multi(t16, fdd, sb_d, nf, S, pass++, c->stream);
+            for (uint32_t b = 0; b < batch; b++)
+                launch_decode_pass_multi(n_sub16, fdd, su_d, nf, su[nf], pass++, c->stream);
             batch = std::min<uint32_t>(2 * batch, 16);
         }
-        // fields whose stream does not decode are left out of the write pass
-        // and the reconstruction (their subsequence state is not trusted)
-        HIPCHK(c, hipMemcpyAsync(sums_h, c->db_sums.p, (size_t)nf * sizeof(DecSummary), hipMemcpyDeviceToHost,
-                                 c->stream));
-        HIPCHK(c, hipStreamSynchronize(c->stream));
+        // fields whose stream does not decode, or whose tables could not be
+        // built, are left out of the write pass and the reconstruction
+        // (their subsequence state is not trusted)
         bool changed = false;
         for (int k = 0; k < nf; k++) {
-            if (status[k] || !sums_h[k].error) continue;
-            status[k] = VECSZ_ECORRUPT;
-            changed = true;
+            if (status[k] || hd[k].root_leaf) continue;
+            redo[k] = meta_h[k].status != 0;
+            if (sums_h[k].error) status[k] = VECSZ_ECORRUPT;
+            changed |= status[k] || redo[k];
         }
         if (changed) {
             for (int k = 0; k < nf; k++) {
-                wu[k + 1] = wu[k] + (status[k] ? 0 : decode_write_units(fd[k].a.nsub));
+                const bool out = status[k] || redo[k];
+                wu[k + 1] = wu[k] + (out || hd[k].root_leaf ? 0 : decode_write_units(fd[k].a.nsub));
                 for (int kind = 0; kind < kRcKinds; kind++)
-                    rk[kind * ns + k + 1] = rk[kind * ns + k] + (!status[k] && fd[k].kind == kind ? recon_tiles(kind, fd[k].ra) : 0);
-                if (status[k]) fd[k].kind = -1;
+                    rk[kind * ns + k + 1] = rk[kind * ns + k] + (!out && fd[k].kind == kind ? recon_tiles(kind, fd[k].ra) : 0);
+                if (out) fd[k].kind = -1;
             }
             memcpy(c->db_pin.p, fd.data(), fd_bytes);
             memcpy(c->db_pin.as<uint8_t>() + fd_bytes, st.data(), st_bytes);
@@ -2228,7 +2247,7 @@ static int decompress_batch_fused_run(vecsz_ctx* c, int nf, const vecsz_params* 
         }
         {
             StageScope s(c, "decode_write");
-            launch_decode_write_multi(t16, max_sub16, fdd, wu_d, nf, wu[nf], uoff, c->stream);
+            launch_decode_write_multi(n_sub16, fdd, wu_d, nf, wu[nf], uoff, c->stream);
         }
         launch_dec_field_totals(wu_d, nf, uoff, c->db_tot.as<uint64_t>(), c->stream);
         HIPCHK(c, hipGetLastError());
@@ -2246,8 +2265,11 @@ static int decompress_batch_fused_run(vecsz_ctx* c, int nf, const vecsz_params* 
     timing_end(c);
     *reported = true;
     for (int k = 0; k < nf; k++) {
-        if (status[k] || c->db_dt[k].root_leaf) continue;
-        if (sums_h[k].error || tot_h[k] < hd[k].n) status[k] = VECSZ_ECORRUPT;
+        if (status[k] || hd[k].root_leaf) continue;
+        if (redo[k])
+            status[k] = decompress_device(c, &p[k], d_in[k], in_bytes[k], d_out[k], out_cap[k], nullptr, 0, true);
+        else if (sums_h[k].error || tot_h[k] < hd[k].n)
+            status[k] = VECSZ_ECORRUPT;
     }
     for (int k = 0; k < nf; k++)
         if (status[k]) {
@@ -2441,11 +2463,10 @@ int vecsz_decompress_batch(vecsz_ctx* c, int nfields, const vecsz_params* p, con
     auto prep = [&](vecsz_ctx* w) {
         (void)hipSetDevice(w->device);
         const uint64_t nsub = bmax * 8 / kSubBits + 2;
-        uint32_t nstripe;
-        uint64_t cap;
-        list_stripes(decode_sync_units(nsub), &nstripe, &cap);
+        SubState ls{};
+        list_stripes(decode_sync_units(nsub), &ls);
         return w->codes.ensure(nmax * 2 + 64) && w->sparse.ensure(nmax * 4 + 64) && w->sub_b.ensure(nsub) &&
-               w->sub_e.ensure(nsub) && w->sub_cz.ensure(nsub * 4) && w->sub_list.ensure(nstripe * cap * 16) &&
+               w->sub_e.ensure(nsub) && w->sub_cz.ensure(nsub * 4) && w->sub_list.ensure(ls.nstripe * ls.stripe_cap * 16) &&
                w->unit_off.ensure((decode_write_units(nsub) + 1) * 16);
     };
     return run_batch(c, nfields, weight.data(), status, prep, [&](vecsz_ctx* w, int k) {

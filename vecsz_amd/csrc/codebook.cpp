@@ -293,7 +293,6 @@ int build_decode_tables(const uint8_t* huff, uint64_t huff_size, DecodeTables& d
         size_t slot;
     };
     std::vector<Pending> todo;
-    std::vector<uint32_t> tab_depth;  // bits consumed before each deeper table
     // Depth-first over the subtree of `node`: a leaf b bits below it fills
     // its 2^(bits - b) entries at once, so a table costs its size plus the
     // nodes it covers.
@@ -341,37 +340,10 @@ int build_decode_tables(const uint8_t* huff, uint64_t huff_size, DecodeTables& d
         if (base + (1u << kSubTabBits) > ((size_t)1 << 24)) return VECSZ_ECORRUPT;
         dt.sub.resize(base + (1u << kSubTabBits));
         (pd.in_lut ? dt.lut : dt.sub)[pd.slot] = kLutSlow | (uint32_t)base;
-        tab_depth.push_back(pd.depth);
         st = fill(pd.node, pd.depth, kSubTabBits, false, base);
         if (st) return st;
     }
 
-    // compact 16-bit form
-    dt.lut16.clear();
-    dt.sub16.clear();
-    bool ok16 = tab_depth.size() <= 4096;
-    auto to16 = [&](uint32_t e, uint32_t depth, uint16_t& out) {
-        if (e == 0) return false;  // invalid path
-        if (e & kLutSlow) {
-            out = (uint16_t)((e & 0x7FFFFFFFu) >> kSubTabBits);
-            return true;
-        }
-        const uint32_t sym = e & 0xFFFF, used = ((e >> 16) & 0x7F) - depth;
-        if (sym >= 4096 || used == 0 || used > 15) return false;
-        out = (uint16_t)((used << 12) | sym);
-        return true;
-    };
-    if (ok16) {
-        dt.lut16.resize(dt.lut.size());
-        for (size_t i = 0; ok16 && i < dt.lut.size(); i++) ok16 = to16(dt.lut[i], 0, dt.lut16[i]);
-        dt.sub16.resize(dt.sub.size());
-        for (size_t i = 0; ok16 && i < dt.sub.size(); i++)
-            ok16 = to16(dt.sub[i], tab_depth[i >> kSubTabBits], dt.sub16[i]);
-    }
-    if (!ok16) {
-        dt.lut16.clear();
-        dt.sub16.clear();
-    }
     return VECSZ_OK;
 }
 

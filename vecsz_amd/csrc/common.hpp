@@ -192,11 +192,16 @@ struct DecSummary {
 //  bit 31 set  : bits 0..30 = first entry of the next-level table
 //  0           : invalid path (corrupt tree)
 constexpr uint32_t kLutSlow = 0x80000000u;
-// Compact tables for symbols below 4096: 16-bit entries, bits 0..11 a symbol
-// or a deeper table's number, bits 12..15 the bits consumed by a leaf in this
-// table (first level: total length 1..12; deeper: 1..kSubTabBits), 0 for a
-// pointer to the next table.
-constexpr uint32_t kMaxSub16 = 12288;  // deeper-table entries kept in LDS
+// Compact tables for symbols below 4096, built on the device: 16-bit entries,
+// bits 0..11 a symbol or a deeper table's number, bits 12..15 the bits
+// consumed by a leaf in this table (first level: total length 1..12; deeper:
+// 1..kSubTabBits), 0 for a pointer to the next table.  The first level also
+// has a counting form, for passes that want no symbols: bits 12..15 the bits
+// of all whole codewords in the pattern (0: none, a pointer as above), 0..3
+// how many they are, 4..7 how many of them decode to symbol 0.
+constexpr uint32_t kMaxSubTabs = 4096;      // deeper tables (their numbers have 12 bits)
+constexpr uint32_t kMaxTreeNodes = 8191;    // of 4096 symbols
+constexpr uint32_t kMaxSub16 = 12288;       // deeper-table entries kept in LDS
 // Node table entry for the bit-serial slow path: child[2*i + bit]
 //  bit 31 set: leaf, bits 0..15 symbol; otherwise internal node index; 0xFFFFFFFF = absent.
 constexpr uint32_t kNodeLeaf = 0x80000000u;

@@ -100,15 +100,33 @@ void launch_pack_multi(const BatchField* fd, int nf, const uint64_t* start, uint
                        int grid_cap, hipStream_t st);
 
 // Decoder (kernels_decompress.hip)
+// Device-built compact tables: whether they could be built (0), and how many
+// deeper entries there are.
+struct TableMeta {
+    uint32_t status, n_sub16;
+    uint32_t pad_[2];
+};
+constexpr size_t table_words(uint32_t cap) { return (2u << kLutBits) + ((size_t)cap << kSubTabBits); }
+struct TableJob {
+    const uint8_t* huff;  // Huffman section: [u32be nodes][u32be dict][tree]
+    uint32_t nodes;       // as in it (0: nothing to build; at most kMaxTreeNodes)
+    uint32_t cap;         // deeper tables tabs has room for (at most kMaxSubTabs)
+    uint16_t* tabs;       // counting first level, first level, deeper tables: table_words(cap)
+    TableMeta* meta;
+    uint32_t* hold;       // list counters whose hold a failure sets, or null
+};
+void launch_decode_tables(const TableJob& job, hipStream_t st);
+void launch_decode_tables_multi(const TableJob* jobs, int n, hipStream_t st);
+
 struct DecodeArgs {
     const uint8_t* stream;   // first byte of the bitstream (any alignment)
     uint64_t stream_bits;    // 8 * stream bytes
     uint64_t n;              // symbols to decode
-    const uint32_t* lut;     // first-level table, 1 << kLutBits entries
+    const uint32_t* lut;     // host-built first level, 1 << kLutBits entries
     const uint32_t* sub;     // deeper tables
-    const uint16_t* lut16;   // compact tables (nullptr: use lut / sub)
-    const uint16_t* sub16;
-    uint32_t n_sub16;        // entries of sub16 the kernels copy to LDS; 0: read in global memory
+    const uint16_t* tabs;    // device-built compact tables (nullptr: use lut / sub), TableJob::tabs
+    const TableMeta* meta;   // of those
+    uint32_t n_sub16;        // deeper compact entries a kernel has LDS room for
     uint64_t nsub;           // subsequences of kSubBits bits
     const uint8_t* outliers; // outlier section of the archive (any alignment)
     uint64_t n_outlier;
@@ -118,19 +136,17 @@ struct SubState {
     // Of subsequence j (its target: bit (j + 1) * kSubBits, or the stream's
     // end): how far past bit j * kSubBits its first codeword starts, and how
     // far past its target the one after its last (both below 64, a codeword's
-    // length); codewords starting in between | those of them that decode to
-    // symbol 0 << 16 (at most kSubBits each).
+    // length, plus 12, a table entry's); codewords starting in between | those
+    // of them that decode to symbol 0 << 16 (at most kSubBits + 11 each).
     uint8_t* b;
     uint8_t* e;
     uint32_t* cz;
     // Re-decode lists, used in alternation by successive passes: subsequence
     // jbase + j | its start (as b) << 48.  A list is nstripe stripes of
-    // stripe_cap entries, each with a counter of its own (list_count): a
-    // counter that every wavefront adds to is a queue at one cache line, at
-    // about 10 ns an addition.
+    // stripe_cap entries, each with a counter of its own (list_counter).
     uint64_t* list[2];
     uint32_t* list_n;
-    uint32_t nstripe;
+    uint32_t nstripe, counter_words, slot_words;
     uint64_t stripe_cap;
     // 0 for one field; in a batch b, e and cz are views of one field's part
     // of batch-wide arrays, and jbase is the batch-wide number of its
@@ -138,14 +154,25 @@ struct SubState {
     uint64_t jbase = 0;
 };
 
-// Counters of a ring of three lists (pass p reads slot p % 3), each on a
-// cache line of its own.
+// Counters of a ring of three lists (pass p reads slot p % 3).  One field's
+// lists: up to kMaxStripes stripes, shared by its workgroups, each counter on
+// a cache line of its own (a counter that every wavefront adds to is a queue
+// at one line, at about 10 ns an addition), and a last one, the hold: set
+// where the tables could not be built, so that what waits for empty lists
+// does not run.  A batch's lists have a stripe per sync unit.
 constexpr uint32_t kMaxStripes = 32;
 constexpr uint32_t kCounterWords = 32;
-constexpr size_t kListCountBytes = (size_t)3 * kMaxStripes * kCounterWords * 4;
-__host__ __device__ inline uint32_t list_slot(uint32_t pass) { return pass % 3 * kMaxStripes * kCounterWords; }
-// Stripes of the lists for `units` sync workgroups, and their entries.
-void list_stripes(uint64_t units, uint32_t* nstripe, uint64_t* cap);
+constexpr uint32_t kSlotWords = (kMaxStripes + 1) * kCounterWords;
+constexpr size_t kListCountBytes = (size_t)3 * kSlotWords * 4;
+__host__ __device__ inline uint32_t list_slot(uint32_t pass) { return pass % 3 * kSlotWords; }
+__host__ __device__ inline uint32_t list_hold(uint32_t pass) { return list_slot(pass) + kMaxStripes * kCounterWords; }
+__host__ __device__ inline uint32_t* list_counter(const SubState& s, uint32_t pass, uint32_t stripe) {
+    return s.list_n + (size_t)(pass % 3) * s.slot_words + (size_t)stripe * s.counter_words;
+}
+// Stripes of one field's lists for `units` sync workgroups, and their entries.
+void list_stripes(uint64_t units, SubState* s);
+// Entries of a stripe that holds one sync unit's.
+uint64_t sync_unit_subs();
 void launch_decode_sync(const DecodeArgs& a, SubState s, DecSummary* sum, hipStream_t st);
 // Re-decode pass `pass` over the list the previous pass (or the sync pass) built.
 void launch_decode_pass(const DecodeArgs& a, SubState s, uint32_t pass, DecSummary* sum, hipStream_t st);
@@ -153,8 +180,8 @@ void launch_scan_u32x2(const uint32_t* a, const uint32_t* b, uint64_t n, uint64_
                        uint64_t* totals, hipStream_t st);
 // Codewords and zeros before each write unit (decode_write_units(nsub) units
 // of consecutive subsequences): off[2 u], off[2 u + 1], the totals behind the
-// last.  guard (nullable): nothing runs while any of the kMaxStripes counters
-// from there on (a list_slot) is nonzero.
+// last.  guard (nullable): nothing runs while any of the counters
+// and the hold from there on (a list_slot) is nonzero.
 void launch_decode_offsets(const SubState& s, uint64_t nsub, uint64_t* off, hipStream_t st, const uint32_t* guard = nullptr);
 void launch_decode_write(const DecodeArgs& a, SubState s, const uint64_t* off, uint16_t* codes, float* sparse,
                          DecSummary* sum, hipStream_t st, const uint32_t* guard = nullptr);
@@ -212,24 +239,21 @@ struct DecField {
     int ndim;
     int kind;                  // ReconKind; -1: not reconstructed
 };
-// t16: every field has compact tables; max_sub16: the largest n_sub16.
-// start: per-field unit starts (nf + 1), nunits = start[nf].
-// The largest deeper-table size of a batch's fields (entries), or 0 when
-// keeping tables that size in LDS would cost the batch's sync pass a
-// resident workgroup per CU (the fields then read them in global memory).
-uint32_t batch_sub16_in_lds(uint32_t max_sub16);
-void launch_decode_sync_multi(bool t16, uint32_t max_sub16, const DecField* fd, const uint64_t* start, int nf,
-                              uint64_t nunits, hipStream_t st);
-// sub_start: batch-wide number of each field's subsequence 0 (nf + 1 entries);
-// S: the batch-wide lists (list, list_n).
-void launch_decode_pass_multi(bool t16, const DecField* fd, const uint64_t* sub_start, int nf, SubState S,
+// start: per-field unit starts (nf + 1), nunits = start[nf].  Compact tables
+// only: a field whose TableMeta says they could not be built is left alone.
+// Deeper compact entries a batch's kernels have LDS room for.
+uint32_t batch_sub16_in_lds();
+void launch_decode_sync_multi(uint32_t n_sub16, const DecField* fd, const uint64_t* start, int nf, uint64_t nunits,
+                              hipStream_t st);
+// start: the sync units (a list's stripes).
+void launch_decode_pass_multi(uint32_t n_sub16, const DecField* fd, const uint64_t* start, int nf, uint64_t nunits,
                               uint32_t pass, hipStream_t st);
 // start: per-field write unit starts (nf + 1), nunits = start[nf]; off as
 // launch_decode_offsets, over the units of every field.
 void launch_decode_offsets_multi(const DecField* fd, const uint64_t* start, int nf, uint64_t nunits, uint64_t* off,
                                  hipStream_t st);
-void launch_decode_write_multi(bool t16, uint32_t max_sub16, const DecField* fd, const uint64_t* start, int nf,
-                               uint64_t nunits, const uint64_t* off, hipStream_t st);
+void launch_decode_write_multi(uint32_t n_sub16, const DecField* fd, const uint64_t* start, int nf, uint64_t nunits,
+                               const uint64_t* off, hipStream_t st);
 // Symbols each field's subsequences hold (tot[f]).
 void launch_dec_field_totals(const uint64_t* start, int nf, const uint64_t* off, uint64_t* tot, hipStream_t st);
 // One reconstruction form over its fields' tiles (start: per-field tile starts).

@@ -109,12 +109,14 @@ struct GlobalWin {
     }
 };
 
-// Whether a list is not empty (every lane of the wavefront calls it).
+// Whether a list is not empty, or held (every lane of the wavefront calls it).
 __device__ __forceinline__ bool listed(const uint32_t* guard) {
     if (!guard) return false;
-    const uint32_t lane = lane_id2();
-    return __any(lane < kMaxStripes && ((GlobalU32)guard)[(lane % kMaxStripes) * kCounterWords] != 0);
+    const uint32_t lane = min(lane_id2(), kMaxStripes);
+    return __any(((GlobalU32)guard)[lane * kCounterWords] != 0);
 }
+// Whether the field's tables could not be built.
+__device__ __forceinline__ bool no_tables(const DecodeArgs& a) { return a.meta && ((GlobalU32)a.meta)[0] != 0; }
 
 // Appends to the list of slot `slot` the lanes with `on` (a subsequence and
 // its start), in stripe `stripe`: one counter addition per wavefront.
@@ -125,48 +127,33 @@ __device__ __forceinline__ void list_append(const SubState& s, uint32_t pass, ui
     const uint32_t lane = lane_id2();
     const int lead = __builtin_ctzll(m);
     uint32_t k = 0;
-    if ((int)lane == lead) k = atomicAdd(&s.list_n[list_slot(pass) + stripe * kCounterWords], (uint32_t)__popcll(m));
+    if ((int)lane == lead) k = atomicAdd(list_counter(s, pass, stripe), (uint32_t)__popcll(m));
     k = (uint32_t)__builtin_amdgcn_readlane((int)k, lead);
     if (on)
         s.list[pass & 1][stripe * s.stripe_cap + k + __popcll(m & ((1ull << lane) - 1))] = (s.jbase + j) | ((uint64_t)first << 48);
 }
 
-// Decode tables as a kernel sees them.
-//   look(w)     first-level entry of the codeword at the top of w
+// Decode tables as a kernel sees them (T16: the compact ones, Decoder<false>:
+// the 32-bit ones).  Decoder yields symbols, CountDecoder counts.
+//   look(w)     first-level entry of the codeword (or codewords) at the top of w
 //   escape(e)   the codeword is longer than the first level (32-bit tables:
 //               or invalid): resolve() walks the deeper tables
-//   len, sym    of an entry (sym: bits above the symbol may be set for the
-//               packing helpers below)
+//   len, sym    of an entry
 //   resolve     e, l <- entry and length of the codeword at lp whose first
 //               32 bits (at least 16 of them valid) are w; l = 0: invalid.
 //               win is read for the bits past those
 template <bool T16>
 struct Decoder;
 
-template <>
-struct Decoder<true> {
-    const uint16_t* lut;
-    LdsU16 sub_lds;  // the first n_lds entries of the deeper tables
+// The deeper compact tables.
+struct Deeper16 {
+    LdsU16 sub_lds;  // the first n_lds entries
     GlobalU16 sub;   // all of them
     uint32_t n_lds;
-    // The tables are in LDS at lds (TableCopy); returns the words they take.
-    __device__ __forceinline__ uint32_t attach(const uint32_t* lds, const DecodeArgs& a) {
-        lut = reinterpret_cast<const uint16_t*>(lds);
-        sub_lds = (LdsU16)(lut + (1u << kLutBits));
-        sub = (GlobalU16)a.sub16;
-        n_lds = a.n_sub16;
-        return ((1u << kLutBits) + n_lds) / 2;
-    }
-    __device__ __forceinline__ uint32_t look(uint32_t w) const { return lut[w >> (32 - kLutBits)]; }
-    static __device__ __forceinline__ bool escape(uint32_t e) { return e < 4096; }
-    static __device__ __forceinline__ uint32_t len(uint32_t e) { return e >> 12; }
-    static __device__ __forceinline__ uint32_t sym(uint32_t e) { return e & 0xFFF; }
-    // Two symbols as the halves of a word.
-    static __device__ __forceinline__ uint32_t pack(uint32_t a, uint32_t b) { return (a | (b << 16)) & 0x0FFF0FFFu; }
-    // Entry i of the deeper tables.  The empty asm makes a global read's wait
-    // part of its own branch: behind the join the wavefronts that read LDS
-    // alone would wait too, for all of their stores in flight.
-    __device__ __forceinline__ uint32_t deeper(uint32_t i) const {
+    // Entry i.  The empty asm makes a global read's wait part of its own
+    // branch: behind the join the wavefronts that read LDS alone would wait
+    // too, for all of their stores in flight.
+    __device__ __forceinline__ uint32_t entry(uint32_t i) const {
         uint32_t e;
         if (i < n_lds) {
             e = sub_lds[i];
@@ -178,7 +165,7 @@ struct Decoder<true> {
     }
     template <typename W>
     __device__ __forceinline__ void resolve(const W& win, uint32_t w, uint32_t lp, uint32_t& e, uint32_t& l) const {
-        e = deeper((e << kSubTabBits) | ((w << kLutBits) >> (32 - kSubTabBits)));
+        e = entry((e << kSubTabBits) | ((w << kLutBits) >> (32 - kSubTabBits)));
         l = e >> 12;
         if (l != 0) {
             l += kLutBits;
@@ -188,7 +175,7 @@ struct Decoder<true> {
         uint32_t used = kLutBits + kSubTabBits;
 #pragma unroll 1
         for (int lv = 1; lv < 16; lv++, used += kSubTabBits) {
-            e = deeper((e << kSubTabBits) | (win(lp + used) >> (32 - kSubTabBits)));
+            e = entry((e << kSubTabBits) | (win(lp + used) >> (32 - kSubTabBits)));
             if (e >> 12) {
                 l = used + (e >> 12);
                 break;
@@ -198,10 +185,37 @@ struct Decoder<true> {
 };
 
 template <>
+struct Decoder<true> {
+    static constexpr bool kInvalid = false;  // no entry is an invalid path
+    const uint16_t* lut;
+    Deeper16 deep;
+    // The tables are in LDS at lds (TableCopy), n_lds deeper entries of them
+    // in a room of a.n_sub16; returns the words they take.
+    __device__ __forceinline__ uint32_t attach(const uint32_t* lds, const DecodeArgs& a, uint32_t n_lds) {
+        lut = reinterpret_cast<const uint16_t*>(lds);
+        deep.sub_lds = (LdsU16)(lut + (1u << kLutBits));
+        deep.sub = (GlobalU16)a.tabs + (2u << kLutBits);
+        deep.n_lds = n_lds;
+        return ((1u << kLutBits) + a.n_sub16) / 2;
+    }
+    __device__ __forceinline__ uint32_t look(uint32_t w) const { return lut[w >> (32 - kLutBits)]; }
+    static __device__ __forceinline__ bool escape(uint32_t e) { return e < 4096; }
+    static __device__ __forceinline__ uint32_t len(uint32_t e) { return e >> 12; }
+    static __device__ __forceinline__ uint32_t sym(uint32_t e) { return e & 0xFFF; }
+    // Two symbols as the halves of a word.
+    static __device__ __forceinline__ uint32_t pack(uint32_t a, uint32_t b) { return (a | (b << 16)) & 0x0FFF0FFFu; }
+    template <typename W>
+    __device__ __forceinline__ void resolve(const W& win, uint32_t w, uint32_t lp, uint32_t& e, uint32_t& l) const {
+        deep.resolve(win, w, lp, e, l);
+    }
+};
+
+template <>
 struct Decoder<false> {
+    static constexpr bool kInvalid = true;
     const uint32_t* lut;
     GlobalU32 sub;
-    __device__ __forceinline__ uint32_t attach(const uint32_t* lds, const DecodeArgs& a) {
+    __device__ __forceinline__ uint32_t attach(const uint32_t* lds, const DecodeArgs& a, uint32_t) {
         lut = lds;
         sub = (GlobalU32)a.sub;
         return 1u << kLutBits;
@@ -217,30 +231,77 @@ struct Decoder<false> {
 #pragma unroll 1
         for (int lv = 0; lv < 16 && (e & kLutSlow); lv++, used += kSubTabBits) {
             e = sub[(e & ~kLutSlow) + (win(lp + used) >> (32 - kSubTabBits))];
-            asm volatile("" : "+v"(e));  // (its wait, as in Decoder<true>::deeper)
+            asm volatile("" : "+v"(e));  // (its wait, as in Deeper16::entry)
         }
         l = (e & kLutSlow) ? 0u : (e >> 16) & 0x7F;
     }
 };
 
-// Copies the tables a kernel keeps in LDS (compact: the first level and the
-// n_sub16 entries behind it, a multiple of 16) with NT threads.  fetch()
-// issues every load of a thread and put() stores them, so a workgroup can
-// have its tables and its bits in flight together and waits for one memory
-// latency; a copy loop of one load per round waited for one latency per
-// round, which was most of a workgroup's time (the indexed decode of the
-// 512^3 field at 1e-3: 0.28 -> 0.16 ms).
-template <bool T16, uint32_t NT>
+// count(e): codewords of an entry (compact: all the whole ones in the 12-bit
+// pattern, 3 on average where a codeword has 3 bits); zeros(e): those that
+// decode to symbol 0.
+template <bool T16>
+struct CountDecoder;
+template <>
+struct CountDecoder<true> {
+    static constexpr bool kInvalid = false;
+    static constexpr uint32_t kStep = kLutBits;  // bits of an entry of several codewords, at most
+    const uint16_t* lut;
+    Deeper16 deep;
+    __device__ __forceinline__ uint32_t attach(const uint32_t* lds, const DecodeArgs& a, uint32_t n_lds) {
+        lut = reinterpret_cast<const uint16_t*>(lds);
+        deep.sub_lds = (LdsU16)(lut + (1u << kLutBits));
+        deep.sub = (GlobalU16)a.tabs + (2u << kLutBits);
+        deep.n_lds = n_lds;
+        return ((1u << kLutBits) + a.n_sub16) / 2;
+    }
+    __device__ __forceinline__ uint32_t look(uint32_t w) const { return lut[w >> (32 - kLutBits)]; }
+    static __device__ __forceinline__ bool escape(uint32_t e) { return e < 4096; }
+    static __device__ __forceinline__ uint32_t len(uint32_t e) { return e >> 12; }
+    static __device__ __forceinline__ uint32_t count(uint32_t e) { return e & 15; }
+    static __device__ __forceinline__ bool any_zero(uint32_t e0, uint32_t e1) { return ((e0 | e1) & 0xF0) != 0; }
+    static __device__ __forceinline__ uint32_t zeros(uint32_t e) { return (e >> 4) & 15; }
+    template <typename W>
+    __device__ __forceinline__ void resolve(const W& win, uint32_t w, uint32_t lp, uint32_t& e, uint32_t& l) const {
+        deep.resolve(win, w, lp, e, l);
+        e = (e & 0xFFF) == 0 ? 0x11u : 0x01u;
+    }
+};
+template <>
+struct CountDecoder<false> : Decoder<false> {
+    static constexpr uint32_t kStep = 0;  // single codewords
+    static __device__ __forceinline__ uint32_t count(uint32_t) { return 1; }
+    static __device__ __forceinline__ bool any_zero(uint32_t e0, uint32_t e1) { return min(sym(e0), sym(e1)) == 0; }
+    static __device__ __forceinline__ uint32_t zeros(uint32_t e) { return sym(e) == 0; }
+};
+
+// Copies the tables a kernel keeps in LDS with NT threads: a first level
+// (compact: the counting one or the other) and, behind it, as many deeper
+// compact entries as there are and fit (n_sub).  fetch() issues every load of
+// a thread and put() stores them, so a workgroup can have its tables and its
+// bits in flight together and waits for one memory latency; a copy loop of
+// one load per round waited for one latency per round, which was most of a
+// workgroup's time (the indexed decode of the 512^3 field at 1e-3: 0.28 ->
+// 0.16 ms).
+template <bool T16, bool COUNT, uint32_t NT>
 struct TableCopy {
-    static constexpr uint32_t kVecs = (((1u << kLutBits) + (T16 ? kMaxSub16 : 0)) * (T16 ? 2 : 4) / 16 + NT - 1) / NT;
+    static constexpr uint32_t kFirst = (1u << kLutBits) * (T16 ? 2 : 4) / 16;  // vectors of the first level
+    static constexpr uint32_t kVecs = (kFirst + (T16 ? kMaxSub16 / 8 : 0) + NT - 1) / NT;
     U32x4 v[kVecs];
-    uint32_t n;
+    uint32_t n, n_sub;
     __device__ __forceinline__ void fetch(const DecodeArgs& a) {
-        n = T16 ? ((1u << kLutBits) + a.n_sub16) / 8 : (1u << kLutBits) / 4;
-        const GlobalU32x4 src = T16 ? (GlobalU32x4)a.lut16 : (GlobalU32x4)a.lut;
+        n_sub = T16 ? min(a.n_sub16, ((GlobalU32)a.meta)[1]) : 0u;
+        n = kFirst + n_sub / 8;
+        const GlobalU32x4 first = T16 ? (GlobalU32x4)(a.tabs + (COUNT ? 0u : 1u << kLutBits)) : (GlobalU32x4)a.lut;
+        const GlobalU32x4 deep = T16 ? (GlobalU32x4)(a.tabs + (2u << kLutBits)) : first;
 #pragma unroll
-        for (uint32_t m = 0; m < kVecs; m++)
-            if (threadIdx.x + m * NT < n) v[m] = src[threadIdx.x + m * NT];
+        for (uint32_t m = 0; m < kVecs; m++) {
+            const uint32_t i = threadIdx.x + m * NT;
+            if (i < kFirst)
+                v[m] = first[i];
+            else if (i < n)
+                v[m] = deep[i - kFirst];
+        }
     }
     __device__ __forceinline__ void put(uint32_t* lds) const {
 #pragma unroll
@@ -281,14 +342,13 @@ struct BitCursor {
     }
 };
 
-// The two codewords from lp on: entries e[], lengths l[] (0: invalid path).
-// One window serves both: its 32 bits hold a codeword of at most 16 bits and
-// the first 16 of the next, which is as far as the first two table levels
-// look.
-template <bool T16, typename W>
-__device__ __forceinline__ void decode_pair(const Decoder<T16>& dec, const W& win, const BitCursor& cur, uint32_t lp,
-                                            uint32_t* e, uint32_t* l) {
-    using D = Decoder<T16>;
+// The two steps from lp on: entries e[], lengths l[] (0: invalid path).  One
+// window serves both: its 32 bits hold a codeword of at most 16 bits (or 12
+// bits of several) and the first 16 of the next, which is as far as the first
+// two table levels look.
+template <class D, typename W>
+__device__ __forceinline__ void decode_pair(const D& dec, const W& win, const BitCursor& cur, uint32_t lp, uint32_t* e,
+                                            uint32_t* l) {
     const uint32_t w = cur.window(lp);
     e[0] = dec.look(w);
     l[0] = D::len(e[0]);
@@ -301,42 +361,66 @@ __device__ __forceinline__ void decode_pair(const Decoder<T16>& dec, const W& wi
     l[1] = D::len(e[1]);
     if (D::escape(e[1])) dec.resolve(win, w2, lp + l[0], e[1], l[1]);
 }
-template <bool T16, typename W>
-__device__ __forceinline__ uint32_t decode_one(const Decoder<T16>& dec, const W& win, uint32_t w, uint32_t lp,
-                                               uint32_t& l) {
+template <class D, typename W>
+__device__ __forceinline__ uint32_t decode_one(const D& dec, const W& win, uint32_t w, uint32_t lp, uint32_t& l) {
     uint32_t e = dec.look(w);
-    l = Decoder<T16>::len(e);
-    if (Decoder<T16>::escape(e)) dec.resolve(win, w, lp, e, l);
-    return Decoder<T16>::sym(e);
+    l = D::len(e);
+    if (D::escape(e)) dec.resolve(win, w, lp, e, l);
+    return e;
 }
 
-// Codewords and zeros (outliers) of the codewords that start in [lp, end),
-// added to cnt and z; lp ends at the first start at or past end, cur with it.
-// Returns whether an invalid codeword was met (it counts as one of one bit).
-template <bool T16, typename W>
-__device__ __forceinline__ bool decode_count(const Decoder<T16>& dec, const W& win, BitCursor& cur, uint32_t& lp,
-                                             uint32_t end, uint32_t& cnt, uint32_t& z) {
-    using D = Decoder<T16>;
+// Codewords and zeros (outliers) of the steps that start in [lp, end), added
+// to cnt and z; lp ends at the first step's start at or past end, cur with it.
+// (A step may hold codewords that start past end: they are this
+// subsequence's, and the next one starts behind them.)  Returns whether an
+// invalid codeword was met (it counts as one of one bit).
+template <class D, typename W>
+__device__ __forceinline__ bool decode_count(const D& dec, const W& win, BitCursor& cur, uint32_t& lp, uint32_t end,
+                                             uint32_t& cnt, uint32_t& z) {
     bool bad = false;
     while (lp < end) {
         uint32_t e[2], l[2];
-        decode_pair<T16>(dec, win, cur, lp, e, l);
-        if constexpr (!T16) {  // (the compact tables hold no invalid path)
+        decode_pair(dec, win, cur, lp, e, l);
+        if constexpr (D::kInvalid) {
             bad |= l[0] == 0;
             l[0] = max(l[0], 1u);
         }
         const bool two = lp + l[0] < end;
-        if constexpr (!T16) {
+        if constexpr (D::kInvalid) {
             bad |= two & (l[1] == 0);
             l[1] = max(l[1], 1u);
         }
-        cnt += two ? 2u : 1u;
+        cnt += D::count(e[0]) + (two ? D::count(e[1]) : 0u);
         lp += l[0] + (two ? l[1] : 0u);
-        const uint32_t s0 = D::sym(e[0]), s1 = D::sym(e[1]);
-        if (min(s0, s1) == 0) z += (uint32_t)(s0 == 0) + (uint32_t)(two & (s1 == 0));
+        if (D::any_zero(e[0], e[1])) z += D::zeros(e[0]) + (two ? D::zeros(e[1]) : 0u);
         cur.advance(win, lp);
     }
     return bad;
+}
+
+// The same where the stream may end: behind its end (bit send, at most an
+// entry's bits past `end` or more) no codeword counts, so the last steps are
+// single codewords, read from the first level in global memory.
+template <class D, typename W>
+__device__ __forceinline__ bool decode_count_to(const D& dec, const W& win, BitCursor& cur, uint32_t& lp, uint32_t end,
+                                                uint32_t send, const DecodeArgs& a, uint32_t& cnt, uint32_t& z) {
+    if constexpr (D::kStep == 0) {
+        return decode_count(dec, win, cur, lp, end, cnt, z);
+    } else {
+        // (a step that starts below lim ends at or before the stream's end)
+        const uint32_t lim = min(end, send > D::kStep ? send - (D::kStep - 1) : 0u);
+        const bool bad = decode_count(dec, win, cur, lp, lim, cnt, z);
+        while (lp < end) {  // (never, where lim is end)
+            const uint32_t w = cur.window(lp);
+            uint32_t e = ((GlobalU16)a.tabs)[(1u << kLutBits) + (w >> (32 - kLutBits))], l = e >> 12;
+            if (l == 0) dec.deep.resolve(win, w, lp, e, l);
+            cnt++;
+            z += (e & 0xFFF) == 0;
+            lp += l;
+            cur.advance(win, lp);
+        }
+        return bad;
+    }
 }
 
 // Whether either half of w is 0 after taking the halves' minima with those of
@@ -419,22 +503,24 @@ template <bool T16>
 __device__ __forceinline__ void decode_sync_unit(const DecodeArgs& a, const SubState& s, DecSummary* sum,
                                                  uint64_t unit, uint32_t stripe) {
     extern __shared__ __align__(16) uint32_t lds[];
-    Decoder<T16> dec;
-    uint32_t* st = lds + dec.attach(lds, a);
-    uint32_t* own_e = st + kSyncStageLds;
+    if (no_tables(a)) return;  // (the whole workgroup)
+    CountDecoder<T16> dec;
+    uint32_t* st;
     StreamView sv;
     sv.setup(a.stream, a.stream_bits);
     const uint64_t J0 = unit * kSyncStride;
     // the stage starts one row before subsequence J0 (but not before the stream)
     const uint64_t Jst = J0 ? J0 - 1 : 0;
     {
-        TableCopy<T16, kSyncWg> tc;
+        TableCopy<T16, true, kSyncWg> tc;
         StageCopy<(kSyncStageWords + 4 * kSyncWg - 1) / (4 * kSyncWg), kSyncWg> sc;
         tc.fetch(a);
         sc.fetch(sv, Jst * kSubWords, (kSyncStageWords + 3) / 4);
+        st = lds + dec.attach(lds, a, tc.n_sub);
         tc.put(lds);
         sc.put_rows(st, kSyncStageWords);
     }
+    uint32_t* own_e = st + kSyncStageLds;
     lds_sync();
     const uint32_t t = threadIdx.x;
     const uint64_t j = J0 + t;
@@ -445,18 +531,20 @@ __device__ __forceinline__ void decode_sync_unit(const DecodeArgs& a, const SubS
     uint32_t first = s0, e0 = s0, cnt = 0, z = 0, lp = s0;
     if (live) {
         const PadWin win{st};
-        e0 += (uint32_t)min<uint64_t>(kSubBits, a.stream_bits - j * kSubBits);
+        const uint64_t left = a.stream_bits - j * kSubBits;
+        e0 += (uint32_t)min<uint64_t>(kSubBits, left);
+        const uint32_t send = s0 + (uint32_t)min<uint64_t>(2 * kSubBits, left);
         BitCursor cur;
         if (j) {
             lp = s0 - kLeadBits;
             cur.seek(win, lp);
             uint32_t lc = 0, lz = 0;
-            (void)decode_count<T16>(dec, win, cur, lp, s0, lc, lz);  // (an invalid path here is a wrong start's)
+            (void)decode_count_to(dec, win, cur, lp, s0, send, a, lc, lz);  // (an invalid path here is a wrong start's)
             first = lp;
         } else {  // the stream starts with a codeword
             cur.seek(win, lp);
         }
-        bad = decode_count<T16>(dec, win, cur, lp, e0, cnt, z);
+        bad = decode_count_to(dec, win, cur, lp, e0, send, a, cnt, z);
         own_e[t] = lp;
     }
     lds_sync();
@@ -516,7 +604,7 @@ __device__ __forceinline__ void stage_row(uint32_t* __restrict__ row, const Stre
 // thread's own LDS row.  Returns whether j + 1 (set) is to be listed, from
 // over bits past its first.
 template <bool T16>
-__device__ __forceinline__ bool redecode_entry(const DecodeArgs& a, const SubState& s, const Decoder<T16>& dec,
+__device__ __forceinline__ bool redecode_entry(const DecodeArgs& a, const SubState& s, const CountDecoder<T16>& dec,
                                                uint32_t* row, uint64_t ent, DecSummary* sum, uint64_t& next,
                                                uint32_t& over) {
     const uint64_t j = (ent & ((1ull << 48) - 1)) - s.jbase;
@@ -525,11 +613,13 @@ __device__ __forceinline__ bool redecode_entry(const DecodeArgs& a, const SubSta
     sv.setup(a.stream, a.stream_bits);
     stage_row(row, sv, j);  // the thread's own row: no barrier
     const RowWin win{row};
-    const uint32_t tl = (uint32_t)min<uint64_t>(kSubBits, a.stream_bits - j * kSubBits) + sv.shift0;
+    const uint64_t left = a.stream_bits - j * kSubBits;
+    const uint32_t tl = (uint32_t)min<uint64_t>(kSubBits, left) + sv.shift0;
+    const uint32_t send = (uint32_t)min<uint64_t>(2 * kSubBits, left) + sv.shift0;
     uint32_t lp = first + sv.shift0, cnt = 0, z = 0;
     BitCursor cur;
     cur.seek(win, lp);
-    if (decode_count<T16>(dec, win, cur, lp, tl, cnt, z)) atomicOr(&sum->error, 1u);
+    if (decode_count_to(dec, win, cur, lp, tl, send, a, cnt, z)) atomicOr(&sum->error, 1u);
     over = lp - tl;
     next = j + 1;
     s.b[j] = (uint8_t)first;
@@ -539,20 +629,21 @@ __device__ __forceinline__ bool redecode_entry(const DecodeArgs& a, const SubSta
     return next < a.nsub;
 }
 
-// Workgroup b takes entries of stripe b % nstripe.  (Whole wavefronts go
+// A pass over stripe `stripe` by workgroups b of nb.  (Whole wavefronts go
 // round together: list_append.)
 template <bool T16>
-__global__ void __launch_bounds__(256) k_decode_pass(DecodeArgs a, SubState s, uint32_t pass, DecSummary* sum) {
-    const uint32_t stripe = blockIdx.x % s.nstripe, nb = gridDim.x / s.nstripe, b = blockIdx.x / s.nstripe;
-    const uint32_t m = s.list_n[list_slot(pass) + stripe * kCounterWords];
-    if (b == 0 && threadIdx.x == 0) s.list_n[list_slot(pass + 2) + stripe * kCounterWords] = 0;  // the list after next
-    if ((uint64_t)b * 256 >= m) return;  // whole workgroup
+__device__ __forceinline__ void decode_pass_stripe(const DecodeArgs& a, const SubState& s, uint32_t pass, DecSummary* sum,
+                                                   uint32_t stripe, uint32_t b, uint32_t nb) {
+    const uint32_t m = *list_counter(s, pass, stripe);
+    if (b == 0 && threadIdx.x == 0) *list_counter(s, pass + 2, stripe) = 0;  // the list after next
+    if ((uint64_t)b * 256 >= m) return;                                      // whole workgroup
     extern __shared__ __align__(16) uint32_t lds[];
-    Decoder<T16> dec;
-    uint32_t* rows = lds + dec.attach(lds, a);
+    CountDecoder<T16> dec;
+    uint32_t* rows;
     {
-        TableCopy<T16, 256> tc;
+        TableCopy<T16, true, 256> tc;
         tc.fetch(a);
+        rows = lds + dec.attach(lds, a, tc.n_sub);
         tc.put(lds);
     }
     lds_sync();  // the tables
@@ -566,6 +657,12 @@ __global__ void __launch_bounds__(256) k_decode_pass(DecodeArgs a, SubState s, u
                                      s.list[pass & 1][stripe * s.stripe_cap + e], sum, next, over);
         list_append(s, pass + 1, stripe, on, next, over);
     }
+}
+
+// Workgroup b takes entries of stripe b % nstripe.
+template <bool T16>
+__global__ void __launch_bounds__(256) k_decode_pass(DecodeArgs a, SubState s, uint32_t pass, DecSummary* sum) {
+    decode_pass_stripe<T16>(a, s, pass, sum, blockIdx.x % s.nstripe, blockIdx.x / s.nstripe, gridDim.x / s.nstripe);
 }
 
 // Device-wide exclusive scan of two u32 arrays into u64 offsets.
@@ -753,11 +850,12 @@ __global__ void __launch_bounds__(256) k_decode_indexed(DecodeArgs a, const uint
     // per 16-byte piece of output
     constexpr uint32_t kFlush = R1D ? 16 : kIdxFlush;
     constexpr uint32_t kPer16 = R1D ? 4 : 8;
+    if (no_tables(a)) return;
     extern __shared__ __align__(16) uint32_t lds[];
     Decoder<T16> dec;
-    const uint32_t tw = dec.attach(lds, a);
-    TableCopy<T16, 256> tc;
+    TableCopy<T16, false, 256> tc;
     tc.fetch(a);
+    const uint32_t tw = dec.attach(lds, a, tc.n_sub);
     tc.put(lds);
     const uint32_t lane = threadIdx.x & 63;
     uint32_t* stage = lds + tw + (threadIdx.x >> 6) * kIdxStageWords;
@@ -846,7 +944,7 @@ __global__ void __launch_bounds__(256) k_decode_indexed(DecodeArgs a, const uint
                 // lp - cw.b0 < 32 here: the codeword's first 32 bits are in buf
                 const uint32_t w = (uint32_t)((cw.buf << (lp - cw.b0)) >> 32);
                 uint32_t len;
-                const uint32_t sym = decode_one<T16>(dec, cw, w, lp, len);
+                const uint32_t sym = Decoder<T16>::sym(decode_one(dec, cw, w, lp, len));
                 // past ns (or at an invalid codeword, an error) the lane
                 // stays where it is: lp ends at the segment's end
                 const bool in = u + k < ns;
@@ -961,16 +1059,17 @@ __global__ void __launch_bounds__(256) k_decode_indexed_staged(DecodeArgs a, con
     StreamView sv;
     sv.setup(a.stream, a.stream_bits);
     const IdxSpan sp = idx_span(index, L, total_bits, sv, blockIdx.x);
-    if (!sp.fits) return;  // (the whole workgroup)
+    if (!sp.fits || no_tables(a)) return;  // (the whole workgroup)
     extern __shared__ __align__(16) uint32_t lds[];
     Decoder<T16> dec;
-    uint32_t* stage = lds + dec.attach(lds, a);
+    uint32_t* stage;
     {
-        TableCopy<T16, 256> tc;
+        TableCopy<T16, false, 256> tc;
         StageCopy<(kIdxSpanWords + 4 * 256 - 1) / (4 * 256), 256> sc;
         const uint32_t nvec = ((uint32_t)sp.nwords + 3) / 4;
         tc.fetch(a);
         sc.fetch(sv, sp.w_lo, nvec);
+        stage = lds + dec.attach(lds, a, tc.n_sub);
         tc.put(lds);
         sc.put(stage, nvec);
     }
@@ -998,7 +1097,7 @@ __global__ void __launch_bounds__(256) k_decode_indexed_staged(DecodeArgs a, con
     // one codeword, or two as the halves of a word
     auto next = [&]() -> uint32_t {
         uint32_t len;
-        const uint32_t sym = decode_one<T16>(dec, win, cur.window(lp), lp, len);
+        const uint32_t sym = Decoder<T16>::sym(decode_one(dec, win, cur.window(lp), lp, len));
         if constexpr (!T16) bad |= len == 0;
         lp += len;
         cur.advance(win, lp);
@@ -1006,7 +1105,7 @@ __global__ void __launch_bounds__(256) k_decode_indexed_staged(DecodeArgs a, con
     };
     auto next2 = [&]() -> uint32_t {
         uint32_t e[2], l[2];
-        decode_pair<T16>(dec, win, cur, lp, e, l);
+        decode_pair(dec, win, cur, lp, e, l);
         if constexpr (!T16) bad |= (l[0] == 0) | (l[1] == 0);
         lp += l[0] + l[1];
         cur.advance(win, lp);
@@ -1214,8 +1313,7 @@ __device__ __forceinline__ void decode_write_unit(const DecodeArgs& a, const Sub
                                                   DecSummary* sum, uint64_t unit) {
     extern __shared__ __align__(16) uint32_t lds[];
     Decoder<T16> dec;
-    uint32_t* st = lds + dec.attach(lds, a);
-    uint32_t* wsum = st + kWriteStageLds;  // counts and zeros of each wavefront
+    uint32_t* st;
     StreamView sv;
     sv.setup(a.stream, a.stream_bits);
     const uint64_t J0 = unit * kWriteWg;
@@ -1223,15 +1321,17 @@ __device__ __forceinline__ void decode_write_unit(const DecodeArgs& a, const Sub
     const bool live = j < a.nsub;
     uint32_t cz, first;
     {
-        TableCopy<T16, kWriteWg> tc;
+        TableCopy<T16, false, kWriteWg> tc;
         StageCopy<(kWriteStageWords + 4 * kWriteWg - 1) / (4 * kWriteWg), kWriteWg> sc;
         tc.fetch(a);
         sc.fetch(sv, J0 * kSubWords, (kWriteStageWords + 3) / 4);
         cz = live ? s.cz[j] : 0u;
         first = live ? s.b[j] : 0u;
+        st = lds + dec.attach(lds, a, tc.n_sub);
         tc.put(lds);
         sc.put_rows(st, kWriteStageWords);
     }
+    uint32_t* wsum = st + kWriteStageLds;  // counts and zeros of each wavefront
     const uint32_t ic = wave_scan_dpp(cz & 0xFFFF), iz = wave_scan_dpp(cz >> 16);
     const uint32_t w = threadIdx.x >> 6;
     if (lane_id2() == 63) {
@@ -1257,7 +1357,7 @@ __device__ __forceinline__ void decode_write_unit(const DecodeArgs& a, const Sub
     // one codeword, or two as the halves of a word
     auto next = [&]() -> uint32_t {
         uint32_t len;
-        const uint32_t sym = decode_one<T16>(dec, win, cur.window(lp), lp, len);
+        const uint32_t sym = Decoder<T16>::sym(decode_one(dec, win, cur.window(lp), lp, len));
         if constexpr (!T16) bad |= len == 0;
         lp += len;
         cur.advance(win, lp);
@@ -1265,7 +1365,7 @@ __device__ __forceinline__ void decode_write_unit(const DecodeArgs& a, const Sub
     };
     auto next2 = [&]() -> uint32_t {
         uint32_t e[2], l[2];
-        decode_pair<T16>(dec, win, cur, lp, e, l);
+        decode_pair(dec, win, cur, lp, e, l);
         if constexpr (!T16) bad |= (l[0] == 0) | (l[1] == 0);
         lp += l[0] + l[1];
         cur.advance(win, lp);
@@ -1844,14 +1944,24 @@ __global__ void __launch_bounds__(256) k_recon_x4(const uint16_t* __restrict__ c
 // write) or its wavefront (reconstruction), so the field lookup and the
 // descriptor reads are scalar.
 
-template <bool T16>
 __global__ void __launch_bounds__(kSyncWg) k_decode_sync_multi(const DecField* __restrict__ fd,
-                                                           const uint64_t* __restrict__ start, int nf) {
+                                                               const uint64_t* __restrict__ start, int nf) {
     const uint64_t u = blockIdx.x;
     const int f = field_of(start, nf, u);
     const DecodeArgs a = fd[f].a;
     const SubState s = fd[f].s;
-    decode_sync_unit<T16>(a, s, fd[f].sum, u - start[f], (uint32_t)(u % s.nstripe));
+    decode_sync_unit<true>(a, s, fd[f].sum, u - start[f], (uint32_t)u);
+}
+
+// Re-decode pass: a workgroup per sync unit, whose listed subsequences are one
+// field's, so that the tables are in LDS.
+__global__ void __launch_bounds__(256) k_decode_pass_multi(const DecField* __restrict__ fd,
+                                                           const uint64_t* __restrict__ start, int nf, uint32_t pass) {
+    const uint64_t u = blockIdx.x;
+    const int f = field_of(start, nf, u);
+    const DecodeArgs a = fd[f].a;
+    const SubState s = fd[f].s;
+    decode_pass_stripe<true>(a, s, pass, fd[f].sum, (uint32_t)u, 0, 1);
 }
 
 __global__ void __launch_bounds__(256) k_decode_sums_multi(const DecField* __restrict__ fd,
@@ -1863,7 +1973,6 @@ __global__ void __launch_bounds__(256) k_decode_sums_multi(const DecField* __res
     decode_sums_unit(fd[f].s.cz, fd[f].a.nsub, u - start[f], sums + 2 * u);
 }
 
-template <bool T16>
 __global__ void __launch_bounds__(kWriteWg) k_decode_write_multi(const DecField* __restrict__ fd,
                                                                  const uint64_t* __restrict__ start, int nf,
                                                                  const uint64_t* __restrict__ off) {
@@ -1871,57 +1980,7 @@ __global__ void __launch_bounds__(kWriteWg) k_decode_write_multi(const DecField*
     const int f = field_of(start, nf, u);
     const DecodeArgs a = fd[f].a;
     const SubState s = fd[f].s;
-    decode_write_unit<T16>(a, s, off + 2 * start[f], off + 2 * u, fd[f].codes, fd[f].sparse, fd[f].sum, u - start[f]);
-}
-
-// The decode tables of a field read from global memory (entries of one
-// re-decode batch may belong to different fields).
-template <bool T16>
-__device__ __forceinline__ Decoder<T16> global_decoder(const DecodeArgs& a);
-template <>
-__device__ __forceinline__ Decoder<true> global_decoder<true>(const DecodeArgs& a) {
-    Decoder<true> d;
-    d.lut = a.lut16;
-    d.sub_lds = nullptr;
-    d.sub = (GlobalU16)a.sub16;
-    d.n_lds = 0;
-    return d;
-}
-template <>
-__device__ __forceinline__ Decoder<false> global_decoder<false>(const DecodeArgs& a) {
-    Decoder<false> d;
-    d.lut = a.lut;
-    d.sub = (GlobalU32)a.sub;
-    return d;
-}
-
-// Re-decode pass over the batch-wide list: as k_decode_pass, but entry J
-// (a batch-wide subsequence number) belongs to field field_of(sub_start, J),
-// whose stream its row is staged from and whose tables decode it.
-template <bool T16>
-__global__ void __launch_bounds__(256) k_decode_pass_multi(const DecField* __restrict__ fd,
-                                                           const uint64_t* __restrict__ sub_start, int nf, SubState S,
-                                                           uint32_t pass) {
-    const uint32_t stripe = blockIdx.x % S.nstripe, nb = gridDim.x / S.nstripe, b = blockIdx.x / S.nstripe;
-    const uint32_t m = S.list_n[list_slot(pass) + stripe * kCounterWords];
-    if (b == 0 && threadIdx.x == 0) S.list_n[list_slot(pass + 2) + stripe * kCounterWords] = 0;  // the list after next
-    if ((uint64_t)b * 256 >= m) return;  // whole workgroup
-    __shared__ uint32_t rows[256 * kRowStride];
-    for (uint64_t e0 = b * 256ull + (threadIdx.x & ~63u); e0 < m; e0 += nb * 256ull) {
-        const uint64_t e = e0 + lane_id2();
-        bool on = false;
-        uint64_t next = 0;
-        uint32_t over = 0;
-        if (e < m) {
-            const uint64_t ent = S.list[pass & 1][stripe * S.stripe_cap + e];
-            const int f = field_of(sub_start, nf, ent & ((1ull << 48) - 1));
-            const DecodeArgs& a = fd[f].a;
-            on = redecode_entry<T16>(a, fd[f].s, global_decoder<T16>(a), rows + threadIdx.x * kRowStride, ent,
-                                     fd[f].sum, next, over);
-            next += fd[f].s.jbase;
-        }
-        list_append(S, pass + 1, stripe, on, next, over);  // (S.jbase 0)
-    }
+    decode_write_unit<true>(a, s, off + 2 * start[f], off + 2 * u, fd[f].codes, fd[f].sparse, fd[f].sum, u - start[f]);
 }
 
 __global__ void k_dec_field_totals(const uint64_t* __restrict__ start, int nf, const uint64_t* __restrict__ off,
@@ -1984,25 +2043,23 @@ static unsigned grid_for(uint64_t threads, unsigned block) { return (unsigned)((
 
 // Dynamic LDS bytes of the decode tables a kernel keeps in LDS.
 static size_t table_lds_bytes(const DecodeArgs& a, bool t16) {
-    return t16 ? (((size_t)(1u << kLutBits) + a.n_sub16 + 1) / 2) * 4 : (size_t)(1u << kLutBits) * 4;
+    return t16 ? ((size_t)(1u << kLutBits) + a.n_sub16) * 2 : (size_t)(1u << kLutBits) * 4;
 }
 
-// The deeper 16-bit tables serve only the codewords over kLutBits bits (a
-// few percent of them at eb 1e-4), so a kernel copies them to LDS only when
-// that costs no resident workgroup per CU, given its other LDS (own_bytes
-// besides the first-level table); otherwise it reads them in global memory
-// (n_sub16 0).  Measured on the 1 GiB field, whose deeper tables took 22 KB:
-// the write pass 0.75 -> 0.53 ms, the sync pass 1.08 -> 1.04 ms in global
-// memory.
+// LDS room for deeper compact tables (n_sub16): what is left of a workgroup's
+// share of the CU when as many workgroups are resident as its other LDS
+// (own_bytes besides the first level) allows.  The tables of codewords of up
+// to 16 bits come first; the rest is read in global memory.  (LDS is given
+// out in units of 1280 bytes: filling up to a KiB granule instead cost the
+// sync pass a workgroup per CU, 0.65 -> 1.0 ms at the 1 GiB field.)
 static DecodeArgs with_lds_sub16(DecodeArgs a, size_t own_bytes) {
-    if (!a.lut16 || !a.n_sub16) return a;
-    constexpr size_t kCuLds = 160 * 1024, kGranule = 1280;  // LDS is allocated in units of 1280 bytes
-    DecodeArgs b = a;
-    b.n_sub16 = 0;
-    const size_t bare = table_lds_bytes(b, true) + own_bytes;
+    a.n_sub16 = 0;
+    if (!a.tabs) return a;
+    constexpr size_t kCuLds = 160 * 1024, kGranule = 1280;
+    const size_t bare = table_lds_bytes(a, true) + own_bytes;
     const size_t share = kCuLds / ((bare + kGranule - 1) / kGranule * kGranule);  // workgroups per CU
     const size_t room = kCuLds / share / kGranule * kGranule - bare;
-    a.n_sub16 = (uint32_t)std::min<size_t>(a.n_sub16, room / 2 & ~(size_t)((1u << kSubTabBits) - 1));
+    a.n_sub16 = (uint32_t)std::min<size_t>(kMaxSub16, room / 2 & ~(size_t)((1u << kSubTabBits) - 1));
     return a;
 }
 
@@ -2025,7 +2082,7 @@ static bool set_big_lds(const void* kernel) {
 void launch_decode_sync(const DecodeArgs& a0, SubState s, DecSummary* sum, hipStream_t st) {
     allow_big_lds(k_decode_sync<true>);
     allow_big_lds(k_decode_sync<false>);
-    const bool t16 = a0.lut16 != nullptr;
+    const bool t16 = a0.tabs != nullptr;
     const DecodeArgs a = with_lds_sub16(a0, (size_t)kSyncLdsWords * 4);
     const size_t lds = table_lds_bytes(a, t16) + (size_t)kSyncLdsWords * 4;
     const dim3 grid(grid_for(a.nsub, kSyncStride));
@@ -2034,17 +2091,20 @@ void launch_decode_sync(const DecodeArgs& a0, SubState s, DecSummary* sum, hipSt
     else
         hipLaunchKernelGGL(k_decode_sync<false>, grid, dim3(kSyncWg), lds, st, a, s, sum);
 }
-void list_stripes(uint64_t units, uint32_t* nstripe, uint64_t* cap) {
-    *nstripe = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(kMaxStripes, units));
-    *cap = (units + *nstripe - 1) / *nstripe * kSyncWg;
+void list_stripes(uint64_t units, SubState* s) {
+    s->nstripe = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(kMaxStripes, units));
+    s->stripe_cap = (units + s->nstripe - 1) / s->nstripe * kSyncWg;
+    s->counter_words = kCounterWords;
+    s->slot_words = kSlotWords;
 }
+uint64_t sync_unit_subs() { return kSyncWg; }
 static unsigned pass_grid(const SubState& s) {
     return s.nstripe * (unsigned)std::max<uint64_t>(1, std::min<uint64_t>(kPassGrid / s.nstripe, (s.stripe_cap + 255) / 256));
 }
 void launch_decode_pass(const DecodeArgs& a0, SubState s, uint32_t pass, DecSummary* sum, hipStream_t st) {
     allow_big_lds(k_decode_pass<true>);
     allow_big_lds(k_decode_pass<false>);
-    const bool t16 = a0.lut16 != nullptr;
+    const bool t16 = a0.tabs != nullptr;
     const DecodeArgs a = with_lds_sub16(a0, (size_t)256 * kRowStride * 4);
     const size_t lds = table_lds_bytes(a, t16) + (size_t)256 * kRowStride * 4;
     // persistent workgroups; those past the listed count return at once
@@ -2064,7 +2124,7 @@ void launch_decode_indexed(const DecodeArgs& a0, const uint64_t* index, uint64_t
     allow_big_lds((k_decode_indexed_staged<false, false>));
     allow_big_lds((k_decode_indexed_staged<true, true>));
     allow_big_lds((k_decode_indexed_staged<false, true>));
-    const bool t16 = a0.lut16 != nullptr;
+    const bool t16 = a0.tabs != nullptr;
     const DecodeArgs a = with_lds_sub16(a0, (size_t)4 * kIdxStageWords * 4);
     const size_t lds = table_lds_bytes(a, t16) + (size_t)4 * kIdxStageWords * 4;
     const IdxLayout L = idx_layout(a.n);
@@ -2122,7 +2182,7 @@ void launch_decode_write(const DecodeArgs& a0, SubState s, const uint64_t* off, 
                          DecSummary* sum, hipStream_t st, const uint32_t* guard) {
     allow_big_lds(k_decode_write<true>);
     allow_big_lds(k_decode_write<false>);
-    const bool t16 = a0.lut16 != nullptr;
+    const bool t16 = a0.tabs != nullptr;
     const DecodeArgs a = with_lds_sub16(a0, (size_t)kWriteLdsWords * 4);
     const size_t lds = table_lds_bytes(a, t16) + (size_t)kWriteLdsWords * 4;
     const dim3 grid((unsigned)decode_write_units(a.nsub));
@@ -2217,35 +2277,33 @@ void launch_reconstruct_fallback(int ndim, int B, const uint16_t* codes, const f
     hipLaunchKernelGGL(k_recon_fallback, dim3(256), dim3(64), 0, st, ndim, B, codes, sparse, out, a, flagged, nflagged);
 }
 
-uint32_t batch_sub16_in_lds(uint32_t max_sub16) {
+static DecodeArgs compact_probe(uint32_t n_sub16) {
     DecodeArgs probe{};
-    probe.lut16 = reinterpret_cast<const uint16_t*>(&probe);  // (only tested for null)
-    probe.n_sub16 = max_sub16;
-    return std::min(with_lds_sub16(probe, (size_t)kSyncLdsWords * 4).n_sub16,
-                    with_lds_sub16(probe, (size_t)kWriteLdsWords * 4).n_sub16);
+    probe.tabs = reinterpret_cast<const uint16_t*>(&probe);  // (only tested for null)
+    probe.n_sub16 = n_sub16;
+    return probe;
+}
+constexpr size_t kPassRowBytes = (size_t)256 * kRowStride * 4;
+uint32_t batch_sub16_in_lds() {
+    const DecodeArgs probe = compact_probe(0);
+    return std::min({with_lds_sub16(probe, (size_t)kSyncLdsWords * 4).n_sub16,
+                     with_lds_sub16(probe, (size_t)kWriteLdsWords * 4).n_sub16,
+                     with_lds_sub16(probe, kPassRowBytes).n_sub16});
 }
 
-void launch_decode_sync_multi(bool t16, uint32_t max_sub16, const DecField* fd, const uint64_t* start, int nf,
-                              uint64_t nunits, hipStream_t st) {
-    allow_big_lds(k_decode_sync_multi<true>);
-    allow_big_lds(k_decode_sync_multi<false>);
+void launch_decode_sync_multi(uint32_t n_sub16, const DecField* fd, const uint64_t* start, int nf, uint64_t nunits,
+                              hipStream_t st) {
+    allow_big_lds(k_decode_sync_multi);
     if (!nunits) return;
-    DecodeArgs probe{};
-    probe.n_sub16 = max_sub16;
-    const size_t lds = table_lds_bytes(probe, t16) + (size_t)kSyncLdsWords * 4;
-    if (t16)
-        hipLaunchKernelGGL(k_decode_sync_multi<true>, dim3((unsigned)nunits), dim3(kSyncWg), lds, st, fd, start, nf);
-    else
-        hipLaunchKernelGGL(k_decode_sync_multi<false>, dim3((unsigned)nunits), dim3(kSyncWg), lds, st, fd, start, nf);
+    const size_t lds = table_lds_bytes(compact_probe(n_sub16), true) + (size_t)kSyncLdsWords * 4;
+    hipLaunchKernelGGL(k_decode_sync_multi, dim3((unsigned)nunits), dim3(kSyncWg), lds, st, fd, start, nf);
 }
-void launch_decode_pass_multi(bool t16, const DecField* fd, const uint64_t* sub_start, int nf, SubState S,
+void launch_decode_pass_multi(uint32_t n_sub16, const DecField* fd, const uint64_t* start, int nf, uint64_t nunits,
                               uint32_t pass, hipStream_t st) {
-    // persistent workgroups; those past the listed count return at once
-    const dim3 grid(pass_grid(S));
-    if (t16)
-        hipLaunchKernelGGL(k_decode_pass_multi<true>, grid, dim3(256), 0, st, fd, sub_start, nf, S, pass);
-    else
-        hipLaunchKernelGGL(k_decode_pass_multi<false>, grid, dim3(256), 0, st, fd, sub_start, nf, S, pass);
+    allow_big_lds(k_decode_pass_multi);
+    if (!nunits) return;
+    const size_t lds = table_lds_bytes(compact_probe(n_sub16), true) + kPassRowBytes;
+    hipLaunchKernelGGL(k_decode_pass_multi, dim3((unsigned)nunits), dim3(256), lds, st, fd, start, nf, pass);
 }
 void launch_decode_offsets_multi(const DecField* fd, const uint64_t* start, int nf, uint64_t nunits, uint64_t* off,
                                  hipStream_t st) {
@@ -2253,18 +2311,12 @@ void launch_decode_offsets_multi(const DecField* fd, const uint64_t* start, int 
         hipLaunchKernelGGL(k_decode_sums_multi, dim3(grid_for(nunits, 4)), dim3(256), 0, st, fd, start, nf, off);
     hipLaunchKernelGGL(k_decode_scan, dim3(1), dim3(1024), 0, st, off, nunits, (const uint32_t*)nullptr);
 }
-void launch_decode_write_multi(bool t16, uint32_t max_sub16, const DecField* fd, const uint64_t* start, int nf,
-                               uint64_t nunits, const uint64_t* off, hipStream_t st) {
-    allow_big_lds(k_decode_write_multi<true>);
-    allow_big_lds(k_decode_write_multi<false>);
+void launch_decode_write_multi(uint32_t n_sub16, const DecField* fd, const uint64_t* start, int nf, uint64_t nunits,
+                               const uint64_t* off, hipStream_t st) {
+    allow_big_lds(k_decode_write_multi);
     if (!nunits) return;
-    DecodeArgs probe{};
-    probe.n_sub16 = max_sub16;
-    const size_t lds = table_lds_bytes(probe, t16) + (size_t)kWriteLdsWords * 4;
-    if (t16)
-        hipLaunchKernelGGL(k_decode_write_multi<true>, dim3((unsigned)nunits), dim3(kWriteWg), lds, st, fd, start, nf, off);
-    else
-        hipLaunchKernelGGL(k_decode_write_multi<false>, dim3((unsigned)nunits), dim3(kWriteWg), lds, st, fd, start, nf, off);
+    const size_t lds = table_lds_bytes(compact_probe(n_sub16), true) + (size_t)kWriteLdsWords * 4;
+    hipLaunchKernelGGL(k_decode_write_multi, dim3((unsigned)nunits), dim3(kWriteWg), lds, st, fd, start, nf, off);
 }
 void launch_dec_field_totals(const uint64_t* start, int nf, const uint64_t* off, uint64_t* tot, hipStream_t st) {
     if (nf > 0)
