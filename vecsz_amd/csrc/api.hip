@@ -267,6 +267,12 @@ constexpr uint64_t kMaxElems = 1ull << 37;
 // Decompress batches whose fields average at most this many elements run
 // fused by default (a 16 MiB f32 field; larger ones take the worker contexts).
 constexpr uint64_t kDBatchFuseElems = 4ull << 20;
+// Batches of at most this many wavefront tiles run every tile form of a stage
+// in one launch: each form's launch alone leaves most of the chip idle, and
+// they wait for one another (48 fields of 64 KiB to 4 MiB: dual quantization
+// 82 -> 51, reconstruction 133 -> 71 us).  Beyond, a launch per form, so that each
+// keeps its own register budget.
+constexpr uint64_t kOneLaunchTiles = 16384;
 
 // Element count of an ndim field with the given extents (x first), each in
 // [1, 2^31); false when an extent is out of range or the product exceeds
@@ -1573,8 +1579,8 @@ static int compress_batch_fused_run(vecsz_ctx* c, int nf, const vecsz_params* p,
         ntot += (n + 63) / 64 * 64;
     }
     // unit starts: range, chunks (the histogram pass borrows them first), then
-    // one dual-quant array per tile form
-    const size_t start_bytes = (2 + kDqKinds) * (size_t)(nf + 1) * 8;
+    // one dual-quant array per tile form and one over all of them
+    const size_t start_bytes = (3 + kDqKinds) * (size_t)(nf + 1) * 8;
     if (!c->codes.ensure(ntot * 2 + 64) || !c->sparse.ensure(ntot * 4 + 64) ||
         !c->b_hist.ensure((size_t)nf * dict * 8) || !c->b_range.ensure((size_t)nf * 8) ||
         !c->b_ebd.ensure((size_t)nf * sizeof(EbDev)) || !c->b_desc.ensure((size_t)nf * sizeof(BatchField)) ||
@@ -1587,10 +1593,10 @@ static int compress_batch_fused_run(vecsz_ctx* c, int nf, const vecsz_params* p,
     // descriptors and unit starts are built here and copied into pinned memory
     // for each upload (the pinned block may be reallocated in between)
     std::vector<BatchField> fd(nf);
-    std::vector<uint64_t> st((2 + kDqKinds) * (size_t)(nf + 1), 0);
+    std::vector<uint64_t> st((3 + kDqKinds) * (size_t)(nf + 1), 0);
     uint64_t* rg0 = st.data();
     uint64_t* ck0 = rg0 + (nf + 1);
-    uint64_t* dqk = rg0 + 2 * (nf + 1);  // dqk + kind * (nf + 1) for each DqKind
+    uint64_t* dqk = rg0 + 2 * (nf + 1);  // dqk + kind * (nf + 1) for each DqKind, and all of them
     std::vector<char> dev_range(nf, 0);
     BatchField* fdd = c->b_desc.as<BatchField>();
     uint64_t tiles3 = 0;  // 3D tiles of whole blocks
@@ -1651,9 +1657,9 @@ static int compress_batch_fused_run(vecsz_ctx* c, int nf, const vecsz_params* p,
         f.out_cap = out_cap[k];
         f.meta_bytes = meta_bytes(ndim);
         rg0[k + 1] = rg0[k] + (dev_range[k] ? range_units(nel[k]) : 0);
-        for (int kind = 0; kind < kDqKinds; kind++) {
+        for (int kind = 0; kind <= kDqKinds; kind++) {
             uint64_t* s0 = dqk + (size_t)kind * (nf + 1);
-            s0[k + 1] = s0[k] + (kind == f.kind ? (f.dq_tiles + 3) / 4 : 0);
+            s0[k + 1] = s0[k] + (kind == f.kind || kind == kDqKinds ? (f.dq_tiles + 3) / 4 : 0);
         }
         status[k] = VECSZ_OK;
         out_bytes[k] = 0;
@@ -1721,11 +1727,16 @@ static int compress_batch_fused_run(vecsz_ctx* c, int nf, const vecsz_params* p,
         static const char* const kDqStage[kDqKinds] = {"dualquant_1d", "dualquant_2d",     "dualquant_2d_x4",
                                                        "dualquant_3d", "dualquant_3d_x4", "dualquant_2d_x4u",
                                                        "dualquant_3d_x4u"};
-        for (int kind = 0; kind < kDqKinds; kind++) {
-            const uint64_t nu = dqk[(size_t)kind * (nf + 1) + nf];
-            if (!nu) continue;
-            StageScope s(c, kDqStage[kind]);
-            launch_dualquant_multi(B, kind, fdd, nf, dqk_d + (size_t)kind * (nf + 1), nu, c->dq_grid, c->stream);
+        if (const uint64_t nu = dqk[(size_t)kDqKinds * (nf + 1) + nf]; nu <= kOneLaunchTiles / 4) {
+            StageScope s(c, "dualquant");
+            launch_dualquant_multi(B, -1, fdd, nf, dqk_d + (size_t)kDqKinds * (nf + 1), nu, c->dq_grid, c->stream);
+        } else {
+            for (int kind = 0; kind < kDqKinds; kind++) {
+                const uint64_t nk = dqk[(size_t)kind * (nf + 1) + nf];
+                if (!nk) continue;
+                StageScope s(c, kDqStage[kind]);
+                launch_dualquant_multi(B, kind, fdd, nf, dqk_d + (size_t)kind * (nf + 1), nk, c->dq_grid, c->stream);
+            }
         }
         {
             StageScope s(c, "histogram");
@@ -2039,11 +2050,11 @@ static int decompress_batch_fused_run(vecsz_ctx* c, int nf, const vecsz_params* 
     uint64_t ntot = 0, tab_tot = 0, nsub_tot = 0, fl_tot = 0;
     const size_t ns = (size_t)nf + 1;
     // starts: sync units, write units, subsequences, then one array per tile form
-    std::vector<uint64_t> st((3 + kRcKinds) * ns, 0);
+    std::vector<uint64_t> st((4 + kRcKinds) * ns, 0);
     uint64_t* su = st.data();
     uint64_t* wu = su + ns;
     uint64_t* sb = wu + ns;
-    uint64_t* rk = sb + ns;  // rk + kind * ns
+    uint64_t* rk = sb + ns;  // rk + kind * ns, and all of them
     std::vector<DecField> fd(nf);
     for (int k = 0; k < nf; k++) {
         DecField& F = fd[k];
@@ -2052,7 +2063,7 @@ static int decompress_batch_fused_run(vecsz_ctx* c, int nf, const vecsz_params* 
         su[k + 1] = su[k];
         wu[k + 1] = wu[k];
         sb[k + 1] = sb[k];
-        for (int kind = 0; kind < kRcKinds; kind++) rk[kind * ns + k + 1] = rk[kind * ns + k];
+        for (int kind = 0; kind <= kRcKinds; kind++) rk[kind * ns + k + 1] = rk[kind * ns + k];
         if (status[k]) continue;
         const Hdr& h = hd[k];
         off[k] = ntot;
@@ -2094,6 +2105,7 @@ static int decompress_batch_fused_run(vecsz_ctx* c, int nf, const vecsz_params* 
         // (code regions start on 64-element boundaries: aligned like a null pointer)
         F.kind = recon_kind(h.ndim, B, ra.d0, nullptr, d_out[k]);
         rk[F.kind * ns + k + 1] = rk[F.kind * ns + k] + recon_tiles(F.kind, ra);
+        rk[kRcKinds * ns + k + 1] = rk[kRcKinds * ns + k] + recon_tiles(F.kind, ra);
         fl_off[k] = fl_tot;
         fl_tot += ((ra.d0 + B - 1) / B) * (h.ndim >= 2 ? (ra.d1 + B - 1) / B : 1) * (h.ndim >= 3 ? (ra.d2 + B - 1) / B : 1);
         F.out = d_out[k];
@@ -2231,8 +2243,10 @@ static int decompress_batch_fused_run(vecsz_ctx* c, int nf, const vecsz_params* 
             for (int k = 0; k < nf; k++) {
                 const bool out = status[k] || redo[k];
                 wu[k + 1] = wu[k] + (out || hd[k].root_leaf ? 0 : decode_write_units(fd[k].a.nsub));
-                for (int kind = 0; kind < kRcKinds; kind++)
-                    rk[kind * ns + k + 1] = rk[kind * ns + k] + (!out && fd[k].kind == kind ? recon_tiles(kind, fd[k].ra) : 0);
+                for (int kind = 0; kind <= kRcKinds; kind++) {
+                    const bool in = !out && fd[k].kind >= 0 && (fd[k].kind == kind || kind == kRcKinds);
+                    rk[kind * ns + k + 1] = rk[kind * ns + k] + (in ? recon_tiles(fd[k].kind, fd[k].ra) : 0);
+                }
                 if (out) fd[k].kind = -1;
             }
             memcpy(c->db_pin.p, fd.data(), fd_bytes);
@@ -2254,8 +2268,11 @@ static int decompress_batch_fused_run(vecsz_ctx* c, int nf, const vecsz_params* 
     }
     {
         StageScope s(c, "reconstruct");
-        for (int kind = 0; kind < kRcKinds; kind++)
-            launch_reconstruct_multi(kind, B, fdd, rk_d + (size_t)kind * ns, nf, rk[kind * ns + nf], c->stream);
+        if (rk[kRcKinds * ns + nf] <= kOneLaunchTiles)
+            launch_reconstruct_multi(-1, B, fdd, rk_d + (size_t)kRcKinds * ns, nf, rk[kRcKinds * ns + nf], c->stream);
+        else
+            for (int kind = 0; kind < kRcKinds; kind++)
+                launch_reconstruct_multi(kind, B, fdd, rk_d + (size_t)kind * ns, nf, rk[kind * ns + nf], c->stream);
         launch_reconstruct_fallback_multi(B, fdd, nf, c->stream);
     }
     HIPCHK(c, hipGetLastError());

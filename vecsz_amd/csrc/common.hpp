@@ -163,6 +163,26 @@ __device__ __forceinline__ uint32_t wave_scan_dpp(uint32_t v) {
 
 __device__ __forceinline__ uint32_t lane63(uint32_t v) { return (uint32_t)__builtin_amdgcn_readlane((int)v, 63); }
 
+// Rows of a tile, kRowsAhead at a time, the next ones' loads in flight while
+// these are processed: a wavefront that loaded each row as it came to it
+// waited for memory on every row, and a small or mid-sized field has too few
+// wavefronts to hide that (201 x 333 x 413, B 16, padded: 182 -> 84 us;
+// 25 x 25 x 26: 32 -> 27 us).
+constexpr int kRowsAhead = 8;
+template <class T>
+struct RowsAhead {
+    T cur[kRowsAhead], next[kRowsAhead];
+    __device__ __forceinline__ void take() {
+#pragma unroll
+        for (int r = 0; r < kRowsAhead; r++) cur[r] = next[r];
+    }
+    template <class F>
+    __device__ __forceinline__ void ahead(const F& load) {
+#pragma unroll
+        for (int r = 0; r < kRowsAhead; r++) next[r] = load(r);
+    }
+};
+
 // Field of work unit u in a batch: the f with start[f] <= u < start[f + 1]
 // (start is nondecreasing, start[0] = 0, start[nf] = total units > u).
 // Where u is uniform across the workgroup the search runs on scalar loads.

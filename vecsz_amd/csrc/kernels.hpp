@@ -78,8 +78,8 @@ void launch_enc_finish(const uint64_t* status, uint64_t n, const uint32_t* outl,
 // start arrays hold nf + 1 unit offsets (see BatchField).
 uint64_t range_units(uint64_t n);
 void launch_range_multi(const BatchField* fd, int nf, const uint64_t* start, uint64_t nunits, hipStream_t st);
-// Dual quantization of the fields whose tile form is `kind` (DqKind); start
-// gives units only to those fields.
+// Dual quantization of the fields whose tile form is `kind` (DqKind; start
+// gives units only to those fields), or, kind -1, of every field.
 void launch_dualquant_multi(int B, int kind, const BatchField* fd, int nf, const uint64_t* start, uint64_t nunits,
                             int grid_cap, hipStream_t st);
 // Histograms of the codes: workgroup g of hist_multi_grid(U) takes units
@@ -223,7 +223,7 @@ void launch_reconstruct_fallback(int ndim, int B, const uint16_t* codes, const f
 // views of the field's part.
 // 64 x per wavefront (kRcN), four x per lane with vector (kRcNx4) or element
 // (kRcNx4u) loads and stores.
-enum ReconKind { kRc1 = 0, kRc1x4, kRc2, kRc2x4, kRc3, kRc3x4, kRc1x4u, kRc2x4u, kRc3x4u, kRcKinds };
+enum ReconKind { kRc1x4 = 0, kRc2, kRc2x4, kRc3, kRc3x4, kRc1x4u, kRc2x4u, kRc3x4u, kRcKinds };
 int recon_kind(int ndim, int B, uint64_t d0, const void* codes, const void* out);
 int recon_kind_ndim(int kind);
 struct DecField {
@@ -256,7 +256,8 @@ void launch_decode_write_multi(uint32_t n_sub16, const DecField* fd, const uint6
                                const uint64_t* off, hipStream_t st);
 // Symbols each field's subsequences hold (tot[f]).
 void launch_dec_field_totals(const uint64_t* start, int nf, const uint64_t* off, uint64_t* tot, hipStream_t st);
-// One reconstruction form over its fields' tiles (start: per-field tile starts).
+// One reconstruction form over its fields' tiles (start: per-field tile
+// starts), or, kind -1, every form in one launch.
 void launch_reconstruct_multi(int kind, int B, const DecField* fd, const uint64_t* start, int nf, uint64_t ntiles,
                               hipStream_t st);
 void launch_reconstruct_fallback_multi(int B, const DecField* fd, int nf, hipStream_t st);

@@ -300,26 +300,6 @@ __device__ __forceinline__ Halo load_halo(const DQArgs& a, bool xin, uint64_t x,
     return h;
 }
 
-// Rows of a tile, kRowsAhead at a time, the next ones' loads in flight while
-// these are processed: a wavefront that loaded each row as it came to it
-// waited for memory on every row, and a small or mid-sized field has too few
-// wavefronts to hide that (201 x 333 x 413, B 16, padded: 182 -> 84 us;
-// 25 x 25 x 26: 32 -> 27 us).
-constexpr int kRowsAhead = 8;
-template <class T>
-struct RowsAhead {
-    T cur[kRowsAhead], next[kRowsAhead];
-    __device__ __forceinline__ void take() {
-#pragma unroll
-        for (int r = 0; r < kRowsAhead; r++) cur[r] = next[r];
-    }
-    template <class F>
-    __device__ __forceinline__ void ahead(const F& load) {
-#pragma unroll
-        for (int r = 0; r < kRowsAhead; r++) next[r] = load(r);
-    }
-};
-
 // PAD: the halo cells hold pad values instead of +0.0 (src/dualquant.hh:
 // 226-246, :553-573): a neighbour across the block's z face reads h.z, else
 // across its y face h.y, else h.x (src/utils/padding.hh:245, :290).
@@ -1802,6 +1782,7 @@ struct NoHist {
 // waves in flight work on neighbouring tiles of the same planes as in the
 // single-field kernels; fields of other forms have no units.  The tile bodies
 // are the single-field kernels'.
+// KIND: the tile form of every field in the queue, or -1: each field's own.
 template <int B, int KIND>
 __global__ void __launch_bounds__(256) k_dualquant_multi(const BatchField* __restrict__ fd,
                                                          const uint64_t* __restrict__ start, int nf,
@@ -1815,9 +1796,11 @@ __global__ void __launch_bounds__(256) k_dualquant_multi(const BatchField* __res
     float* sparse = nullptr;
     uint64_t ntiles = 0, ub = 0, ue = 0;
     bool aligned = false;
+    int kind = KIND;
     for (uint64_t u = blockIdx.x; u < nunits; u += gridDim.x) {
         if (u >= ue) {  // next field (uniform)
             const int f = field_of(start, nf, u);
+            if (KIND < 0) kind = fd[f].kind;
             a = fd[f].a;
             dq_resolve(a);
             in = fd[f].in;
@@ -1830,17 +1813,15 @@ __global__ void __launch_bounds__(256) k_dualquant_multi(const BatchField* __res
         }
         const uint64_t t = (u - ub) * 4 + wave;
         if (t >= ntiles) continue;
-        if constexpr (KIND == kDq3x4 || KIND == kDq3x4u) {
-            if constexpr (B <= 16) dq3_x4_at<B, KIND == kDq3x4>(in, codes, sparse, H, a, t, lane);
-        } else if constexpr (KIND == kDq3) {
-            dq3_tile<B, false>(in, codes, sparse, H, a, t, lane);
-        } else if constexpr (KIND == kDq2x4 || KIND == kDq2x4u) {
-            dq2_x4_tile<B, KIND == kDq2x4>(in, codes, sparse, H, a, t, lane);
-        } else if constexpr (KIND == kDq2) {
-            dq2_tile<B, false>(in, codes, sparse, H, a, t, lane);
-        } else {
-            dq1_tile<B, false>(in, codes, sparse, H, a, t * 64, lane, aligned);
+        if constexpr (B <= 16) {
+            if (kind == kDq3x4) dq3_x4_at<B, true>(in, codes, sparse, H, a, t, lane);
+            if (kind == kDq3x4u) dq3_x4_at<B, false>(in, codes, sparse, H, a, t, lane);
         }
+        if (kind == kDq3) dq3_tile<B, false>(in, codes, sparse, H, a, t, lane);
+        if (kind == kDq2x4) dq2_x4_tile<B, true>(in, codes, sparse, H, a, t, lane);
+        if (kind == kDq2x4u) dq2_x4_tile<B, false>(in, codes, sparse, H, a, t, lane);
+        if (kind == kDq2) dq2_tile<B, false>(in, codes, sparse, H, a, t, lane);
+        if (kind == kDq1) dq1_tile<B, false>(in, codes, sparse, H, a, t * 64, lane, aligned);
     }
 }
 
@@ -2284,7 +2265,7 @@ void launch_dualquant_multi(int B, int kind, const BatchField* fd, int nf, const
 #define DQM(BB, KK)                                                                                              \
     if (B == BB && kind == KK)                                                                                   \
         hipLaunchKernelGGL((k_dualquant_multi<BB, KK>), dim3(grid), dim3(256), 0, st, fd, start, nf, nunits);
-#define DQM_B(BB) DQM(BB, kDq1) DQM(BB, kDq2) DQM(BB, kDq2x4) DQM(BB, kDq2x4u) DQM(BB, kDq3)
+#define DQM_B(BB) DQM(BB, -1) DQM(BB, kDq1) DQM(BB, kDq2) DQM(BB, kDq2x4) DQM(BB, kDq2x4u) DQM(BB, kDq3)
     DQM_B(8) DQM_B(16) DQM_B(32) DQM_B(64)
     DQM(8, kDq3x4) DQM(16, kDq3x4) DQM(8, kDq3x4u) DQM(16, kDq3x4u)
 #undef DQM_B

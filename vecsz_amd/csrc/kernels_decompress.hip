@@ -1458,20 +1458,39 @@ __device__ __forceinline__ float scale_out(int32_t s, double twoeb) { return (fl
 // non-outlier s is never -0.0: pred + (float)(code - R) with a +0.0 addend).
 __device__ __forceinline__ float scale_outlier(float v, double twoeb) { return (float)((double)v * twoeb); }
 
-// Inclusive segmented scan over segments of B lanes: a lane with f set starts
-// a new run.
+// Value of the lane D below, in the same row of 16 lanes (else 0): a DPP move,
+// where __shfl_up is an LDS permute with an LDS round trip's latency on the
+// scan's chain.
+template <int D>
+__device__ __forceinline__ int32_t lane_below(int32_t v) {
+    return (int32_t)dpp_move<0x110 + D>((uint32_t)v);
+}
+
+// Inclusive segmented scan over segments of L lanes: v, and whether the lane
+// or one before it in its segment starts a new run (f set).  Rows of 16 lanes
+// first, then a segment's rows: row 0's last lane to row 1 and row 2's to row
+// 3, and the last lane of the first two to the others.
+template <int L, int D = 1>
+__device__ __forceinline__ void seg_scan_lanes(int32_t& v, int32_t& f) {
+    if constexpr (D < L) {
+        int32_t nv, nf;  // (every lane is active here: 0 where it has no source)
+        if constexpr (D < 16) {
+            nv = lane_below<D>(v), nf = lane_below<D>(f);
+            if (lane_id2() % L % 16 < (uint32_t)D) nv = nf = 0;
+        } else if constexpr (D == 16) {
+            nv = (int32_t)dpp_move<0x142, 0xA>((uint32_t)v), nf = (int32_t)dpp_move<0x142, 0xA>((uint32_t)f);
+        } else {
+            nv = (int32_t)dpp_move<0x143, 0xC>((uint32_t)v), nf = (int32_t)dpp_move<0x143, 0xC>((uint32_t)f);
+        }
+        if (!f) v += nv;
+        f |= nf;
+        seg_scan_lanes<L, 2 * D>(v, f);
+    }
+}
 template <int B>
 __device__ __forceinline__ int32_t seg_scan(int32_t v, bool f) {
-    const uint32_t lib = lane_id2() % B;
-#pragma unroll
-    for (int d = 1; d < B; d <<= 1) {
-        int32_t nv = __shfl_up(v, d, B);
-        int nf = __shfl_up((int)f, d, B);
-        if (lib >= (uint32_t)d) {
-            if (!f) v += nv;
-            f = f || nf;
-        }
-    }
+    int32_t g = f;
+    seg_scan_lanes<B>(v, g);
     return v;
 }
 
@@ -1541,6 +1560,12 @@ __device__ __forceinline__ void recon_3d_tile(uint64_t t, const uint16_t* __rest
         int32_t prevplane[B];
 #pragma unroll
         for (int j = 0; j < B; j++) prevplane[j] = 0;
+        auto load = [&](int zz, int yy) -> uint32_t {
+            return xin && zz < B && z0 + zz < a.d2 && y0 + yy < a.d1 ? codes[x + (y0 + yy) * sy + (z0 + zz) * sz]
+                                                                     : (uint32_t)a.radius;
+        };
+        RowsAhead<uint32_t> rows;
+        rows.ahead([&](int r) { return load(0, r); });
         for (int zz = 0; zz < B; zz++) {
             const uint64_t z = z0 + zz;
             if (z >= a.d2) break;
@@ -1548,9 +1573,14 @@ __device__ __forceinline__ void recon_3d_tile(uint64_t t, const uint16_t* __rest
 #pragma unroll
             for (int yy = 0; yy < B; yy++) {
                 const uint64_t y = y0 + yy;
+                if (yy % kRowsAhead == 0) {
+                    rows.take();
+                    const int ny = yy + kRowsAhead < B ? yy + kRowsAhead : 0;
+                    rows.ahead([&](int r) { return load(ny ? zz : zz + 1, ny + r); });
+                }
                 if (y < a.d1) {
                     const uint64_t idx = x + y * sy + z * sz;
-                    const uint32_t c = xin ? codes[idx] : (uint32_t)a.radius;
+                    const uint32_t c = rows.cur[yy % kRowsAhead];
                     const bool isout = xin && c == 0;
                     const int32_t Y = yy > 0 ? srow : h.y;
                     const int32_t Z = zz > 0 ? prevplane[yy] : h.z;
@@ -1612,12 +1642,21 @@ __device__ __forceinline__ void recon_2d_tile(uint64_t t, const uint16_t* __rest
             bad = !h.exact;
         }
         int32_t srow = 0;
+        auto load = [&](int yy) -> uint32_t {
+            return xin && yy < B && y0 + yy < a.d1 ? codes[x + (y0 + yy) * a.d0] : (uint32_t)a.radius;
+        };
+        RowsAhead<uint32_t> rows;
+        rows.ahead([&](int r) { return load(r); });
 #pragma unroll
         for (int yy = 0; yy < B; yy++) {
             const uint64_t y = y0 + yy;
+            if (yy % kRowsAhead == 0) {
+                rows.take();
+                rows.ahead([&](int r) { return load(yy + kRowsAhead + r); });
+            }
             if (y < a.d1) {
                 const uint64_t idx = x + y * a.d0;
-                const uint32_t c = xin ? codes[idx] : (uint32_t)a.radius;
+                const uint32_t c = rows.cur[yy % kRowsAhead];
                 const bool isout = xin && c == 0;
                 const int32_t N = yy > 0 ? srow : h.y;
                 int32_t g0;
@@ -1785,20 +1824,11 @@ __device__ __forceinline__ void row_scan4(int32_t (&D)[4], const int32_t (&g)[4]
 #pragma unroll
     for (int i = 1; i < 4; i++) D[i] = rs[i] ? g[i] : D[i - 1] + g[i];
     if constexpr (L > 1) {
-        const uint32_t lib = lane_id2() % L;
         int32_t T = D[3];
-        int f = rs[0] | rs[1] | rs[2] | rs[3];
-#pragma unroll
-        for (int d = 1; d < L; d <<= 1) {
-            const int32_t t2 = __shfl_up(T, d, L);
-            const int f2 = __shfl_up(f, d, L);
-            if (lib >= (uint32_t)d) {
-                if (!f) T += t2;
-                f |= f2;
-            }
-        }
-        int32_t carry = __shfl_up(T, 1, L);
-        if (lib == 0) carry = 0;
+        int32_t f = rs[0] | rs[1] | rs[2] | rs[3];
+        seg_scan_lanes<L>(T, f);
+        int32_t carry = lane_below<1>(T);
+        if (lane_id2() % L == 0) carry = 0;
         bool open = true;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
@@ -1841,6 +1871,27 @@ __device__ __forceinline__ void recon_x4_tile(uint64_t t, const uint16_t* __rest
         for (int j = 0; j < (ZB > 1 ? B : 1); j++)
 #pragma unroll
             for (int i = 0; i < 4; i++) prev[j][i] = 0;
+        // a row's four codes, two to a word (the radius code outside the field)
+        auto load = [&](int zz, int yy) -> uint2 {
+            const uint64_t y = ND >= 2 ? ty * B + yy : 0, z = ND >= 3 ? tz * B + zz : 0;
+            uint2 cw = make_uint2(R | (R << 16), R | (R << 16));
+            if (zz < ZB && yy < YB && y < a.d1 && z < a.d2) {
+                const uint16_t* p = codes + x0 + y * sy + z * sz;
+                if constexpr (ALN) {
+                    if (xin) cw = *reinterpret_cast<const uint2*>(p);
+                } else {
+                    if (ein[3]) {
+                        __builtin_memcpy(&cw, p, 8);
+                    } else if (xin) {
+                        cw.x = p[0] | ((ein[1] ? (uint32_t)p[1] : R) << 16);
+                        if (ein[2]) cw.y = p[2] | (R << 16);
+                    }
+                }
+            }
+            return cw;
+        };
+        RowsAhead<uint2> rows;
+        if constexpr (ND > 1) rows.ahead([&](int r) { return load(0, r); });
         for (int zz = 0; zz < ZB; zz++) {
             const uint64_t z = ND >= 3 ? tz * B + zz : 0;
             if (z >= a.d2) break;
@@ -1848,20 +1899,15 @@ __device__ __forceinline__ void recon_x4_tile(uint64_t t, const uint16_t* __rest
 #pragma unroll
             for (int yy = 0; yy < YB; yy++) {
                 const uint64_t y = ND >= 2 ? ty * B + yy : 0;
+                if (ND > 1 && yy % kRowsAhead == 0) {
+                    rows.take();
+                    const int ny = yy + kRowsAhead < YB ? yy + kRowsAhead : 0;
+                    rows.ahead([&](int r) { return load(ny ? zz : zz + 1, ny + r); });
+                }
                 if (y < a.d1) {
                     const uint64_t idx = x0 + y * sy + z * sz;
-                    uint32_t c[4];
-                    if constexpr (ALN) {
-                        uint2 cw = make_uint2(R | (R << 16), R | (R << 16));
-                        if (xin) cw = *reinterpret_cast<const uint2*>(codes + idx);
-                        c[0] = cw.x & 0xFFFF;
-                        c[1] = cw.x >> 16;
-                        c[2] = cw.y & 0xFFFF;
-                        c[3] = cw.y >> 16;
-                    } else {
-#pragma unroll
-                        for (int i = 0; i < 4; i++) c[i] = ein[i] ? (uint32_t)codes[idx + i] : R;
-                    }
+                    const uint2 cw = ND > 1 ? rows.cur[yy % kRowsAhead] : load(0, 0);
+                    const uint32_t c[4] = {cw.x & 0xFFFF, cw.x >> 16, cw.y & 0xFFFF, cw.y >> 16};
                     int32_t g[4], base[4], Zv[4], D[4];
                     bool rs[4], isout[4];
                     float v[4];
@@ -1910,9 +1956,13 @@ __device__ __forceinline__ void recon_x4_tile(uint64_t t, const uint16_t* __rest
                     if constexpr (ALN) {
                         if (xin) *reinterpret_cast<float4*>(out + idx) = make_float4(o[0], o[1], o[2], o[3]);
                     } else {
+                        if (ein[3]) {
+                            __builtin_memcpy(out + idx, o, 16);
+                        } else {
 #pragma unroll
-                        for (int i = 0; i < 4; i++)
-                            if (ein[i]) out[idx + i] = o[i];
+                            for (int i = 0; i < 3; i++)
+                                if (ein[i]) out[idx + i] = o[i];
+                        }
                     }
                 }
             }
@@ -1921,8 +1971,10 @@ __device__ __forceinline__ void recon_x4_tile(uint64_t t, const uint16_t* __rest
     }
 }
 
+// (3D, B 8: four wavefronts per SIMD for a few spilled registers; with the
+// 135 it would take, three, the 1 GiB field ran 371 -> 400 us.)
 template <int ND, int B, bool ALN>
-__global__ void __launch_bounds__(256) k_recon_x4(const uint16_t* __restrict__ codes, const float* __restrict__ sparse,
+__global__ void __launch_bounds__(256, ND == 3 && B == 8 ? 4 : 1) k_recon_x4(const uint16_t* __restrict__ codes, const float* __restrict__ sparse,
                                                   float* __restrict__ out, ReconArgs a, uint32_t* flagged,
                                                   uint32_t* nflagged) {
     if (listed(a.guard)) return;  // decode output not final: a later launch redoes this
@@ -1989,9 +2041,10 @@ __global__ void k_dec_field_totals(const uint64_t* __restrict__ start, int nf, c
     if (f < nf) tot[f] = off[2 * start[f + 1]] - off[2 * start[f]];
 }
 
+// KIND: the tile form of every field in the queue, or -1: each field's own.
 template <int KIND, int B>
-__global__ void __launch_bounds__(256) k_recon_multi(const DecField* __restrict__ fd,
-                                                     const uint64_t* __restrict__ start, int nf, uint64_t ntot) {
+__global__ void __launch_bounds__(256, (KIND == kRc3x4 || KIND == kRc3x4u || KIND < 0) && B == 8 ? 4 : 1)
+    k_recon_multi(const DecField* __restrict__ fd, const uint64_t* __restrict__ start, int nf, uint64_t ntot) {
     const uint64_t wave = blockIdx.x * 4ull + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint64_t nwaves = gridDim.x * 4ull;
     for (uint64_t T = wave; T < ntot; T += nwaves) {
@@ -2003,24 +2056,17 @@ __global__ void __launch_bounds__(256) k_recon_multi(const DecField* __restrict_
         float* out = fd[f].out;
         uint32_t* fl = fd[f].flagged;
         uint32_t* nfl = fd[f].nflagged;
-        if constexpr (KIND == kRc1x4)
-            recon_x4_tile<1, B, true>(t, codes, sparse, out, ra, fl, nfl);
-        else if constexpr (KIND == kRc2x4)
-            recon_x4_tile<2, B, true>(t, codes, sparse, out, ra, fl, nfl);
-        else if constexpr (KIND == kRc3x4)
-            recon_x4_tile<3, B, true>(t, codes, sparse, out, ra, fl, nfl);
-        else if constexpr (KIND == kRc1x4u)
-            recon_x4_tile<1, B, false>(t, codes, sparse, out, ra, fl, nfl);
-        else if constexpr (KIND == kRc2x4u)
-            recon_x4_tile<2, B, false>(t, codes, sparse, out, ra, fl, nfl);
-        else if constexpr (KIND == kRc3x4u)
-            recon_x4_tile<3, B, false>(t, codes, sparse, out, ra, fl, nfl);
-        else if constexpr (KIND == kRc3)
-            recon_3d_tile<B, false>(t, codes, sparse, out, ra, fl, nfl);
-        else if constexpr (KIND == kRc2)
-            recon_2d_tile<B, false>(t, codes, sparse, out, ra, fl, nfl);
-        else
-            recon_1d_tile<B, false>(t, codes, sparse, out, ra, fl, nfl);
+        const int kind = KIND < 0 ? fd[f].kind : KIND;
+        if (kind == kRc1x4) recon_x4_tile<1, B, true>(t, codes, sparse, out, ra, fl, nfl);
+        if (kind == kRc2x4) recon_x4_tile<2, B, true>(t, codes, sparse, out, ra, fl, nfl);
+        if (kind == kRc1x4u) recon_x4_tile<1, B, false>(t, codes, sparse, out, ra, fl, nfl);
+        if (kind == kRc2x4u) recon_x4_tile<2, B, false>(t, codes, sparse, out, ra, fl, nfl);
+        if constexpr (B <= 16) {
+            if (kind == kRc3x4) recon_x4_tile<3, B, true>(t, codes, sparse, out, ra, fl, nfl);
+            if (kind == kRc3x4u) recon_x4_tile<3, B, false>(t, codes, sparse, out, ra, fl, nfl);
+        }
+        if (kind == kRc3) recon_3d_tile<B, false>(t, codes, sparse, out, ra, fl, nfl);
+        if (kind == kRc2) recon_2d_tile<B, false>(t, codes, sparse, out, ra, fl, nfl);
     }
 }
 
@@ -2226,7 +2272,7 @@ void launch_reconstruct(int ndim, int B, const uint16_t* codes, const float* spa
         return;
     }
     const int kind = recon_kind(ndim, B, a.d0, codes, out);
-    if (kind != kRc1 && kind != kRc2 && kind != kRc3) {
+    if (kind != kRc2 && kind != kRc3) {
         const uint64_t work = recon_tiles(kind, a);
         const dim3 g4((unsigned)std::max<uint64_t>(1, std::min<uint64_t>((work + 3) / 4, 2048)));
         const bool aln = kind == kRc1x4 || kind == kRc2x4 || kind == kRc3x4;
@@ -2265,10 +2311,6 @@ void launch_reconstruct(int ndim, int B, const uint16_t* codes, const float* spa
     RC_CASE(2, k_recon_2d, 16)
     RC_CASE(2, k_recon_2d, 32)
     RC_CASE(2, k_recon_2d, 64)
-    RC_CASE(1, k_recon_1d, 8)
-    RC_CASE(1, k_recon_1d, 16)
-    RC_CASE(1, k_recon_1d, 32)
-    RC_CASE(1, k_recon_1d, 64)
 #undef RC_CASE
 }
 
@@ -2324,7 +2366,7 @@ void launch_dec_field_totals(const uint64_t* start, int nf, const uint64_t* off,
 }
 int recon_kind_ndim(int kind) {
     switch (kind) {
-        case kRc1: case kRc1x4: case kRc1x4u: return 1;
+        case kRc1x4: case kRc1x4u: return 1;
         case kRc2: case kRc2x4: case kRc2x4u: return 2;
         default: return 3;
     }
@@ -2334,6 +2376,10 @@ int recon_kind(int ndim, int B, uint64_t d0, const void* codes, const void* out)
     // not fit (B > 16); vector loads and stores when rows are whole multiples
     // of 4 and codes / output are 8- / 16-byte aligned
     if (ndim == 3 && B > 16) return kRc3;
+    // under 128 wide the 4-wide tiles' 256 columns are half empty, and a row
+    // costs a wavefront four elements' instructions: 64 columns, one element
+    // a lane (25 x 25 x 26: stage 47 -> 26 us)
+    if (ndim > 1 && d0 < 128) return ndim == 2 ? kRc2 : kRc3;
     const bool aln = d0 % 4 == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0 &&
                      (reinterpret_cast<uintptr_t>(codes) & 7) == 0;
     if (ndim == 1) return aln ? kRc1x4 : kRc1x4u;
@@ -2341,7 +2387,7 @@ int recon_kind(int ndim, int B, uint64_t d0, const void* codes, const void* out)
     return aln ? kRc3x4 : kRc3x4u;
 }
 uint64_t recon_tiles(int kind, const ReconArgs& a) {
-    const bool x4 = kind != kRc1 && kind != kRc2 && kind != kRc3;
+    const bool x4 = kind != kRc2 && kind != kRc3;
     const int nd = recon_kind_ndim(kind);
     const uint64_t tx = x4 ? (a.d0 + 255) / 256 : a.ntiles_x;
     return tx * (nd >= 2 ? a.ntiles_y : 1) * (nd >= 3 ? a.ntiles_z : 1);
@@ -2355,38 +2401,10 @@ void launch_reconstruct_multi(int kind, int B, const DecField* fd, const uint64_
         hipLaunchKernelGGL((k_recon_multi<K, BB>), grid, dim3(256), 0, st, fd, start, nf, ntiles); \
         return;                                                                                  \
     }
-    RM(kRc3x4, 8)
-    RM(kRc3x4, 16)
-    RM(kRc2x4, 8)
-    RM(kRc2x4, 16)
-    RM(kRc2x4, 32)
-    RM(kRc2x4, 64)
-    RM(kRc1x4, 8)
-    RM(kRc1x4, 16)
-    RM(kRc1x4, 32)
-    RM(kRc1x4, 64)
-    RM(kRc3, 8)
-    RM(kRc3, 16)
-    RM(kRc3, 32)
-    RM(kRc3, 64)
-    RM(kRc2, 8)
-    RM(kRc2, 16)
-    RM(kRc2, 32)
-    RM(kRc2, 64)
-    RM(kRc1, 8)
-    RM(kRc1, 16)
-    RM(kRc1, 32)
-    RM(kRc1, 64)
-    RM(kRc3x4u, 8)
-    RM(kRc3x4u, 16)
-    RM(kRc2x4u, 8)
-    RM(kRc2x4u, 16)
-    RM(kRc2x4u, 32)
-    RM(kRc2x4u, 64)
-    RM(kRc1x4u, 8)
-    RM(kRc1x4u, 16)
-    RM(kRc1x4u, 32)
-    RM(kRc1x4u, 64)
+#define RM_B(BB) RM(-1, BB) RM(kRc1x4, BB) RM(kRc1x4u, BB) RM(kRc2, BB) RM(kRc2x4, BB) RM(kRc2x4u, BB) RM(kRc3, BB)
+    RM_B(8) RM_B(16) RM_B(32) RM_B(64)
+    RM(kRc3x4, 8) RM(kRc3x4, 16) RM(kRc3x4u, 8) RM(kRc3x4u, 16)
+#undef RM_B
 #undef RM
 }
 uint64_t decode_sync_units(uint64_t nsub) { return (nsub + kSyncStride - 1) / kSyncStride; }
