@@ -949,13 +949,38 @@ __device__ __forceinline__ void load_syms(const uint16_t* __restrict__ codes, ui
     }
 }
 
+// Copies n words (any alignment of src) to LDS with a workgroup of 256, four
+// 16-byte loads of a thread in flight: a loop of one load a round waited for a
+// memory latency each, 16 or more a table (25 x 25 x 26: chunk bits 8.4 ->
+// 3.7 us, pack 9.8 -> 5.9 us).
+__device__ __forceinline__ void table_to_lds(uint32_t* dst, const void* __restrict__ src, uint32_t n) {
+    const uint8_t* s = static_cast<const uint8_t*>(src);
+    for (uint32_t i0 = threadIdx.x; i0 < n / 4; i0 += 4 * 256) {
+        uint4 v[4];
+#pragma unroll
+        for (uint32_t k = 0; k < 4; k++)
+            if (i0 + 256 * k < n / 4) __builtin_memcpy(&v[k], s + 16 * (size_t)(i0 + 256 * k), 16);
+#pragma unroll
+        for (uint32_t k = 0; k < 4; k++)
+            if (i0 + 256 * k < n / 4) {
+                uint32_t* d = dst + 4 * (i0 + 256 * k);
+                d[0] = v[k].x, d[1] = v[k].y, d[2] = v[k].z, d[3] = v[k].w;
+            }
+    }
+    for (uint32_t i = n / 4 * 4 + threadIdx.x; i < n; i += 256) __builtin_memcpy(dst + i, s + 4 * (size_t)i, 4);
+}
+// The code lengths (dict bytes, dict even) as n / 4 words and the bytes left.
+__device__ __forceinline__ void lengths_to_lds(uint8_t* dst, const uint8_t* __restrict__ src, uint32_t dict) {
+    table_to_lds(reinterpret_cast<uint32_t*>(dst), src, dict / 4);
+    for (uint32_t i = dict / 4 * 4 + threadIdx.x; i < dict; i += 256) dst[i] = src[i];
+}
+
 template <bool LDS_TAB>
 __global__ void __launch_bounds__(256) k_chunk_bits(const uint16_t* __restrict__ codes, uint64_t n, uint64_t nchunks,
                                                     const uint8_t* __restrict__ len_tab, int dict,
                                                     uint32_t* __restrict__ chunk_bits, uint32_t* __restrict__ chunk_zeros) {
-    __shared__ uint8_t slen[LDS_TAB ? kMaxLdsLenTab : 4];
-    if (LDS_TAB)
-        for (int i = threadIdx.x; i < dict; i += blockDim.x) slen[i] = len_tab[i];
+    __shared__ __align__(4) uint8_t slen[LDS_TAB ? kMaxLdsLenTab : 4];
+    if (LDS_TAB) lengths_to_lds(slen, len_tab, dict);
     lds_sync();
     const uint32_t lane = lane_id();
     const uint64_t nw = (uint64_t)gridDim.x * (blockDim.x >> 6);
@@ -1044,11 +1069,17 @@ __global__ void k_enc_summary_dev(const uint64_t* __restrict__ totals, EncSummar
 // global atomics.  Lane L holds 16 consecutive symbols; a wavefront scan gives
 // its first bit inside the chunk.  The lanes OR their codewords into a
 // wave-private LDS image of the 32-bit words the chunk touches; the wavefront
-// completes the chunk's last word with the leading bits of the next chunk
-// (fewer than 32 bits, always inside the next chunk's first 32 codewords since
-// a codeword has at least one bit) and stores the image with coalesced dword
-// writes.  A word shared by two chunks belongs to the earlier one; the stream's
-// first word keeps the tree bytes in front of it.
+// stores the image with coalesced dword writes.  A wavefront packs a run of
+// chunks and hands the word that two of them share on from one to the next;
+// the run's last word is completed with the leading bits of the chunk after it
+// (fewer than 32 bits, always inside that chunk's first 32 codewords since a
+// codeword has at least one bit), and belongs to the earlier run.  The
+// stream's first word keeps the tree bytes in front of it.
+// Bounded by instruction issue and the stage's LDS traffic, not by memory (1.9
+// bytes read and 0.5 written a symbol): 264 us at 1 GiB and 64 at 67M values
+// with every codeword ORed in alone, every chunk's last word completed from
+// the next one's codes and the next chunk's loads waited for at once; 230 and
+// 50 with four codewords to an OR group, runs, and the loads in flight.
 struct Code {
     uint32_t lo, hi, len;  // codeword = hi:lo, right-aligned, len bits
 };
@@ -1083,39 +1114,43 @@ __device__ __forceinline__ void wave_lds_sync() {
 }
 
 // Raw codes of one chunk as lane L sees them: its 16 symbols (two 16-byte
-// loads), how many of them exist, and, for lanes 0..31, symbol L of the next
-// chunk (the next chunk's leading bits complete this chunk's last word).
+// loads), how many of them exist, and, at the end of a run, for lanes 0..31,
+// symbol L of the next chunk (whose leading bits complete the run's last word).
 struct ChunkRaw {
     uint32_t w[8];
     uint32_t nvalid;
     uint32_t next;  // 0xFFFFFFFF: none
-    uint64_t bit_off, out_off, nz;  // nz: outliers in the chunk
+    uint64_t bit_off, out_off, out_end;  // out_end: the first outlier after the chunk's
 };
 
 // Symbols past the field read as `fill` (an LDS table slot that holds 0).
 __device__ __forceinline__ void load_chunk(const uint16_t* __restrict__ codes, uint64_t n, uint64_t nchunks,
                                            const uint64_t* __restrict__ bit_off,
                                            const uint64_t* __restrict__ out_off, uint64_t n_outlier, uint64_t k,
-                                           uint32_t lane, uint32_t fill, ChunkRaw& r) {
+                                           bool last, uint32_t lane, uint32_t fill, ChunkRaw& r) {
     const uint64_t base = k * kChunk + lane * kSymPerThread;
-    r.nvalid = base >= n ? 0u : (uint32_t)min<uint64_t>(kSymPerThread, n - base);
-    if (r.nvalid == kSymPerThread) {
+    if ((k + 1) * kChunk <= n) {  // (for the whole wavefront: a lane's own test had the loads waited for at once)
         const uint4* p = reinterpret_cast<const uint4*>(codes + base);
         const uint4 u0 = p[0], u1 = p[1];
         r.w[0] = u0.x, r.w[1] = u0.y, r.w[2] = u0.z, r.w[3] = u0.w;
         r.w[4] = u1.x, r.w[5] = u1.y, r.w[6] = u1.z, r.w[7] = u1.w;
+        r.nvalid = kSymPerThread;
     } else {
+        r.nvalid = base >= n ? 0u : (uint32_t)min<uint64_t>(kSymPerThread, n - base);
 #pragma unroll
         for (int j = 0; j < 8; j++) r.w[j] = 0;
 #pragma unroll
         for (int j = 0; j < kSymPerThread; j++)
             r.w[j >> 1] |= ((uint32_t)j < r.nvalid ? (uint32_t)codes[base + j] : fill) << (16 * (j & 1));
     }
-    const uint64_t i = (k + 1) * kChunk + lane;
-    r.next = (lane < 32 && k + 1 < nchunks && i < n) ? (uint32_t)codes[i] : 0xFFFFFFFFu;
+    r.next = 0xFFFFFFFFu;
+    if (last) {
+        const uint64_t i = (k + 1) * kChunk + lane;
+        if (lane < 32 && k + 1 < nchunks && i < n) r.next = codes[i];
+    }
     r.bit_off = bit_off[k];
     r.out_off = out_off[k];
-    r.nz = (k + 1 < nchunks ? out_off[k + 1] : n_outlier) - r.out_off;
+    r.out_end = k + 1 < nchunks ? out_off[k + 1] : n_outlier;
 }
 
 // Codebook layouts of k_pack: the global tables; LDS entries (codeword << 6)
@@ -1126,6 +1161,31 @@ enum { kBookGlobal = 0, kBookPacked = 1, kBookSplit = 2 };
 
 __host__ __device__ constexpr uint32_t book_words(int book, int dict) {
     return book == kBookPacked ? (uint32_t)dict + 1 : book == kBookSplit ? (uint32_t)dict + 1 + ((uint32_t)dict + 4) / 4 : 0;
+}
+
+// The LDS book of a workgroup of 256 (the caller's barrier follows).
+template <int BOOK>
+__device__ __forceinline__ void book_to_lds(uint32_t* tab, uint8_t* tlen, const uint32_t* __restrict__ cw_lo,
+                                            const uint8_t* __restrict__ len_tab, int dict) {
+    if constexpr (BOOK == kBookPacked) {
+        constexpr int U = 8;
+        for (int i0 = threadIdx.x; i0 <= dict; i0 += U * 256) {
+            uint32_t l[U], cw[U];
+#pragma unroll
+            for (int k = 0; k < U; k++) {
+                const int i = i0 + 256 * k;
+                l[k] = i < dict ? len_tab[i] : 0u;
+                cw[k] = i < dict ? cw_lo[i] : 0u;
+            }
+#pragma unroll
+            for (int k = 0; k < U; k++)
+                if (i0 + 256 * k <= dict) tab[i0 + 256 * k] = l[k] == 0 ? 0u : l[k] <= 26 ? (cw[k] << 6) | l[k] : kLongCode;
+        }
+    } else if constexpr (BOOK == kBookSplit) {
+        table_to_lds(tab, cw_lo, dict);
+        lengths_to_lds(tlen, len_tab, dict);
+        if (threadIdx.x == 0) tab[dict] = 0, tlen[dict] = 0;
+    }
 }
 
 // Chunks of one decode-index group (its segments' bit offsets are stored
@@ -1158,7 +1218,21 @@ __device__ __forceinline__ PackTarget pack_target(const EncSummary& S, uint8_t* 
     return T;
 }
 
+// Words of a wavefront's stage: those one chunk can touch (1024 codewords of
+// at most max_len bits and the partial words at either end) and the two after
+// them, where a group's last word may OR a zero.
+constexpr uint32_t stage_words_of(int max_len) { return 32u * (uint32_t)(max_len > 1 ? max_len : 1) + 4; }
+
+// Four codewords as one number of `l` bits in `v`.
+struct Quad {
+    uint64_t v;
+    uint32_t l;
+};
+
 // Packs chunk k (codes already in `cur`) into the archive; see k_pack.
+// first / last: the chunk begins / ends its wavefront's run of chunks; inside
+// a run the partial word between two chunks is handed on in `carry`.  The
+// stage is all zero on entry and on return.
 // index: the decode index (layout L), or null; gbits / gouts: the first bit
 // and outlier rank of the chunk's index group (its first chunk's offsets).
 template <int BOOK>
@@ -1167,46 +1241,73 @@ __device__ __forceinline__ void pack_chunk(const ChunkRaw& cur, uint64_t k, uint
                                            const uint32_t* __restrict__ cw_hi, const uint32_t* __restrict__ cw_lo,
                                            const uint8_t* __restrict__ len_tab, const PackTarget& T,
                                            const float* __restrict__ sparse, uint8_t* __restrict__ archive,
-                                           uint32_t* stage, uint64_t* __restrict__ index = nullptr,
-                                           IdxLayout L = IdxLayout{}, uint64_t gbits = 0, uint64_t gouts = 0) {
+                                           uint32_t* stage, bool first, bool last, uint32_t& carry,
+                                           uint64_t* __restrict__ index = nullptr, IdxLayout L = IdxLayout{},
+                                           uint64_t gbits = 0, uint64_t gouts = 0) {
     constexpr bool LDS_BOOK = BOOK != kBookGlobal;
     uint32_t* out32 = reinterpret_cast<uint32_t*>(archive);
     const uint64_t base = k * kChunk + lane * kSymPerThread;
-
-    // the LDS books keep the raw entries (one or two registers per symbol)
-    uint32_t ent[LDS_BOOK ? kSymPerThread : 1];
-    uint32_t elen[BOOK == kBookSplit ? kSymPerThread : 1];
-    Code c[LDS_BOOK ? 1 : kSymPerThread];
-    uint32_t tbits = 0, tz = 0, long_mask = 0;
+    uint32_t w[8];
 #pragma unroll
-    for (int j = 0; j < kSymPerThread; j++) {
-        const uint32_t sj = (cur.w[j >> 1] >> (16 * (j & 1))) & 0xFFFF;
-        if constexpr (BOOK == kBookPacked) {
-            ent[j] = tab[sj];
-            const uint32_t l = ent[j] & 63;
-            tbits += l;
-            long_mask |= (uint32_t)(l == kLongCode) << j;
-        } else if constexpr (BOOK == kBookSplit) {
-            ent[j] = tab[sj];
-            elen[j] = tlen[sj];
-            tbits += elen[j];
-        } else {
-            const bool valid = (uint32_t)j < cur.nvalid;
+    for (int j = 0; j < 8; j++) w[j] = cur.w[j];
+    auto sym = [&](int j) { return (w[j >> 1] >> (16 * (j & 1))) & 0xFFFF; };
+    // Before the rare paths: what they derive from the codes is not kept in
+    // registers from the common path on (119 vector registers and 52 spilled
+    // scalar ones, else).
+    auto forget = [&] {
+#pragma unroll
+        for (int j = 0; j < 8; j++) asm("" : "+v"(w[j]));
+    };
+
+    // LDS books: the lane's codewords joined by fours, where every two of them
+    // fit 32 bits (all but a few chunks); else symbol by symbol
+    Quad q[LDS_BOOK ? kSymPerThread / 4 : 1];
+    Code c[LDS_BOOK ? 1 : kSymPerThread];
+    uint32_t tbits = 0, tz = 0;
+    bool slow = false;
+    auto entry = [&](int j) {  // of an LDS book, as (codeword, length)
+        const uint32_t s = sym(j);
+        if constexpr (BOOK == kBookSplit) return uint2{tab[s], tlen[s]};
+        const uint32_t e = tab[s];
+        return uint2{e >> 6, e & 63};
+    };
+    if constexpr (LDS_BOOK) {
+        uint2 e[kSymPerThread];
+#pragma unroll
+        for (int j = 0; j < kSymPerThread; j++) e[j] = entry(j);  // absent symbols: 0, 0
+        uint32_t longest = 0;
+#pragma unroll
+        for (int g = 0; g < kSymPerThread / 4; g++) {
+            const uint2 *a = e + 4 * g;
+            const uint32_t l0 = a[0].y + a[1].y, l1 = a[2].y + a[3].y;
+            const uint32_t p0 = (a[0].x << (a[1].y & 31)) | a[1].x;  // (length 32 there: none here, and codeword 0)
+            const uint32_t p1 = (a[2].x << (a[3].y & 31)) | a[3].x;
+            q[g] = Quad{((uint64_t)p0 << (l1 & 63)) | p1, l0 + l1};
+            tbits += q[g].l;
+            longest = max(longest, max(l0, l1));
+        }
+        slow = __any(longest > 32);  // (kLongCode alone is more)
+        if (BOOK == kBookPacked && slow) {
+            forget();
+            tbits = 0;
+#pragma unroll
+            for (int j = 0; j < kSymPerThread; j++) {
+                const uint32_t l = entry(j).y;
+                tbits += l == kLongCode ? (uint32_t)len_tab[sym(j)] : l;
+            }
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < kSymPerThread; j++) {
             c[j] = Code{0, 0, 0};
-            if (valid) c[j] = lookup_global(sj, cw_hi, cw_lo, len_tab);
+            if ((uint32_t)j < cur.nvalid) c[j] = lookup_global(sym(j), cw_hi, cw_lo, len_tab);
             tbits += c[j].len;
         }
     }
-    if (cur.nz) {  // outliers are rare: count them per lane only in chunks that hold some
+    if (cur.out_end != cur.out_off) {  // outliers are rare: count them per lane only in chunks that hold some
+        forget();
 #pragma unroll
-        for (int j = 0; j < kSymPerThread; j++)
-            tz += (uint32_t)j < cur.nvalid && ((cur.w[j >> 1] >> (16 * (j & 1))) & 0xFFFF) == 0;
-    }
-    if (BOOK == kBookPacked && long_mask) {
-        // codewords of more than 26 bits: true lengths from the global table
-#pragma unroll
-        for (int j = 0; j < kSymPerThread; j++)
-            if ((long_mask >> j) & 1) tbits += (uint32_t)len_tab[(cur.w[j >> 1] >> (16 * (j & 1))) & 0xFFFF] - kLongCode;
+        for (int j = 0; j < kSymPerThread; j++) tz += (LDS_BOOK || (uint32_t)j < cur.nvalid) && sym(j) == 0;
     }
     // bits (low 17) and outliers (high 15) in one wavefront scan
     const uint32_t v = tbits | (tz << 17);
@@ -1234,11 +1335,11 @@ __device__ __forceinline__ void pack_chunk(const ChunkRaw& cur, uint64_t k, uint
 
     // outlier compaction, index order
     if (tz) {
+        forget();
         uint64_t r = cur.out_off + (excl >> 17);
 #pragma unroll
         for (int j = 0; j < kSymPerThread; j++) {
-            const uint32_t sj = (cur.w[j >> 1] >> (16 * (j & 1))) & 0xFFFF;
-            if ((uint32_t)j < cur.nvalid && sj == 0) {
+            if ((LDS_BOOK || (uint32_t)j < cur.nvalid) && sym(j) == 0) {  // (an LDS book's absent symbols: dict)
                 const uint32_t bv = __float_as_uint(sparse[base + j]);
                 uint8_t* dst = T.outl + 4 * r;
                 dst[0] = (uint8_t)bv;
@@ -1257,13 +1358,12 @@ __device__ __forceinline__ void pack_chunk(const ChunkRaw& cur, uint64_t k, uint
     const uint64_t wbase = Ak >> 5;
     const uint32_t a0 = (uint32_t)(Ak & 31);
     const uint32_t nwords = (a0 + cbits + 31) >> 5;
-    for (uint32_t i = lane; i < nwords; i += kWave) stage[i] = 0;
-    wave_lds_sync();
 
-    // Each codeword is ORed into the one or two stage words it overlaps
-    // (codeword at bit offset o of word w, MSB first).  The second OR may
-    // add zero to the word after the chunk's last; the stage has room.
+    // Every codeword, or four as one, is ORed into the stage words it overlaps
+    // (bit offset o of word w, MSB first); an OR of zero may reach two words
+    // past the chunk's last.
     uint32_t pos = a0 + (excl & 0x1FFFF);
+    if (!first && lane == 0) atomicOr(stage, carry);
     auto place = [&](uint32_t cw, uint32_t l) {  // l <= 32; l = 0 places nothing (cw = 0)
         const uint32_t o = pos & 31;
         const uint64_t v = (uint64_t)cw << ((64 - o - l) & 63);
@@ -1280,31 +1380,37 @@ __device__ __forceinline__ void pack_chunk(const ChunkRaw& cur, uint64_t k, uint
             place(c.lo, c.len);
         }
     };
-    if constexpr (BOOK == kBookSplit) {
-#pragma unroll
-        for (int j = 0; j < kSymPerThread; j++) place(ent[j], elen[j]);  // absent symbols: length 0
-    } else if constexpr (BOOK == kBookPacked) {
-        if (!__any(long_mask != 0)) {
-#pragma unroll
-            for (int j = 0; j < kSymPerThread; j++) place(ent[j] >> 6, ent[j] & 63);  // absent symbols: ent 0
-        } else {
-#pragma unroll
-            for (int j = 0; j < kSymPerThread; j++) {
-                const uint32_t l = ent[j] & 63;
-                if (l == kLongCode)
-                    place_code(lookup_global((cur.w[j >> 1] >> (16 * (j & 1))) & 0xFFFF, cw_hi, cw_lo, len_tab));
-                else if (l)
-                    place(ent[j] >> 6, l);
-            }
-        }
-    } else {
+    if constexpr (!LDS_BOOK) {
 #pragma unroll
         for (int j = 0; j < kSymPerThread; j++) place_code(c[j]);
+    } else if (!slow) {
+#pragma unroll
+        for (int g = 0; g < kSymPerThread / 4; g++) {  // l <= 64; l = 0: v = 0
+            const uint64_t t = q[g].v << ((64 - q[g].l) & 63);
+            const uint32_t hi = (uint32_t)(t >> 32), lo = (uint32_t)t;
+            uint32_t* w = stage + (pos >> 5);
+            atomicOr(w, __builtin_amdgcn_alignbit(0, hi, pos));  // (the shift is pos mod 32)
+            atomicOr(w + 1, __builtin_amdgcn_alignbit(hi, lo, pos));
+            atomicOr(w + 2, __builtin_amdgcn_alignbit(lo, 0, pos));
+            pos += q[g].l;
+        }
+    } else {
+        forget();
+#pragma unroll
+        for (int j = 0; j < kSymPerThread; j++) {
+            const uint2 e = entry(j);
+            if (BOOK == kBookPacked && e.y == kLongCode)
+                place_code(lookup_global(sym(j), cw_hi, cw_lo, len_tab));
+            else
+                place(e.x, e.y);
+        }
     }
 
-    // complete the last word with the next chunk's leading bits
+    // the word after the last complete one: the run's next chunk's, or
+    // completed here with the next chunk's leading bits
     const uint32_t e = (a0 + cbits) & 31;
-    if (e != 0 && k + 1 < nchunks) {
+    const bool open = e != 0 && k + 1 < nchunks;
+    if (open && last) {
         Code d{0, 0, 0};
         if (cur.next != 0xFFFFFFFFu) {
             if constexpr (BOOK == kBookSplit)
@@ -1324,26 +1430,56 @@ __device__ __forceinline__ void pack_chunk(const ChunkRaw& cur, uint64_t k, uint
     }
     wave_lds_sync();
 
-    for (uint32_t i = ((a0 != 0 && k != 0) ? 1u : 0u) + lane; i < nwords; i += kWave) {
-        const uint64_t Wg = wbase + i;
-        uint32_t wv = stage[i];
-        if (k == 0 && i == 0 && a0) {
-            // keep the tree bytes that precede the stream in this word
-            const uint32_t mask = ~0u << (32 - a0);
-            wv = (__builtin_bswap32(out32[Wg]) & mask) | (wv & ~mask);
+    const uint32_t i0 = first && a0 != 0 && k != 0 ? 1u : 0u;
+    const uint32_t i1 = nwords - (open && !last ? 1u : 0u);
+    if (open && !last) carry = stage[nwords - 1];
+    else carry = 0;
+    // bytes at or past the stream end are not the stream's; bytes at or
+    // past cap are outside the buffer (a stream byte there: too small)
+    const uint64_t lim = end_byte < T.cap ? end_byte : T.cap;
+    if (lim == ~0ull && (k != 0 || a0 == 0)) {
+        uint32_t* o = out32 + wbase;
+        for (uint32_t i = lane; i < nwords; i += 4 * kWave) {
+            uint32_t wv[4];
+#pragma unroll
+            for (uint32_t u = 0; u < 4; u++) {
+                const uint32_t iu = min(i + kWave * u, nwords);  // (the word after the last is zero)
+                wv[u] = stage[iu];
+                stage[iu] = 0;
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < 4; u++) {
+                const uint32_t iu = i + kWave * u;
+                if (iu >= i0 && iu < i1) o[iu] = __builtin_bswap32(wv[u]);
+            }
         }
-        // bytes at or past the stream end are not the stream's; bytes at or
-        // past cap are outside the buffer (a stream byte there: too small)
-        const uint64_t lim = end_byte < T.cap ? end_byte : T.cap;
-        if ((Wg + 1) * 4 > lim) {
-            uint8_t* bp = archive + Wg * 4;
-            for (int j = 0; j < 4; j++)
-                if (Wg * 4 + j < lim) bp[j] = (uint8_t)(wv >> (24 - 8 * j));
-            if (T.cap < min(end_byte, (Wg + 1) * 4)) atomicOr(T.err, 1u);
-        } else {
-            out32[Wg] = __builtin_bswap32(wv);
+    } else {
+        for (uint32_t i = lane; i < nwords; i += kWave) {
+            const uint64_t Wg = wbase + i;
+            uint32_t wv = stage[i];
+            stage[i] = 0;
+            if (i < i0 || i >= i1) continue;
+            if (k == 0 && i == 0 && a0) {
+                // keep the tree bytes that precede the stream in this word
+                const uint32_t mask = ~0u << (32 - a0);
+                wv = (__builtin_bswap32(out32[Wg]) & mask) | (wv & ~mask);
+            }
+            if ((Wg + 1) * 4 > lim) {
+                uint8_t* bp = archive + Wg * 4;
+                for (int j = 0; j < 4; j++)
+                    if (Wg * 4 + j < lim) bp[j] = (uint8_t)(wv >> (24 - 8 * j));
+                if (T.cap < min(end_byte, (Wg + 1) * 4)) atomicOr(T.err, 1u);
+            } else {
+                out32[Wg] = __builtin_bswap32(wv);
+            }
         }
     }
+    wave_lds_sync();
+}
+
+// Zeroes a wavefront's stage (see pack_chunk).
+__device__ __forceinline__ void clear_stage(uint32_t* stage, uint32_t words, uint32_t lane) {
+    for (uint32_t i = lane; i < words; i += kWave) stage[i] = 0;
     wave_lds_sync();
 }
 
@@ -1354,44 +1490,42 @@ __global__ void __launch_bounds__(256) k_pack(const uint16_t* __restrict__ codes
                                               const uint64_t* __restrict__ bit_off, const uint64_t* __restrict__ out_off,
                                               uint64_t nchunks, const EncSummary* __restrict__ sum,
                                               const float* __restrict__ sparse, uint8_t* __restrict__ archive,
-                                              const uint32_t* __restrict__ err, uint32_t stage_words,
+                                              const uint32_t* __restrict__ err, uint32_t stage_words, uint32_t run,
                                               uint64_t* __restrict__ index, IdxLayout L) {
     constexpr bool LDS_BOOK = BOOK != kBookGlobal;
     if (*err) return;
     extern __shared__ uint32_t lds[];
     uint32_t* tab = lds;                                                        // packed entries, or split codewords
     uint8_t* tlen = reinterpret_cast<uint8_t*>(lds + (uint32_t)dict + 1);       // split lengths
-    if (BOOK == kBookPacked) {
-        for (int i = threadIdx.x; i <= dict; i += blockDim.x) {
-            const uint32_t l = i < dict ? len_tab[i] : 0u;
-            tab[i] = l == 0 ? 0u : l <= 26 ? (cw_lo[i] << 6) | l : kLongCode;
-        }
-    } else if (BOOK == kBookSplit) {
-        for (int i = threadIdx.x; i <= dict; i += blockDim.x) {
-            tab[i] = i < dict ? cw_lo[i] : 0u;
-            tlen[i] = i < dict ? len_tab[i] : 0u;
-        }
-    }
+    book_to_lds<BOOK>(tab, tlen, cw_lo, len_tab, dict);
     lds_sync();
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     uint32_t* stage = lds + book_words(BOOK, dict) + wave * stage_words;
-    const EncSummary S = *sum;
     const uint32_t lane = lane_id();
+    // the wavefront's runs of `run` chunks (a power of two), one in nw
     const uint64_t nw = (uint64_t)gridDim.x * (blockDim.x >> 6);
-    uint64_t k = blockIdx.x * (uint64_t)(blockDim.x >> 6) + wave;
+    uint64_t k = (blockIdx.x * (uint64_t)(blockDim.x >> 6) + wave) * run;
     if (k >= nchunks) return;  // no workgroup barrier follows
+    clear_stage(stage, stage_words, lane);
+    const EncSummary S = *sum;
 
     // software pipeline: the next chunk's loads are in flight while this one is packed
     const uint32_t fill = LDS_BOOK ? (uint32_t)dict : 0u;
+    const auto ends_run = [&](uint64_t q) { return ((q + 1) & (run - 1)) == 0 || q + 1 == nchunks; };
     ChunkRaw nxt;
-    load_chunk(codes, n, nchunks, bit_off, out_off, S.n_outlier, k, lane, fill, nxt);
+    load_chunk(codes, n, nchunks, bit_off, out_off, S.n_outlier, k, ends_run(k), lane, fill, nxt);
     const PackTarget T = pack_target(S, archive);
-    for (; k < nchunks; k += nw) {
+    uint32_t carry = 0;
+    while (k < nchunks) {
         const ChunkRaw cur = nxt;
-        if (k + nw < nchunks) load_chunk(codes, n, nchunks, bit_off, out_off, S.n_outlier, k + nw, lane, fill, nxt);
+        const bool last = ends_run(k);
+        const uint64_t kn = last ? k + 1 + (nw - 1) * run : k + 1;
+        if (kn < nchunks) load_chunk(codes, n, nchunks, bit_off, out_off, S.n_outlier, kn, ends_run(kn), lane, fill, nxt);
         const uint64_t k0 = k / kChunksPerGroup * kChunksPerGroup;  // the index group's first chunk
-        pack_chunk<BOOK>(cur, k, nchunks, lane, tab, tlen, cw_hi, cw_lo, len_tab, T, sparse, archive, stage, index, L,
-                         index ? bit_off[k0] : 0, index ? out_off[k0] : 0);
+        pack_chunk<BOOK>(cur, k, nchunks, lane, tab, tlen, cw_hi, cw_lo, len_tab, T, sparse, archive, stage,
+                         (k & (run - 1)) == 0, last, carry, index, L, index ? bit_off[k0] : 0,
+                         index ? out_off[k0] : 0);
+        k = kn;
     }
 }
 
@@ -1542,21 +1676,12 @@ __global__ void __launch_bounds__(256) k_encode(const uint16_t* __restrict__ cod
     __shared__ uint64_t s_lb[24];  // look-back masks and sums
     uint32_t* tab = lds;
     uint8_t* tlen = reinterpret_cast<uint8_t*>(lds + (uint32_t)dict + 1);
-    if (BOOK == kBookPacked) {
-        for (int i = threadIdx.x; i <= dict; i += blockDim.x) {
-            const uint32_t l = i < dict ? len_tab[i] : 0u;
-            tab[i] = l == 0 ? 0u : l <= 26 ? (cw_lo[i] << 6) | l : kLongCode;
-        }
-    } else {
-        for (int i = threadIdx.x; i <= dict; i += blockDim.x) {
-            tab[i] = i < dict ? cw_lo[i] : 0u;
-            tlen[i] = i < dict ? len_tab[i] : 0u;
-        }
-    }
+    book_to_lds<BOOK>(tab, tlen, cw_lo, len_tab, dict);
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     uint32_t* stage = lds + book_words(BOOK, dict) + wave * stage_words;
     const uint32_t lane = lane_id();
     const uint32_t fill = (uint32_t)dict;  // symbols past the field: an LDS slot holding 0
+    clear_stage(stage, stage_words, lane);
     for (;;) {
         if (threadIdx.x == 0) s_part = atomicAdd(part_ctr, 1u);
         lds_sync();  // (also orders the codebook fill before the first lookup)
@@ -1621,6 +1746,7 @@ __global__ void __launch_bounds__(256) k_encode(const uint16_t* __restrict__ cod
         }
 
         // pass 2: pack each chunk from its first bit and outlier rank
+        uint32_t carry = 0;
         uint64_t cb = eb, cz = ez;
         for (uint32_t w = 0; w < wave; w++) {
             cb += s_wb[w];
@@ -1645,13 +1771,14 @@ __global__ void __launch_bounds__(256) k_encode(const uint16_t* __restrict__ cod
             for (int j = 0; j < 8; j++) cur.w[j] = keep[0][j];
             const uint64_t base = k * kChunk + lane * kSymPerThread;
             cur.nvalid = base >= n ? 0u : (uint32_t)min<uint64_t>(kSymPerThread, n - base);
+            const bool last = i + 1 == WC || k + 1 == nchunks;
             const uint64_t nx = (k + 1) * kChunk + lane;
-            cur.next = (lane < 32 && k + 1 < nchunks && nx < n) ? (uint32_t)codes[nx] : 0xFFFFFFFFu;
+            cur.next = (last && lane < 32 && k + 1 < nchunks && nx < n) ? (uint32_t)codes[nx] : 0xFFFFFFFFu;
             cur.bit_off = cb;
             cur.out_off = cz;
-            cur.nz = ctot[0] >> 17;
-            pack_chunk<BOOK>(cur, k, nchunks, lane, tab, tlen, cw_hi, cw_lo, len_tab, T, sparse, archive, stage,
-                             index, L, gbits, gouts);
+            cur.out_end = cz + (ctot[0] >> 17);
+            pack_chunk<BOOK>(cur, k, nchunks, lane, tab, tlen, cw_hi, cw_lo, len_tab, T, sparse, archive, stage, i == 0,
+                             last, carry, index, L, gbits, gouts);
             cb += ctot[0] & 0x1FFFF;
             cz += ctot[0] >> 17;
             // the next chunk's totals and codes move to the front (registers,
@@ -1886,12 +2013,27 @@ __global__ void __launch_bounds__(256) k_hist_reduce_multi(const uint32_t* __res
 
 // Copies each field's staged header (metadata, Huffman header, tree) to the
 // front of its archive; one workgroup per field.
-__global__ void k_place_heads(const BatchField* __restrict__ fd, int nf, const uint32_t* __restrict__ errs) {
+// Each archive's header, tree included (up to 73 KB), 16 bytes a load and a
+// store at any alignment, eight in flight per thread: byte by byte the largest
+// tree of a batch took 40 us.  blockIdx.x: the field.
+__global__ void __launch_bounds__(256) k_place_heads(const BatchField* __restrict__ fd, int nf,
+                                                     const uint32_t* __restrict__ errs) {
     const int f = blockIdx.x;
     if (f >= nf || errs[f]) return;
     const uint8_t* src = fd[f].head;
     uint8_t* dst = fd[f].archive;
-    for (uint64_t i = threadIdx.x; i < fd[f].head_bytes; i += blockDim.x) dst[i] = src[i];
+    const uint64_t n = fd[f].head_bytes, nv = n / 16;
+    constexpr uint32_t U = 8;
+    for (uint64_t i0 = threadIdx.x; i0 < nv; i0 += 256 * U) {
+        uint4 v[U];
+#pragma unroll
+        for (uint32_t k = 0; k < U; k++)
+            if (i0 + 256 * k < nv) __builtin_memcpy(&v[k], src + 16 * (i0 + 256 * k), 16);
+#pragma unroll
+        for (uint32_t k = 0; k < U; k++)
+            if (i0 + 256 * k < nv) __builtin_memcpy(dst + 16 * (i0 + 256 * k), &v[k], 16);
+    }
+    for (uint64_t i = 16 * nv + threadIdx.x; i < n; i += 256) dst[i] = src[i];
 }
 
 // Bits and outliers of every chunk of every field (as k_chunk_bits); a unit
@@ -1900,7 +2042,7 @@ __global__ void __launch_bounds__(256) k_chunk_bits_multi(const BatchField* __re
                                                           const uint64_t* __restrict__ start, int nf, uint64_t nunits,
                                                           int dict, uint32_t* __restrict__ chunk_bits,
                                                           uint32_t* __restrict__ chunk_zeros) {
-    __shared__ uint8_t slen[kMaxLdsBook];
+    __shared__ __align__(4) uint8_t slen[kMaxLdsBook];
     const uint32_t lane = lane_id();
     const uint32_t wave = threadIdx.x >> 6;
     uint64_t u = nunits * blockIdx.x / gridDim.x;
@@ -1911,7 +2053,7 @@ __global__ void __launch_bounds__(256) k_chunk_bits_multi(const BatchField* __re
         if (u >= ue) continue;
         const uint8_t* len_tab = reinterpret_cast<const uint8_t*>(fd[f].book + 2 * dict);
         lds_sync();
-        for (int i = threadIdx.x; i < dict; i += blockDim.x) slen[i] = len_tab[i];
+        lengths_to_lds(slen, len_tab, dict);
         lds_sync();
         const uint16_t* codes = fd[f].codes;
         const uint64_t n = fd[f].a.n, nch = fd[f].nchunks, c0 = fd[f].chunk0, ub = start[f];
@@ -1977,24 +2119,15 @@ __global__ void __launch_bounds__(256) k_pack_multi(const BatchField* __restrict
     uint64_t u = nunits * blockIdx.x / gridDim.x;
     const uint64_t u1 = nunits * (blockIdx.x + 1) / gridDim.x;
     if (u >= u1) return;
+    clear_stage(stage, stage_words, lane);
     for (int f = field_of(start, nf, u); u < u1; f++) {
-        const uint64_t ue = min(u1, start[f + 1]);
+        const uint64_t ue = min<uint64_t>(u1, start[f + 1]);
         if (u >= ue) continue;
         const uint32_t* cw_hi = fd[f].book;
         const uint32_t* cw_lo = cw_hi + dict;
         const uint8_t* len_tab = reinterpret_cast<const uint8_t*>(cw_hi + 2 * dict);
         lds_sync();
-        if (BOOK == kBookPacked) {
-            for (int i = threadIdx.x; i <= dict; i += blockDim.x) {
-                const uint32_t l = i < dict ? len_tab[i] : 0u;
-                tab[i] = l == 0 ? 0u : l <= 26 ? (cw_lo[i] << 6) | l : kLongCode;
-            }
-        } else {
-            for (int i = threadIdx.x; i <= dict; i += blockDim.x) {
-                tab[i] = i < dict ? cw_lo[i] : 0u;
-                tlen[i] = i < dict ? len_tab[i] : 0u;
-            }
-        }
+        book_to_lds<BOOK>(tab, tlen, cw_lo, len_tab, dict);
         lds_sync();
         if (!errs[f]) {
             const EncSummary S = sums[f];
@@ -2003,20 +2136,24 @@ __global__ void __launch_bounds__(256) k_pack_multi(const BatchField* __restrict
             uint8_t* archive = fd[f].archive;
             const uint64_t n = fd[f].a.n, nch = fd[f].nchunks, c0 = fd[f].chunk0, ub = start[f];
             const uint64_t bb = bit_off[c0], zb = out_off[c0];
-            // software pipeline: the next unit's chunk is in flight while this one is packed
+            // the wavefront's run of the units' chunks; the next chunk is in
+            // flight while one is packed
+            const uint64_t ca = (u - ub) * 4, cn = min<uint64_t>(nch, (ue - ub) * 4) - ca;
+            const uint64_t kb = ca + cn * wave / 4, ke = ca + cn * (wave + 1) / 4;
             ChunkRaw nxt;
-            uint64_t k = (u - ub) * 4 + wave;
-            if (k < nch) load_chunk(codes, n, nch, bit_off + c0, out_off + c0, zb + S.n_outlier, k, lane, fill, nxt);
-            for (uint64_t v = u; v < ue; v++, k += 4) {
-                const ChunkRaw cur = nxt;
-                if (v + 1 < ue && k + 4 < nch)
-                    load_chunk(codes, n, nch, bit_off + c0, out_off + c0, zb + S.n_outlier, k + 4, lane, fill, nxt);
-                if (k >= nch) continue;
-                ChunkRaw c = cur;
+            if (kb < ke)
+                load_chunk(codes, n, nch, bit_off + c0, out_off + c0, zb + S.n_outlier, kb, kb + 1 == ke, lane, fill, nxt);
+            uint32_t carry = 0;
+            for (uint64_t k = kb; k < ke; k++) {
+                ChunkRaw c = nxt;
+                if (k + 1 < ke)
+                    load_chunk(codes, n, nch, bit_off + c0, out_off + c0, zb + S.n_outlier, k + 1, k + 2 == ke, lane,
+                               fill, nxt);
                 c.bit_off -= bb;
                 c.out_off -= zb;
+                c.out_end -= zb;
                 pack_chunk<BOOK>(c, k, nch, lane, tab, tlen, cw_hi, cw_lo, len_tab, pack_target(S, archive), sparse,
-                                 archive, stage);
+                                 archive, stage, k == kb, k + 1 == ke, carry);
             }
         }
         u = ue;
@@ -2183,19 +2320,26 @@ void launch_enc_summary_dev(const uint64_t* totals, EncSummary* sum, uint8_t* ar
                        out_cap, err, index);
 }
 
+// k_pack: four workgroups a CU, all resident at once (six fit; 2048 queued
+// ones: 244 us at 1 GiB, 16.2 at 1800 x 3600, against 240 and 14.0), and runs
+// of at most eight chunks (1: 319 us at 1 GiB, 8: 240, 16: 245, 32: 252, where
+// a wavefront's distance from its neighbours is a large power of two).
+constexpr int kPackGrid = 1024;
+constexpr uint32_t kPackRun = 8;
+
 void launch_pack(const uint16_t* codes, uint64_t n, const uint32_t* cw_hi, const uint32_t* cw_lo, const uint8_t* len_tab,
                  int dict, const uint64_t* bit_off, const uint64_t* out_off, uint64_t nchunks, const EncSummary* sum,
                  const float* sparse, uint8_t* archive, const uint32_t* err, int max_len, int grid_cap,
                  uint64_t* index, hipStream_t st) {
     const IdxLayout L = idx_layout(index ? n : 0);
-    const unsigned grid = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>((nchunks + 3) / 4, grid_cap));
-    // words one chunk can touch: 1024 codewords of at most max_len bits, plus
-    // the partial words at either end
-    const uint32_t stage_words = 32u * (uint32_t)std::max(max_len, 1) + 2;
+    const unsigned grid = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>((nchunks + 3) / 4, std::min(grid_cap, kPackGrid)));
+    uint32_t run = 1;  // as long as each wavefront still gets a run
+    while (run < kPackRun && nchunks >= 8ull * grid * run) run *= 2;
+    const uint32_t stage_words = stage_words_of(max_len);
     const int book = dict > kMaxLdsBook ? kBookGlobal : max_len <= 32 ? kBookSplit : kBookPacked;
     const size_t lds = ((size_t)book_words(book, dict) + 4 * (size_t)stage_words) * 4;
 #define PACK_ARGS \
-    codes, n, cw_hi, cw_lo, len_tab, dict, bit_off, out_off, nchunks, sum, sparse, archive, err, stage_words, index, L
+    codes, n, cw_hi, cw_lo, len_tab, dict, bit_off, out_off, nchunks, sum, sparse, archive, err, stage_words, run, index, L
     if (book == kBookSplit)
         hipLaunchKernelGGL(k_pack<kBookSplit>, dim3(grid), dim3(256), lds, st, PACK_ARGS);
     else if (book == kBookPacked)
@@ -2224,7 +2368,7 @@ void launch_encode(const uint16_t* codes, uint64_t n, const uint32_t* cw_hi, con
     T.err = err;
     T.no_stream = no_stream;
     const unsigned grid = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>(nparts, (uint64_t)grid_cap));
-    const uint32_t stage_words = 32u * (uint32_t)std::max(max_len, 1) + 2;
+    const uint32_t stage_words = stage_words_of(max_len);
     const int book = max_len <= 32 ? kBookSplit : kBookPacked;
     const size_t lds = ((size_t)book_words(book, dict) + 4 * (size_t)stage_words) * 4;
     uint64_t* sb = status;
@@ -2308,7 +2452,7 @@ void launch_pack_multi(const BatchField* fd, int nf, const uint64_t* start, uint
                        int grid_cap, hipStream_t st) {
     if (!nunits) return;
     const unsigned grid = (unsigned)std::min<uint64_t>(nunits, grid_cap);
-    const uint32_t stage_words = 32u * (uint32_t)std::max(max_len, 1) + 2;
+    const uint32_t stage_words = stage_words_of(max_len);
     const int book = max_len <= 32 ? kBookSplit : kBookPacked;
     const size_t lds = ((size_t)book_words(book, dict) + 4 * (size_t)stage_words) * 4;
     if (book == kBookSplit)
