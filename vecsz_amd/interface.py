@@ -13,6 +13,7 @@ one HIP stream.
 from __future__ import annotations
 
 import ctypes
+import struct
 from dataclasses import dataclass, field
 from typing import Optional, Sequence
 
@@ -193,13 +194,13 @@ def params_from_sidecar(record: bytes) -> Params:
 def header_fields(head: bytes) -> dict:
     """ndim, dims (x first) and eb from the first bytes of an archive payload
     (datapack layout, src/utils/datapack.hh:33-47); no section-size checks."""
-    nd = int(np.frombuffer(head[:4], dtype=np.int32)[0])
+    nd = struct.unpack_from("<i", head)[0] if len(head) >= 4 else int(np.frombuffer(head[:4], dtype=np.int32)[0])
     if not 1 <= nd <= 3 or len(head) < 4 * (nd + 1) + 8:
         raise VecszError(_lib.VECSZ_ECORRUPT, "archive header is corrupt")
-    dims = tuple(int(v) for v in np.frombuffer(head[4:4 + 4 * nd], dtype=np.int32))
+    *dims, eb = struct.unpack_from(f"<{nd}id", head, 4)
+    dims = tuple(dims)
     if min(dims) <= 0:
         raise VecszError(_lib.VECSZ_ECORRUPT, "archive header is corrupt")
-    eb = float(np.frombuffer(head[4 * (nd + 1):4 * (nd + 1) + 8], dtype=np.float64)[0])
     return {"ndim": nd, "dims": dims, "eb": eb}
 
 
@@ -428,8 +429,13 @@ class Context:
         modes = list(modes) if isinstance(modes, (list, tuple)) else [modes] * nf
         vrs = list(value_ranges) if isinstance(value_ranges, (list, tuple)) else [value_ranges] * nf
         params, outs = [], []
-        for a, m, vr in zip(archives, modes, vrs):
-            info = header_fields(a[:64].cpu().numpy().tobytes())
+        # every archive's header in one copy (a copy each was 0.8 ms for 48)
+        heads = [a[:64] for a in archives]
+        raw = torch.cat(heads).cpu().numpy().tobytes() if heads else b""
+        at = 0
+        for a, h, m, vr in zip(archives, heads, modes, vrs):
+            info = header_fields(raw[at:at + h.numel()])
+            at += h.numel()
             shape = tuple(reversed(info["dims"]))
             params.append(make_params((1,), 1e-4, m, block, dict_size, vr))
             outs.append(torch.empty(shape, dtype=torch.float32, device=a.device))
