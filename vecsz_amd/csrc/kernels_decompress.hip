@@ -80,22 +80,24 @@ struct StreamView {
 constexpr uint32_t kSubWords = kSubBits / 32;
 __device__ __forceinline__ uint32_t pad_idx(uint32_t w) { return w + w / kSubWords; }
 
-// 32-bit window whose MSB is bit `lp` of the staged words.
-__device__ __forceinline__ uint32_t win32(const uint32_t* st, uint32_t lp) {
-    const uint32_t i0 = pad_idx(lp >> 5);
-    return __builtin_elementwise_fshl(st[i0], st[i0 + 1], lp & 31);
-}
-struct PadWin {  // the rows staging above
+// 32-bit window whose MSB is bit `lp` of staged words: the words around the
+// end of bit lp - 1, so that one alignbit joins them (lp = 0 takes nothing of
+// the word before the first, which is only read).
+struct PadWin {  // the rows staging above, a copy of word 0 at st[-1]
     const uint32_t* st;
-    __device__ __forceinline__ uint32_t word(uint32_t w) const { return st[pad_idx(w)]; }
-    __device__ __forceinline__ uint32_t operator()(uint32_t lp) const { return win32(st, lp); }
+    __device__ __forceinline__ uint32_t operator()(uint32_t lp) const {
+        const int32_t t = (int32_t)lp - 1;
+        int32_t i = (t >> 5) + (t >> 9);
+        asm("" : "+v"(i));  // (else two shifts and two masks for the byte address)
+        return __builtin_amdgcn_alignbit(st[i], st[i + 1], ~(uint32_t)t);
+    }
 };
+static_assert(kSubBits == 512, "rows of 16 words");
 struct RowWin {  // plain consecutive words
     const uint32_t* row;
-    __device__ __forceinline__ uint32_t word(uint32_t w) const { return row[w]; }
     __device__ __forceinline__ uint32_t operator()(uint32_t lp) const {
-        const uint32_t i0 = lp >> 5;
-        return __builtin_elementwise_fshl(row[i0], row[i0 + 1], lp & 31);
+        const int32_t t = (int32_t)lp - 1, i = t >> 5;
+        return __builtin_amdgcn_alignbit(row[i], row[i + 1], ~(uint32_t)t);
     }
 };
 
@@ -198,7 +200,11 @@ struct Decoder<true> {
         deep.n_lds = n_lds;
         return ((1u << kLutBits) + a.n_sub16) / 2;
     }
-    __device__ __forceinline__ uint32_t look(uint32_t w) const { return lut[w >> (32 - kLutBits)]; }
+    __device__ __forceinline__ uint32_t look(uint32_t w) const {
+        uint32_t i = w >> (32 - kLutBits);
+        asm("" : "+v"(i));  // (else a shift, a mask and an addition)
+        return lut[i];
+    }
     static __device__ __forceinline__ bool escape(uint32_t e) { return e < 4096; }
     static __device__ __forceinline__ uint32_t len(uint32_t e) { return e >> 12; }
     static __device__ __forceinline__ uint32_t sym(uint32_t e) { return e & 0xFFF; }
@@ -220,7 +226,11 @@ struct Decoder<false> {
         sub = (GlobalU32)a.sub;
         return 1u << kLutBits;
     }
-    __device__ __forceinline__ uint32_t look(uint32_t w) const { return lut[w >> (32 - kLutBits)]; }
+    __device__ __forceinline__ uint32_t look(uint32_t w) const {
+        uint32_t i = w >> (32 - kLutBits);
+        asm("" : "+v"(i));  // (else a shift, a mask and an addition)
+        return lut[i];
+    }
     static __device__ __forceinline__ bool escape(uint32_t e) { return (int32_t)e <= 0; }
     static __device__ __forceinline__ uint32_t len(uint32_t e) { return e >> 16; }
     static __device__ __forceinline__ uint32_t sym(uint32_t e) { return e & 0xFFFF; }
@@ -237,9 +247,9 @@ struct Decoder<false> {
     }
 };
 
-// count(e): codewords of an entry (compact: all the whole ones in the 12-bit
-// pattern, 3 on average where a codeword has 3 bits); zeros(e): those that
-// decode to symbol 0.
+// The compact counting entry: length << 12 | zeros << 4 | codewords, all the
+// whole ones in the 12-bit pattern (3 on average where a codeword has 3 bits);
+// zeros are those that decode to symbol 0.
 template <bool T16>
 struct CountDecoder;
 template <>
@@ -255,24 +265,24 @@ struct CountDecoder<true> {
         deep.n_lds = n_lds;
         return ((1u << kLutBits) + a.n_sub16) / 2;
     }
-    __device__ __forceinline__ uint32_t look(uint32_t w) const { return lut[w >> (32 - kLutBits)]; }
+    __device__ __forceinline__ uint32_t look(uint32_t w) const {
+        uint32_t i = w >> (32 - kLutBits);
+        asm("" : "+v"(i));  // (else a shift, a mask and an addition)
+        return lut[i];
+    }
     static __device__ __forceinline__ bool escape(uint32_t e) { return e < 4096; }
     static __device__ __forceinline__ uint32_t len(uint32_t e) { return e >> 12; }
-    static __device__ __forceinline__ uint32_t count(uint32_t e) { return e & 15; }
     static __device__ __forceinline__ bool any_zero(uint32_t e0, uint32_t e1) { return ((e0 | e1) & 0xF0) != 0; }
     static __device__ __forceinline__ uint32_t zeros(uint32_t e) { return (e >> 4) & 15; }
     template <typename W>
     __device__ __forceinline__ void resolve(const W& win, uint32_t w, uint32_t lp, uint32_t& e, uint32_t& l) const {
         deep.resolve(win, w, lp, e, l);
-        e = (e & 0xFFF) == 0 ? 0x11u : 0x01u;
+        e = (l << 12) | ((e & 0xFFF) == 0 ? 0x11u : 0x01u);
     }
 };
 template <>
 struct CountDecoder<false> : Decoder<false> {
     static constexpr uint32_t kStep = 0;  // single codewords
-    static __device__ __forceinline__ uint32_t count(uint32_t) { return 1; }
-    static __device__ __forceinline__ bool any_zero(uint32_t e0, uint32_t e1) { return min(sym(e0), sym(e1)) == 0; }
-    static __device__ __forceinline__ uint32_t zeros(uint32_t e) { return sym(e) == 0; }
 };
 
 // Copies the tables a kernel keeps in LDS with NT threads: a first level
@@ -310,46 +320,13 @@ struct TableCopy {
     }
 };
 
-// A lane's place in its staged bits: words iw, iw + 1 and iw + 2 are held in
-// registers, iw the word before bit lp - 1 ends ((lp - 1) >> 5, so that the
-// window at lp is one alignbit: 1 to 32 bits into a).  The word that a step
-// will need is read one step ahead, so a codeword waits for its table
-// lookup only, not for the window before it.
-struct BitCursor {
-    uint32_t a, b, c;
-    int32_t iw;
-    template <typename W>
-    __device__ __forceinline__ void seek(const W& win, uint32_t lp) {
-        iw = (int32_t)(lp - 1) >> 5;
-        a = iw >= 0 ? win.word((uint32_t)iw) : 0u;
-        b = win.word((uint32_t)(iw + 1));
-        c = win.word((uint32_t)(iw + 2));
-    }
-    __device__ __forceinline__ uint32_t window(uint32_t lp) const { return __builtin_amdgcn_alignbit(a, b, 0u - lp); }
-    // To the new position lp (forward).
-    template <typename W>
-    __device__ __forceinline__ void advance(const W& win, uint32_t lp) {
-        const int32_t w = (int32_t)(lp - 1) >> 5;
-        if (w > iw + 1) {  // more than 32 bits: a long codeword
-            seek(win, lp);
-        } else {
-            const bool over = w != iw;
-            a = over ? b : a;
-            b = over ? c : b;
-            c = win.word((uint32_t)(w + 2));
-            iw = w;
-        }
-    }
-};
-
 // The two steps from lp on: entries e[], lengths l[] (0: invalid path).  One
 // window serves both: its 32 bits hold a codeword of at most 16 bits (or 12
 // bits of several) and the first 16 of the next, which is as far as the first
 // two table levels look.
 template <class D, typename W>
-__device__ __forceinline__ void decode_pair(const D& dec, const W& win, const BitCursor& cur, uint32_t lp, uint32_t* e,
-                                            uint32_t* l) {
-    const uint32_t w = cur.window(lp);
+__device__ __forceinline__ void decode_pair(const D& dec, const W& win, uint32_t lp, uint32_t* e, uint32_t* l) {
+    const uint32_t w = win(lp);
     e[0] = dec.look(w);
     l[0] = D::len(e[0]);
     uint32_t w2 = w << (l[0] & 31);
@@ -370,54 +347,74 @@ __device__ __forceinline__ uint32_t decode_one(const D& dec, const W& win, uint3
 }
 
 // Codewords and zeros (outliers) of the steps that start in [lp, end), added
-// to cnt and z; lp ends at the first step's start at or past end, cur with it.
+// to cnt and z; lp ends at the first step's start at or past end.
 // (A step may hold codewords that start past end: they are this
 // subsequence's, and the next one starts behind them.)  Returns whether an
 // invalid codeword was met (it counts as one of one bit).
+//
+// Bound by the instructions it issues, so a round is two looks at one window
+// and little else (24 vector instructions; 45 and more with the words around
+// lp kept in registers, counts taken out of every entry and both looks able to
+// walk the deeper tables: the 1 GiB field's sync pass 409 -> 303 us, a 1800 x 3600 slice's 52 -> 40).
+// Entries are summed whole: length, zeros and count are the sum's digits, once
+// the lengths (lp's own way) and the zeros (rare, summed beside) are taken
+// off.  A second look at a longer codeword is dropped; the next round's first
+// meets it.
 template <class D, typename W>
-__device__ __forceinline__ bool decode_count(const D& dec, const W& win, BitCursor& cur, uint32_t& lp, uint32_t end,
-                                             uint32_t& cnt, uint32_t& z) {
-    bool bad = false;
-    while (lp < end) {
-        uint32_t e[2], l[2];
-        decode_pair(dec, win, cur, lp, e, l);
-        if constexpr (D::kInvalid) {
-            bad |= l[0] == 0;
-            l[0] = max(l[0], 1u);
+__device__ __forceinline__ bool decode_count(const D& dec, const W& win, uint32_t& lp, uint32_t end, uint32_t& cnt,
+                                             uint32_t& z) {
+    if constexpr (D::kInvalid) {
+        bool bad = false;
+        while (lp < end) {
+            uint32_t e[2], l[2];
+            decode_pair(dec, win, lp, e, l);
+            const bool two = lp + max(l[0], 1u) < end;
+            bad |= (l[0] == 0) | (two & (l[1] == 0));
+            cnt += two ? 2 : 1;
+            z += (D::sym(e[0]) == 0) + (two & (D::sym(e[1]) == 0));
+            lp += max(l[0], 1u) + (two ? max(l[1], 1u) : 0u);
         }
-        const bool two = lp + l[0] < end;
-        if constexpr (D::kInvalid) {
-            bad |= two & (l[1] == 0);
-            l[1] = max(l[1], 1u);
+        return bad;
+    } else {
+        const uint32_t lp0 = lp, z0 = z;
+        uint32_t sum = 0;
+        while (lp < end) {
+            const uint32_t w = win(lp);
+            uint32_t e0 = dec.look(w), l0 = D::len(e0);
+            uint32_t e1 = dec.look(w << l0);
+            if (D::escape(e0)) {
+                dec.resolve(win, w, lp, e0, l0);
+                e1 = 0;
+            }
+            e1 = (!D::escape(e1) & (lp + l0 < end)) ? e1 : 0u;
+            sum += e0 + e1;
+            lp += l0 + D::len(e1);
+            if (__builtin_expect(__any(D::any_zero(e0, e1)), 0)) z += D::zeros(e0) + D::zeros(e1);
         }
-        cnt += D::count(e[0]) + (two ? D::count(e[1]) : 0u);
-        lp += l[0] + (two ? l[1] : 0u);
-        if (D::any_zero(e[0], e[1])) z += D::zeros(e[0]) + (two ? D::zeros(e[1]) : 0u);
-        cur.advance(win, lp);
+        cnt += sum - ((lp - lp0) << 12) - ((z - z0) << 4);
+        return false;
     }
-    return bad;
 }
 
 // The same where the stream may end: behind its end (bit send, at most an
 // entry's bits past `end` or more) no codeword counts, so the last steps are
 // single codewords, read from the first level in global memory.
 template <class D, typename W>
-__device__ __forceinline__ bool decode_count_to(const D& dec, const W& win, BitCursor& cur, uint32_t& lp, uint32_t end,
+__device__ __forceinline__ bool decode_count_to(const D& dec, const W& win, uint32_t& lp, uint32_t end,
                                                 uint32_t send, const DecodeArgs& a, uint32_t& cnt, uint32_t& z) {
     if constexpr (D::kStep == 0) {
-        return decode_count(dec, win, cur, lp, end, cnt, z);
+        return decode_count(dec, win, lp, end, cnt, z);
     } else {
         // (a step that starts below lim ends at or before the stream's end)
         const uint32_t lim = min(end, send > D::kStep ? send - (D::kStep - 1) : 0u);
-        const bool bad = decode_count(dec, win, cur, lp, lim, cnt, z);
+        const bool bad = decode_count(dec, win, lp, lim, cnt, z);
         while (lp < end) {  // (never, where lim is end)
-            const uint32_t w = cur.window(lp);
+            const uint32_t w = win(lp);
             uint32_t e = ((GlobalU16)a.tabs)[(1u << kLutBits) + (w >> (32 - kLutBits))], l = e >> 12;
             if (l == 0) dec.deep.resolve(win, w, lp, e, l);
             cnt++;
             z += (e & 0xFFF) == 0;
             lp += l;
-            cur.advance(win, lp);
         }
         return bad;
     }
@@ -461,7 +458,7 @@ struct StageCopy {
             }
         }
     }
-    // Into rows (pad_idx), the first nw words.
+    // Into rows (pad_idx), the first nw words; st[-1] is written too.
     __device__ __forceinline__ void put_rows(uint32_t* st, uint32_t nw) const {
 #pragma unroll
         for (uint32_t m = 0; m < VECS; m++) {
@@ -473,7 +470,7 @@ struct StageCopy {
                 d[1] = v[m].y;
                 d[2] = v[m].z;
                 d[3] = v[m].w;
-                if (k % kSubWords == 0 && k > 0) d[-1] = v[m].x;  // the previous row's copy of its successor
+                if (k % kSubWords == 0) d[-1] = v[m].x;  // the previous row's copy of its successor (word 0's: PadWin)
             }
         }
     }
@@ -496,7 +493,7 @@ static_assert(kLeadBits <= kSubBits, "the lead lies in one row");
 // 72 + 64 bits on (the deepest table walk of an invalid path, words read ahead).
 constexpr uint32_t kSyncStageWords = (kSyncWg + 1) * kSubWords + 12;
 constexpr uint32_t kSyncStageLds = kSyncStageWords + kSyncStageWords / kSubWords + 1;
-constexpr uint32_t kSyncLdsWords = kSyncStageLds + kSyncWg;  // dynamic LDS after the tables
+constexpr uint32_t kSyncLdsWords = 1 + kSyncStageLds + kSyncWg;  // dynamic LDS after the tables
 
 // Workgroup `unit` of the sync pass: subsequences unit * kSyncStride on.
 template <bool T16>
@@ -516,7 +513,7 @@ __device__ __forceinline__ void decode_sync_unit(const DecodeArgs& a, const SubS
         StageCopy<(kSyncStageWords + 4 * kSyncWg - 1) / (4 * kSyncWg), kSyncWg> sc;
         tc.fetch(a);
         sc.fetch(sv, Jst * kSubWords, (kSyncStageWords + 3) / 4);
-        st = lds + dec.attach(lds, a, tc.n_sub);
+        st = lds + dec.attach(lds, a, tc.n_sub) + 1;
         tc.put(lds);
         sc.put_rows(st, kSyncStageWords);
     }
@@ -534,17 +531,13 @@ __device__ __forceinline__ void decode_sync_unit(const DecodeArgs& a, const SubS
         const uint64_t left = a.stream_bits - j * kSubBits;
         e0 += (uint32_t)min<uint64_t>(kSubBits, left);
         const uint32_t send = s0 + (uint32_t)min<uint64_t>(2 * kSubBits, left);
-        BitCursor cur;
         if (j) {
             lp = s0 - kLeadBits;
-            cur.seek(win, lp);
             uint32_t lc = 0, lz = 0;
-            (void)decode_count_to(dec, win, cur, lp, s0, send, a, lc, lz);  // (an invalid path here is a wrong start's)
+            (void)decode_count_to(dec, win, lp, s0, send, a, lc, lz);  // (an invalid path here is a wrong start's)
             first = lp;
-        } else {  // the stream starts with a codeword
-            cur.seek(win, lp);
-        }
-        bad = decode_count_to(dec, win, cur, lp, e0, send, a, cnt, z);
+        }  // (the stream starts with a codeword)
+        bad = decode_count_to(dec, win, lp, e0, send, a, cnt, z);
         own_e[t] = lp;
     }
     lds_sync();
@@ -617,9 +610,7 @@ __device__ __forceinline__ bool redecode_entry(const DecodeArgs& a, const SubSta
     const uint32_t tl = (uint32_t)min<uint64_t>(kSubBits, left) + sv.shift0;
     const uint32_t send = (uint32_t)min<uint64_t>(2 * kSubBits, left) + sv.shift0;
     uint32_t lp = first + sv.shift0, cnt = 0, z = 0;
-    BitCursor cur;
-    cur.seek(win, lp);
-    if (decode_count_to(dec, win, cur, lp, tl, send, a, cnt, z)) atomicOr(&sum->error, 1u);
+    if (decode_count_to(dec, win, lp, tl, send, a, cnt, z)) atomicOr(&sum->error, 1u);
     over = lp - tl;
     next = j + 1;
     s.b[j] = (uint8_t)first;
@@ -1092,23 +1083,19 @@ __global__ void __launch_bounds__(256) k_decode_indexed_staged(DecodeArgs a, con
     // the loops count symbols, so an invalid codeword (len 0, an error)
     // needs no forced progress; a damaged stream stays within kIdxSpanOver
     // words past the span
-    BitCursor cur;
-    cur.seek(win, lp);
     // one codeword, or two as the halves of a word
     auto next = [&]() -> uint32_t {
         uint32_t len;
-        const uint32_t sym = Decoder<T16>::sym(decode_one(dec, win, cur.window(lp), lp, len));
+        const uint32_t sym = Decoder<T16>::sym(decode_one(dec, win, win(lp), lp, len));
         if constexpr (!T16) bad |= len == 0;
         lp += len;
-        cur.advance(win, lp);
         return sym;
     };
     auto next2 = [&]() -> uint32_t {
         uint32_t e[2], l[2];
-        decode_pair(dec, win, cur, lp, e, l);
+        decode_pair(dec, win, lp, e, l);
         if constexpr (!T16) bad |= (l[0] == 0) | (l[1] == 0);
         lp += l[0] + l[1];
-        cur.advance(win, lp);
         return Decoder<T16>::pack(e[0], e[1]);
     };
     auto outlier = [&](uint64_t i) {
@@ -1303,7 +1290,7 @@ __global__ void __launch_bounds__(1024) k_decode_scan(uint64_t* __restrict__ off
 // a predecessor).  Only the field's last unit may be partial.
 constexpr uint32_t kWriteStageWords = kWriteWg * kSubWords + 32;  // + up to 7 codewords past the last range
 constexpr uint32_t kWriteStageLds = kWriteStageWords + kWriteStageWords / kSubWords + 1;
-constexpr uint32_t kWriteLdsWords = kWriteStageLds + 2 * (kWriteWg / 64);  // dynamic LDS after the tables
+constexpr uint32_t kWriteLdsWords = 1 + kWriteStageLds + 2 * (kWriteWg / 64);  // dynamic LDS after the tables
 // base, off: the field's first unit's offsets and this unit's (field_base of
 // a batch's earlier fields is subtracted).
 template <bool T16>
@@ -1327,7 +1314,7 @@ __device__ __forceinline__ void decode_write_unit(const DecodeArgs& a, const Sub
         sc.fetch(sv, J0 * kSubWords, (kWriteStageWords + 3) / 4);
         cz = live ? s.cz[j] : 0u;
         first = live ? s.b[j] : 0u;
-        st = lds + dec.attach(lds, a, tc.n_sub);
+        st = lds + dec.attach(lds, a, tc.n_sub) + 1;
         tc.put(lds);
         sc.put_rows(st, kWriteStageWords);
     }
@@ -1352,23 +1339,19 @@ __device__ __forceinline__ void decode_write_unit(const DecodeArgs& a, const Sub
     // the loops below count symbols, so an invalid codeword (len 0, an
     // error) needs no forced progress
     const PadWin win{st};
-    BitCursor cur;
-    cur.seek(win, lp);
     // one codeword, or two as the halves of a word
     auto next = [&]() -> uint32_t {
         uint32_t len;
-        const uint32_t sym = Decoder<T16>::sym(decode_one(dec, win, cur.window(lp), lp, len));
+        const uint32_t sym = Decoder<T16>::sym(decode_one(dec, win, win(lp), lp, len));
         if constexpr (!T16) bad |= len == 0;
         lp += len;
-        cur.advance(win, lp);
         return sym;
     };
     auto next2 = [&]() -> uint32_t {
         uint32_t e[2], l[2];
-        decode_pair(dec, win, cur, lp, e, l);
+        decode_pair(dec, win, lp, e, l);
         if constexpr (!T16) bad |= (l[0] == 0) | (l[1] == 0);
         lp += l[0] + l[1];
-        cur.advance(win, lp);
         return Decoder<T16>::pack(e[0], e[1]);
     };
     auto outlier = [&](uint64_t i) {
