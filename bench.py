@@ -756,7 +756,7 @@ def measure_single(args, workload, full=True):
     # element); the packer writes the archive (A bytes).  The u16 code array
     # they pass along is scratch, counted in `traffic`, not in `achieved`.
     kern = {"range": ("k_range", 4 * n), "dualquant": (dq_kernel_name(len(dims), args.block), 4 * n),
-            "chunk_bits": ("k_chunk_bits<true>", 0), "scan": ("k_scan_local", 0), "pack": ("k_pack", size),
+            "chunk_bits": ("k_chunk_bits<true>", 0), "scan": ("k_scan_tiles", 0), "pack": ("k_pack", size),
             "encode": ("k_encode", size)}
     dom = max((k for k in cst if k in kern), key=lambda k: cst[k])
     kname, abytes = kern[dom]

@@ -4,7 +4,7 @@
 //   [r2r] k_range -> k_ebfam (eb family on the device, src/types.cc:84-93)
 //   [padding] pad values and halos
 //   k_dualquant -> histogram to host -> codebook + tree bytes (codebook.cpp)
-//   header + tree H2D -> k_chunk_bits -> chunk scan -> k_enc_summary -> k_pack
+//   header + tree H2D -> k_chunk_bits -> chunk scan and sizes -> k_pack
 //   Batches: the same stages once for all fields (k_*_multi launches).
 // Decompress (vecsz::interface::Decompress, src/vecsz_interface.hh:232-375):
 //   header D2H -> k_decode_tables -> k_decode_sync -> k_decode_pass
@@ -700,7 +700,7 @@ int compress_run(vecsz_ctx* c, const vecsz_params* p, const float* d_in, uint8_t
         if (rc) CFAIL(rc, "codebook construction failed");
         max_len = cb.max_len;
 
-        // Header: datapack metadata (huff_size / n_outlier filled by k_enc_summary),
+        // Header: datapack metadata (huff_size / n_outlier filled after the chunk scan),
         // Huffman header [u32be nodeCount][u32be dict] (src/huffman.hh:649-653) and
         // tree; then the codebook tables.  Both staged in pinned memory.
         tb = cb.tree.size();
@@ -753,7 +753,7 @@ int compress_run(vecsz_ctx* c, const vecsz_params* p, const float* d_in, uint8_t
     if (dev_cb) launch_zero_u32(S.err, 4, c->stream);  // (the host path's upload cleared it)
     if (NA ? c->pin2.cap < 512 : !c->pin2.ensure(512)) CFAIL(VECSZ_ENOMEM, "pinned buffer");
     if (d_index) {
-        // index header words 0-2 and 5; k_enc_summary writes words 3 and 4
+        // index header words 0-2 and 5; the chunk scan writes words 3 and 4
         uint64_t* ih = reinterpret_cast<uint64_t*>(c->pin2.as<uint8_t>() + 192);
         ih[0] = kIdxMagic;
         ih[1] = n;
@@ -800,14 +800,18 @@ int compress_run(vecsz_ctx* c, const vecsz_params* p, const float* d_in, uint8_t
         }
         {
             StageScope s(c, "scan");
-            launch_scan_u32x2(S.chunk_bits, S.chunk_zeros, nchunks, S.bit_off, S.out_off, S.scan_tmp, S.scan_tot,
+            EncTail T;
+            T.sum = S.summary;
+            T.archive = d_out;
+            T.meta_bytes = mb;
+            T.pad_bytes = pad_bytes;
+            T.tree_bytes = tb;
+            T.out_cap = out_cap;
+            T.err = S.err;
+            T.index = d_index;
+            T.info = dev_cb ? c->cbinfo.as<CodebookInfo>() : nullptr;
+            launch_scan_u32x2(S.chunk_bits, S.chunk_zeros, nchunks, S.bit_off, S.out_off, S.scan_tmp, S.scan_tot, T,
                               c->stream);
-            if (dev_cb)
-                launch_enc_summary_dev(S.scan_tot, S.summary, d_out, mb, pad_bytes, c->cbinfo.as<CodebookInfo>(),
-                                       out_cap, S.err, d_index, c->stream);
-            else
-                launch_enc_summary(S.scan_tot, S.summary, d_out, mb, pad_bytes, tb, out_cap, S.err, d_index,
-                                   c->stream);
         }
         {
             StageScope s(c, "pack");
@@ -1882,7 +1886,7 @@ static int compress_batch_fused_run(vecsz_ctx* c, int nf, const vecsz_params* p,
                 StageScope s(c, "scan");
                 launch_scan_u32x2(c->chunk_bits.as<uint32_t>(), c->chunk_zeros.as<uint32_t>(), ctot,
                                   c->bit_off.as<uint64_t>(), c->out_off.as<uint64_t>(), c->scan_tmp.as<uint64_t>(),
-                                  c->scan_tot.as<uint64_t>(), c->stream);
+                                  c->scan_tot.as<uint64_t>(), EncTail{}, c->stream);
                 launch_enc_summary_multi(fdd, nf, c->bit_off.as<uint64_t>(), c->out_off.as<uint64_t>(),
                                          c->scan_tot.as<uint64_t>(), ctot, c->b_sums.as<EncSummary>(), errs_d,
                                          c->stream);

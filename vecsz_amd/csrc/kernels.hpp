@@ -31,10 +31,6 @@ bool dualquant_x4_aligned(const float* in, uint64_t d0);
 // does not depend on it).
 void launch_chunk_bits(const uint16_t* codes, uint64_t n, const uint8_t* len_tab, int dict, uint32_t* cb, uint32_t* cz,
                        uint64_t nchunks, int grid_cap, hipStream_t st);
-// index (nullable): decode index whose header words 3 and 4 get the totals.
-void launch_enc_summary(const uint64_t* totals, EncSummary* sum, uint8_t* archive, uint64_t meta_bytes,
-                        uint64_t pad_bytes, uint64_t tree_bytes, uint64_t out_cap, uint32_t* err, uint64_t* index,
-                        hipStream_t st);
 void launch_pack(const uint16_t* codes, uint64_t n, const uint32_t* cw_hi, const uint32_t* cw_lo, const uint8_t* len_tab,
                  int dict, const uint64_t* bit_off, const uint64_t* out_off, uint64_t nchunks, const EncSummary* sum,
                  const float* sparse, uint8_t* archive, const uint32_t* err, int max_len, int grid_cap,
@@ -51,11 +47,21 @@ struct CodebookInfo {
 size_t codebook_lds_bytes(int dict);
 void launch_codebook(const unsigned long long* hist, int dict, uint32_t* book, uint8_t* huff, uint64_t huff_cap,
                      CodebookInfo* info, hipStream_t st);
-// k_enc_summary with the tree size from a device-built codebook (a failed
-// build sets err to 2 and writes nothing).
-void launch_enc_summary_dev(const uint64_t* totals, EncSummary* sum, uint8_t* archive, uint64_t meta_bytes,
-                            uint64_t pad_bytes, const CodebookInfo* info, uint64_t out_cap, uint32_t* err,
-                            uint64_t* index, hipStream_t st);
+// What the chunk scan ends with (sum null: nothing more than the totals): the
+// archive's sizes, the tree's from the host or, info set, from a device-built
+// codebook (a failed build sets err to 2 and writes nothing).  index
+// (nullable): decode index whose header words 3 and 4 get the totals.
+struct EncTail {
+    EncSummary* sum = nullptr;
+    uint8_t* archive = nullptr;
+    uint64_t meta_bytes = 0, pad_bytes = 0, tree_bytes = 0, out_cap = 0;
+    uint32_t* err = nullptr;
+    uint64_t* index = nullptr;
+    const CodebookInfo* info = nullptr;
+};
+// Exclusive scans of n words each; tile_tmp: 2 words a tile of 4096.
+void launch_scan_u32x2(const uint32_t* a, const uint32_t* b, uint64_t n, uint64_t* oa, uint64_t* ob, uint64_t* tile_tmp,
+                       uint64_t* totals, const EncTail& T, hipStream_t st);
 
 // Fused single-pass encode (bits, prefix by decoupled look-back, packing) for
 // dictionaries whose codebook fits in LDS (encode_fused_ok).  status: 2 *
@@ -176,8 +182,6 @@ uint64_t sync_unit_subs();
 void launch_decode_sync(const DecodeArgs& a, SubState s, DecSummary* sum, hipStream_t st);
 // Re-decode pass `pass` over the list the previous pass (or the sync pass) built.
 void launch_decode_pass(const DecodeArgs& a, SubState s, uint32_t pass, DecSummary* sum, hipStream_t st);
-void launch_scan_u32x2(const uint32_t* a, const uint32_t* b, uint64_t n, uint64_t* oa, uint64_t* ob, uint64_t* block_tmp,
-                       uint64_t* totals, hipStream_t st);
 // Codewords and zeros before each write unit (decode_write_units(nsub) units
 // of consecutive subsequences): off[2 u], off[2 u + 1], the totals behind the
 // last.  guard (nullable): nothing runs while any of the counters

@@ -5,7 +5,7 @@
 //                  quant-code histogram (c_lorenzo_{1,2,3}d1l, src/dualquant.hh:18-913;
 //                  initHuffman's frequency loop, src/huffman.hh:239-242)
 //   k_chunk_bits   bits and outliers per 1024-symbol chunk (HuffmanEncode sizes, src/huffman.hh:268-341)
-//   k_enc_summary  archive sizes from the scanned chunk totals (src/vecsz_interface.hh:189-202)
+//   k_scan*        bit and outlier offsets of the chunks, then the archive sizes (src/vecsz_interface.hh:189-202)
 //   k_pack         MSB-first bit packing into the archive + outlier compaction in index order
 //                  (HuffmanEncode; outlier gather, src/vecsz_interface.hh:166-170)
 //
@@ -1045,24 +1045,147 @@ __device__ __forceinline__ void enc_summary(uint64_t tb, uint64_t tz, EncSummary
     }
 }
 
-__global__ void k_enc_summary(const uint64_t* __restrict__ totals, EncSummary* __restrict__ sum,
-                              uint8_t* __restrict__ archive, uint64_t meta_bytes, uint64_t pad_bytes,
-                              uint64_t tree_bytes, uint64_t out_cap, uint32_t* __restrict__ err,
-                              uint64_t* __restrict__ index) {
-    if (threadIdx.x == 0 && blockIdx.x == 0)
-        enc_summary(totals[0], totals[1], sum, archive, meta_bytes, pad_bytes, tree_bytes, out_cap, err, index);
+__device__ __forceinline__ uint64_t wave_sum_u64(uint64_t v) {
+#pragma unroll
+    for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d);
+    return v;
 }
 
-__global__ void k_enc_summary_dev(const uint64_t* __restrict__ totals, EncSummary* __restrict__ sum,
-                                  uint8_t* __restrict__ archive, uint64_t meta_bytes, uint64_t pad_bytes,
-                                  const CodebookInfo* __restrict__ info, uint64_t out_cap, uint32_t* __restrict__ err,
-                                  uint64_t* __restrict__ index) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
-    if (info->status != 0) {
-        *err = 2;
-        return;
+// The archive sizes of an EncTail (sum null: none).
+__device__ __forceinline__ void enc_tail(const EncTail& T, uint64_t tb, uint64_t tz) {
+    if (!T.sum) return;
+    uint64_t tree = T.tree_bytes;
+    if (T.info) {
+        if (T.info->status != 0) {
+            *T.err = 2;
+            return;
+        }
+        tree = T.info->tree_bytes;
     }
-    enc_summary(totals[0], totals[1], sum, archive, meta_bytes, pad_bytes, info->tree_bytes, out_cap, err, index);
+    enc_summary(tb, tz, T.sum, T.archive, T.meta_bytes, T.pad_bytes, tree, T.out_cap, T.err, T.index);
+}
+
+// Exclusive scan of two u32 arrays (a chunk's bits and outliers) into u64
+// offsets, kScanBlock elements a tile: up to kScanOneTiles tiles by one
+// workgroup, more by two launches (the tiles' sums; then each tile scanned
+// from the sum of the sums before it).  Either ends with the totals and the
+// archive's sizes.  A call's time here is launches and their gaps (three
+// scans of 4 to 7 us and the sizes' own kernel before): stage 15.8 -> 6.3 us
+// at 25 x 25 x 26, 15.6 -> 8.0 at 1800 x 3600, 18.9 -> 12.0 at 1 GiB.
+constexpr int kScanPer = 4;
+constexpr int kScanBlock = 1024 * kScanPer;
+constexpr uint64_t kScanOneTiles = 4;
+
+struct ScanTile {
+    uint32_t a[kScanPer], b[kScanPer];
+    __device__ __forceinline__ void load(const uint32_t* __restrict__ pa, const uint32_t* __restrict__ pb, uint64_t n,
+                                         uint64_t tile) {
+        const uint64_t base = tile * kScanBlock + threadIdx.x * kScanPer;
+        if (base + kScanPer <= n) {
+            __builtin_memcpy(a, pa + base, sizeof a);
+            __builtin_memcpy(b, pb + base, sizeof b);
+            return;
+        }
+#pragma unroll
+        for (int i = 0; i < kScanPer; i++) {
+            a[i] = base + i < n ? pa[base + i] : 0;
+            b[i] = base + i < n ? pb[base + i] : 0;
+        }
+    }
+    // The wavefronts' sums into sh (32 words; the caller's barrier follows)
+    // and the thread's own inclusive sums.  (A tile's bits fit 32: 4096
+    // chunks of 1024 codewords of at most 64.)
+    __device__ __forceinline__ void sums(uint32_t* sh, uint32_t& ia, uint32_t& ib, uint32_t& ta, uint32_t& tb) const {
+        ta = tb = 0;
+#pragma unroll
+        for (int i = 0; i < kScanPer; i++) ta += a[i], tb += b[i];
+        ia = wave_scan_dpp(ta), ib = wave_scan_dpp(tb);
+        if (lane_id() == 63) sh[threadIdx.x >> 6] = ia, sh[16 + (threadIdx.x >> 6)] = ib;
+    }
+    // The tile's offsets from (ca, cb) on, which move to its end.
+    __device__ __forceinline__ void scan(uint32_t* sh, uint64_t n, uint64_t tile, uint64_t& ca, uint64_t& cb,
+                                         uint64_t* __restrict__ oa, uint64_t* __restrict__ ob) const {
+        uint32_t ia, ib, ta, tb;
+        sums(sh, ia, ib, ta, tb);
+        lds_sync();
+        const uint32_t w = threadIdx.x >> 6;
+        uint64_t pa = ca + ia - ta, pb = cb + ib - tb;
+        for (uint32_t i = 0; i < 16; i++) {
+            if (i < w) pa += sh[i], pb += sh[16 + i];
+            ca += sh[i], cb += sh[16 + i];
+        }
+        const uint64_t base = tile * kScanBlock + threadIdx.x * kScanPer;
+        uint64_t va[kScanPer], vb[kScanPer];
+#pragma unroll
+        for (int i = 0; i < kScanPer; i++) {
+            va[i] = pa, vb[i] = pb;
+            pa += a[i], pb += b[i];
+        }
+        if (base + kScanPer <= n) {
+            __builtin_memcpy(oa + base, va, sizeof va);
+            __builtin_memcpy(ob + base, vb, sizeof vb);
+            return;
+        }
+#pragma unroll
+        for (int i = 0; i < kScanPer; i++)
+            if (base + i < n) oa[base + i] = va[i], ob[base + i] = vb[i];
+    }
+};
+
+__global__ void __launch_bounds__(1024) k_scan(const uint32_t* __restrict__ a, const uint32_t* __restrict__ b,
+                                               uint64_t n, uint64_t* __restrict__ oa, uint64_t* __restrict__ ob,
+                                               uint64_t* __restrict__ totals, EncTail T) {
+    __shared__ uint32_t sh[2][32];  // by turns: a tile's is read while the next one's is written
+    uint64_t ca = 0, cb = 0;
+    ScanTile nxt;
+    nxt.load(a, b, n, 0);
+    for (uint64_t tile = 0; tile * kScanBlock < n; tile++) {
+        const ScanTile cur = nxt;
+        nxt.load(a, b, n, tile + 1);
+        cur.scan(sh[tile & 1], n, tile, ca, cb, oa, ob);
+    }
+    if (threadIdx.x == 0) {
+        totals[0] = ca;
+        totals[1] = cb;
+        enc_tail(T, ca, cb);
+    }
+}
+
+__global__ void __launch_bounds__(1024) k_scan_sums(const uint32_t* __restrict__ a, const uint32_t* __restrict__ b,
+                                                    uint64_t n, uint64_t* __restrict__ bsum) {
+    __shared__ uint32_t sh[32];
+    ScanTile t;
+    t.load(a, b, n, blockIdx.x);
+    uint32_t ia, ib, ta, tb;
+    t.sums(sh, ia, ib, ta, tb);
+    lds_sync();
+    if (threadIdx.x >= 2) return;
+    uint64_t s = 0;
+    for (uint32_t i = 0; i < 16; i++) s += sh[16 * threadIdx.x + i];
+    bsum[2 * blockIdx.x + threadIdx.x] = s;
+}
+
+__global__ void __launch_bounds__(1024) k_scan_tiles(const uint32_t* __restrict__ a, const uint32_t* __restrict__ b,
+                                                     uint64_t n, const uint64_t* __restrict__ bsum,
+                                                     uint64_t* __restrict__ oa, uint64_t* __restrict__ ob,
+                                                     uint64_t* __restrict__ totals, EncTail T) {
+    __shared__ uint32_t sh[32];
+    __shared__ uint64_t before[2][16];
+    ScanTile t;
+    t.load(a, b, n, blockIdx.x);
+    uint64_t sa = 0, sb = 0;
+    for (uint32_t i = threadIdx.x; i < blockIdx.x; i += 1024) sa += bsum[2 * i], sb += bsum[2 * i + 1];
+    sa = wave_sum_u64(sa), sb = wave_sum_u64(sb);
+    if (lane_id() == 0) before[0][threadIdx.x >> 6] = sa, before[1][threadIdx.x >> 6] = sb;
+    lds_sync();
+    uint64_t ca = 0, cb = 0;
+    for (uint32_t i = 0; i < 16; i++) ca += before[0][i], cb += before[1][i];
+    t.scan(sh, n, blockIdx.x, ca, cb, oa, ob);
+    if (threadIdx.x == 0 && blockIdx.x + 1 == gridDim.x) {
+        totals[0] = ca;
+        totals[1] = cb;
+        enc_tail(T, ca, cb);
+    }
 }
 
 // Bit packing, one wavefront per 1024-symbol chunk, no workgroup barriers or
@@ -1531,7 +1654,7 @@ __global__ void __launch_bounds__(256) k_pack(const uint16_t* __restrict__ codes
 
 // ------------------------------------------------------------------ fused single-pass encode
 //
-// k_encode does the work of k_chunk_bits, the chunk scan, k_enc_summary and
+// k_encode does the work of k_chunk_bits, the chunk scan and
 // k_pack in one pass, so the field's codes are read from HBM once (a
 // wavefront keeps its chunks' codes in registers until it packs them).  The
 // chunks are cut into partitions of kEncPartChunks (kEncWaveChunks per
@@ -1558,12 +1681,6 @@ __device__ __forceinline__ uint64_t ld_status(const uint64_t* p) {
 }
 __device__ __forceinline__ void st_status(uint64_t* p, uint64_t v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-__device__ __forceinline__ uint64_t wave_sum_u64(uint64_t v) {
-#pragma unroll
-    for (int d = 32; d >= 1; d >>= 1) v += __shfl_xor(v, d);
-    return v;
 }
 
 // Exclusive prefixes (bits, outliers) of partition `part` from the status
@@ -2306,18 +2423,15 @@ void launch_chunk_bits(const uint16_t* codes, uint64_t n, const uint8_t* len_tab
         hipLaunchKernelGGL(k_chunk_bits<false>, dim3(grid), dim3(256), 0, st, codes, n, nchunks, len_tab, dict, cb, cz);
 }
 
-void launch_enc_summary(const uint64_t* totals, EncSummary* sum, uint8_t* archive, uint64_t meta_bytes,
-                        uint64_t pad_bytes, uint64_t tree_bytes, uint64_t out_cap, uint32_t* err, uint64_t* index,
-                        hipStream_t st) {
-    hipLaunchKernelGGL(k_enc_summary, dim3(1), dim3(64), 0, st, totals, sum, archive, meta_bytes, pad_bytes,
-                       tree_bytes, out_cap, err, index);
-}
-
-void launch_enc_summary_dev(const uint64_t* totals, EncSummary* sum, uint8_t* archive, uint64_t meta_bytes,
-                            uint64_t pad_bytes, const CodebookInfo* info, uint64_t out_cap, uint32_t* err,
-                            uint64_t* index, hipStream_t st) {
-    hipLaunchKernelGGL(k_enc_summary_dev, dim3(1), dim3(64), 0, st, totals, sum, archive, meta_bytes, pad_bytes, info,
-                       out_cap, err, index);
+void launch_scan_u32x2(const uint32_t* a, const uint32_t* b, uint64_t n, uint64_t* oa, uint64_t* ob, uint64_t* tile_tmp,
+                       uint64_t* totals, const EncTail& T, hipStream_t st) {
+    const uint64_t nt = (n + kScanBlock - 1) / kScanBlock;
+    if (nt <= kScanOneTiles) {
+        hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, st, a, b, n, oa, ob, totals, T);
+        return;
+    }
+    hipLaunchKernelGGL(k_scan_sums, dim3((unsigned)nt), dim3(1024), 0, st, a, b, n, tile_tmp);
+    hipLaunchKernelGGL(k_scan_tiles, dim3((unsigned)nt), dim3(1024), 0, st, a, b, n, tile_tmp, oa, ob, totals, T);
 }
 
 // k_pack: four workgroups a CU, all resident at once (six fit; 2048 queued

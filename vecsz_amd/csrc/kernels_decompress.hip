@@ -656,108 +656,6 @@ __global__ void __launch_bounds__(256) k_decode_pass(DecodeArgs a, SubState s, u
     decode_pass_stripe<T16>(a, s, pass, sum, blockIdx.x % s.nstripe, blockIdx.x / s.nstripe, gridDim.x / s.nstripe);
 }
 
-// Device-wide exclusive scan of two u32 arrays into u64 offsets.
-constexpr int kScanPer = 4;
-constexpr int kScanBlock = 1024 * kScanPer;
-
-__global__ void __launch_bounds__(1024) k_scan_local(const uint32_t* __restrict__ a, const uint32_t* __restrict__ b,
-                                                     uint64_t n, uint64_t* __restrict__ oa, uint64_t* __restrict__ ob,
-                                                     uint64_t* __restrict__ bsum) {
-    __shared__ uint64_t sa[16], sbb[16];
-    const uint64_t base = blockIdx.x * (uint64_t)kScanBlock + threadIdx.x * kScanPer;
-    uint64_t va[kScanPer], vb[kScanPer], ta = 0, tb = 0;
-#pragma unroll
-    for (int i = 0; i < kScanPer; i++) {
-        va[i] = base + i < n ? a[base + i] : 0;
-        vb[i] = base + i < n ? b[base + i] : 0;
-        ta += va[i];
-        tb += vb[i];
-    }
-    uint64_t ia = ta, ib = tb;
-    const uint32_t lane = lane_id2();
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-        uint64_t xa = __shfl_up(ia, d), xb = __shfl_up(ib, d);
-        if (lane >= (uint32_t)d) {
-            ia += xa;
-            ib += xb;
-        }
-    }
-    const int w = threadIdx.x >> 6;
-    if (lane == 63) {
-        sa[w] = ia;
-        sbb[w] = ib;
-    }
-    lds_sync();
-    uint64_t pa = 0, pb = 0, tot_a = 0, tot_b = 0;
-    for (int i = 0; i < 16; i++) {
-        if (i < w) {
-            pa += sa[i];
-            pb += sbb[i];
-        }
-        tot_a += sa[i];
-        tot_b += sbb[i];
-    }
-    pa += ia - ta;
-    pb += ib - tb;
-#pragma unroll
-    for (int i = 0; i < kScanPer; i++) {
-        if (base + i < n) {
-            oa[base + i] = pa;
-            ob[base + i] = pb;
-        }
-        pa += va[i];
-        pb += vb[i];
-    }
-    if (threadIdx.x == 0) {
-        bsum[2 * blockIdx.x] = tot_a;
-        bsum[2 * blockIdx.x + 1] = tot_b;
-    }
-}
-
-// Exclusive scan of the per-block sums, 1024 at a time on one workgroup
-// (an LDS Hillis-Steele scan per pass, carried across passes).
-__global__ void __launch_bounds__(1024) k_scan_blocks(uint64_t* __restrict__ bsum, uint64_t nb, uint64_t* __restrict__ totals) {
-    __shared__ uint64_t sa[1024], sb[1024];
-    const uint32_t t = threadIdx.x;
-    uint64_t ca = 0, cb = 0;
-    for (uint64_t base = 0; base < nb; base += 1024) {
-        const uint64_t i = base + t;
-        const uint64_t x = i < nb ? bsum[2 * i] : 0, y = i < nb ? bsum[2 * i + 1] : 0;
-        sa[t] = x;
-        sb[t] = y;
-        lds_sync();
-        for (uint32_t d = 1; d < 1024; d <<= 1) {
-            const uint64_t ax = t >= d ? sa[t - d] : 0, bx = t >= d ? sb[t - d] : 0;
-            lds_sync();
-            sa[t] += ax;
-            sb[t] += bx;
-            lds_sync();
-        }
-        if (i < nb) {
-            bsum[2 * i] = ca + sa[t] - x;
-            bsum[2 * i + 1] = cb + sb[t] - y;
-        }
-        ca += sa[1023];
-        cb += sb[1023];
-        lds_sync();
-    }
-    if (t == 0) {
-        totals[0] = ca;
-        totals[1] = cb;
-    }
-}
-
-__global__ void __launch_bounds__(1024) k_scan_add(uint64_t* __restrict__ oa, uint64_t* __restrict__ ob, uint64_t n,
-                                                   const uint64_t* __restrict__ bsum) {
-    const uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x;
-    if (i < n) {
-        const uint64_t blk = i / kScanBlock;
-        oa[i] += bsum[2 * blk];
-        ob[i] += bsum[2 * blk + 1];
-    }
-}
-
 __device__ __forceinline__ float read_f32_bytes(const uint8_t* p) {
     uint32_t v = (uint32_t)p[0] | ((uint32_t)p[1] << 8) | ((uint32_t)p[2] << 16) | ((uint32_t)p[3] << 24);
     return __uint_as_float(v);
@@ -2194,13 +2092,6 @@ void launch_decode_indexed(const DecodeArgs& a0, const uint64_t* index, uint64_t
             DI(false, false);
     }
 #undef DI
-}
-void launch_scan_u32x2(const uint32_t* a, const uint32_t* b, uint64_t n, uint64_t* oa, uint64_t* ob, uint64_t* block_tmp,
-                       uint64_t* totals, hipStream_t st) {
-    const uint64_t nb = (n + kScanBlock - 1) / kScanBlock;
-    hipLaunchKernelGGL(k_scan_local, dim3((unsigned)nb), dim3(1024), 0, st, a, b, n, oa, ob, block_tmp);
-    hipLaunchKernelGGL(k_scan_blocks, dim3(1), dim3(1024), 0, st, block_tmp, nb, totals);
-    hipLaunchKernelGGL(k_scan_add, dim3(grid_for(n, 1024)), dim3(1024), 0, st, oa, ob, n, block_tmp);
 }
 void launch_decode_offsets(const SubState& s, uint64_t nsub, uint64_t* off, hipStream_t st, const uint32_t* guard) {
     const uint64_t nu = decode_write_units(nsub);
