@@ -1153,10 +1153,11 @@ int decompress_device(vecsz_ctx* c, const vecsz_params* p, const uint8_t* d_in, 
         // after the write.  (The longest chain of wrong starts grows with
         // their number: the 1 GiB field needs three or four passes, a 26 MB
         // one two; a pass over empty lists takes about 4 us, a host check
-        // with its repeated launches about 35.)  Otherwise passes run
-        // in growing batches between host checks while the lists ask for more
-        // (each pass resolves at least the first subsequence of every chain,
-        // so nsub passes suffice), and then the scan and the write again.
+        // with its repeated launches about 35.)  Otherwise passes run in
+        // growing batches while the lists ask for more (each pass resolves at
+        // least the first subsequence of every chain, so nsub passes suffice),
+        // each batch with launch_decode_tail for what a short list still
+        // holds, the scan and the write again, and a host check.
         const uint32_t ahead = nsub < (1u << 17) ? 2 : nsub < (1u << 21) ? 3 : 4;
         uint32_t pass = 0;
         {
@@ -1195,19 +1196,19 @@ int decompress_device(vecsz_ctx* c, const vecsz_params* p, const uint8_t* d_in, 
         if (tm.status)  // (nothing has run behind the tables)
             return decompress_device(c, p, d_in, in_bytes, d_out, out_cap, nullptr, 0, true);
         if (left) {
-            for (uint32_t batch = 2; left; batch = std::min<uint32_t>(2 * batch, 16)) {
+            for (uint32_t batch = 4; left; batch = std::min<uint32_t>(2 * batch, 16)) {
                 if (pass > nsub + 2) return fail(c, VECSZ_ECORRUPT, "subsequence boundaries do not converge");
                 // (a pass over an empty list does nothing but clear the list after next)
                 {
                     StageScope s(c, "decode_redo");
                     for (uint32_t b = 0; b < batch; b++) launch_decode_pass(da, ss, pass++, dsum, c->stream);
+                    launch_decode_tail(da, ss, pass, dsum, c->stream);
                 }
+                scan_write(ss.list_n + list_slot(pass));
+                if (!fused_1d) reconstruct(ss.list_n + list_slot(pass));
+                HIPCHK(c, hipGetLastError());
                 if (int rc2 = check()) return rc2;
             }
-            scan_write(nullptr);
-            if (!fused_1d) reconstruct(nullptr);
-            HIPCHK(c, hipGetLastError());
-            if (int rc2 = check()) return rc2;
         }
         if (tot < n) return fail(c, VECSZ_ECORRUPT, "bitstream holds fewer symbols than the field");
         }

@@ -656,6 +656,67 @@ __global__ void __launch_bounds__(256) k_decode_pass(DecodeArgs a, SubState s, u
     decode_pass_stripe<T16>(a, s, pass, sum, blockIdx.x % s.nstripe, blockIdx.x / s.nstripe, gridDim.x / s.nstripe);
 }
 
+// The end of a redo that a few chains of wrong starts make long: one
+// workgroup resolves pass `pass`'s list in place, all passes' worth, when it
+// holds at most kTailWg entries (else it does nothing).  A pass over such a
+// list is latency: about 4 us of launch and tables around 5 of work, and a
+// host check with its launches every so many passes (67M values whose phase a
+// start picks by chance, 33 passes long: decompress 710 -> 606 us).
+// Rounds are passes as k_decode_pass makes them, with the lists in LDS and a
+// barrier between them that also orders the subsequences' state.  Bounded:
+// what is left after kTailRounds goes back to the list.
+constexpr uint32_t kTailWg = 1024;
+constexpr uint32_t kTailRounds = 512;
+template <bool T16>
+__global__ void __launch_bounds__(kTailWg) k_decode_tail(DecodeArgs a, SubState s, uint32_t pass, DecSummary* sum) {
+    extern __shared__ __align__(16) uint32_t lds[];
+    if (no_tables(a)) return;
+    const uint32_t t = threadIdx.x;
+    // entry t of the stripes one after the other (nstripe <= 32: a lane each)
+    const uint32_t k = lane_id2() < s.nstripe ? min(*list_counter(s, pass, lane_id2()), 2 * kTailWg) : 0u;
+    const uint32_t ends = wave_scan_dpp(k);
+    uint32_t m = lane63(ends);
+    if (m > kTailWg) return;  // (the whole workgroup)
+    uint64_t at = 0;
+    for (uint32_t q = 0; q < s.nstripe; q++) {
+        const uint32_t q1 = (uint32_t)__builtin_amdgcn_readlane((int)ends, (int)q);
+        const uint32_t q0 = q1 - (uint32_t)__builtin_amdgcn_readlane((int)k, (int)q);
+        if (t >= q0 && t < q1) at = q * s.stripe_cap + (t - q0);
+    }
+    if (m == 0) return;
+    uint64_t* list = s.list[pass & 1];
+    CountDecoder<T16> dec;
+    uint32_t* p = lds;
+    {
+        TableCopy<T16, true, kTailWg> tc;
+        tc.fetch(a);
+        p += dec.attach(lds, a, tc.n_sub);
+        tc.put(lds);
+    }
+    uint32_t* rows = p;
+    uint64_t* ents = reinterpret_cast<uint64_t*>(rows + kTailWg * kRowStride);  // two lists, by turns
+    uint32_t* n_ents = reinterpret_cast<uint32_t*>(ents + 2 * kTailWg);         // their counters
+    if (t < 2) n_ents[t] = 0;
+    uint64_t ent = t < m ? list[at] : 0;
+    mem_sync();
+    uint32_t cur = 0;
+    for (uint32_t r = 0; m && r < kTailRounds; r++, cur ^= 1) {
+        if (t < m) {
+            uint64_t next = 0;
+            uint32_t over = 0;
+            if (redecode_entry<T16>(a, s, dec, rows + t * kRowStride, ent, sum, next, over))
+                ents[cur * kTailWg + atomicAdd(n_ents + cur, 1u)] = (s.jbase + next) | ((uint64_t)over << 48);
+        }
+        mem_sync();
+        m = n_ents[cur];
+        ent = t < m ? ents[cur * kTailWg + t] : 0;
+        if (t == 0) n_ents[cur ^ 1] = 0;  // the next round's
+        mem_sync();
+    }
+    if (t < m) list[t] = ent;
+    if (t < s.nstripe) *list_counter(s, pass, t) = t == 0 ? m : 0u;
+}
+
 __device__ __forceinline__ float read_f32_bytes(const uint8_t* p) {
     uint32_t v = (uint32_t)p[0] | ((uint32_t)p[1] << 8) | ((uint32_t)p[2] << 16) | ((uint32_t)p[3] << 24);
     return __uint_as_float(v);
@@ -2092,6 +2153,18 @@ void launch_decode_indexed(const DecodeArgs& a0, const uint64_t* index, uint64_t
             DI(false, false);
     }
 #undef DI
+}
+void launch_decode_tail(const DecodeArgs& a0, SubState s, uint32_t pass, DecSummary* sum, hipStream_t st) {
+    allow_big_lds(k_decode_tail<true>);
+    allow_big_lds(k_decode_tail<false>);
+    const bool t16 = a0.tabs != nullptr;
+    constexpr size_t kOwn = (size_t)kTailWg * (kRowStride * 4 + 2 * 8) + 16;
+    const DecodeArgs a = with_lds_sub16(a0, kOwn);
+    const size_t lds = table_lds_bytes(a, t16) + kOwn;
+    if (t16)
+        hipLaunchKernelGGL(k_decode_tail<true>, dim3(1), dim3(kTailWg), lds, st, a, s, pass, sum);
+    else
+        hipLaunchKernelGGL(k_decode_tail<false>, dim3(1), dim3(kTailWg), lds, st, a, s, pass, sum);
 }
 void launch_decode_offsets(const SubState& s, uint64_t nsub, uint64_t* off, hipStream_t st, const uint32_t* guard) {
     const uint64_t nu = decode_write_units(nsub);
