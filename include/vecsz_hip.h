@@ -156,10 +156,9 @@ int vecsz_archive_info(const uint8_t* h_archive, uint64_t bytes, int* ndim, uint
  * set_workers host threads).  Decompress of two or more archives with one
  * block size and dict_size (at most 4096), no pad section and output
  * capacities of at most 4M elements on average runs fused the same way (see
- * vecsz_ctx_set_batch_fused): one copy of every archive's header and tree to the host, the
- * decode tables built on host threads, then one launch per stage (sync pass,
- * re-decode passes over one batch-wide list, scan, write pass, one
- * reconstruction launch per tile form).  Other batches are spread, largest
+ * vecsz_ctx_set_batch_fused): one copy of every archive's header to the host,
+ * then one launch per stage (decode tables, a workgroup per field; sync pass,
+ * re-decode passes, scan, write pass, reconstruction).  Other batches are spread, largest
  * first, over worker contexts (own HIP stream and scratch each, set_workers
  * of them), so small fields overlap on the GPU and host codebook work
  * overlaps kernels.  status[k] receives each field's VECSZ_*
