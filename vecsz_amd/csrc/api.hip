@@ -157,7 +157,7 @@ struct vecsz_ctx {
     HostBuf vpin;
     // decompress scratch
     // dec_small: decoder summary, symbol and zero totals, list counts (kDecSmall*)
-    DevBuf tabs, sub_b, sub_e, sub_cz, sub_list, sub_ln, unit_off, scan_tmp, scan_tot, dec_small, flagged, nflagged;
+    DevBuf tabs, sub_b, sub_e, sub_cz, sub_list, sub_ln, unit_off, scan_tmp, scan_tot, dec_small, flagged;
     // host staging
     DevBuf stage_in, stage_out;
     HostBuf pin, pin2, pin_tab;
@@ -412,9 +412,11 @@ CScratch small_scratch(CScratch s, uint8_t* block, int dict) {
 // The small state of a single-field decompress in one block: [decoder
 // summary | state of the device-built tables | the re-decode list counters].
 constexpr size_t kDecSmallTables = 64;
+constexpr size_t kDecSmallFlagged = 96;  // u32: blocks listed for the fp32 reconstruction
 constexpr size_t kDecSmallLists = 128;
 constexpr size_t kDecSmallBytes = kDecSmallLists + kListCountBytes;
-static_assert(sizeof(DecSummary) <= kDecSmallTables && kDecSmallTables + sizeof(TableMeta) <= kDecSmallLists,
+static_assert(sizeof(DecSummary) <= kDecSmallTables && kDecSmallTables + sizeof(TableMeta) <= kDecSmallFlagged &&
+                  kDecSmallFlagged + 4 <= kDecSmallLists,
               "the slots hold their structs");
 
 // Whether the list pass `pass` reads holds entries (counters: the host's copy).
@@ -1059,19 +1061,22 @@ int decompress_device(vecsz_ctx* c, const vecsz_params* p, const uint8_t* d_in, 
     const uint64_t nblocks = ((d0 + B - 1) / B) * (ndim >= 2 ? (d1 + B - 1) / B : 1) * (ndim >= 3 ? (d2 + B - 1) / B : 1);
     const uint64_t rwork = ra.ntiles_x * ra.ntiles_y * ra.ntiles_z;
     const int rgrid = (int)std::max<uint64_t>(1, std::min<uint64_t>((rwork + 3) / 4, 2048));
-    if (!fused_1d && (!c->flagged.ensure(nblocks * 4 + 16) || !c->nflagged.ensure(16)))
+    if ((!fused_1d && !c->flagged.ensure(nblocks * 4 + 16)) || !c->dec_small.ensure(kDecSmallBytes))
         return fail(c, VECSZ_ENOMEM, "device scratch allocation failed");
     // Lorenzo reconstruction; guard: as the write pass's (nonzero: nothing
     // runs, the decode is not final yet)
     bool recon_issued = false;
+    // (the reconstruction's counter with it: one launch less than its own
+    // fill, and it stays zero until the one reconstruction that runs)
+    HIPCHK(c, hipMemsetAsync(c->dec_small.p, 0, kDecSmallBytes, c->stream));
+    uint32_t* nflagged = reinterpret_cast<uint32_t*>(c->dec_small.as<uint8_t>() + kDecSmallFlagged);
     auto reconstruct = [&](const uint32_t* guard) {
-        launch_zero_u32(c->nflagged.as<uint32_t>(), 1, c->stream);
         StageScope s(c, "reconstruct");
         ra.guard = guard;
-        launch_reconstruct(ndim, B, codes, sparse, d_out, ra, c->flagged.as<uint32_t>(), c->nflagged.as<uint32_t>(),
+        launch_reconstruct(ndim, B, codes, sparse, d_out, ra, c->flagged.as<uint32_t>(), nflagged,
                            rgrid, c->stream);
         launch_reconstruct_fallback(ndim, B, codes, sparse, d_out, ra, c->flagged.as<uint32_t>(),
-                                    c->nflagged.as<uint32_t>(), c->stream);
+                                    nflagged, c->stream);
         recon_issued = true;
     };
 
@@ -1090,8 +1095,7 @@ int decompress_device(vecsz_ctx* c, const vecsz_params* p, const uint8_t* d_in, 
         list_stripes(decode_sync_units(nsub), &ss);
         const uint64_t list_cap = ss.nstripe * ss.stripe_cap;
         if (!c->sub_b.ensure(nsub) || !c->sub_e.ensure(nsub) || !c->sub_cz.ensure(nsub * 4) ||
-            !c->sub_list.ensure(list_cap * 16) || !c->unit_off.ensure((nunits + 1) * 16) ||
-            !c->dec_small.ensure(kDecSmallBytes))
+            !c->sub_list.ensure(list_cap * 16) || !c->unit_off.ensure((nunits + 1) * 16))
             return fail(c, VECSZ_ENOMEM, "device scratch allocation failed");
         DecodeArgs da;
         da.stream = d_stream;
@@ -1101,7 +1105,6 @@ int decompress_device(vecsz_ctx* c, const vecsz_params* p, const uint8_t* d_in, 
         da.tabs = nullptr;
         da.meta = nullptr;
         da.n_sub16 = 0;
-        HIPCHK(c, hipMemsetAsync(c->dec_small.p, 0, kDecSmallBytes, c->stream));
         if (t16) {
             const uint32_t cap = std::min<uint32_t>(kMaxSubTabs, nodes / 2);
             if (!c->tabs.ensure(table_words(cap) * 2)) return fail(c, VECSZ_ENOMEM, "decode table allocation failed");
