@@ -1094,8 +1094,9 @@ int decompress_device(vecsz_ctx* c, const vecsz_params* p, const uint8_t* d_in, 
         SubState ss{};  // jbase 0: list entries are this field's subsequence numbers
         list_stripes(decode_sync_units(nsub), &ss);
         const uint64_t list_cap = ss.nstripe * ss.stripe_cap;
-        if (!c->sub_b.ensure(nsub) || !c->sub_e.ensure(nsub) || !c->sub_cz.ensure(nsub * 4) ||
-            !c->sub_list.ensure(list_cap * 16) || !c->unit_off.ensure((nunits + 1) * 16))
+        // (a decode from an index finds no subsequences)
+        if (!d_index && (!c->sub_b.ensure(nsub) || !c->sub_e.ensure(nsub) || !c->sub_cz.ensure(nsub * 4) ||
+                         !c->sub_list.ensure(list_cap * 16) || !c->unit_off.ensure((nunits + 1) * 16)))
             return fail(c, VECSZ_ENOMEM, "device scratch allocation failed");
         DecodeArgs da;
         da.stream = d_stream;
