@@ -12,8 +12,10 @@
 //     k_decode_pass   listed subsequences re-decode from their predecessor's
 //                     end; a moved end lists the successor for the next
 //                     pass, until no list is left
+//     k_decode_tail   the same, passes to the end of a short list in one
+//                     workgroup
 //     k_decode_sums,  codeword and zero counts per write unit, and their
-//     k_decode_scan   prefixes
+//     k_decode_scan   prefixes (k_decode_offsets: both for a few units)
 //     k_decode_write  final decode from the true starts: quant codes in
 //                     16-byte stores + outlier scatter
 //                     (src/vecsz_interface.hh:313-317)
