@@ -398,9 +398,24 @@ __device__ __forceinline__ bool decode_count(const D& dec, const W& win, uint32_
     }
 }
 
-// The same where the stream may end: behind its end (bit send, at most an
+// Single codewords (and the zeros among them) from lp until one starts at or
+// past end, by the symbols' first level in global memory: for a few bits.
+template <typename W>
+__device__ __forceinline__ void count_singles(const CountDecoder<true>& dec, const W& win, uint32_t& lp, uint32_t end,
+                                              const DecodeArgs& a, uint32_t& cnt, uint32_t& z) {
+    while (lp < end) {
+        const uint32_t w = win(lp);
+        uint32_t e = ((GlobalU16)a.tabs)[(1u << kLutBits) + (w >> (32 - kLutBits))], l = e >> 12;
+        if (l == 0) dec.deep.resolve(win, w, lp, e, l);
+        cnt++;
+        z += (e & 0xFFF) == 0;
+        lp += l;
+    }
+}
+
+// decode_count where the stream may end: behind its end (bit send, at most an
 // entry's bits past `end` or more) no codeword counts, so the last steps are
-// single codewords, read from the first level in global memory.
+// single codewords.
 template <class D, typename W>
 __device__ __forceinline__ bool decode_count_to(const D& dec, const W& win, uint32_t& lp, uint32_t end,
                                                 uint32_t send, const DecodeArgs& a, uint32_t& cnt, uint32_t& z) {
@@ -410,14 +425,7 @@ __device__ __forceinline__ bool decode_count_to(const D& dec, const W& win, uint
         // (a step that starts below lim ends at or before the stream's end)
         const uint32_t lim = min(end, send > D::kStep ? send - (D::kStep - 1) : 0u);
         const bool bad = decode_count(dec, win, lp, lim, cnt, z);
-        while (lp < end) {  // (never, where lim is end)
-            const uint32_t w = win(lp);
-            uint32_t e = ((GlobalU16)a.tabs)[(1u << kLutBits) + (w >> (32 - kLutBits))], l = e >> 12;
-            if (l == 0) dec.deep.resolve(win, w, lp, e, l);
-            cnt++;
-            z += (e & 0xFFF) == 0;
-            lp += l;
-        }
+        count_singles(dec, win, lp, end, a, cnt, z);  // (none, where lim is end)
         return bad;
     }
 }
@@ -546,11 +554,33 @@ __device__ __forceinline__ void decode_sync_unit(const DecodeArgs& a, const SubS
     bool wrong = false;
     uint32_t pred = s0;
     if (live && (t > 0 || j == 0)) {
+        if (t > 0) pred = own_e[t - 1];
+        wrong = t > 0 && pred != first;
+        if constexpr (T16) {
+            // The lead and the subsequence before each stopped behind a step,
+            // of several codewords maybe: up to 11 bits past s0 and, in
+            // general, not at the same codeword.  A start on the codewords of
+            // the other is right all the same, and only the ones in between
+            // change hands.  (Compared as they are, subsequences in a run of
+            // one short codeword, a constant stretch of a field, never settle:
+            // with 2^21 noise values and 2^21 of one 2-bit codeword every
+            // start of the run was listed in each of 8,190 passes, 92 ms a
+            // call where it is 0.15 now.)
+            const uint32_t to = max(pred, first);
+            if (wrong && to <= e0) {
+                uint32_t at = min(pred, first), n = 0, nz = 0;
+                count_singles(dec, PadWin{st}, at, to, a, n, nz);
+                if (at == to) {
+                    cnt += first > pred ? n : 0u - n;
+                    z += first > pred ? nz : 0u - nz;
+                    first = pred;
+                    wrong = false;
+                }
+            }
+        }
         s.b[j] = (uint8_t)(first - s0);
         s.e[j] = (uint8_t)(lp - e0);
         s.cz[j] = cnt | (z << 16);
-        if (t > 0) pred = own_e[t - 1];
-        wrong = t > 0 && pred != first;
         if (bad && !wrong) atomicOr(&sum->error, 1u);
     }
     list_append(s, 0, stripe, wrong, j, pred - s0);
@@ -612,12 +642,28 @@ __device__ __forceinline__ bool redecode_entry(const DecodeArgs& a, const SubSta
     const uint32_t tl = (uint32_t)min<uint64_t>(kSubBits, left) + sv.shift0;
     const uint32_t send = (uint32_t)min<uint64_t>(2 * kSubBits, left) + sv.shift0;
     uint32_t lp = first + sv.shift0, cnt = 0, z = 0;
-    if (decode_count_to(dec, win, lp, tl, send, a, cnt, z)) atomicOr(&sum->error, 1u);
-    over = lp - tl;
+    const uint32_t old = s.e[j];
     next = j + 1;
+    if constexpr (T16) {
+        // in two parts: up to where a step may reach past the target, and on
+        (void)decode_count(dec, win, lp, tl > dec.kStep ? tl - (dec.kStep - 1) : 0u, cnt, z);
+        uint32_t lp1 = lp, cnt1 = cnt, z1 = z;
+        (void)decode_count_to(dec, win, lp, tl, send, a, cnt, z);
+        const uint32_t to = tl + old;
+        if (lp != to && to <= send) {
+            // another end than j + 1 starts from, which does as well if these
+            // codewords meet it (as in decode_sync_unit): they are j's up to it
+            if (lp < to) lp1 = lp, cnt1 = cnt, z1 = z;
+            count_singles(dec, win, lp1, to, a, cnt1, z1);
+            if (lp1 == to) lp = lp1, cnt = cnt1, z = z1;
+        }
+    } else {
+        if (decode_count_to(dec, win, lp, tl, send, a, cnt, z)) atomicOr(&sum->error, 1u);
+    }
+    over = lp - tl;
     s.b[j] = (uint8_t)first;
     s.cz[j] = cnt | (z << 16);
-    if (over == s.e[j]) return false;
+    if (over == old) return false;
     s.e[j] = (uint8_t)over;
     return next < a.nsub;
 }
