@@ -218,7 +218,9 @@ constexpr uint32_t kLutSlow = 0x80000000u;
 // 1..kSubTabBits), 0 for a pointer to the next table.  The first level also
 // has a counting form, for passes that want no symbols: bits 12..15 the bits
 // of all whole codewords in the pattern (0: none, a pointer as above), 0..3
-// how many they are, 4..7 how many of them decode to symbol 0.
+// how many they are, 4..7 how many of them decode to symbol 0.  Beside it, the
+// ends of those codewords: bits 1..12 whether one ends behind that many bits
+// of the pattern, bit 0 whether one decodes to symbol 0.
 constexpr uint32_t kMaxSubTabs = 4096;      // deeper tables (their numbers have 12 bits)
 constexpr uint32_t kMaxTreeNodes = 8191;    // of 4096 symbols
 constexpr uint32_t kMaxSub16 = 12288;       // deeper-table entries kept in LDS

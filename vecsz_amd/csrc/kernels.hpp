@@ -112,12 +112,15 @@ struct TableMeta {
     uint32_t status, n_sub16;
     uint32_t pad_[2];
 };
-constexpr size_t table_words(uint32_t cap) { return (2u << kLutBits) + ((size_t)cap << kSubTabBits); }
+// First words of the tables in a field's: the counting first level, the first
+// level, the ends of each pattern's codewords, the deeper tables.
+constexpr uint32_t kTabLut = 1u << kLutBits, kTabEnds = 2u << kLutBits, kTabDeep = 3u << kLutBits;
+constexpr size_t table_words(uint32_t cap) { return kTabDeep + ((size_t)cap << kSubTabBits); }
 struct TableJob {
     const uint8_t* huff;  // Huffman section: [u32be nodes][u32be dict][tree]
     uint32_t nodes;       // as in it (0: nothing to build; at most kMaxTreeNodes)
     uint32_t cap;         // deeper tables tabs has room for (at most kMaxSubTabs)
-    uint16_t* tabs;       // counting first level, first level, deeper tables: table_words(cap)
+    uint16_t* tabs;       // table_words(cap)
     TableMeta* meta;
     uint32_t* hold;       // list counters whose hold a failure sets, or null
 };

@@ -198,7 +198,7 @@ struct Decoder<true> {
     __device__ __forceinline__ uint32_t attach(const uint32_t* lds, const DecodeArgs& a, uint32_t n_lds) {
         lut = reinterpret_cast<const uint16_t*>(lds);
         deep.sub_lds = (LdsU16)(lut + (1u << kLutBits));
-        deep.sub = (GlobalU16)a.tabs + (2u << kLutBits);
+        deep.sub = (GlobalU16)a.tabs + kTabDeep;
         deep.n_lds = n_lds;
         return ((1u << kLutBits) + a.n_sub16) / 2;
     }
@@ -263,7 +263,7 @@ struct CountDecoder<true> {
     __device__ __forceinline__ uint32_t attach(const uint32_t* lds, const DecodeArgs& a, uint32_t n_lds) {
         lut = reinterpret_cast<const uint16_t*>(lds);
         deep.sub_lds = (LdsU16)(lut + (1u << kLutBits));
-        deep.sub = (GlobalU16)a.tabs + (2u << kLutBits);
+        deep.sub = (GlobalU16)a.tabs + kTabDeep;
         deep.n_lds = n_lds;
         return ((1u << kLutBits) + a.n_sub16) / 2;
     }
@@ -304,8 +304,8 @@ struct TableCopy {
     __device__ __forceinline__ void fetch(const DecodeArgs& a) {
         n_sub = T16 ? min(a.n_sub16, ((GlobalU32)a.meta)[1]) : 0u;
         n = kFirst + n_sub / 8;
-        const GlobalU32x4 first = T16 ? (GlobalU32x4)(a.tabs + (COUNT ? 0u : 1u << kLutBits)) : (GlobalU32x4)a.lut;
-        const GlobalU32x4 deep = T16 ? (GlobalU32x4)(a.tabs + (2u << kLutBits)) : first;
+        const GlobalU32x4 first = T16 ? (GlobalU32x4)(a.tabs + (COUNT ? 0u : kTabLut)) : (GlobalU32x4)a.lut;
+        const GlobalU32x4 deep = T16 ? (GlobalU32x4)(a.tabs + kTabDeep) : first;
 #pragma unroll
         for (uint32_t m = 0; m < kVecs; m++) {
             const uint32_t i = threadIdx.x + m * NT;
@@ -349,7 +349,8 @@ __device__ __forceinline__ uint32_t decode_one(const D& dec, const W& win, uint3
 }
 
 // Codewords and zeros (outliers) of the steps that start in [lp, end), added
-// to cnt and z; lp ends at the first step's start at or past end.
+// to cnt and z; lp ends at the first step's start at or past end, `last` is
+// the start of the last round's first step.
 // (A step may hold codewords that start past end: they are this
 // subsequence's, and the next one starts behind them.)  Returns whether an
 // invalid codeword was met (it counts as one of one bit).
@@ -364,7 +365,7 @@ __device__ __forceinline__ uint32_t decode_one(const D& dec, const W& win, uint3
 // meets it.
 template <class D, typename W>
 __device__ __forceinline__ bool decode_count(const D& dec, const W& win, uint32_t& lp, uint32_t end, uint32_t& cnt,
-                                             uint32_t& z) {
+                                             uint32_t& z, uint32_t& last) {
     if constexpr (D::kInvalid) {
         bool bad = false;
         while (lp < end) {
@@ -380,8 +381,9 @@ __device__ __forceinline__ bool decode_count(const D& dec, const W& win, uint32_
     } else {
         const uint32_t lp0 = lp, z0 = z;
         uint32_t sum = 0;
+        last = lp;
         while (lp < end) {
-            const uint32_t w = win(lp);
+            const uint32_t w = win(last = lp);
             uint32_t e0 = dec.look(w), l0 = D::len(e0);
             uint32_t e1 = dec.look(w << l0);
             if (D::escape(e0)) {
@@ -398,19 +400,40 @@ __device__ __forceinline__ bool decode_count(const D& dec, const W& win, uint32_
     }
 }
 
-// Single codewords (and the zeros among them) from lp until one starts at or
-// past end, by the symbols' first level in global memory: for a few bits.
+// The codeword at lp, by the symbols' first level in global memory (a kernel
+// that counts keeps the other one in LDS), added to cnt and z.
 template <typename W>
-__device__ __forceinline__ void count_singles(const CountDecoder<true>& dec, const W& win, uint32_t& lp, uint32_t end,
-                                              const DecodeArgs& a, uint32_t& cnt, uint32_t& z) {
-    while (lp < end) {
-        const uint32_t w = win(lp);
-        uint32_t e = ((GlobalU16)a.tabs)[(1u << kLutBits) + (w >> (32 - kLutBits))], l = e >> 12;
-        if (l == 0) dec.deep.resolve(win, w, lp, e, l);
-        cnt++;
-        z += (e & 0xFFF) == 0;
-        lp += l;
+__device__ __forceinline__ void count_single(const CountDecoder<true>& dec, const W& win, uint32_t& lp,
+                                             const DecodeArgs& a, uint32_t& cnt, uint32_t& z) {
+    const uint32_t w = win(lp);
+    uint32_t e = ((GlobalU16)a.tabs)[kTabLut + (w >> (32 - kLutBits))], l = e >> 12;
+    if (l == 0) dec.deep.resolve(win, w, lp, e, l);
+    cnt++;
+    z += (e & 0xFFF) == 0;
+    lp += l;
+}
+
+// Whether the codewords from p on come to bit `to`, and those up to it, added
+// to cnt and z.  `to` is a few bits away: one look at the ends of a pattern's
+// codewords, mostly (a codeword at a time, each a load, took a re-decode pass
+// from 27 to 29 us and the 1 GiB field's sync pass from 302 to 308).
+template <typename W>
+__device__ __forceinline__ bool count_meet(const CountDecoder<true>& dec, const W& win, uint32_t p, uint32_t to,
+                                           const DecodeArgs& a, uint32_t& cnt, uint32_t& z) {
+    while (p < to) {
+        const uint32_t d = min(to - p, (uint32_t)kLutBits);
+        const uint32_t m = ((GlobalU16)a.tabs)[kTabEnds + (win(p) >> (32 - kLutBits))];
+        const uint32_t in = m & ((2u << d) - 2);  // ends in the next d bits
+        if (to - p <= kLutBits && !(in >> d)) return false;
+        if (in == 0 || (m & 1)) {
+            // a codeword of more than d bits, or a zero, which has to be found
+            count_single(dec, win, p, a, cnt, z);
+        } else {
+            cnt += __popc(in);
+            p += 31 - __clz(in);
+        }
     }
+    return p == to;
 }
 
 // decode_count where the stream may end: behind its end (bit send, at most an
@@ -418,14 +441,15 @@ __device__ __forceinline__ void count_singles(const CountDecoder<true>& dec, con
 // single codewords.
 template <class D, typename W>
 __device__ __forceinline__ bool decode_count_to(const D& dec, const W& win, uint32_t& lp, uint32_t end,
-                                                uint32_t send, const DecodeArgs& a, uint32_t& cnt, uint32_t& z) {
+                                                uint32_t send, const DecodeArgs& a, uint32_t& cnt, uint32_t& z,
+                                                uint32_t& last) {
     if constexpr (D::kStep == 0) {
-        return decode_count(dec, win, lp, end, cnt, z);
+        return decode_count(dec, win, lp, end, cnt, z, last);
     } else {
         // (a step that starts below lim ends at or before the stream's end)
         const uint32_t lim = min(end, send > D::kStep ? send - (D::kStep - 1) : 0u);
-        const bool bad = decode_count(dec, win, lp, lim, cnt, z);
-        count_singles(dec, win, lp, end, a, cnt, z);  // (none, where lim is end)
+        const bool bad = decode_count(dec, win, lp, lim, cnt, z, last);
+        while (lp < end) count_single(dec, win, lp, a, cnt, z);  // (never, where lim is end)
         return bad;
     }
 }
@@ -535,7 +559,7 @@ __device__ __forceinline__ void decode_sync_unit(const DecodeArgs& a, const SubS
     bool bad = false;
     // stage bits: the subsequence's first bit, its first codeword, its target
     const uint32_t s0 = (uint32_t)(j - Jst) * kSubBits + sv.shift0;
-    uint32_t first = s0, e0 = s0, cnt = 0, z = 0, lp = s0;
+    uint32_t first = s0, e0 = s0, cnt = 0, z = 0, lp = s0, last;
     if (live) {
         const PadWin win{st};
         const uint64_t left = a.stream_bits - j * kSubBits;
@@ -544,10 +568,10 @@ __device__ __forceinline__ void decode_sync_unit(const DecodeArgs& a, const SubS
         if (j) {
             lp = s0 - kLeadBits;
             uint32_t lc = 0, lz = 0;
-            (void)decode_count_to(dec, win, lp, s0, send, a, lc, lz);  // (an invalid path here is a wrong start's)
+            (void)decode_count_to(dec, win, lp, s0, send, a, lc, lz, last);  // (an invalid path here is a wrong start's)
             first = lp;
         }  // (the stream starts with a codeword)
-        bad = decode_count_to(dec, win, lp, e0, send, a, cnt, z);
+        bad = decode_count_to(dec, win, lp, e0, send, a, cnt, z, last);
         own_e[t] = lp;
     }
     lds_sync();
@@ -568,9 +592,8 @@ __device__ __forceinline__ void decode_sync_unit(const DecodeArgs& a, const SubS
             // call where it is 0.15 now.)
             const uint32_t to = max(pred, first);
             if (wrong && to <= e0) {
-                uint32_t at = min(pred, first), n = 0, nz = 0;
-                count_singles(dec, PadWin{st}, at, to, a, n, nz);
-                if (at == to) {
+                uint32_t n = 0, nz = 0;
+                if (count_meet(dec, PadWin{st}, min(pred, first), to, a, n, nz)) {
                     cnt += first > pred ? n : 0u - n;
                     z += first > pred ? nz : 0u - nz;
                     first = pred;
@@ -642,23 +665,26 @@ __device__ __forceinline__ bool redecode_entry(const DecodeArgs& a, const SubSta
     const uint32_t tl = (uint32_t)min<uint64_t>(kSubBits, left) + sv.shift0;
     const uint32_t send = (uint32_t)min<uint64_t>(2 * kSubBits, left) + sv.shift0;
     uint32_t lp = first + sv.shift0, cnt = 0, z = 0;
-    const uint32_t old = s.e[j];
+    const uint32_t old = s.e[j], to = tl + old;
     next = j + 1;
+    uint32_t last = lp;
+    if (decode_count_to(dec, win, lp, tl, send, a, cnt, z, last)) atomicOr(&sum->error, 1u);
     if constexpr (T16) {
-        // in two parts: up to where a step may reach past the target, and on
-        (void)decode_count(dec, win, lp, tl > dec.kStep ? tl - (dec.kStep - 1) : 0u, cnt, z);
-        uint32_t lp1 = lp, cnt1 = cnt, z1 = z;
-        (void)decode_count_to(dec, win, lp, tl, send, a, cnt, z);
-        const uint32_t to = tl + old;
+        // Another end than j + 1 starts from, which does as well if these
+        // codewords come to it (see decode_sync_unit): they are j's up to it.
         if (lp != to && to <= send) {
-            // another end than j + 1 starts from, which does as well if these
-            // codewords meet it (as in decode_sync_unit): they are j's up to it
-            if (lp < to) lp1 = lp, cnt1 = cnt, z1 = z;
-            count_singles(dec, win, lp1, to, a, cnt1, z1);
-            if (lp1 == to) lp = lp1, cnt = cnt1, z = z1;
+            uint32_t n = 0, nz = 0;
+            if (count_meet(dec, win, lp < to ? lp : last, to, a, n, nz)) {
+                if (lp < to) {
+                    cnt += n, z += nz;
+                } else {
+                    n = nz = 0;
+                    (void)count_meet(dec, win, to, lp, a, n, nz);
+                    cnt -= n, z -= nz;
+                }
+                lp = to;
+            }
         }
-    } else {
-        if (decode_count_to(dec, win, lp, tl, send, a, cnt, z)) atomicOr(&sum->error, 1u);
     }
     over = lp - tl;
     s.b[j] = (uint8_t)first;

@@ -107,15 +107,16 @@ __global__ void __launch_bounds__(kThreads) k_decode_tables(TableJob one, const 
     uint32_t tables = 0;
     if (!fail) {
         // first level: the first codeword of each 12-bit pattern (lut16), and
-        // all the codewords that lie in it whole (lut_count); a pattern that
-        // is no whole codeword gets a table
+        // all the codewords that lie in it whole (lut_count, ends); a pattern
+        // that is no whole codeword gets a table
         uint16_t* lut_count = job.tabs;
-        uint16_t* lut16 = job.tabs + (1u << kLutBits);
-        uint16_t* sub16 = lut16 + (1u << kLutBits);
+        uint16_t* lut16 = job.tabs + kTabLut;
+        uint16_t* ends = job.tabs + kTabEnds;
+        uint16_t* sub16 = job.tabs + kTabDeep;
 #pragma unroll
         for (uint32_t q = 0; q < (1u << kLutBits) / kThreads; q++) {
             const uint32_t idx = t + q * kThreads;
-            uint32_t node = 0, first = 0, end = 0, n = 0, z = 0;
+            uint32_t node = 0, first = 0, end = 0, n = 0, z = 0, at_end = 0;
 #pragma unroll
             for (uint32_t b = 0; b < (uint32_t)kLutBits; b++) {
                 const uint32_t cw = child[node];
@@ -125,6 +126,7 @@ __global__ void __launch_bounds__(kThreads) k_decode_tables(TableJob one, const 
                 n += at;
                 z += at && (k & 0xFFF) == 0;
                 end = at ? b + 1 : end;
+                at_end |= (uint32_t)at << (b + 1);
                 node = at ? 0 : k;
             }
             uint32_t e16 = first, ec = (end << 12) | (z << 4) | n;
@@ -135,6 +137,7 @@ __global__ void __launch_bounds__(kThreads) k_decode_tables(TableJob one, const 
             }
             lut16[idx] = (uint16_t)e16;
             lut_count[idx] = (uint16_t)ec;
+            ends[idx] = (uint16_t)(at_end | (z != 0));
         }
         lds_sync();
         uint32_t nf = nnext;
