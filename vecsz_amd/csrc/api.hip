@@ -1224,7 +1224,11 @@ int decompress_device(vecsz_ctx* c, const vecsz_params* p, const uint8_t* d_in, 
         }
     }
 
-    if (!fused_1d && !recon_issued) reconstruct(nullptr);
+    // (an indexed decode whose tables could not be built has left no codes:
+    // the hold keeps the reconstruction from an earlier call's)
+    if (!fused_1d && !recon_issued)
+        reconstruct(indexed ? reinterpret_cast<const uint32_t*>(c->dec_small.as<uint8_t>() + kDecSmallLists) + list_slot(0)
+                            : nullptr);
     HIPCHK(c, hipGetLastError());
     if (indexed) HIPCHK(c, hipMemcpyAsync(h, c->dec_small.p, kDecSmallLists, hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
