@@ -93,3 +93,13 @@ def test_masked_field(gpu_ctx):
     x = datagen.grf((32, 160, 192), seed=5)
     x = np.where(x < np.quantile(x, 0.9), 0, x).astype(np.float32)
     _check(gpu_ctx, x, 1e-3, True, 1, 5)
+
+
+# streams of 21,721 and 77,592 subsequences whose first pass leaves a list
+# that one workgroup takes (964 and 106 entries): one host check
+@pytest.mark.parametrize("data", ["walk", "grf"])
+def test_short_list_of_a_long_stream(gpu_ctx, data):
+    from vecsz_amd import datagen
+
+    x = datagen.walk_spikes_1d(1 << 22) if data == "walk" else datagen.grf((64, 256, 256), seed=3)
+    _check(gpu_ctx, x.astype(np.float32), 1e-4, True, 1, 5)

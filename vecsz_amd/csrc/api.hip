@@ -419,12 +419,12 @@ static_assert(sizeof(DecSummary) <= kDecSmallTables && kDecSmallTables + sizeof(
                   kDecSmallFlagged + 4 <= kDecSmallLists,
               "the slots hold their structs");
 
-// Whether the list pass `pass` reads holds entries (counters: the host's copy).
-bool any_listed(const uint8_t* counters, uint32_t pass) {
+// Entries of the list pass `pass` reads (counters: the host's copy).
+uint64_t listed_entries(const uint8_t* counters, uint32_t pass) {
     const uint32_t* n = reinterpret_cast<const uint32_t*>(counters) + list_slot(pass);
-    for (uint32_t i = 0; i < kMaxStripes; i++)
-        if (n[i * kCounterWords]) return true;
-    return false;
+    uint64_t sum = 0;
+    for (uint32_t i = 0; i < kMaxStripes; i++) sum += n[i * kCounterWords];
+    return sum;
 }
 
 // ---- allocation-free compress (vecsz_compress_noalloc)
@@ -1151,28 +1151,26 @@ int decompress_device(vecsz_ctx* c, const vecsz_params* p, const uint8_t* d_in, 
             StageScope s(c, "decode_sync");
             launch_decode_sync(da, ss, dsum, c->stream);
         }
-        // Re-decode passes, a few without a host check, then the scan and the
-        // write pass, which do nothing unless the list the next pass would
-        // read is empty: in the common case the decode needs one host check,
-        // after the write.  (The longest chain of wrong starts grows with
-        // their number: the 1 GiB field needs three or four passes, a 26 MB
-        // one two; a pass over empty lists takes about 4 us, a host check
-        // with its repeated launches about 35.)  Otherwise passes run in
-        // growing batches while the lists ask for more (each pass resolves at
-        // least the first subsequence of every chain, so nsub passes suffice),
-        // each batch with launch_decode_tail for what a short list still
-        // holds, the scan and the write again, and a host check.
-        // A short stream's second pass is launch_decode_tail: what the first
-        // leaves there is a list it takes (an empty one costs the same 4 us),
-        // so chains need no further host check (a 2^18-value walk: 263 ->
-        // 222 us).
-        const bool short_stream = nsub < (1u << 14);
-        const uint32_t ahead = short_stream ? 1 : nsub < (1u << 17) ? 2 : nsub < (1u << 21) ? 3 : 4;
+        // Re-decode passes without a host check and launch_decode_tail for the
+        // short list they leave, then the scan and the write pass, which do
+        // nothing unless the list is empty: in the common case the decode
+        // needs one host check, after the write.  Otherwise more of the same,
+        // by the list's length, until nothing is left (each pass resolves at
+        // least the first subsequence of every chain, so nsub passes suffice).
+        // A list's length depends on the codewords: of a turbulence field's
+        // subsequences 9% are listed at first and 0.2% after a pass, of a
+        // walk's 13% and then six tenths of the last list each pass.  The
+        // passes ahead are what brings the former under the tail's kTailList
+        // (a pass or a tail with nothing to do is about 4 us, a host check
+        // with its repeated launches about 55); a walk goes on from what the
+        // check has counted (2^26 values: 3 checks after 3, 7 and 15 passes,
+        // by guess -> 2).
+        const uint32_t ahead = nsub < (1u << 19) ? 1 : nsub < (1u << 21) ? 2 : 3;
         uint32_t pass = 0;
         {
             StageScope s(c, "decode_redo");
             for (; pass < ahead; pass++) launch_decode_pass(da, ss, pass, dsum, c->stream);
-            if (short_stream) launch_decode_tail(da, ss, pass, dsum, c->stream);
+            launch_decode_tail(da, ss, pass, dsum, c->stream);
         }
         auto scan_write = [&](const uint32_t* guard) {
             {
@@ -1191,7 +1189,7 @@ int decompress_device(vecsz_ctx* c, const vecsz_params* p, const uint8_t* d_in, 
         DecSummary ds;
         uint64_t tot;
         TableMeta tm;
-        bool left = false;
+        uint64_t left = 0;
         auto check = [&]() -> int {  // summary, the pending list count and the symbol total
             HIPCHK(c, hipMemcpyAsync(h, c->dec_small.p, kDecSmallBytes, hipMemcpyDeviceToHost, c->stream));
             HIPCHK(c, hipMemcpyAsync(h + kDecSmallBytes, off + 2 * nunits, 8, hipMemcpyDeviceToHost, c->stream));
@@ -1199,26 +1197,29 @@ int decompress_device(vecsz_ctx* c, const vecsz_params* p, const uint8_t* d_in, 
             memcpy(&ds, h, sizeof(ds));
             memcpy(&tot, h + kDecSmallBytes, 8);
             memcpy(&tm, h + kDecSmallTables, sizeof(tm));
-            left = any_listed(h + kDecSmallLists, pass);
+            left = listed_entries(h + kDecSmallLists, pass);
             return ds.error ? fail(c, VECSZ_ECORRUPT, "bitstream does not decode") : VECSZ_OK;
         };
         if (int rc2 = check()) return rc2;
         if (tm.status)  // (nothing has run behind the tables)
             return decompress_device(c, p, d_in, in_bytes, d_out, out_cap, nullptr, 0, true);
-        if (left) {
-            for (uint32_t batch = 4; left; batch = std::min<uint32_t>(2 * batch, 16)) {
-                if (pass > nsub + 2) return fail(c, VECSZ_ECORRUPT, "subsequence boundaries do not converge");
-                // (a pass over an empty list does nothing but clear the list after next)
-                {
-                    StageScope s(c, "decode_redo");
-                    for (uint32_t b = 0; b < batch; b++) launch_decode_pass(da, ss, pass++, dsum, c->stream);
-                    launch_decode_tail(da, ss, pass, dsum, c->stream);
-                }
-                scan_write(ss.list_n + list_slot(pass));
-                if (!fused_1d) reconstruct(ss.list_n + list_slot(pass));
-                HIPCHK(c, hipGetLastError());
-                if (int rc2 = check()) return rc2;
+        for (uint32_t least = 1; left; least = std::min<uint32_t>(std::max<uint32_t>(2 * least, 4), 16)) {
+            if (pass > nsub + 2) return fail(c, VECSZ_ECORRUPT, "subsequence boundaries do not converge");
+            // as many passes as bring a list that loses a third of its entries
+            // each under the tail's (a walk's loses four tenths), more where
+            // that was not enough
+            uint32_t batch = 0;
+            for (uint64_t m = left; m > kTailList && batch < 16; m -= m / 3) batch++;
+            batch = std::max(batch, least);
+            {
+                StageScope s(c, "decode_redo");
+                for (uint32_t b = 0; b < batch; b++) launch_decode_pass(da, ss, pass++, dsum, c->stream);
+                launch_decode_tail(da, ss, pass, dsum, c->stream);
             }
+            scan_write(ss.list_n + list_slot(pass));
+            if (!fused_1d) reconstruct(ss.list_n + list_slot(pass));
+            HIPCHK(c, hipGetLastError());
+            if (int rc2 = check()) return rc2;
         }
         if (tot < n) return fail(c, VECSZ_ECORRUPT, "bitstream holds fewer symbols than the field");
         }

@@ -185,7 +185,8 @@ uint64_t sync_unit_subs();
 void launch_decode_sync(const DecodeArgs& a, SubState s, DecSummary* sum, hipStream_t st);
 // Re-decode pass `pass` over the list the previous pass (or the sync pass) built.
 void launch_decode_pass(const DecodeArgs& a, SubState s, uint32_t pass, DecSummary* sum, hipStream_t st);
-// Resolves pass `pass`'s list in place if it is short (one workgroup).
+// Resolves pass `pass`'s list in place if it holds at most kTailList entries (one workgroup).
+constexpr uint32_t kTailList = 1024;
 void launch_decode_tail(const DecodeArgs& a, SubState s, uint32_t pass, DecSummary* sum, hipStream_t st);
 // Codewords and zeros before each write unit (decode_write_units(nsub) units
 // of consecutive subsequences): off[2 u], off[2 u + 1], the totals behind the

@@ -739,7 +739,7 @@ __global__ void __launch_bounds__(256) k_decode_pass(DecodeArgs a, SubState s, u
 // Rounds are passes as k_decode_pass makes them, with the lists in LDS and a
 // barrier between them that also orders the subsequences' state.  Bounded:
 // what is left after kTailRounds goes back to the list.
-constexpr uint32_t kTailWg = 1024;
+constexpr uint32_t kTailWg = kTailList;  // an entry per thread
 constexpr uint32_t kTailRounds = 512;
 template <bool T16>
 __global__ void __launch_bounds__(kTailWg) k_decode_tail(DecodeArgs a, SubState s, uint32_t pass, DecSummary* sum) {
