@@ -947,21 +947,31 @@ int decompress_device(vecsz_ctx* c, const vecsz_params* p, const uint8_t* d_in, 
     if (rc) return rc;
     HIPCHK(c, hipSetDevice(c->device));
     timing_begin(c);
-    // One round trip for the metadata and the Huffman header; where the host
-    // builds the tables, a second copy brings the tree.
-    constexpr uint64_t kHeadRead = 256;
-    if (!c->pin.ensure(std::max<uint64_t>(kHeadRead + 64, kDecSmallBytes + 64)))
-        return fail(c, VECSZ_ENOMEM, "pinned buffer");
+    // One round trip for the metadata and the Huffman header, behind up to
+    // 32,000 pad values, and, where the host builds the tables, a tree of up to
+    // 14,000 nodes; what lies further takes another.  (A copy of 128 KiB to
+    // pinned memory takes 13 us, one of 256 bytes 16, a round trip more 16.
+    // With the index's header behind it only a small copy is as cheap, 22 us
+    // for both against 23 and, in a call, 7 more: 4,000 pad values then, unless
+    // the tree is for the host.)
+    constexpr uint64_t kHeadMost = 1 << 17;
+    const uint64_t head_read = d_index && p->dict_size <= kMaxLdsBook ? 1 << 14 : kHeadMost;
+    static_assert(kHeadMost >= kDecSmallBytes + 8, "the checks' copies fit too");
+    if (!c->pin.ensure(kHeadMost + 64)) return fail(c, VECSZ_ENOMEM, "pinned buffer");
     uint8_t* h = c->pin.as<uint8_t>();
-    const uint64_t head_avail = std::min<uint64_t>(in_bytes, kHeadRead);
+    const uint64_t head_avail = std::min<uint64_t>(in_bytes, head_read);
     HIPCHK(c, hipMemcpyAsync(h, d_in, head_avail, hipMemcpyDeviceToHost, c->stream));
     uint64_t ih[kIdxHead] = {0, 0, 0, 0, 0, 0};
     if (d_index) {
         if (index_words < kIdxHead) return fail(c, VECSZ_EINVAL, "decode index too short");
-        HIPCHK(c, hipMemcpyAsync(h + kHeadRead, d_index, 8 * kIdxHead, hipMemcpyDeviceToHost, c->stream));
+        HIPCHK(c, hipMemcpyAsync(h + head_read, d_index, 8 * kIdxHead, hipMemcpyDeviceToHost, c->stream));
     }
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    if (d_index) memcpy(ih, h + kHeadRead, sizeof(ih));
+    auto wait_header = [c]() {
+        HostTimer ht(c, "header");
+        return hipStreamSynchronize(c->stream);
+    };
+    HIPCHK(c, wait_header());
+    if (d_index) memcpy(ih, h + head_read, sizeof(ih));
     int ndim;
     uint64_t dims[3], pad_len, huff_size, nout;
     double ebu;
@@ -990,7 +1000,7 @@ int decompress_device(vecsz_ctx* c, const vecsz_params* p, const uint8_t* d_in, 
             if (!c->pin2.ensure(64)) return fail(c, VECSZ_ENOMEM, "pinned buffer");
             hp = c->pin2.as<uint8_t>();
             HIPCHK(c, hipMemcpyAsync(c->pin2.p, d_huff, 8, hipMemcpyDeviceToHost, c->stream));
-            HIPCHK(c, hipStreamSynchronize(c->stream));
+            HIPCHK(c, wait_header());
         }
         int32_t ncs = (int32_t)(((uint32_t)hp[0] << 24) | ((uint32_t)hp[1] << 16) | ((uint32_t)hp[2] << 8) | hp[3]);
         if (ncs <= 0) return fail(c, VECSZ_ECORRUPT, "Huffman node count");
@@ -1000,10 +1010,13 @@ int decompress_device(vecsz_ctx* c, const vecsz_params* p, const uint8_t* d_in, 
         t16 = !host_tables && device_tables_ok(nodes, p->dict_size);
         if (!t16) {
             HostTimer ht(c, "host_tables");
-            if (!c->pin2.ensure(8 + tb)) return fail(c, VECSZ_ENOMEM, "pinned buffer");
-            HIPCHK(c, hipMemcpyAsync(c->pin2.p, d_huff, 8 + tb, hipMemcpyDeviceToHost, c->stream));
-            HIPCHK(c, hipStreamSynchronize(c->stream));
-            rc = build_decode_tables(c->pin2.as<uint8_t>(), huff_size, dt);
+            if (hoff + 8 + tb > head_avail) {
+                if (!c->pin2.ensure(8 + tb)) return fail(c, VECSZ_ENOMEM, "pinned buffer");
+                hp = c->pin2.as<uint8_t>();
+                HIPCHK(c, hipMemcpyAsync(c->pin2.p, d_huff, 8 + tb, hipMemcpyDeviceToHost, c->stream));
+                HIPCHK(c, wait_header());
+            }
+            rc = build_decode_tables(hp, huff_size, dt);
             if (rc) return fail(c, rc, "Huffman tree is corrupt");
             if (!dt.root_leaf && !tree_is_full(dt)) return fail(c, VECSZ_ECORRUPT, "Huffman tree is not full");
         }
