@@ -1201,8 +1201,9 @@ __global__ void __launch_bounds__(1024) k_scan_tiles(const uint32_t* __restrict_
 // Bounded by instruction issue and the stage's LDS traffic, not by memory (1.9
 // bytes read and 0.5 written a symbol): 264 us at 1 GiB and 64 at 67M values
 // with every codeword ORed in alone, every chunk's last word completed from
-// the next one's codes and the next chunk's loads waited for at once; 230 and
-// 50 with four codewords to an OR group, runs, and the loads in flight.
+// the next one's codes and the next chunk's loads waited for at once; 212 and
+// 51 with four codewords to an OR group, runs, and the loads in flight; 201
+// and 50 with four of the stage's words read at a time on the way out.
 struct Code {
     uint32_t lo, hi, len;  // codeword = hi:lo, right-aligned, len bits
 };
@@ -1558,9 +1559,10 @@ __device__ __forceinline__ void pack_chunk(const ChunkRaw& cur, uint64_t k, uint
     if (open && !last) carry = stage[nwords - 1];
     else carry = 0;
     // bytes at or past the stream end are not the stream's; bytes at or
-    // past cap are outside the buffer (a stream byte there: too small)
+    // past cap are outside the buffer (a stream byte there: too small); a
+    // chunk whose words all lie before both goes out four of them at a time
     const uint64_t lim = end_byte < T.cap ? end_byte : T.cap;
-    if (lim == ~0ull && (k != 0 || a0 == 0)) {
+    if ((wbase + nwords) * 4 <= lim && (k != 0 || a0 == 0)) {
         uint32_t* o = out32 + wbase;
         for (uint32_t i = lane; i < nwords; i += 4 * kWave) {
             uint32_t wv[4];
@@ -2435,8 +2437,8 @@ void launch_scan_u32x2(const uint32_t* a, const uint32_t* b, uint64_t n, uint64_
 }
 
 // k_pack: four workgroups a CU, all resident at once (six fit; 2048 queued
-// ones: 244 us at 1 GiB, 16.2 at 1800 x 3600, against 240 and 14.0), and runs
-// of at most eight chunks (1: 319 us at 1 GiB, 8: 240, 16: 245, 32: 252, where
+// ones: 198 us at 1 GiB, 14.4 at 1800 x 3600, against 200 and 13.1), and runs
+// of at most eight chunks (1: 214 us at 1 GiB, 8: 200, 16: 203, 32: 207, where
 // a wavefront's distance from its neighbours is a large power of two).
 constexpr int kPackGrid = 1024;
 constexpr uint32_t kPackRun = 8;
