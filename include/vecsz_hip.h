@@ -228,7 +228,8 @@ int vecsz_autotune(vecsz_ctx* ctx, const vecsz_params* params, const float* d_in
                    vecsz_tune* out);
 /* Sets the launch shapes vecsz_autotune chooses (e.g. from a stored result):
  * workgroup caps of the dual quantization and of the encode kernels, each in
- * [1, 65536] (defaults 768 and 2048). */
+ * [1, 65536] (defaults 768 and 2048; a single field's pack takes half of the
+ * latter where that is 1024 or more). */
 int vecsz_ctx_set_launch_shape(vecsz_ctx* ctx, int dq_grid, int enc_grid);
 
 /* Served form: a request server on one GPU (no counterpart in the

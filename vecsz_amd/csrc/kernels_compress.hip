@@ -2439,7 +2439,9 @@ void launch_scan_u32x2(const uint32_t* a, const uint32_t* b, uint64_t n, uint64_
 // k_pack: four workgroups a CU, all resident at once (six fit; 2048 queued
 // ones: 198 us at 1 GiB, 14.4 at 1800 x 3600, against 200 and 13.1), and runs
 // of at most eight chunks (1: 214 us at 1 GiB, 8: 200, 16: 203, 32: 207, where
-// a wavefront's distance from its neighbours is a large power of two).
+// a wavefront's distance from its neighbours is a large power of two).  The
+// default launch shape's 2048 is for the chunk bits; above kPackGrid the packer
+// takes half of a shape's workgroups, so that a tuned one reaches it as well.
 constexpr int kPackGrid = 1024;
 constexpr uint32_t kPackRun = 8;
 
@@ -2448,7 +2450,8 @@ void launch_pack(const uint16_t* codes, uint64_t n, const uint32_t* cw_hi, const
                  const float* sparse, uint8_t* archive, const uint32_t* err, int max_len, int grid_cap,
                  uint64_t* index, hipStream_t st) {
     const IdxLayout L = idx_layout(index ? n : 0);
-    const unsigned grid = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>((nchunks + 3) / 4, std::min(grid_cap, kPackGrid)));
+    const int cap = grid_cap <= kPackGrid ? grid_cap : std::max(kPackGrid, grid_cap / 2);
+    const unsigned grid = (unsigned)std::max<uint64_t>(1, std::min<uint64_t>((nchunks + 3) / 4, cap));
     uint32_t run = 1;  // as long as each wavefront still gets a run
     while (run < kPackRun && nchunks >= 8ull * grid * run) run *= 2;
     const uint32_t stage_words = stage_words_of(max_len);
