@@ -750,14 +750,13 @@ __global__ void __launch_bounds__(kTailWg) k_decode_tail(DecodeArgs a, SubState 
     const uint32_t k = lane_id2() < s.nstripe ? min(*list_counter(s, pass, lane_id2()), 2 * kTailWg) : 0u;
     const uint32_t ends = wave_scan_dpp(k);
     uint32_t m = lane63(ends);
-    if (m > kTailWg) return;  // (the whole workgroup)
+    if (m == 0 || m > kTailWg) return;  // (the whole workgroup)
     uint64_t at = 0;
     for (uint32_t q = 0; q < s.nstripe; q++) {
         const uint32_t q1 = (uint32_t)__builtin_amdgcn_readlane((int)ends, (int)q);
         const uint32_t q0 = q1 - (uint32_t)__builtin_amdgcn_readlane((int)k, (int)q);
         if (t >= q0 && t < q1) at = q * s.stripe_cap + (t - q0);
     }
-    if (m == 0) return;
     uint64_t* list = s.list[pass & 1];
     CountDecoder<T16> dec;
     uint32_t* p = lds;
