@@ -948,14 +948,13 @@ int decompress_device(vecsz_ctx* c, const vecsz_params* p, const uint8_t* d_in, 
     HIPCHK(c, hipSetDevice(c->device));
     timing_begin(c);
     // One round trip for the metadata and the Huffman header, behind up to
-    // 32,000 pad values, and, where the host builds the tables, a tree of up to
-    // 14,000 nodes; what lies further takes another.  (A copy of 128 KiB to
-    // pinned memory takes 13 us, one of 256 bytes 16, a round trip more 16.
-    // With the index's header behind it only a small copy is as cheap, 22 us
-    // for both against 23 and, in a call, 7 more: 4,000 pad values then, unless
-    // the tree is for the host.)
+    // 8,000 pad values, or, where the host builds the tables, with a tree of
+    // up to 14,000 nodes; what lies further takes another, about 16 us.  (A
+    // first read of 256 bytes to 32 KiB costs a call the same, 64 KiB 1 us
+    // more, 128 KiB 2.5.  With the index's header behind it, 16 KiB is the
+    // most that costs nothing and 32 KiB to 128 KiB are 7 us.)
     constexpr uint64_t kHeadMost = 1 << 17;
-    const uint64_t head_read = d_index && p->dict_size <= kMaxLdsBook ? 1 << 14 : kHeadMost;
+    const uint64_t head_read = p->dict_size > kMaxLdsBook ? kHeadMost : d_index ? 1 << 14 : 1 << 15;
     static_assert(kHeadMost >= kDecSmallBytes + 8, "the checks' copies fit too");
     if (!c->pin.ensure(kHeadMost + 64)) return fail(c, VECSZ_ENOMEM, "pinned buffer");
     uint8_t* h = c->pin.as<uint8_t>();
