@@ -430,7 +430,7 @@ class Context:
         vrs = list(value_ranges) if isinstance(value_ranges, (list, tuple)) else [value_ranges] * nf
         params, outs = [], []
         # every archive's header in one copy (a copy each was 0.8 ms for 48)
-        heads = [a[:64] for a in archives]
+        heads = [a[:64].view(torch.uint8) for a in archives]  # (cat would widen bytes of mixed types)
         raw = torch.cat(heads).cpu().numpy().tobytes() if heads else b""
         at = 0
         for a, h, m, vr in zip(archives, heads, modes, vrs):
