@@ -156,7 +156,7 @@ struct vecsz_ctx {
     DevBuf vparts;
     HostBuf vpin;
     // decompress scratch
-    // dec_small: decoder summary, symbol and zero totals, list counts (kDecSmall*)
+    // dec_small: decoder summary, state of the tables, list counts (kDecSmall*)
     DevBuf tabs, sub_b, sub_e, sub_cz, sub_list, sub_ln, unit_off, scan_tmp, scan_tot, dec_small, flagged;
     // host staging
     DevBuf stage_in, stage_out;
@@ -1980,7 +1980,7 @@ static int compress_batch_fused(vecsz_ctx* c, int nf, const vecsz_params* p, con
 // archive's metadata and Huffman header to the host, and then each stage is
 // one launch over all fields: the decode tables (a workgroup per tree), the
 // sync pass, the re-decode passes, the offsets, the write pass, and the
-// reconstruction (one launch per tile form) with its fp32 fallback.  A field
+// reconstruction (one launch, or one per tile form) with its fp32 fallback.  A field
 // whose tables the device could not build takes the per-field path behind
 // the batch.  Outputs are the single-field path's.
 static bool dbatch_fusable(const vecsz_ctx* c, int nf, const vecsz_params* p, const uint8_t* const* d_in,

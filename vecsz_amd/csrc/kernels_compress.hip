@@ -2130,11 +2130,10 @@ __global__ void __launch_bounds__(256) k_hist_reduce_multi(const uint32_t* __res
     if (s) atomicAdd(&hist[(uint64_t)f * dict + b], (unsigned long long)s);
 }
 
-// Copies each field's staged header (metadata, Huffman header, tree) to the
-// front of its archive; one workgroup per field.
-// Each archive's header, tree included (up to 73 KB), 16 bytes a load and a
-// store at any alignment, eight in flight per thread: byte by byte the largest
-// tree of a batch took 40 us.  blockIdx.x: the field.
+// Copies each field's staged header (metadata, Huffman header, tree: up to 73
+// KB) to the front of its archive, a workgroup per field: 16 bytes a load and a
+// store at any alignment, eight in flight per thread (byte by byte the largest
+// tree of a batch took 40 us).
 __global__ void __launch_bounds__(256) k_place_heads(const BatchField* __restrict__ fd, int nf,
                                                      const uint32_t* __restrict__ errs) {
     const int f = blockIdx.x;

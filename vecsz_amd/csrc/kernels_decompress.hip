@@ -733,9 +733,10 @@ __global__ void __launch_bounds__(256) k_decode_pass(DecodeArgs a, SubState s, u
 // The end of a redo that a few chains of wrong starts make long: one
 // workgroup resolves pass `pass`'s list in place, all passes' worth, when it
 // holds at most kTailWg entries (else it does nothing).  A pass over such a
-// list is latency: about 4 us of launch and tables around 5 of work, and a
-// host check with its launches every so many passes (67M values whose phase a
-// start picks by chance, 33 passes long: decompress 710 -> 606 us).
+// list is latency: about 4 us of launch and tables around 5 to 13 of work, and
+// a host check with its launches every so many passes (a walk of 2^26 values,
+// 24 passes: decompress 933 us with passes alone, 770 with the last 16 of them
+// in here).
 // Rounds are passes as k_decode_pass makes them, with the lists in LDS and a
 // barrier between them that also orders the subsequences' state.  Bounded:
 // what is left after kTailRounds goes back to the list.
