@@ -146,7 +146,7 @@ struct SubState {
     // end): how far past bit j * kSubBits its first codeword starts, and how
     // far past its target the one after its last (both below 64, a codeword's
     // length, plus 12, a table entry's); codewords starting in between | those
-    // of them that decode to symbol 0 << 16 (at most kSubBits + 11 each).
+    // of them that decode to symbol 0 << 16 (at most kSubBits + 75 each).
     uint8_t* b;
     uint8_t* e;
     uint32_t* cz;

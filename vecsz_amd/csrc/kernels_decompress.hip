@@ -7,11 +7,11 @@
 //                     decoding from kLeadBits before it (two decodes of one
 //                     stream soon agree, wherever they started), then
 //                     decodes the subsequence: start, end and counts.  A
-//                     start other than the end its predecessor found lists
-//                     the subsequence
+//                     start that is not on the codewords of its predecessor
+//                     lists the subsequence
 //     k_decode_pass   listed subsequences re-decode from their predecessor's
-//                     end; a moved end lists the successor for the next
-//                     pass, until no list is left
+//                     end; codewords that do not come to the successor's
+//                     start list it for the next pass, until no list is left
 //     k_decode_tail   the same, passes to the end of a short list in one
 //                     workgroup
 //     k_decode_sums,  codeword and zero counts per write unit, and their
