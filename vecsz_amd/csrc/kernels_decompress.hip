@@ -527,6 +527,7 @@ static_assert(kLeadBits <= kSubBits, "the lead lies in one row");
 // 72 + 64 bits on (the deepest table walk of an invalid path, words read ahead).
 constexpr uint32_t kSyncStageWords = (kSyncWg + 1) * kSubWords + 12;
 constexpr uint32_t kSyncStageLds = kSyncStageWords + kSyncStageWords / kSubWords + 1;
+constexpr int kManyWrong = 16;  // of a wavefront's starts (see decode_sync_unit)
 constexpr uint32_t kSyncLdsWords = 1 + kSyncStageLds + kSyncWg;  // dynamic LDS after the tables
 
 // Workgroup `unit` of the sync pass: subsequences unit * kSyncStride on.
@@ -589,9 +590,13 @@ __device__ __forceinline__ void decode_sync_unit(const DecodeArgs& a, const SubS
             // one short codeword, a constant stretch of a field, never settle:
             // with 2^21 noise values and 2^21 of one 2-bit codeword every
             // start of the run was listed in each of 8,190 passes, 92 ms a
-            // call where it is 0.15 now.)
+            // call where it is 0.15 now.)  Only where it is so for many of a
+            // wavefront, as in a run: the five or six of other fields, mostly
+            // on other codewords indeed, can as well be listed, and looking at
+            // them in every wavefront took the 1 GiB field's sync pass from
+            // 304 to 308 us.
             const uint32_t to = max(pred, first);
-            if (wrong && to <= e0) {
+            if (__popcll(__ballot(wrong)) >= kManyWrong && wrong && to <= e0) {
                 uint32_t n = 0, nz = 0;
                 if (count_meet(dec, PadWin{st}, min(pred, first), to, a, n, nz)) {
                     cnt += first > pred ? n : 0u - n;
