@@ -590,7 +590,7 @@ __device__ __forceinline__ void decode_sync_unit(const DecodeArgs& a, const SubS
             // one short codeword, a constant stretch of a field, never settle:
             // with 2^21 noise values and 2^21 of one 2-bit codeword every
             // start of the run was listed in each of 8,190 passes, 92 ms a
-            // call where it is 0.15 now.)  Only where it is so for many of a
+            // call where it is 0.16 now.)  Only where it is so for many of a
             // wavefront, as in a run: the five or six of other fields, mostly
             // on other codewords indeed, can as well be listed, and looking at
             // them in every wavefront took the 1 GiB field's sync pass from
