@@ -416,7 +416,7 @@ __device__ __forceinline__ void count_single(const CountDecoder<true>& dec, cons
 // Whether the codewords from p on come to bit `to`, and those up to it, added
 // to cnt and z.  `to` is a few bits away: one look at the ends of a pattern's
 // codewords, mostly (a codeword at a time, each a load, took a re-decode pass
-// from 27 to 29 us and the 1 GiB field's sync pass from 302 to 308).
+// from 27 to 29 us).
 template <typename W>
 __device__ __forceinline__ bool count_meet(const CountDecoder<true>& dec, const W& win, uint32_t p, uint32_t to,
                                            const DecodeArgs& a, uint32_t& cnt, uint32_t& z) {
